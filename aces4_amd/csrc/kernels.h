@@ -191,15 +191,22 @@ hipError_t launch_slice(const SliceArgs &a, bool insert, double *tens, double *s
                         hipStream_t st);
 
 // ---------------------------------------------------------------- triples --
-// The (T) energy with W kept on chip (triples.hip).  Indices are cut into
-// 5-blocks within their segments; a box is one 5-block per W index.
+// The (T) energy with W kept on chip (triples.hip).  The virtual and the
+// occupied index range are each cut into 5-blocks (block s starts at global
+// index 5 s, across segment boundaries, so only the last is shorter: cut
+// inside each segment instead, segments of 17, 18, 17, 14 | 13, 14 had
+// 729,000 partly empty boxes, not 592,704, 296 ms a sum against 40 with the
+// images of a box shared); a box is one 5-block per W index.
 constexpr int kTriplesBox = 5;
 constexpr int kTriplesSums = 4096; // partial sums of the final reduction
-struct TriplesBlk {
-    int seg;    // segment
-    int off;    // offset of the 5-block inside the segment
-    int ext;    // extent, 1..5
-    int gstart; // global orbital index of its first element
+// A class of super-boxes (two 5-blocks per index) that differ by a
+// permutation of the pairs (a,i), (b,j), (c,k): p holds the pairs' super
+// coordinates (virtual + occupied * virtual count), ascending; the class's
+// 6, 3 or 1 distinct arrangements are the super-boxes first, first + 1, ...
+struct TriplesOrbit {
+    int p[3];
+    int pad;
+    long long first;
 };
 // Packs PA (side 0: sets (x, y1, y2) over vblk x oblk x oblk) or PB (side 1:
 // sets (x2, x3, y3) over vblk x vblk x oblk) from the blocks of T(a,d,i,j),
@@ -210,7 +217,6 @@ struct TriplesPackArgs {
     long long total; // doubles of the panel array
     int side, nkp, kd, kl;
     int n1, n2;      // 5-block counts of the second and third set index
-    const TriplesBlk *blk0, *blk1, *blk2;
     int nv, no;      // segment counts
     const int *vext, *oext;             // segment extents
     const int *vseg_of, *oseg_of;       // segment of each global index
@@ -220,17 +226,22 @@ struct TriplesPackArgs {
 struct TriplesArgs {
     const double *PA, *PB;
     int nkp, nvb, nob;
-    const TriplesBlk *vblk, *oblk;
+    int kd, kl;     // virtual and occupied index totals
     const double *e_vir, *e_occ;
     double *partial;
-    // global mode: linear box ids [box0, box0 + nbox) of the super-box order
-    long long box0, nbox, per_xcd;
-    int super[6], nblk[6];
-    // tuple mode: the boxes first[d] .. first[d] + count[d] - 1
+    // global mode: one box per (class, position in its super-box) for the
+    // classes orbits[0 .. norbits), each result stored for the box's images
+    // among slots [box0, box0 + nbox)
+    const TriplesOrbit *orbits;
+    long long norbits, per_xcd;
+    long long box0, nbox;
+    int super_v;
+    // tuple mode: the boxes first[d] .. first[d] + count[d] - 1, limited to
+    // the tuple's global index ranges [lo[d], lo[d] + wdims[d])
     int tuple_mode;
     int first[6], count[6];
     double *wout;   // tuple mode, optional: W of the tuple (column-major)
-    int wdims[6];
+    int lo[6], wdims[6];
 };
 hipError_t launch_triples_pack(const TriplesPackArgs &a, hipStream_t s);
 // grid workgroups of 512; hipErrorInvalidConfiguration at 2^23 workgroups or more

@@ -1,9 +1,9 @@
 // triples.cpp -- host side of the on-chip-W (T) energy (triples.hip).
 //
-// A plan holds the 5-block tables of the virtual and occupied index
-// ranges, the two packed operand panel arrays (PA over row sets
-// (x, y1, y2), PB over column sets (x2, x3, y3)), and one energy partial
-// per box slot.  sipgpu_triples_pack fills the panels from the T, V1 and V2
+// A plan holds the classes of super-boxes that differ by a permutation of
+// the pairs (a,i), (b,j), (c,k), the two packed operand panel arrays (PA over
+// row sets (x, y1, y2), PB over column sets (x2, x3, y3)), and one energy
+// partial per box slot.  sipgpu_triples_pack fills the panels from the T, V1 and V2
 // blocks; sipgpu_triples_run computes the partials of a range of box
 // slots (one workgroup per box); sipgpu_triples_energy sums all partials in
 // slot order into the energy (deterministic).
@@ -12,24 +12,27 @@
 #include <algorithm>
 #include <cstring>
 #include <memory>
+#include <new>
+#include <numeric>
 #include <vector>
 
 #include "../../include/sipgpu.h"
 #include "internal.h"
 #include "kernels.h"
 
-using sipgpu::TriplesBlk;
+using sipgpu::TriplesOrbit;
 using sipgpu::rt::fail;
 using sipgpu::rt::hip_fail;
 
 struct sipgpu_triples_s {
     int nv = 0, no = 0;
     std::vector<int> vseg, oseg;
-    std::vector<TriplesBlk> vblk, oblk;
+    std::vector<TriplesOrbit> orbits; // ascending in `first`
+    int nvb = 0, nob = 0;             // 5-blocks of the virtual / occupied range
     int kd = 0, kl = 0, nkp = 0;
     // device memory
-    void *tables = nullptr; // TriplesBlk vblk | oblk, ints, pointer tables
-    const TriplesBlk *d_vblk = nullptr, *d_oblk = nullptr;
+    void *tables = nullptr; // orbits, ints, pointer tables
+    const TriplesOrbit *d_orbits = nullptr;
     const int *d_vext = nullptr, *d_oext = nullptr, *d_vseg_of = nullptr, *d_oseg_of = nullptr;
     const int *d_vseg_start = nullptr, *d_oseg_start = nullptr;
     const double *const *d_T = nullptr, *const *d_V1 = nullptr, *const *d_V2 = nullptr;
@@ -38,31 +41,42 @@ struct sipgpu_triples_s {
     long long pa_doubles = 0, pb_doubles = 0;
     double *partial = nullptr, *sums = nullptr, *tuple_partial = nullptr;
     long long slots = 0;   // box slots of the super-box order
-    int super[6] = {}, nblk[6] = {};
-    int max_tuple_boxes = 0;
+    int super_v = 0;       // super-boxes along a virtual index
     bool packed = false;
 };
 
 namespace {
 
-void cut_blocks(const std::vector<int> &seg, std::vector<TriplesBlk> &out) {
-    int g = 0;
-    for (int s = 0; s < (int)seg.size(); ++s) {
-        for (int off = 0; off < seg[s]; off += sipgpu::kTriplesBox)
-            out.push_back(TriplesBlk{s, off, std::min(sipgpu::kTriplesBox, seg[s] - off), g + off});
-        g += seg[s];
-    }
+// Classes of super-boxes over n super pairs and, per class, its first
+// super-box: the 6, 3 or 1 distinct arrangements of a class are consecutive.
+std::vector<TriplesOrbit> super_box_classes(int n) {
+    std::vector<TriplesOrbit> out;
+    long long first = 0;
+    for (int p = 0; p < n; ++p)
+        for (int q = p; q < n; ++q)
+            for (int r = q; r < n; ++r) {
+                out.push_back(TriplesOrbit{{p, q, r}, 0, first});
+                first += p == q && q == r ? 1 : p == q || q == r ? 3 : 6;
+            }
+    return out;
 }
 
-// first 5-block of each segment, and the count
-void seg_blocks(const std::vector<TriplesBlk> &blk, int s, int &first, int &count) {
-    first = -1;
-    count = 0;
-    for (int i = 0; i < (int)blk.size(); ++i)
-        if (blk[i].seg == s) {
-            if (first < 0) first = i;
-            ++count;
-        }
+// the 5-blocks that a segment at global index g touches
+void seg_blocks(int g, int ext, int &first, int &count) {
+    first = g / sipgpu::kTriplesBox;
+    count = (g + ext - 1) / sipgpu::kTriplesBox - first + 1;
+}
+
+// most 5-blocks that one segment touches
+int max_seg_blocks(const std::vector<int> &seg) {
+    int most = 0, g = 0;
+    for (int x : seg) {
+        int first, count;
+        seg_blocks(g, x, first, count);
+        most = std::max(most, count);
+        g += x;
+    }
+    return most;
 }
 
 } // namespace
@@ -86,29 +100,54 @@ int sipgpu_triples_create(int nv, const int *v_seg, int no, const int *o_seg,
         if (x < 1) return fail(SIPGPU_EARG, "triples: segment extents must be positive");
     for (int x : P->oseg)
         if (x < 1) return fail(SIPGPU_EARG, "triples: segment extents must be positive");
-    cut_blocks(P->vseg, P->vblk);
-    cut_blocks(P->oseg, P->oblk);
     for (int x : P->vseg) P->kd += x;
     for (int x : P->oseg) P->kl += x;
     // K padded to whole pairs of k-pairs (the kernel loads two per trip)
     P->nkp = ((P->kd + P->kl + 15) / 16) * 2;
-    const long long nvb = (long long)P->vblk.size(), nob = (long long)P->oblk.size();
+    P->nvb = (P->kd + sipgpu::kTriplesBox - 1) / sipgpu::kTriplesBox;
+    P->nob = (P->kl + sipgpu::kTriplesBox - 1) / sipgpu::kTriplesBox;
+    const long long nvb = P->nvb, nob = P->nob;
     const long long per_set = 8LL * P->nkp * 128;
     P->pa_doubles = nvb * nob * nob * per_set;
     P->pb_doubles = nvb * nvb * nob * per_set;
-    const int nblk[6] = {(int)nvb, (int)nvb, (int)nvb, (int)nob, (int)nob, (int)nob};
-    P->slots = 64;
-    for (int d = 0; d < 6; ++d) {
-        P->nblk[d] = nblk[d];
-        P->super[d] = (nblk[d] + 1) / 2;
-        P->slots *= P->super[d];
-    }
-    int vmax = 0, omax = 0;
-    for (int s = 0; s < nv; ++s) vmax = std::max(vmax, (P->vseg[s] + 4) / 5);
-    for (int s = 0; s < no; ++s) omax = std::max(omax, (P->oseg[s] + 4) / 5);
-    P->max_tuple_boxes = vmax * vmax * vmax * omax * omax * omax;
+    P->super_v = (P->nvb + 1) / 2;
+    const long long pairs = (long long)P->super_v * ((P->nob + 1) / 2);
+    P->slots = 64 * pairs * pairs * pairs;
+    const long long vmax = max_seg_blocks(P->vseg), omax = max_seg_blocks(P->oseg);
+    const long long max_tuple_boxes = vmax * vmax * vmax * omax * omax * omax;
 
-    // tables: blocks, then int arrays, then pointer tables (8-byte aligned)
+    const size_t nT = (size_t)nv * nv * no * no, nV1 = (size_t)nv * nv * nv * no,
+                 nV2 = (size_t)no * nv * no * no;
+    for (size_t i = 0; i < nT; ++i)
+        if (!T[i]) return fail(SIPGPU_EARG, "triples: null T block");
+    for (size_t i = 0; i < nV1; ++i)
+        if (!V1[i]) return fail(SIPGPU_EARG, "triples: null V1 block");
+    for (size_t i = 0; i < nV2; ++i)
+        if (!V2[i]) return fail(SIPGPU_EARG, "triples: null V2 block");
+
+    auto no_memory = [&]() {
+        for (void *p : {(void *)P->tables, (void *)P->PA, (void *)P->PB, (void *)P->partial,
+                        (void *)P->sums, (void *)P->tuple_partial})
+            if (p) (void)hipFree(p);
+        (void)hipGetLastError();
+        return fail(SIPGPU_ENOMEM, "triples: device memory for the packed operands");
+    };
+    hipError_t e = hipMalloc(&P->PA, (size_t)P->pa_doubles * sizeof(double));
+    if (e == hipSuccess) e = hipMalloc(&P->PB, (size_t)P->pb_doubles * sizeof(double));
+    if (e == hipSuccess) e = hipMalloc(&P->partial, (size_t)P->slots * sizeof(double));
+    if (e == hipSuccess) e = hipMalloc(&P->sums, (size_t)sipgpu::kTriplesSums * sizeof(double));
+    if (e == hipSuccess)
+        e = hipMalloc(&P->tuple_partial, (size_t)max_tuple_boxes * sizeof(double));
+    if (e != hipSuccess) return no_memory();
+    // built once the device holds a partial per slot: the host's classes are
+    // then at most a hundredth of that
+    try {
+        P->orbits = super_box_classes((int)pairs);
+    } catch (const std::bad_alloc &) {
+        return no_memory();
+    }
+
+    // tables: super-box classes, then int arrays, then pointer tables (16-byte aligned)
     std::vector<int> vseg_of(P->kd), oseg_of(P->kl), vstart(nv), ostart(no);
     for (int s = 0, g = 0; s < nv; g += P->vseg[s], ++s) {
         vstart[s] = g;
@@ -118,8 +157,6 @@ int sipgpu_triples_create(int nv, const int *v_seg, int no, const int *o_seg,
         ostart[s] = g;
         for (int q = 0; q < P->oseg[s]; ++q) oseg_of[g + q] = s;
     }
-    const size_t nT = (size_t)nv * nv * no * no, nV1 = (size_t)nv * nv * nv * no,
-                 nV2 = (size_t)no * nv * no * no;
     std::vector<unsigned char> img;
     auto put = [&](const void *p, size_t bytes) {
         const size_t at = (img.size() + 15) & ~(size_t)15;
@@ -127,8 +164,7 @@ int sipgpu_triples_create(int nv, const int *v_seg, int no, const int *o_seg,
         std::memcpy(img.data() + at, p, bytes);
         return at;
     };
-    const size_t o_vblk = put(P->vblk.data(), P->vblk.size() * sizeof(TriplesBlk));
-    const size_t o_oblk = put(P->oblk.data(), P->oblk.size() * sizeof(TriplesBlk));
+    const size_t o_orbits = put(P->orbits.data(), P->orbits.size() * sizeof(TriplesOrbit));
     const size_t o_vext = put(P->vseg.data(), nv * sizeof(int));
     const size_t o_oext = put(P->oseg.data(), no * sizeof(int));
     const size_t o_vso = put(vseg_of.data(), vseg_of.size() * sizeof(int));
@@ -138,38 +174,12 @@ int sipgpu_triples_create(int nv, const int *v_seg, int no, const int *o_seg,
     const size_t o_T = put(T, nT * sizeof(double *));
     const size_t o_V1 = put(V1, nV1 * sizeof(double *));
     const size_t o_V2 = put(V2, nV2 * sizeof(double *));
-    for (size_t i = 0; i < nT; ++i)
-        if (!T[i]) return fail(SIPGPU_EARG, "triples: null T block");
-    for (size_t i = 0; i < nV1; ++i)
-        if (!V1[i]) return fail(SIPGPU_EARG, "triples: null V1 block");
-    for (size_t i = 0; i < nV2; ++i)
-        if (!V2[i]) return fail(SIPGPU_EARG, "triples: null V2 block");
-
-    auto cleanup = [&]() {
-        if (P->tables) (void)hipFree(P->tables);
-        if (P->PA) (void)hipFree(P->PA);
-        if (P->PB) (void)hipFree(P->PB);
-        if (P->partial) (void)hipFree(P->partial);
-        if (P->sums) (void)hipFree(P->sums);
-        if (P->tuple_partial) (void)hipFree(P->tuple_partial);
-    };
-    hipError_t e = hipMalloc(&P->tables, img.size());
+    e = hipMalloc(&P->tables, img.size());
     if (e == hipSuccess)
         e = hipMemcpy(P->tables, img.data(), img.size(), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMalloc(&P->PA, (size_t)P->pa_doubles * sizeof(double));
-    if (e == hipSuccess) e = hipMalloc(&P->PB, (size_t)P->pb_doubles * sizeof(double));
-    if (e == hipSuccess) e = hipMalloc(&P->partial, (size_t)P->slots * sizeof(double));
-    if (e == hipSuccess) e = hipMalloc(&P->sums, (size_t)sipgpu::kTriplesSums * sizeof(double));
-    if (e == hipSuccess)
-        e = hipMalloc(&P->tuple_partial, (size_t)P->max_tuple_boxes * sizeof(double));
-    if (e != hipSuccess) {
-        cleanup();
-        (void)hipGetLastError();
-        return fail(SIPGPU_ENOMEM, "triples: device memory for the packed operands");
-    }
+    if (e != hipSuccess) return no_memory();
     const unsigned char *base = static_cast<const unsigned char *>(P->tables);
-    P->d_vblk = reinterpret_cast<const TriplesBlk *>(base + o_vblk);
-    P->d_oblk = reinterpret_cast<const TriplesBlk *>(base + o_oblk);
+    P->d_orbits = reinterpret_cast<const TriplesOrbit *>(base + o_orbits);
     P->d_vext = reinterpret_cast<const int *>(base + o_vext);
     P->d_oext = reinterpret_cast<const int *>(base + o_oext);
     P->d_vseg_of = reinterpret_cast<const int *>(base + o_vso);
@@ -217,11 +227,8 @@ int sipgpu_triples_pack(sipgpu_triples_t P, sipgpu_stream_t s) {
         a.nkp = P->nkp;
         a.kd = P->kd;
         a.kl = P->kl;
-        a.n1 = side == 0 ? (int)P->oblk.size() : (int)P->vblk.size();
-        a.n2 = (int)P->oblk.size();
-        a.blk0 = P->d_vblk;
-        a.blk1 = side == 0 ? P->d_oblk : P->d_vblk;
-        a.blk2 = P->d_oblk;
+        a.n1 = side == 0 ? P->nob : P->nvb;
+        a.n2 = P->nob;
         a.nv = P->nv;
         a.no = P->no;
         a.vext = P->d_vext;
@@ -248,16 +255,13 @@ sipgpu::TriplesArgs box_args(const sipgpu_triples_s &P) {
     a.PA = P.PA;
     a.PB = P.PB;
     a.nkp = P.nkp;
-    a.nvb = (int)P.vblk.size();
-    a.nob = (int)P.oblk.size();
-    a.vblk = P.d_vblk;
-    a.oblk = P.d_oblk;
+    a.nvb = P.nvb;
+    a.nob = P.nob;
+    a.kd = P.kd;
+    a.kl = P.kl;
+    a.super_v = P.super_v;
     a.e_vir = P.e_vir;
     a.e_occ = P.e_occ;
-    for (int d = 0; d < 6; ++d) {
-        a.super[d] = P.super[d];
-        a.nblk[d] = P.nblk[d];
-    }
     return a;
 }
 
@@ -272,13 +276,22 @@ int sipgpu_triples_run(sipgpu_triples_t P, long long box0, long long nbox, sipgp
     sipgpu::TriplesArgs a = box_args(*P);
     a.partial = P->partial;
     const hipStream_t hs = sipgpu::rt::stream_of(s);
+    // class that holds a slot's super-box
+    auto class_of = [&](long long slot) {
+        return std::upper_bound(P->orbits.begin(), P->orbits.end(), slot / 64,
+                                [](long long s, const TriplesOrbit &o) { return s < o.first; }) -
+               P->orbits.begin() - 1;
+    };
     // one launch per SIPGPU_TRIPLES_LAUNCH_BOXES slots: a dispatch holds
-    // fewer than 2^32 work-items (8.4M boxes of 512), and a launch stays
-    // near a second of the whole sum's ~20 s on one GPU
+    // fewer than 2^32 work-items (8.4M workgroups of 512).  A class that a
+    // cut divides is computed by both launches.
     for (long long b = box0; b < box0 + nbox; b += SIPGPU_TRIPLES_LAUNCH_BOXES) {
         a.box0 = b;
         a.nbox = std::min<long long>(SIPGPU_TRIPLES_LAUNCH_BOXES, box0 + nbox - b);
-        a.per_xcd = (a.nbox + 7) / 8;
+        const long long c0 = class_of(b), c1 = class_of(b + a.nbox - 1);
+        a.orbits = P->d_orbits + c0;
+        a.norbits = c1 - c0 + 1;
+        a.per_xcd = a.norbits * 8;
         SIPGPU_HIP_TRY(sipgpu::launch_triples_boxes(a, 8 * a.per_xcd, hs));
     }
     return 0;
@@ -301,11 +314,12 @@ int sipgpu_triples_tuple(sipgpu_triples_t P, const int *tuple, double factor, do
     a.wout = w_out;
     long long grid = 1;
     for (int d = 0; d < 6; ++d) {
-        const bool virt = d < 3;
-        const int nseg = virt ? P->nv : P->no;
-        if (tuple[d] < 0 || tuple[d] >= nseg) return fail(SIPGPU_EARG, "triples: tuple outside the segments");
-        seg_blocks(virt ? P->vblk : P->oblk, tuple[d], a.first[d], a.count[d]);
-        a.wdims[d] = (virt ? P->vseg : P->oseg)[tuple[d]];
+        const std::vector<int> &seg = d < 3 ? P->vseg : P->oseg;
+        if (tuple[d] < 0 || tuple[d] >= (int)seg.size())
+            return fail(SIPGPU_EARG, "triples: tuple outside the segments");
+        a.lo[d] = std::accumulate(seg.begin(), seg.begin() + tuple[d], 0);
+        a.wdims[d] = seg[tuple[d]];
+        seg_blocks(a.lo[d], a.wdims[d], a.first[d], a.count[d]);
         grid *= a.count[d];
     }
     const hipStream_t hs = sipgpu::rt::stream_of(s);

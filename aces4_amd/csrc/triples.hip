@@ -71,12 +71,15 @@ __global__ __launch_bounds__(256) void triples_pack_kernel(TriplesPackArgs a) {
             const int s2 = (int)(set % a.n2);
             const int s1 = (int)((set / a.n2) % a.n1);
             const int s0 = (int)(set / ((long long)a.n2 * a.n1));
-            const TriplesBlk b0 = a.blk0[s0], b1 = a.blk1[s1], b2 = a.blk2[s2];
-            if (r0 < b0.ext && r1 < b1.ext && r2d < b2.ext) {
-                // global indices (segment, offset within segment) of the row
-                const int g0s = b0.seg, g0o = b0.off + r0;
-                const int g1s = b1.seg, g1o = b1.off + r1;
-                const int g2s = b2.seg, g2o = b2.off + r2d;
+            // global indices of the row; the first is virtual, the last
+            // occupied, the middle one occupied in PA and virtual in PB
+            const int g0 = s0 * kBoxE + r0, g1 = s1 * kBoxE + r1, g2 = s2 * kBoxE + r2d;
+            if (g0 < a.kd && g1 < (a.side == 0 ? a.kl : a.kd) && g2 < a.kl) {
+                // segment and offset within it
+                const int g0s = a.vseg_of[g0], g0o = g0 - a.vseg_start[g0s];
+                const int g1s = a.side == 0 ? a.oseg_of[g1] : a.vseg_of[g1];
+                const int g1o = g1 - (a.side == 0 ? a.oseg_start[g1s] : a.vseg_start[g1s]);
+                const int g2s = a.oseg_of[g2], g2o = g2 - a.oseg_start[g2s];
                 if (a.side == 0) {
                     // PA row (x, y1, y2)
                     if (k < a.kd) { // T(x, d, y1, y2)
@@ -114,41 +117,81 @@ __global__ __launch_bounds__(256) void triples_pack_kernel(TriplesPackArgs a) {
 
 // ---------------------------------------------------------------- boxes --
 
-// Box coordinates (5-block indices of a, b, c, i, j, k) of this workgroup;
-// false for a workgroup without a box.  Global mode: linear ids in
-// 2x2x2x2x2x2 super-boxes (consecutive ids are neighbours in all six
-// indices), workgroup w on XCD w % 8 taking ids in order within its XCD's
-// share, so the boxes running together on one XCD share operand sets in its
-// L2.  Tuple mode: the boxes of one tuple, first index fastest.
-// Returns 0 (no slot: past the launch's range), 1 (a slot whose box lies in
-// the padding of the super-box grid: its partial is zero) or 2 (a box).
-__device__ __forceinline__ int box_of(const TriplesArgs &a, int (&bc)[6], long long &slot) {
+// W is unchanged when the pairs (a,i), (b,j), (c,k) are permuted together
+// with their indices (its six terms only change places), and so is D: the up
+// to six boxes that differ by such a permutation have one energy.  The kernel
+// computes it once, on the box whose pairs are in ascending order, and stores
+// it for every image: a whole sum runs a sixth of its boxes (o = 30, v = 60,
+// segments of 20 and 10: 373,248 slots, 64,824 boxes; 133 -> 25.8 ms).  A slot's
+// value does not depend on which range of slots a call covers.
+//
+// Global mode: workgroup (class, q) owns position q (one bit per index) of a
+// class's ascending super-box.  Slots number the 64 boxes of every super-box,
+// the arrangements of a class next to each other, so that any range of slots
+// holds most images of the boxes it computes.  Workgroup w runs on XCD w % 8
+// and takes ids in order within that XCD's share: the boxes running together
+// on one XCD are neighbours in all six indices and share operand sets in its
+// L2.
+struct BoxId {
+    TriplesOrbit orbit;
+    int sub[3]; // bit 0: which virtual 5-block of the super-box, bit 1: occupied
+};
+
+// Slot of the arrangement g of the box's pairs (position t holds pair kPerm[g][t]).
+__device__ __forceinline__ long long image_slot(const BoxId &b, int g) {
+    const int t0 = kPerm[g][0], t1 = kPerm[g][1], t2 = kPerm[g][2];
+    const bool eq01 = b.orbit.p[0] == b.orbit.p[1], eq12 = b.orbit.p[1] == b.orbit.p[2];
+    // distinct arrangements of the class: by g, by the place of the pair that
+    // differs from the other two, or just one
+    int rank = g;
+    if (eq01 && eq12)
+        rank = 0;
+    else if (eq01)
+        rank = t0 == 2 ? 0 : t1 == 2 ? 1 : 2;
+    else if (eq12)
+        rank = t0 == 0 ? 0 : t1 == 0 ? 1 : 2;
+    const int s0 = b.sub[t0], s1 = b.sub[t1], s2 = b.sub[t2];
+    const int q = (s0 & 1) | (s1 & 1) << 1 | (s2 & 1) << 2 | (s0 >> 1) << 3 | (s1 >> 1) << 4 |
+                  (s2 >> 1) << 5;
+    return (b.orbit.first + rank) * 64 + q;
+}
+
+// Box coordinates (5-block indices of a, b, c, i, j, k) of this workgroup.
+// Returns false where there is nothing to compute: no work id, a position
+// whose ascending form is another one, no image among the call's slots, or a
+// box past the index ranges (padding of the super-boxes; its partial stays
+// the zero that packing stores).  Tuple mode: the boxes of one tuple, first
+// index fastest.
+__device__ __forceinline__ bool box_of(const TriplesArgs &a, int (&bc)[6], BoxId &id) {
     if (a.tuple_mode) {
         long long q = blockIdx.x;
-        slot = q;
 #pragma unroll
         for (int d = 0; d < 6; ++d) {
             bc[d] = a.first[d] + (int)(q % a.count[d]);
             q /= a.count[d];
         }
-        return 2;
+        return true;
     }
     const long long w = blockIdx.x;
     const long long local = (w & 7) * a.per_xcd + (w >> 3);
-    if (local >= a.nbox) return 0;
-    const long long L = a.box0 + local;
-    slot = L;
-    const int q = (int)(L & 63);
-    long long r = L >> 6;
-    bool ok = true;
+    if (local >= a.norbits * 64) return false;
+    id.orbit = a.orbits[local >> 6];
+    const int q = (int)(local & 63);
 #pragma unroll
-    for (int d = 0; d < 6; ++d) {
-        const int sd = (int)(r % a.super[d]);
-        r /= a.super[d];
-        bc[d] = 2 * sd + ((q >> d) & 1);
-        ok = ok && bc[d] < a.nblk[d];
+    for (int m = 0; m < 3; ++m) {
+        id.sub[m] = ((q >> m) & 1) | ((q >> (3 + m)) & 1) << 1;
+        bc[m] = 2 * (id.orbit.p[m] % a.super_v) + (id.sub[m] & 1);
+        bc[3 + m] = 2 * (id.orbit.p[m] / a.super_v) + (id.sub[m] >> 1);
+        if (bc[m] >= a.nvb || bc[3 + m] >= a.nob) return false;
     }
-    return ok ? 2 : 1;
+    if (id.orbit.p[0] == id.orbit.p[1] && id.sub[0] > id.sub[1]) return false;
+    if (id.orbit.p[1] == id.orbit.p[2] && id.sub[1] > id.sub[2]) return false;
+    bool any = false;
+    for (int g = 0; g < 6; ++g) {
+        const long long slot = image_slot(id, g) - a.box0;
+        any = any || (slot >= 0 && slot < a.nbox);
+    }
+    return any;
 }
 
 // One workgroup: one 5^6 box of W, all six GEMMs, the energy partial.
@@ -157,7 +200,7 @@ __device__ __forceinline__ int box_of(const TriplesArgs &a, int (&bc)[6], long l
 __global__ __launch_bounds__(kThreads) void triples_box_kernel(TriplesArgs a) {
     __shared__ double W[kBoxElems];
     __shared__ double eps[6][kBoxE];
-    __shared__ int ext[6];
+    __shared__ int lo[6], hi[6]; // the box's elements that count, per index
     __shared__ double red[kThreads / 64];
     __shared__ double occ[kBoxRows];
     // box offsets of product row / column x (< 128) under permutation g
@@ -166,21 +209,20 @@ __global__ __launch_bounds__(kThreads) void triples_box_kernel(TriplesArgs a) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave & 1, wn = wave >> 1;
     int bc[6];
-    long long slot = 0;
-    const int kind = box_of(a, bc, slot);
-    if (kind < 2) {
-        if (kind == 1 && tid == 0) a.partial[slot] = 0.0;
-        return;
-    }
-    if (tid < 6) {
-        const TriplesBlk b = tid < 3 ? a.vblk[bc[tid]] : a.oblk[bc[tid]];
-        ext[tid] = b.ext;
-    }
+    BoxId id;
+    if (!box_of(a, bc, id)) return;
     if (tid < 30) {
         const int d = tid / kBoxE, q = tid % kBoxE;
-        const TriplesBlk b = d < 3 ? a.vblk[bc[d]] : a.oblk[bc[d]];
+        const int g = bc[d] * kBoxE + q, total = d < 3 ? a.kd : a.kl;
         const double *e = d < 3 ? a.e_vir : a.e_occ;
-        eps[d][q] = q < b.ext ? e[b.gstart + q] : 0.0;
+        eps[d][q] = g < total ? e[g] : 0.0;
+    }
+    if (tid < 6) {
+        const int g0 = bc[tid] * kBoxE, total = tid < 3 ? a.kd : a.kl;
+        const int first = a.tuple_mode ? a.lo[tid] : 0;
+        const int end = a.tuple_mode ? a.lo[tid] + a.wdims[tid] : total;
+        lo[tid] = max(0, first - g0);
+        hi[tid] = min(kBoxE, end - g0);
     }
 
     for (int t = tid; t < 6 * 128; t += kThreads) {
@@ -311,13 +353,15 @@ __global__ __launch_bounds__(kThreads) void triples_box_kernel(TriplesArgs a) {
     if (!a.wout) {
         if (tid < kBoxRows) {
             const int i = tid % kBoxE, j = (tid / kBoxE) % kBoxE, k = tid / (kBoxE * kBoxE);
-            const bool in = i < ext[3] && j < ext[4] && k < ext[5];
+            const bool in = i >= lo[3] && i < hi[3] && j >= lo[4] && j < hi[4] && k >= lo[5] &&
+                            k < hi[5];
             occ[tid] = in ? eps[3][i] + eps[4][j] + eps[5][k] : __builtin_nan("");
         }
         __syncthreads(); // the box and the occupied sums are complete
         const int abc = tid & 127;
         const int ea_i = abc % kBoxE, eb_i = (abc / kBoxE) % kBoxE, ec_i = abc / (kBoxE * kBoxE);
-        if (abc < kBoxRows && ea_i < ext[0] && eb_i < ext[1] && ec_i < ext[2]) {
+        if (abc < kBoxRows && ea_i >= lo[0] && ea_i < hi[0] && eb_i >= lo[1] && eb_i < hi[1] &&
+            ec_i >= lo[2] && ec_i < hi[2]) {
             const double ea = eps[0][ea_i], eb = eps[1][eb_i], ec = eps[2][ec_i];
             for (int ijk = tid >> 7; ijk < kBoxRows; ijk += kThreads / 128) {
                 const double o = occ[ijk];
@@ -338,7 +382,7 @@ __global__ __launch_bounds__(kThreads) void triples_box_kernel(TriplesArgs a) {
         for (int d = 0; d < 6; ++d) {
             dg[d] = q % kBoxE;
             q /= kBoxE;
-            in = in && dg[d] < ext[d];
+            in = in && dg[d] >= lo[d] && dg[d] < hi[d];
         }
         if (!in) continue;
         const double w = W[e];
@@ -350,7 +394,7 @@ __global__ __launch_bounds__(kThreads) void triples_box_kernel(TriplesArgs a) {
             long long o = 0;
 #pragma unroll
             for (int d = 5; d >= 0; --d)
-                o = o * a.wdims[d] + ((bc[d] - a.first[d]) * kBoxE + dg[d]);
+                o = o * a.wdims[d] + (bc[d] * kBoxE + dg[d] - a.lo[d]);
             a.wout[o] = w;
         }
     }
@@ -362,7 +406,15 @@ __global__ __launch_bounds__(kThreads) void triples_box_kernel(TriplesArgs a) {
     if (tid == 0) {
         double t = red[0];
         for (int w = 1; w < kThreads / 64; ++w) t += red[w];
-        a.partial[slot] = t;
+        if (a.tuple_mode) {
+            a.partial[blockIdx.x] = t;
+        } else {
+            // images that coincide store the same value twice
+            for (int g = 0; g < 6; ++g) {
+                const long long slot = image_slot(id, g);
+                if (slot >= a.box0 && slot < a.box0 + a.nbox) a.partial[slot] = t;
+            }
+        }
     }
 }
 

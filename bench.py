@@ -645,14 +645,21 @@ def triples_fused_bench(steps, warmup):
     # sipgpu_triples_run makes one kernel launch per tp.LAUNCH_BOXES slots:
     # the roofline divides a step by its launches (one at 12 steps or more)
     kernels = -(-chunk // tp.LAUNCH_BOXES)
-    per_launch = flops * chunk / ft.slots / kernels
+    # The six boxes of W that differ by a permutation of the pairs (a,i), (b,j),
+    # (c,k) have one energy and are computed once: `value` counts the sum's
+    # flop, the roofline the flop of the boxes that are computed.
+    pairs = (v // 5) * (o // 5)
+    boxes = pairs * (pairs + 1) * (pairs + 2) // 6
+    flop_per_box = flops / pairs ** 3
+    per_launch = flop_per_box * boxes / steps / kernels
     res = {"wall_s": wall, "flops": flops, "energy": energy, "pack_ms": pack_ms,
-           "slots": ft.slots, "boxes_per_launch": chunk / kernels, "boxes_per_step": chunk,
+           "slots": ft.slots, "slots_per_launch": chunk / kernels, "slots_per_step": chunk,
+           "boxes_computed": boxes, "boxes_per_launch": boxes / steps / kernels,
            "kernels_per_step": kernels,
            "launch_ms": launch_ms / kernels, "flop_per_launch": per_launch,
            "panel_bytes": ft.panel_bytes,
            "mfma_flop_issued_per_box": ft.mfma_flop_per_box,
-           "algorithmic_flop_per_box": flops / ft.slots,
+           "algorithmic_flop_per_box": flop_per_box,
            "v_segments": w["v_segs"], "o_segments": w["o_segs"], "o": o, "v": v}
     return w, ft, res
 
@@ -993,7 +1000,8 @@ def main():
                            "energy reduced in the epilogue); operands packed once into MFMA-order "
                            "panels",
                    "pack_ms": tri["pack_ms"], "slots": tri["slots"],
-                   "boxes_per_step": tri["boxes_per_step"],
+                   "slots_per_step": tri["slots_per_step"],
+                   "boxes_computed": tri["boxes_computed"],
                    "kernel_launches_per_step": kernels,
                    "tflops_including_pack": tri["flops"] / (tri["wall_s"] + tri["pack_ms"] * 1e-3)
                    / 1e12},

@@ -102,6 +102,72 @@ def test_fused_whole_sum_vs_oracle(small):
     assert outs[0] == outs[1]
 
 
+def dense(arr):
+    """A DeviceBlocks array as one numpy array."""
+    out = np.zeros([sum(s) for s in arr.segs])
+    host = arr.dev.download()
+    for blk in arr.offset:
+        at = [tp.seg_offset(s, b) for s, b in zip(arr.segs, blk)]
+        out[tuple(slice(a, a + n) for a, n in zip(at, arr.dims(blk)))] = \
+            arr.download_block(blk, host).reshape(arr.dims(blk), order="F")
+    return out
+
+
+# Boxes whose pairs are all equal, two equal and all different; 5-blocks
+# across segment boundaries; one box; odd and even 5-block counts (super-boxes
+# with and without padding).
+@pytest.mark.parametrize("v_segs, o_segs", [((1,), (1,)), ((7, 4), (6, 6)), ((7, 9, 8), (2, 2)),
+                                            ((2, 3, 1, 4), (3, 1, 7))])
+def test_fused_classes_vs_dense(v_segs, o_segs):
+    """The whole sum, its bits over any cut of the slots, and every tuple's
+    energy and W against a dense numpy build of W (sums of one sign: the
+    relative error is that of the products, far below 1e-13)."""
+    print("fused classes", v_segs, o_segs, flush=True)
+    w = tp.triples(o_segs=o_segs, v_segs=v_segs, seed=8)
+    tp.to_device(w)
+    V1, V2, T = (dense(w[k]) for k in ("V1", "V2", "T"))
+    base = np.einsum("bcdk,adij->abcijk", V1, T, optimize=True) + \
+        np.einsum("lcjk,abil->abcijk", V2, T, optimize=True)
+    W = sum(base.transpose(*[p.index(n) for n in range(3)], *[3 + p.index(n) for n in range(3)])
+            for p in itertools.permutations(range(3)))
+    e_o, e_v = w["e_occ"], w["e_vir"]
+    D = np.add.outer(np.add.outer(-e_v, -e_v), -e_v)[..., None, None, None] + \
+        np.add.outer(np.add.outer(e_o, e_o), e_o)
+    E = W * W / D
+    ft = tp.FusedTriples(w)
+    out = sg.DeviceArray(1)
+    got = []
+    cut = ft.slots // 3 + 1
+    for ranges in ([(0, ft.slots)], [(0, cut), (cut, ft.slots - cut)],
+                   [(i, min(37, ft.slots - i)) for i in range(0, ft.slots, 37)][:400]):
+        ft.pack()
+        for r in ranges:
+            ft.run(*r)
+        done = ranges[-1][0] + ranges[-1][1]
+        if done < ft.slots:
+            ft.run(done, ft.slots - done)
+        out.zero()
+        ft.energy(out.ptr)
+        sg.synchronize()
+        got.append(float(out.download()[0]))
+    assert abs(got[0] - E.sum()) <= 1e-13 * abs(E.sum())
+    assert got[0] == got[1] == got[2]
+    nv, no = len(v_segs), len(o_segs)
+    wbuf = sg.DeviceArray(max(v_segs) ** 3 * max(o_segs) ** 3)
+    for tup in itertools.product(*([range(nv)] * 3 + [range(no)] * 3)):
+        segs = [v_segs] * 3 + [o_segs] * 3
+        at = tuple(slice(tp.seg_offset(s, b), tp.seg_offset(s, b) + s[b])
+                   for s, b in zip(segs, tup))
+        out.zero()
+        ft.tuple(tup, out.ptr, w_out=wbuf.ptr)
+        sg.synchronize()
+        n = W[at].size
+        assert rel_fro(wbuf.download()[:n], W[at].ravel(order="F")) <= 1e-13
+        want = E[at].sum()
+        assert abs(float(out.download()[0]) - want) <= 1e-13 * abs(want)
+    ft.destroy()
+
+
 def test_fused_full_size_tuple():
     """One 20^6 tuple of the triples configuration (o = 30 in 20, 10; v = 240
     in 12 x 20): its energy against the twelve-batch FP64 path (oracle-pinned
