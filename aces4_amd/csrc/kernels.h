@@ -233,7 +233,7 @@ struct TriplesArgs {
     // classes orbits[0 .. norbits), each result stored for the box's images
     // among slots [box0, box0 + nbox)
     const TriplesOrbit *orbits;
-    long long norbits, per_xcd;
+    long long norbits;
     long long box0, nbox;
     int super_v;
     // tuple mode: the boxes first[d] .. first[d] + count[d] - 1, limited to

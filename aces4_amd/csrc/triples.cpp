@@ -291,8 +291,8 @@ int sipgpu_triples_run(sipgpu_triples_t P, long long box0, long long nbox, sipgp
         const long long c0 = class_of(b), c1 = class_of(b + a.nbox - 1);
         a.orbits = P->d_orbits + c0;
         a.norbits = c1 - c0 + 1;
-        a.per_xcd = a.norbits * 8;
-        SIPGPU_HIP_TRY(sipgpu::launch_triples_boxes(a, 8 * a.per_xcd, hs));
+        // 64 workgroups a class, the classes in groups of one per XCD
+        SIPGPU_HIP_TRY(sipgpu::launch_triples_boxes(a, (a.norbits + 7) / 8 * 512, hs));
     }
     return 0;
 }

@@ -37,6 +37,8 @@ constexpr int kBoxE = kTriplesBox;                 // box extent per index
 constexpr int kBoxRows = kBoxE * kBoxE * kBoxE;     // 125 rows / columns per P
 constexpr int kBoxElems = kBoxRows * kBoxRows;      // 15625
 constexpr int kThreads = 512;
+constexpr int kFinalThreads = 1024;
+static_assert(kTriplesSums % kFinalThreads == 0, "the final sum's split");
 
 // the permutations P of (0, 1, 2), in the order W sums them
 __constant__ int kPerm[6][3] = {{0, 1, 2}, {0, 2, 1}, {1, 0, 2}, {1, 2, 0}, {2, 0, 1}, {2, 1, 0}};
@@ -172,11 +174,11 @@ __device__ __forceinline__ bool box_of(const TriplesArgs &a, int (&bc)[6], BoxId
         }
         return true;
     }
-    const long long w = blockIdx.x;
-    const long long local = (w & 7) * a.per_xcd + (w >> 3);
-    if (local >= a.norbits * 64) return false;
-    id.orbit = a.orbits[local >> 6];
-    const int q = (int)(local & 63);
+    // XCD x takes the classes x, x + 8, ... of the call, 64 workgroups each
+    const long long w = blockIdx.x, cls = (w >> 9) * 8 + (w & 7);
+    if (cls >= a.norbits) return false;
+    id.orbit = a.orbits[cls];
+    const int q = (int)(w >> 3) & 63;
 #pragma unroll
     for (int m = 0; m < 3; ++m) {
         id.sub[m] = ((q >> m) & 1) | ((q >> (3 + m)) & 1) << 1;
@@ -418,8 +420,8 @@ __global__ __launch_bounds__(kThreads) void triples_box_kernel(TriplesArgs a) {
     }
 }
 
-// out[0] += factor * sum of partial[0 .. n) in index order: per-workgroup
-// sums of contiguous ranges, then one thread over them.
+// out[0] += factor * sum of partial[0 .. n) in a fixed order: per-workgroup
+// sums of contiguous ranges, then one workgroup over them.
 __global__ __launch_bounds__(256) void triples_reduce_kernel(const double *partial, long long n,
                                                              long long chunk, double *sums) {
     __shared__ double red[4];
@@ -434,11 +436,24 @@ __global__ __launch_bounds__(256) void triples_reduce_kernel(const double *parti
     if (threadIdx.x == 0) sums[blockIdx.x] = ((red[0] + red[1]) + red[2]) + red[3];
 }
 
-__global__ void triples_final_kernel(const double *sums, int n, double factor, double *out) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    double t = 0.0;
-    for (int i = 0; i < n; ++i) t += sums[i];
-    out[0] += factor * t;
+// One workgroup over the at most kTriplesSums sums: thread t its consecutive
+// ones, then a fixed tree.  (One thread over all of them, a chain of 4096
+// dependent loads and adds, took 214 us of every energy.)
+__global__ __launch_bounds__(kFinalThreads) void triples_final_kernel(const double *sums, int n,
+                                                                      double factor,
+                                                                      double *out) {
+    __shared__ double red[kFinalThreads];
+    constexpr int per = kTriplesSums / kFinalThreads;
+    const int t = threadIdx.x;
+    double s = 0.0;
+#pragma unroll
+    for (int i = 0; i < per; ++i) s += t * per + i < n ? sums[t * per + i] : 0.0;
+    red[t] = s;
+    for (int m = kFinalThreads / 2; m >= 1; m >>= 1) {
+        __syncthreads();
+        if (t < m) red[t] += red[t + m];
+    }
+    if (t == 0) out[0] += factor * red[0];
 }
 
 } // namespace
@@ -464,7 +479,7 @@ hipError_t launch_triples_reduce(const double *partial, long long n, double *sum
     const long long chunk = (n + kTriplesSums - 1) / kTriplesSums;
     const int blocks = (int)((n + chunk - 1) / chunk);
     triples_reduce_kernel<<<blocks, 256, 0, s>>>(partial, n, chunk, sums);
-    triples_final_kernel<<<1, 64, 0, s>>>(sums, blocks, factor, out);
+    triples_final_kernel<<<1, kFinalThreads, 0, s>>>(sums, blocks, factor, out);
     return hipGetLastError();
 }
 
