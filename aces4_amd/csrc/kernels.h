@@ -229,23 +229,26 @@ struct TriplesArgs {
     int kd, kl;     // virtual and occupied index totals
     const double *e_vir, *e_occ;
     double *partial;
-    // global mode: one box per (class, position in its super-box) for the
-    // classes orbits[0 .. norbits), each result stored for the box's images
+    // global mode: XCD x runs the boxes items[begin[x] .. end[x]) (class * 64 +
+    // position in its super-box) and stores each result for the box's images
     // among slots [box0, box0 + nbox)
     const TriplesOrbit *orbits;
-    long long norbits;
+    const unsigned *items;
+    unsigned begin[8], end[8];
     long long box0, nbox;
     int super_v;
-    // tuple mode: the boxes first[d] .. first[d] + count[d] - 1, limited to
-    // the tuple's global index ranges [lo[d], lo[d] + wdims[d])
+    // tuple mode: boxes 0 .. end[0] - 1 of first[d] .. first[d] + count[d] - 1
+    // (first index fastest).  Elements count that lie in the global index
+    // ranges [lo[d], lo[d] + wdims[d]) (both modes)
     int tuple_mode;
     int first[6], count[6];
     double *wout;   // tuple mode, optional: W of the tuple (column-major)
     int lo[6], wdims[6];
 };
 hipError_t launch_triples_pack(const TriplesPackArgs &a, hipStream_t s);
-// grid workgroups of 512; hipErrorInvalidConfiguration at 2^23 workgroups or more
-hipError_t launch_triples_boxes(const TriplesArgs &a, long long grid, hipStream_t s);
+// One workgroup of 512 per CU (fewer for fewer boxes).
+constexpr unsigned kTriplesGroups = 256;
+hipError_t launch_triples_boxes(const TriplesArgs &a, hipStream_t s);
 // out[0] += factor * sum of partial[0 .. n) in a fixed order (sums: kTriplesSums doubles)
 hipError_t launch_triples_reduce(const double *partial, long long n, double *sums, double factor,
                                  double *out, hipStream_t s);

@@ -28,11 +28,15 @@ struct sipgpu_triples_s {
     int nv = 0, no = 0;
     std::vector<int> vseg, oseg;
     std::vector<TriplesOrbit> orbits; // ascending in `first`
+    // boxes to compute (class * 64 + position), XCD by XCD, ascending in each
+    std::vector<unsigned> items;
+    size_t xcd_first[9] = {};
     int nvb = 0, nob = 0;             // 5-blocks of the virtual / occupied range
     int kd = 0, kl = 0, nkp = 0;
     // device memory
     void *tables = nullptr; // orbits, ints, pointer tables
     const TriplesOrbit *d_orbits = nullptr;
+    const unsigned *d_items = nullptr;
     const int *d_vext = nullptr, *d_oext = nullptr, *d_vseg_of = nullptr, *d_oseg_of = nullptr;
     const int *d_vseg_start = nullptr, *d_oseg_start = nullptr;
     const double *const *d_T = nullptr, *const *d_V1 = nullptr, *const *d_V2 = nullptr;
@@ -59,6 +63,38 @@ std::vector<TriplesOrbit> super_box_classes(int n) {
                 first += p == q && q == r ? 1 : p == q || q == r ? 3 : 6;
             }
     return out;
+}
+
+// The boxes to compute: positions whose 5-blocks exist and whose pairs are
+// ascending (another order of equal super pairs is an image), the classes
+// dealt to the XCDs in turn.  Bit q of a mask stands for position q.
+void list_boxes(sipgpu_triples_s &P) {
+    uint64_t zero[6] = {}, asc01 = 0, asc12 = 0; // zero[d]: positions with bit d clear
+    for (unsigned q = 0; q < 64; ++q) {
+        const uint64_t bit = 1ull << q;
+        int sub[3];
+        for (int m = 0; m < 3; ++m) sub[m] = ((q >> m) & 1) | ((q >> (3 + m)) & 1) << 1;
+        for (int d = 0; d < 6; ++d)
+            if (!((q >> d) & 1)) zero[d] |= bit;
+        if (sub[0] <= sub[1]) asc01 |= bit;
+        if (sub[1] <= sub[2]) asc12 |= bit;
+    }
+    for (int x = 0; x < 8; ++x) {
+        P.xcd_first[x] = P.items.size();
+        for (size_t c = x; c < P.orbits.size(); c += 8) {
+            const int *p = P.orbits[c].p;
+            uint64_t boxes = ~0ull;
+            for (int m = 0; m < 3; ++m) {
+                if (2 * (p[m] % P.super_v) + 1 >= P.nvb) boxes &= zero[m];
+                if (2 * (p[m] / P.super_v) + 1 >= P.nob) boxes &= zero[3 + m];
+            }
+            if (p[0] == p[1]) boxes &= asc01;
+            if (p[1] == p[2]) boxes &= asc12;
+            for (; boxes; boxes &= boxes - 1)
+                P.items.push_back((unsigned)(c * 64) | (unsigned)__builtin_ctzll(boxes));
+        }
+    }
+    P.xcd_first[8] = P.items.size();
 }
 
 // the 5-blocks that a segment at global index g touches
@@ -102,8 +138,9 @@ int sipgpu_triples_create(int nv, const int *v_seg, int no, const int *o_seg,
         if (x < 1) return fail(SIPGPU_EARG, "triples: segment extents must be positive");
     for (int x : P->vseg) P->kd += x;
     for (int x : P->oseg) P->kl += x;
-    // K padded to whole pairs of k-pairs (the kernel loads two per trip)
-    P->nkp = ((P->kd + P->kl + 15) / 16) * 2;
+    // K in k-pairs of 8, at least four (the kernel's loads run two ahead and
+    // cross one permutation boundary at a time)
+    P->nkp = std::max(4, (P->kd + P->kl + 7) / 8);
     P->nvb = (P->kd + sipgpu::kTriplesBox - 1) / sipgpu::kTriplesBox;
     P->nob = (P->kl + sipgpu::kTriplesBox - 1) / sipgpu::kTriplesBox;
     const long long nvb = P->nvb, nob = P->nob;
@@ -143,6 +180,7 @@ int sipgpu_triples_create(int nv, const int *v_seg, int no, const int *o_seg,
     // then at most a hundredth of that
     try {
         P->orbits = super_box_classes((int)pairs);
+        list_boxes(*P);
     } catch (const std::bad_alloc &) {
         return no_memory();
     }
@@ -165,6 +203,7 @@ int sipgpu_triples_create(int nv, const int *v_seg, int no, const int *o_seg,
         return at;
     };
     const size_t o_orbits = put(P->orbits.data(), P->orbits.size() * sizeof(TriplesOrbit));
+    const size_t o_items = put(P->items.data(), P->items.size() * sizeof(unsigned));
     const size_t o_vext = put(P->vseg.data(), nv * sizeof(int));
     const size_t o_oext = put(P->oseg.data(), no * sizeof(int));
     const size_t o_vso = put(vseg_of.data(), vseg_of.size() * sizeof(int));
@@ -180,6 +219,7 @@ int sipgpu_triples_create(int nv, const int *v_seg, int no, const int *o_seg,
     if (e != hipSuccess) return no_memory();
     const unsigned char *base = static_cast<const unsigned char *>(P->tables);
     P->d_orbits = reinterpret_cast<const TriplesOrbit *>(base + o_orbits);
+    P->d_items = reinterpret_cast<const unsigned *>(base + o_items);
     P->d_vext = reinterpret_cast<const int *>(base + o_vext);
     P->d_oext = reinterpret_cast<const int *>(base + o_oext);
     P->d_vseg_of = reinterpret_cast<const int *>(base + o_vso);
@@ -260,6 +300,9 @@ sipgpu::TriplesArgs box_args(const sipgpu_triples_s &P) {
     a.kd = P.kd;
     a.kl = P.kl;
     a.super_v = P.super_v;
+    a.orbits = P.d_orbits;
+    a.items = P.d_items;
+    for (int d = 0; d < 6; ++d) a.wdims[d] = d < 3 ? P.kd : P.kl;
     a.e_vir = P.e_vir;
     a.e_occ = P.e_occ;
     return a;
@@ -282,17 +325,21 @@ int sipgpu_triples_run(sipgpu_triples_t P, long long box0, long long nbox, sipgp
                                 [](long long s, const TriplesOrbit &o) { return s < o.first; }) -
                P->orbits.begin() - 1;
     };
-    // one launch per SIPGPU_TRIPLES_LAUNCH_BOXES slots: a dispatch holds
-    // fewer than 2^32 work-items (8.4M workgroups of 512).  A class that a
-    // cut divides is computed by both launches.
+    // one launch per SIPGPU_TRIPLES_LAUNCH_BOXES slots (about 0.3 s of the
+    // whole sum at o = 30, v = 240).  A class that a cut divides is computed
+    // by both launches.
     for (long long b = box0; b < box0 + nbox; b += SIPGPU_TRIPLES_LAUNCH_BOXES) {
         a.box0 = b;
         a.nbox = std::min<long long>(SIPGPU_TRIPLES_LAUNCH_BOXES, box0 + nbox - b);
-        const long long c0 = class_of(b), c1 = class_of(b + a.nbox - 1);
-        a.orbits = P->d_orbits + c0;
-        a.norbits = c1 - c0 + 1;
-        // 64 workgroups a class, the classes in groups of one per XCD
-        SIPGPU_HIP_TRY(sipgpu::launch_triples_boxes(a, (a.norbits + 7) / 8 * 512, hs));
+        const unsigned i0 = (unsigned)class_of(b) * 64,
+                       i1 = ((unsigned)class_of(b + a.nbox - 1) + 1) * 64;
+        for (int x = 0; x < 8; ++x) {
+            const auto f = P->items.begin() + P->xcd_first[x],
+                       l = P->items.begin() + P->xcd_first[x + 1];
+            a.begin[x] = (unsigned)(std::lower_bound(f, l, i0) - P->items.begin());
+            a.end[x] = (unsigned)(std::lower_bound(f, l, i1) - P->items.begin());
+        }
+        SIPGPU_HIP_TRY(sipgpu::launch_triples_boxes(a, hs));
     }
     return 0;
 }
@@ -323,7 +370,8 @@ int sipgpu_triples_tuple(sipgpu_triples_t P, const int *tuple, double factor, do
         grid *= a.count[d];
     }
     const hipStream_t hs = sipgpu::rt::stream_of(s);
-    SIPGPU_HIP_TRY(sipgpu::launch_triples_boxes(a, grid, hs));
+    a.end[0] = (unsigned)grid;
+    SIPGPU_HIP_TRY(sipgpu::launch_triples_boxes(a, hs));
     SIPGPU_HIP_TRY(sipgpu::launch_triples_reduce(P->tuple_partial, grid, P->sums, factor, out, hs));
     return 0;
 }

@@ -24,6 +24,8 @@
 // of two MFMA k-steps with one 16-byte load per lane, 1 KiB contiguous per
 // wave.  Every P reads the same two arrays: P only changes which box
 // coordinates select the row and column sets.
+#include <type_traits>
+
 #include "kernels.h"
 
 namespace sipgpu {
@@ -37,6 +39,7 @@ constexpr int kBoxE = kTriplesBox;                 // box extent per index
 constexpr int kBoxRows = kBoxE * kBoxE * kBoxE;     // 125 rows / columns per P
 constexpr int kBoxElems = kBoxRows * kBoxRows;      // 15625
 constexpr int kThreads = 512;
+constexpr int kOutside = 1 << 20; // byte offset of a padded row or column: past any box
 constexpr int kFinalThreads = 1024;
 static_assert(kTriplesSums % kFinalThreads == 0, "the final sum's split");
 
@@ -127,22 +130,28 @@ __global__ __launch_bounds__(256) void triples_pack_kernel(TriplesPackArgs a) {
 // segments of 20 and 10: 373,248 slots, 64,824 boxes; 133 -> 25.8 ms).  A slot's
 // value does not depend on which range of slots a call covers.
 //
-// Global mode: workgroup (class, q) owns position q (one bit per index) of a
-// class's ascending super-box.  Slots number the 64 boxes of every super-box,
-// the arrangements of a class next to each other, so that any range of slots
-// holds most images of the boxes it computes.  Workgroup w runs on XCD w % 8
-// and takes ids in order within that XCD's share: the boxes running together
-// on one XCD are neighbours in all six indices and share operand sets in its
-// L2.
+// Global mode: item 64 c + q is position q (one bit per index) of class c's
+// ascending super-box; the plan lists the items that are boxes (inside the
+// index ranges, their pairs ascending) XCD by XCD, the classes dealt to the
+// XCDs in turn.  Slots number the 64 boxes of every super-box, the
+// arrangements of a class next to each other, so that any range of slots
+// holds most images of the boxes it computes.
 struct BoxId {
-    TriplesOrbit orbit;
-    int sub[3]; // bit 0: which virtual 5-block of the super-box, bit 1: occupied
+    int p[3];        // the class's super pairs
+    long long first; // its first super-box
+    int sub[3];      // bit 0: which virtual 5-block of the super-box, bit 1: occupied
 };
+
+// the p-th of three values (an array indexed at run time would leave the
+// registers)
+__device__ __forceinline__ int pick(int x0, int x1, int x2, int p) {
+    return p == 0 ? x0 : p == 1 ? x1 : x2;
+}
 
 // Slot of the arrangement g of the box's pairs (position t holds pair kPerm[g][t]).
 __device__ __forceinline__ long long image_slot(const BoxId &b, int g) {
     const int t0 = kPerm[g][0], t1 = kPerm[g][1], t2 = kPerm[g][2];
-    const bool eq01 = b.orbit.p[0] == b.orbit.p[1], eq12 = b.orbit.p[1] == b.orbit.p[2];
+    const bool eq01 = b.p[0] == b.p[1], eq12 = b.p[1] == b.p[2];
     // distinct arrangements of the class: by g, by the place of the pair that
     // differs from the other two, or just one
     int rank = g;
@@ -152,125 +161,138 @@ __device__ __forceinline__ long long image_slot(const BoxId &b, int g) {
         rank = t0 == 2 ? 0 : t1 == 2 ? 1 : 2;
     else if (eq12)
         rank = t0 == 0 ? 0 : t1 == 0 ? 1 : 2;
-    const int s0 = b.sub[t0], s1 = b.sub[t1], s2 = b.sub[t2];
+    const int s0 = pick(b.sub[0], b.sub[1], b.sub[2], t0), s1 = pick(b.sub[0], b.sub[1], b.sub[2], t1), s2 = pick(b.sub[0], b.sub[1], b.sub[2], t2);
     const int q = (s0 & 1) | (s1 & 1) << 1 | (s2 & 1) << 2 | (s0 >> 1) << 3 | (s1 >> 1) << 4 |
                   (s2 >> 1) << 5;
-    return (b.orbit.first + rank) * 64 + q;
+    return (b.first + rank) * 64 + q;
 }
 
-// Box coordinates (5-block indices of a, b, c, i, j, k) of this workgroup.
-// Returns false where there is nothing to compute: no work id, a position
-// whose ascending form is another one, no image among the call's slots, or a
-// box past the index ranges (padding of the super-boxes; its partial stays
-// the zero that packing stores).  Tuple mode: the boxes of one tuple, first
-// index fastest.
-__device__ __forceinline__ bool box_of(const TriplesArgs &a, int (&bc)[6], BoxId &id) {
+// Box coordinates (5-block indices of a, b, c, i, j, k) of work item t.
+// Tuple mode: the boxes of one tuple, first index fastest.
+__device__ __forceinline__ void box_of(const TriplesArgs &a, unsigned t, int (&bc)[6], BoxId &id) {
     if (a.tuple_mode) {
-        long long q = blockIdx.x;
+        unsigned q = t;
 #pragma unroll
         for (int d = 0; d < 6; ++d) {
             bc[d] = a.first[d] + (int)(q % a.count[d]);
             q /= a.count[d];
         }
-        return true;
+        return;
     }
-    // XCD x takes the classes x, x + 8, ... of the call, 64 workgroups each
-    const long long w = blockIdx.x, cls = (w >> 9) * 8 + (w & 7);
-    if (cls >= a.norbits) return false;
-    id.orbit = a.orbits[cls];
-    const int q = (int)(w >> 3) & 63;
+    const unsigned item = a.items[t];
+    const TriplesOrbit o = a.orbits[item >> 6];
+    id.first = o.first;
 #pragma unroll
     for (int m = 0; m < 3; ++m) {
-        id.sub[m] = ((q >> m) & 1) | ((q >> (3 + m)) & 1) << 1;
-        bc[m] = 2 * (id.orbit.p[m] % a.super_v) + (id.sub[m] & 1);
-        bc[3 + m] = 2 * (id.orbit.p[m] / a.super_v) + (id.sub[m] >> 1);
-        if (bc[m] >= a.nvb || bc[3 + m] >= a.nob) return false;
+        id.p[m] = o.p[m];
+        id.sub[m] = ((item >> m) & 1) | ((item >> (3 + m)) & 1) << 1;
+        bc[m] = 2 * (o.p[m] % a.super_v) + (id.sub[m] & 1);
+        bc[3 + m] = 2 * (o.p[m] / a.super_v) + (id.sub[m] >> 1);
     }
-    if (id.orbit.p[0] == id.orbit.p[1] && id.sub[0] > id.sub[1]) return false;
-    if (id.orbit.p[1] == id.orbit.p[2] && id.sub[1] > id.sub[2]) return false;
-    bool any = false;
-    for (int g = 0; g < 6; ++g) {
-        const long long slot = image_slot(id, g) - a.box0;
-        any = any || (slot >= 0 && slot < a.nbox);
-    }
-    return any;
 }
 
-// One workgroup: one 5^6 box of W, all six GEMMs, the energy partial.
-// Eight waves in 2 x 4, each a 64 x 32 tile (4 x 2 MFMA blocks): two waves
-// per SIMD, so one issues MFMAs while the other waits for its operands.
+// *w += x in LDS, no value returned: the wave does not wait for the sum
+// before it goes on with the next product (read, add, write: 21.7 ms a sum of
+// o = 30, v = 60, this 20.9).  Each element is added to once between two
+// barriers, so the order of the sums is fixed.
+__device__ __forceinline__ void lds_add(double *w, double x) {
+    __builtin_amdgcn_ds_atomic_fadd_f64((__attribute__((address_space(3))) double *)w, x);
+}
+
+// A barrier that the waves of a workgroup may reach at different places of
+// the program, the same number of times each.
+__device__ __forceinline__ void group_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
+// A workgroup runs boxes one after another, each with all six GEMMs and the
+// energy partial.  Eight waves in 2 x 4, each a 64 x 32 tile (4 x 2 MFMA
+// blocks): two waves per SIMD, so one issues MFMAs while the other waits for
+// its operands.  The box fills the LDS, so a CU holds one workgroup and
+// nothing else covers its start and end: one workgroup per CU stays and
+// fetches its next box's first operands and energies during the present one.
+// Adding a product into the box is 16384 LDS operations without a branch: with
+// the bounds tested per element, the waits between them and both waves of a
+// SIMD adding at once, the sum of o = 30, v = 60 took 24.9 ms; 20.9 now, of
+// which the MFMAs alone take 15.8 (76% busy; was 65%).
+template <int REST>
 __global__ __launch_bounds__(kThreads) void triples_box_kernel(TriplesArgs a) {
-    __shared__ double W[kBoxElems];
+    __shared__ double W[kBoxElems + 64]; // 64: where the padded rows and columns go
     __shared__ double eps[6][kBoxE];
     __shared__ int lo[6], hi[6]; // the box's elements that count, per index
     __shared__ double red[kThreads / 64];
     __shared__ double occ[kBoxRows];
-    // box offsets of product row / column x (< 128) under permutation g
-    __shared__ int rofs[6][128], cofs[6][128];
+    // byte offsets in the box of the product's rows and columns under
+    // permutation g: rows by (wave row, lane / 16, block, register), columns
+    // by x; past the 125th far outside the box
+    __shared__ int rofs[6][2][4][16], cofs[6][128];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave & 1, wn = wave >> 1;
-    int bc[6];
+    // this workgroup's work items: item, item + stride, ... < end
+    unsigned item, end, stride;
+    if (a.tuple_mode) {
+        item = blockIdx.x;
+        end = a.end[0];
+        stride = gridDim.x;
+    } else {
+        const int x = blockIdx.x & 7;
+        item = a.begin[x] + (blockIdx.x >> 3);
+        end = a.end[x];
+        stride = gridDim.x >> 3;
+    }
+    if (item >= end) return;
+    int bc[6]; // the box being loaded
     BoxId id;
-    if (!box_of(a, bc, id)) return;
-    if (tid < 30) {
-        const int d = tid / kBoxE, q = tid % kBoxE;
-        const int g = bc[d] * kBoxE + q, total = d < 3 ? a.kd : a.kl;
-        const double *e = d < 3 ? a.e_vir : a.e_occ;
-        eps[d][q] = g < total ? e[g] : 0.0;
-    }
-    if (tid < 6) {
-        const int g0 = bc[tid] * kBoxE, total = tid < 3 ? a.kd : a.kl;
-        const int first = a.tuple_mode ? a.lo[tid] : 0;
-        const int end = a.tuple_mode ? a.lo[tid] + a.wdims[tid] : total;
-        lo[tid] = max(0, first - g0);
-        hi[tid] = min(kBoxE, end - g0);
-    }
+    box_of(a, item, bc, id);
 
     for (int t = tid; t < 6 * 128; t += kThreads) {
         const int g = t >> 7, x = t & 127;
         const int p0 = kPerm[g][0], p1 = kPerm[g][1], p2 = kPerm[g][2];
         const int d0 = x % kBoxE, d1 = (x / kBoxE) % kBoxE, d2 = x / (kBoxE * kBoxE);
         // row (x1, y1, y2), column (x2, x3, y3)
-        rofs[g][x] = d0 * box_stride(p0) + d1 * box_stride(3 + p0) + d2 * box_stride(3 + p1);
-        cofs[g][x] = d0 * box_stride(p1) + d1 * box_stride(p2) + d2 * box_stride(3 + p2);
+        const int r = d0 * box_stride(p0) + d1 * box_stride(3 + p0) + d2 * box_stride(3 + p1);
+        const int c = d0 * box_stride(p1) + d1 * box_stride(p2) + d2 * box_stride(3 + p2);
+        // row x = 64 wm + 16 i + 4 r + lane / 16
+        rofs[g][x >> 6][x & 3][(x >> 2) & 15] = x < kBoxRows ? 8 * r : kOutside;
+        cofs[g][x] = x < kBoxRows ? 8 * c : kOutside;
     }
 
     const int nkp = a.nkp;
-    // operand pointers of permutation g: its row set (x1, y1, y2) in PA and
-    // column set (x2, x3, y3) in PB, at this wave's first 16-row block
+    // operand pointers of permutation g of the box being loaded: its row set
+    // (x1, y1, y2) in PA and column set (x2, x3, y3) in PB, at this wave's
+    // first 16-row block
     auto panels = [&](int g, const f64x2 *&pa, const f64x2 *&pb) {
         const int p0 = kPerm[g][0], p1 = kPerm[g][1], p2 = kPerm[g][2];
-        const long long rowset = ((long long)bc[p0] * a.nob + bc[3 + p0]) * a.nob + bc[3 + p1];
-        const long long colset = ((long long)bc[p1] * a.nvb + bc[p2]) * a.nob + bc[3 + p2];
+        const int x1 = pick(bc[0], bc[1], bc[2], p0), y1 = pick(bc[3], bc[4], bc[5], p0);
+        const int x2 = pick(bc[0], bc[1], bc[2], p1), y2 = pick(bc[3], bc[4], bc[5], p1);
+        const int x3 = pick(bc[0], bc[1], bc[2], p2), y3 = pick(bc[3], bc[4], bc[5], p2);
+        const long long rowset = ((long long)x1 * a.nob + y1) * a.nob + y2;
+        const long long colset = ((long long)x2 * a.nvb + x3) * a.nob + y3;
         pa = reinterpret_cast<const f64x2 *>(a.PA) + ((rowset * 8 + wm * 4) * nkp) * 64 + lane;
         pb = reinterpret_cast<const f64x2 *>(a.PB) + ((colset * 8 + wn * 2) * nkp) * 64 + lane;
     };
+    // The k-pairs of the six permutations of all boxes form one stream;
+    // loads run two k-pairs ahead of the MFMAs through three register sets,
+    // across the permutation and box boundaries (nkp >= 4).  Load cursor:
+    // k-pair lkp of (lpa, lpb), then the next permutation's (npa, npb).
     f64x2 fa[3][4], fb[3][2];
-    auto load = [&](int st, const f64x2 *pa, const f64x2 *pb, int kp) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) fa[st][i] = pa[((long long)i * nkp + kp) * 64];
-#pragma unroll
-        for (int j = 0; j < 2; ++j) fb[st][j] = pb[((long long)j * nkp + kp) * 64];
-    };
-    // The k-pairs of the six permutations form one stream; loads run two
-    // k-pairs ahead of the MFMAs through three register sets, across the
-    // permutation boundaries.  Load cursor: permutation lg, k-pair lkp
-    // (past the last k-pair of the last permutation it reloads that one,
-    // which nothing reads).
-    int lg = 0, lkp = 0;
-    const f64x2 *lpa, *lpb;
+    const f64x2 *lpa, *lpb, *npa, *npb;
     panels(0, lpa, lpb);
+    npa = lpa;
+    npb = lpb;
+    int lkp = 0;
     auto load_next = [&](int st) {
-        load(st, lpa, lpb, lkp);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) fa[st][i] = lpa[((long long)i * nkp + lkp) * 64];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) fb[st][j] = lpb[((long long)j * nkp + lkp) * 64];
         if (++lkp == nkp) {
-            if (lg < 5) {
-                lkp = 0;
-                ++lg;
-                panels(lg, lpa, lpb);
-            } else {
-                lkp = nkp - 1;
-            }
+            lkp = 0;
+            lpa = npa;
+            lpb = npb;
         }
     };
     f64x4 acc[4][2];
@@ -288,135 +310,195 @@ __global__ __launch_bounds__(kThreads) void triples_box_kernel(TriplesArgs a) {
                     acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[st][i][h], fb[st][j][h],
                                                                      acc[i][j], 0, 0, 0);
     };
-    // add permutation g's product into the box: row (x1, y1, y2), column
-    // (x2, x3, y3); the first permutation assigns
-    auto scatter = [&](int g) {
-        // the previous P's adds into the box are complete
-        __syncthreads();
-        int coff[2];
-        bool cok[2];
+    // this thread's share of the box's tables, stored once the previous box's
+    // energy is done: an orbital energy (tid < 30), an index's range (tid < 6)
+    double my_eps = 0.0;
+    int my_lo = 0, my_hi = 0;
+    auto fetch_tables = [&]() {
+        if (tid < 30) {
+            const int d = tid / kBoxE;
+            int blk = bc[0];
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int c = (wn * 2 + j) * 16 + (lane & 15);
-            cok[j] = c < kBoxRows;
-            coff[j] = cofs[g][c];
+            for (int e = 1; e < 6; ++e) blk = d == e ? bc[e] : blk;
+            const int g = blk * kBoxE + tid % kBoxE, total = d < 3 ? a.kd : a.kl;
+            my_eps = g < total ? (d < 3 ? a.e_vir : a.e_occ)[g] : 0.0;
         }
+        if (tid < 6) {
+            int g0 = bc[0], first = a.lo[0], ext = a.wdims[0];
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = (wm * 4 + i) * 16 + 4 * r + (lane >> 4);
-                if (row >= kBoxRows) continue;
-                const int roff = rofs[g][row];
-#pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    if (!cok[j]) continue;
-                    double &w = W[roff + coff[j]];
-                    w = g == 0 ? acc[i][j][r] : w + acc[i][j][r];
-                }
+            for (int e = 1; e < 6; ++e) {
+                g0 = tid == e ? bc[e] : g0;
+                first = tid == e ? a.lo[e] : first;
+                ext = tid == e ? a.wdims[e] : ext;
             }
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) acc[i][j] = f64x4{0.0, 0.0, 0.0, 0.0};
-    };
-    // compute cursor: permutation cg, k-pairs done ckp
-    int cg = 0, ckp = 0;
-    auto step = [&](int st) {
-        mma(st);
-        if (++ckp == nkp) {
-            scatter(cg);
-            ckp = 0;
-            ++cg;
+            my_lo = max(0, first - g0 * kBoxE);
+            my_hi = min(kBoxE, first + ext - g0 * kBoxE);
         }
     };
-    load_next(0);
-    load_next(1);
-    const int total = 6 * nkp;
-    for (int t = 0; t < total; t += 3) {
-        load_next(2);
-        step(0);
-        if (t + 1 < total) {
-            load_next(0);
-            step(1);
-        }
-        if (t + 2 < total) {
-            load_next(1);
-            step(2);
-        }
-    }
-    // energy of the box: sum over its elements inside the blocks' extents.
-    // Element e = abc + 125 ijk (abc = a + 5 b + 25 c, ijk = i + 5 j + 25 k).
-    // D = ((((e_i + e_j) + e_k) - e_a) - e_b) - e_c: the occupied sums of the
-    // box's 125 (i, j, k) are formed once (NaN marks an (i, j, k) outside the
-    // extents); a thread keeps one abc, its virtual energies in registers,
-    // and runs over ijk.
-    double sum = 0.0;
-    if (!a.wout) {
-        if (tid < kBoxRows) {
+    // add permutation g's product into the box: row (x1, y1, y2), column
+    // (x2, x3, y3); the first permutation assigns.  The previous P's adds into
+    // the box (the previous box's energy) are complete.
+    auto scatter = [&](int g) {
+        if (g == 0) {
+            if (tid < 30) eps[tid / kBoxE][tid % kBoxE] = my_eps;
+            if (tid < 6) {
+                lo[tid] = my_lo;
+                hi[tid] = my_hi;
+            }
+        } else if (g == 1 && tid < kBoxRows) {
+            // the occupied sums of the box (see the energy below)
             const int i = tid % kBoxE, j = (tid / kBoxE) % kBoxE, k = tid / (kBoxE * kBoxE);
             const bool in = i >= lo[3] && i < hi[3] && j >= lo[4] && j < hi[4] && k >= lo[5] &&
                             k < hi[5];
             occ[tid] = in ? eps[3][i] + eps[4][j] + eps[5][k] : __builtin_nan("");
         }
-        __syncthreads(); // the box and the occupied sums are complete
-        const int abc = tid & 127;
-        const int ea_i = abc % kBoxE, eb_i = (abc / kBoxE) % kBoxE, ec_i = abc / (kBoxE * kBoxE);
-        if (abc < kBoxRows && ea_i >= lo[0] && ea_i < hi[0] && eb_i >= lo[1] && eb_i < hi[1] &&
-            ec_i >= lo[2] && ec_i < hi[2]) {
-            const double ea = eps[0][ea_i], eb = eps[1][eb_i], ec = eps[2][ec_i];
-            for (int ijk = tid >> 7; ijk < kBoxRows; ijk += kThreads / 128) {
-                const double o = occ[ijk];
-                if (o != o) continue; // (i, j, k) outside the extents
-                const double w = W[abc + kBoxRows * ijk];
-                const double D = ((o - ea) - eb) - ec;
-                sum += (w / D) * w;
-            }
-        }
-    }
-    __syncthreads();
-
-    // tuple mode with W written out: every element's global position
-    for (int e = a.wout ? tid : kBoxElems; e < kBoxElems; e += kThreads) {
-        int q = e, dg[6];
-        bool in = true;
+        int roff[16], coff[2];
 #pragma unroll
-        for (int d = 0; d < 6; ++d) {
-            dg[d] = q % kBoxE;
-            q /= kBoxE;
-            in = in && dg[d] >= lo[d] && dg[d] < hi[d];
-        }
-        if (!in) continue;
-        const double w = W[e];
-        // occupied energies in index order, then the virtual ones subtracted
-        const double D = eps[3][dg[3]] + eps[4][dg[4]] + eps[5][dg[5]] - eps[0][dg[0]] -
-                         eps[1][dg[1]] - eps[2][dg[2]];
-        sum += (w / D) * w;
-        if (a.wout) {
-            long long o = 0;
+        for (int q = 0; q < 16; ++q) roff[q] = rofs[g][wm][lane >> 4][q];
 #pragma unroll
-            for (int d = 5; d >= 0; --d)
-                o = o * a.wdims[d] + (bc[d] * kBoxE + dg[d] - a.lo[d]);
-            a.wout[o] = w;
-        }
-    }
-    // fixed-order reduction: lanes by xor butterfly, then waves in order
+        for (int j = 0; j < 2; ++j) coff[j] = cofs[g][(wn * 2 + j) * 16 + (lane & 15)];
+        // no branch per element: what lies outside goes to 64 spare doubles
+        const unsigned outside = 8 * (kBoxElems + lane);
+        auto at = [&](int i, int r, int j) {
+            const unsigned o = min((unsigned)(roff[4 * i + r] + coff[j]), outside);
+            return reinterpret_cast<double *>(reinterpret_cast<char *>(W) + o);
+        };
+        if (g == 0) {
 #pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) sum += __shfl_xor(sum, m);
-    if (lane == 0) red[wave] = sum;
-    __syncthreads();
-    if (tid == 0) {
-        double t = red[0];
-        for (int w = 1; w < kThreads / 64; ++w) t += red[w];
-        if (a.tuple_mode) {
-            a.partial[blockIdx.x] = t;
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) *at(i, r, j) = acc[i][j][r];
         } else {
-            // images that coincide store the same value twice
-            for (int g = 0; g < 6; ++g) {
-                const long long slot = image_slot(id, g);
-                if (slot >= a.box0 && slot < a.box0 + a.nbox) a.partial[slot] = t;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) lds_add(at(i, r, j), acc[i][j][r]);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[i][j] = f64x4{0.0, 0.0, 0.0, 0.0};
+    };
+    // The two waves of a SIMD (w and w + 4) run half a product apart: one adds
+    // its product into the box while the other multiplies (together: 21.6 ms,
+    // apart: 20.9).  Each passes one
+    // barrier a product, the first four waves at its end, the others at its
+    // middle: behind it every wave has added the product before.
+    const bool late = wave >= 4;
+    const int middle = nkp / 2 / 3 * 3;
+    // Permutation g, its first k-pair in register set S: nkp = 3 n + REST
+    // k-pairs, so that the sets of three permutations are known here.
+    auto product = [&](int g, auto first_set) {
+        constexpr int S = decltype(first_set)::value;
+        // what is loaded after this permutation: the next one, then the next
+        // box (after the last box its own operands, which nothing reads)
+        if (g == 5 && item + stride < end) box_of(a, item + stride, bc, id);
+        panels(g == 5 ? 0 : g + 1, npa, npb);
+        for (int kp = 0; kp + 3 <= nkp; kp += 3) {
+            if (late && kp == middle) group_barrier();
+            load_next((S + 2) % 3);
+            mma(S);
+            load_next(S);
+            mma((S + 1) % 3);
+            load_next((S + 1) % 3);
+            mma((S + 2) % 3);
+        }
+        if (REST >= 1) {
+            load_next((S + 2) % 3);
+            mma(S);
+        }
+        if (REST == 2) {
+            load_next(S);
+            mma((S + 1) % 3);
+        }
+        if (!late) group_barrier();
+        scatter(g);
+    };
+    load_next(0);
+    load_next(1);
+    while (true) {
+        fetch_tables();
+        for (int g = 0; g < 6; g += 3) {
+            product(g, std::integral_constant<int, 0>{});
+            product(g + 1, std::integral_constant<int, REST>{});
+            product(g + 2, std::integral_constant<int, 2 * REST % 3>{});
+        }
+        // energy of the box: sum over its elements inside the blocks' extents.
+        // Element e = abc + 125 ijk (abc = a + 5 b + 25 c, ijk = i + 5 j + 25 k).
+        // D = ((((e_i + e_j) + e_k) - e_a) - e_b) - e_c: the occupied sums of the
+        // box's 125 (i, j, k) are formed once (NaN marks an (i, j, k) outside the
+        // extents); a thread keeps one abc, its virtual energies in registers,
+        // and runs over ijk.
+        double sum = 0.0;
+        __syncthreads(); // the box is complete
+        if (!a.wout) {
+            const int abc = tid & 127;
+            const int ea_i = abc % kBoxE, eb_i = (abc / kBoxE) % kBoxE, ec_i = abc / (kBoxE * kBoxE);
+            if (abc < kBoxRows && ea_i >= lo[0] && ea_i < hi[0] && eb_i >= lo[1] && eb_i < hi[1] &&
+                ec_i >= lo[2] && ec_i < hi[2]) {
+                const double ea = eps[0][ea_i], eb = eps[1][eb_i], ec = eps[2][ec_i];
+                for (int ijk = tid >> 7; ijk < kBoxRows; ijk += kThreads / 128) {
+                    const double o = occ[ijk];
+                    if (o != o) continue; // (i, j, k) outside the extents
+                    const double w = W[abc + kBoxRows * ijk];
+                    const double D = ((o - ea) - eb) - ec;
+                    sum += (w / D) * w;
+                }
             }
         }
+        // tuple mode with W written out: every element's global position
+        if (a.wout) box_of(a, item, bc, id);
+        for (int e = a.wout ? tid : kBoxElems; e < kBoxElems; e += kThreads) {
+            int q = e, dg[6];
+            bool in = true;
+#pragma unroll
+            for (int d = 0; d < 6; ++d) {
+                dg[d] = q % kBoxE;
+                q /= kBoxE;
+                in = in && dg[d] >= lo[d] && dg[d] < hi[d];
+            }
+            if (!in) continue;
+            const double w = W[e];
+            // occupied energies in index order, then the virtual ones subtracted
+            const double D = eps[3][dg[3]] + eps[4][dg[4]] + eps[5][dg[5]] - eps[0][dg[0]] -
+                             eps[1][dg[1]] - eps[2][dg[2]];
+            sum += (w / D) * w;
+            if (a.wout) {
+                long long o = 0;
+#pragma unroll
+                for (int d = 5; d >= 0; --d)
+                    o = o * a.wdims[d] + (bc[d] * kBoxE + dg[d] - a.lo[d]);
+                a.wout[o] = w;
+            }
+        }
+        // fixed-order reduction: lanes by xor butterfly, then waves in order
+#pragma unroll
+        for (int m = 32; m >= 1; m >>= 1) sum += __shfl_xor(sum, m);
+        if (lane == 0) red[wave] = sum;
+        __syncthreads();
+        if (tid == 0) {
+            double t = red[0];
+            for (int w = 1; w < kThreads / 64; ++w) t += red[w];
+            if (a.tuple_mode) {
+                a.partial[item] = t;
+            } else {
+                int unused[6];
+                BoxId id;
+                box_of(a, item, unused, id);
+                // images that coincide store the same value twice
+                for (int g = 0; g < 6; ++g) {
+                    const long long slot = image_slot(id, g);
+                    if (slot >= a.box0 && slot < a.box0 + a.nbox) a.partial[slot] = t;
+                }
+            }
+        }
+        item += stride;
+        if (item >= end) break;
+        if (a.wout) box_of(a, item, bc, id);
     }
 }
 
@@ -465,11 +547,19 @@ hipError_t launch_triples_pack(const TriplesPackArgs &a, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t launch_triples_boxes(const TriplesArgs &a, long long grid, hipStream_t s) {
-    if (grid <= 0) return hipSuccess;
-    // a dispatch holds at most 2^32 - 1 work-items per dimension
-    if (grid * kThreads >= (1LL << 32)) return hipErrorInvalidConfiguration;
-    triples_box_kernel<<<(unsigned)grid, kThreads, 0, s>>>(a);
+hipError_t launch_triples_boxes(const TriplesArgs &a, hipStream_t s) {
+    unsigned most = 0; // work items of the longest list
+    for (int x = 0; x < (a.tuple_mode ? 1 : 8); ++x) most = std::max(most, a.end[x] - a.begin[x]);
+    if (most == 0) return hipSuccess;
+    const unsigned grid = a.tuple_mode ? std::min(most, kTriplesGroups)
+                                       : 8 * std::min(most, kTriplesGroups / 8);
+    if (a.nkp < 4) return hipErrorInvalidValue;
+    if (a.nkp % 3 == 0)
+        triples_box_kernel<0><<<grid, kThreads, 0, s>>>(a);
+    else if (a.nkp % 3 == 1)
+        triples_box_kernel<1><<<grid, kThreads, 0, s>>>(a);
+    else
+        triples_box_kernel<2><<<grid, kThreads, 0, s>>>(a);
     return hipGetLastError();
 }
 

@@ -634,8 +634,7 @@ int sipgpu_permute_rhs_to_lhs(int lrank, const int *lhs_ids, const int *rhs_ids,
  * box slots [box0, box0 + nbox) (all `slots` slots cover the whole sum; boxes
  * that differ by a permutation of the pairs (a,i), (b,j), (c,k) have one
  * energy, and those of a call are computed once for all their slots), in
- * one kernel launch per SIPGPU_TRIPLES_LAUNCH_BOXES slots (a launch of
- * 512-thread workgroups holds fewer than 2^32 work-items; 2^21 slots of
+ * one kernel launch per SIPGPU_TRIPLES_LAUNCH_BOXES slots (2^21 slots of
  * o = 30, v = 240 run ~0.3 s on one MI355X);
  * sipgpu_triples_energy adds factor * (sum of all partials, in slot order)
  * to *out (a device double).  sipgpu_triples_tuple computes one tuple's
