@@ -166,18 +166,10 @@ void gemm_f64_kernel(GemmArgs args) {
     double vb[TileLoader<BN, NT, kBK>::kItems];
 
     for (int t = blockIdx.x; t < args.ntiles; t += gridDim.x) {
-        // a single contraction split along K: segment ks of the tile
-        const bool split = !args.tiles && args.ksplit > 1;
-        const int ks = split ? t / (args.ntiles / args.ksplit) : 0;
-        const int tt = t - ks * (split ? args.ntiles / args.ksplit : 0);
         const GemmTile tile = args.tiles ? args.tiles[t]
-                                         : GemmTile{0, tt % args.tilesM, tt / args.tilesM, 0};
+                                         : GemmTile{0, t % args.tilesM, t / args.tilesM, 0};
         if (tile.task < 0) continue; // padding slot of the XCD schedule
-        GemmTask task = args.tiles ? args.tasks[tile.task] : args.task0;
-        if (ks > 0) {
-            task.D = args.ws + (ks - 1) * args.ws_stride;
-            task.beta = 0;
-        }
+        const GemmTask task = args.tiles ? args.tasks[tile.task] : args.task0;
         const int m0 = tile.mt * BM, n0 = tile.nt * BN;
         // rows / columns of this wave's sub-tile that lie inside the block
         const int mlive = __builtin_amdgcn_readfirstlane(task.M - (m0 + wm * TM));
@@ -190,13 +182,7 @@ void gemm_f64_kernel(GemmArgs args) {
             for (int j = 0; j < FN; ++j) acc[i][j] = f64x4{0.0, 0.0, 0.0, 0.0};
 
         for (int p = task.first; p < task.first + task.npairs; ++p) {
-            GemmPair pr = args.tiles ? args.pairs[p] : args.pair0;
-            if (split) { // this segment's k range: the tables from k0 on
-                const int k0 = ks * args.kseg;
-                pr.kL += k0;
-                pr.kR += k0;
-                pr.K = min(pr.K - k0, args.kseg);
-            }
+            const GemmPair pr = args.tiles ? args.pairs[p] : args.pair0;
             la.pair(pr.flags & 1, pr.L, args.tab + pr.kL, pr.K, args.tab + pr.mL, m0, task.M, tid);
             lb.pair(pr.flags & 2, pr.R, args.tab + pr.kR, pr.K, args.tab + pr.nR, n0, task.N, tid);
             la.lookup(0, tid);
@@ -682,6 +668,251 @@ __global__ __launch_bounds__(WM *WN * 64) void gemm_f64_lds_kernel(GemmArgs args
     }
 }
 
+// ---------------------------------------------------------------------------
+// Tiles of 32 x 32 whose K is split over the waves of a workgroup.
+//
+// A result block of a SIAL program is small (100 x 100 to a few hundred
+// squared), so a few blocks are a few 64 x 64 tiles, each a serial chain of K
+// stages on one CU while the others idle.  Here a tile is 32 x 32 and each of
+// the workgroup's eight waves sums its own contiguous eighth of the task's
+// k-steps (all its pairs, four k a step) straight from global memory into
+// registers: no LDS staging, no barrier in the loop.  The eight partial tiles
+// are added through LDS in wave order at the end.  The split depends on the
+// task alone, so a block's bits do not depend on its batch.
+//
+// What bounds it: for few tiles the latency of a wave's chain (tables, loads,
+// MFMAs of its eighth), for many the cache lines its gathers touch.  107
+// registers keep two workgroups on a CU; stages of four k-steps need 197 and
+// ran 10-30% slower.  256 pairs of 100^3 into 16 blocks: 169 us in 64 x 64
+// tiles, 27 here; one 100^3 product 13.2 -> 5.9 us, one 450^3 22 + 4 -> 14.
+//
+// Per wave, a stage is two k-steps: its eight loads are in flight while the
+// previous stage's MFMAs run, also across pairs.  A lane holds the k offsets
+// of 64 k of its pair (one load) and hands them out by lane permutes.
+
+constexpr int kSplitWaves = 8;
+constexpr int kSplitSteps = 2; // k-steps (of 4 k) per stage
+
+template <int MB, int NB>
+struct SplitTile {
+    // One operand pair: where its elements are, and the k range [k, ke).
+    struct Pair {
+        gptr_t L, R;
+        gitab_t kL, kR;
+        int mo[MB], no[NB]; // this lane's row and column offsets
+        int kA, kB;         // k offsets of k = chunk + lane
+        int chunk, k, ke, K;
+    };
+    struct Stage {
+        double a[kSplitSteps][MB], b[kSplitSteps][NB];
+    };
+
+    const GemmArgs &args;
+    const GemmTask &task;
+    const GemmPair &pair0; // of a single contraction
+    int m0, n0, lane, li, lk;
+    f64x4 acc[MB][NB];
+
+    __device__ SplitTile(const GemmArgs &a, const GemmTask &t, const GemmPair &p0, int m0_, int n0_)
+        : args(a), task(t), pair0(p0), m0(m0_), n0(n0_), lane(threadIdx.x & 63), li(lane & 15),
+          lk(lane >> 4) {
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j) acc[i][j] = f64x4{0.0, 0.0, 0.0, 0.0};
+    }
+
+    // Steps [first, last) of the task that lie in pair pr.
+    __device__ Pair pair(const GemmPair &pr, int first, int last) const {
+        Pair q;
+        q.L = (gptr_t)pr.L;
+        q.R = (gptr_t)pr.R;
+        q.kL = (gitab_t)(args.tab + pr.kL);
+        q.kR = (gitab_t)(args.tab + pr.kR);
+        gitab_t mt = (gitab_t)(args.tab + pr.mL), nt = (gitab_t)(args.tab + pr.nR);
+#pragma unroll
+        for (int i = 0; i < MB; ++i) q.mo[i] = mt[min(m0 + i * 16 + li, task.M - 1)];
+#pragma unroll
+        for (int j = 0; j < NB; ++j) q.no[j] = nt[min(n0 + j * 16 + li, task.N - 1)];
+        q.K = pr.K;
+        q.k = max(0, first - pr.s0) * 4;
+        q.ke = min(pr.K, (last - pr.s0) * 4);
+        lookup(q);
+        return q;
+    }
+    // The k offsets of the 64 k from q.k on, clamped into the pair.
+    __device__ void lookup(Pair &q) const {
+        q.chunk = q.k;
+        const int k = min(q.k + lane, q.K - 1);
+        q.kA = q.kL[k];
+        q.kB = q.kR[k];
+    }
+    // Issues the loads of the stage at q.k (past the pair's K: its last k).
+    __device__ void issue(const Pair &q, Stage &s) const {
+#pragma unroll
+        for (int u = 0; u < kSplitSteps; ++u) {
+            const int from = (q.k - q.chunk) + 4 * u + lk;
+            const int oa = __shfl(q.kA, from), ob = __shfl(q.kB, from);
+#pragma unroll
+            for (int i = 0; i < MB; ++i) s.a[u][i] = q.L[oa + q.mo[i]];
+#pragma unroll
+            for (int j = 0; j < NB; ++j) s.b[u][j] = q.R[ob + q.no[j]];
+        }
+    }
+    // Multiplies a stage of which `left` k remain in the pair's range.
+    __device__ void mma(Stage &s, int left) {
+        if (left < 4 * kSplitSteps) {
+#pragma unroll
+            for (int u = 0; u < kSplitSteps; ++u) {
+                if (4 * u + lk < left) continue;
+#pragma unroll
+                for (int i = 0; i < MB; ++i) s.a[u][i] = 0.0;
+#pragma unroll
+                for (int j = 0; j < NB; ++j) s.b[u][j] = 0.0;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kSplitSteps; ++u) {
+            if (4 * u >= left) break;
+#pragma unroll
+            for (int i = 0; i < MB; ++i)
+#pragma unroll
+                for (int j = 0; j < NB; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(s.a[u][i], s.b[u][j],
+                                                                     acc[i][j], 0, 0, 0);
+        }
+    }
+
+    // Steps [first, last) of the task, which begin in pair p.
+    __device__ void run(int p, int first, int last) {
+        auto record = [&](int at) { return args.tiles ? args.pairs[at] : pair0; };
+        const int end = task.first + task.npairs;
+        Pair cur = pair(record(p), first, last);
+        Stage now, ahead;
+        issue(cur, now);
+        while (true) {
+            // the next pair, if this wave's range reaches it
+            Pair next = cur;
+            bool more = false;
+            if (p + 1 < end) {
+                const GemmPair pr = record(p + 1);
+                more = pr.s0 < last;
+                if (more) next = pair(pr, first, last);
+            }
+            while (true) {
+                const int left = cur.ke - cur.k;
+                const bool inside = left > 4 * kSplitSteps;
+                if (inside) {
+                    cur.k += 4 * kSplitSteps;
+                    if (cur.k - cur.chunk == 64) lookup(cur);
+                    issue(cur, ahead);
+                } else if (more) {
+                    issue(next, ahead);
+                }
+                mma(now, left);
+                now = ahead;
+                if (!inside) break;
+            }
+            if (!more) break;
+            cur = next;
+            ++p;
+        }
+    }
+};
+
+template <int MB, int NB>
+__device__ __forceinline__ void split_tile(const GemmArgs &args, const GemmTask &task,
+                                           const GemmPair &pair0, int m0, int n0, int p, int first,
+                                           int last, double *part) {
+    SplitTile<MB, NB> t(args, task, pair0, m0, n0);
+    if (first < last) t.run(p, first, last);
+    // this wave's partial tile, block by block in accumulator order
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                part[((wave * 4 + i * 2 + j) * 4 + r) * 64 + lane] = t.acc[i][j][r];
+}
+
+__global__ __launch_bounds__(kSplitWaves * 64) void gemm_f64_ksplit_kernel(GemmArgs args) {
+    __shared__ double part[kSplitWaves * 32 * 32];
+    // a single contraction in K segments: segment seg of the tile
+    const bool segments = !args.tiles && args.ksplit > 1;
+    const int per = segments ? args.ntiles / args.ksplit : 0;
+    const int seg = segments ? (int)blockIdx.x / per : 0, t = (int)blockIdx.x - seg * per;
+    const GemmTile tile =
+        args.tiles ? args.tiles[t] : GemmTile{0, t % args.tilesM, t / args.tilesM, 0};
+    if (tile.task < 0) return; // padding slot of the XCD schedule
+    GemmTask task = args.tiles ? args.tasks[tile.task] : args.task0;
+    GemmPair pair0 = args.pair0;
+    if (segments) {
+        const int k0 = seg * args.kseg;
+        pair0.kL += k0;
+        pair0.kR += k0;
+        pair0.K = min(pair0.K - k0, args.kseg);
+        if (seg > 0) {
+            task.D = args.ws + (seg - 1) * args.ws_stride;
+            task.beta = 0;
+        }
+    }
+    const int m0 = tile.mt * 32, n0 = tile.nt * 32;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+
+    // this wave's steps of the task, and the pair they begin in
+    int base = 0, steps = 0;
+    if (task.npairs > 0) {
+        const GemmPair tail = args.tiles ? args.pairs[task.first + task.npairs - 1] : pair0;
+        base = args.tiles ? args.pairs[task.first].s0 : 0;
+        steps = tail.s0 + (tail.K + 3) / 4 - base;
+    }
+    const int first = base + (int)((long long)steps * wave / kSplitWaves);
+    const int last = base + (int)((long long)steps * (wave + 1) / kSplitWaves);
+    int p = task.first;
+    if (args.tiles)
+        for (int q = 0; q < task.npairs; q += 64) { // pairs that begin at or before `first`
+            const int at = q + lane;
+            const bool before = at < task.npairs && args.pairs[task.first + at].s0 <= first;
+            const int n = __popcll(__ballot(before));
+            if (n == 0) break;
+            p = task.first + q + n - 1;
+            if (n < 64) break;
+        }
+
+    const bool m2 = m0 + 16 < task.M, n2 = n0 + 16 < task.N;
+    if (m2 && n2)
+        split_tile<2, 2>(args, task, pair0, m0, n0, p, first, last, part);
+    else if (m2)
+        split_tile<2, 1>(args, task, pair0, m0, n0, p, first, last, part);
+    else if (n2)
+        split_tile<1, 2>(args, task, pair0, m0, n0, p, first, last, part);
+    else
+        split_tile<1, 1>(args, task, pair0, m0, n0, p, first, last, part);
+    __syncthreads();
+
+    // sum the waves' partial tiles in order and scatter them
+    gitab_t mtab = (gitab_t)(args.tab + task.mD);
+    gitab_t ntab = (gitab_t)(args.tab + task.nD);
+    __attribute__((address_space(1))) double *D =
+        (__attribute__((address_space(1))) double *)task.D;
+#pragma unroll
+    for (int h = 0; h < 1024 / (kSplitWaves * 64); ++h) {
+        const int e = h * (kSplitWaves * 64) + threadIdx.x;
+        const int block = e >> 8, r = (e >> 6) & 3;
+        const int m = m0 + (block >> 1) * 16 + 4 * r + (lane >> 4);
+        const int n = n0 + (block & 1) * 16 + (lane & 15);
+        if (m >= task.M || n >= task.N) continue;
+        double v = part[e];
+#pragma unroll
+        for (int w = 1; w < kSplitWaves; ++w) v += part[w * 1024 + e];
+        const int off = mtab[m] + ntab[n];
+        if (task.beta) v += D[off];
+        D[off] = v;
+    }
+}
+
 __global__ void scale_scatter_kernel(double *D, const int32_t *moffD, const double *X,
                                      const int32_t *moffX, const double *s, int M) {
     // tensor_block_add_ on a zeroed destination (tensor_dil_omp.F90:394-436):
@@ -756,6 +987,7 @@ constexpr CfgShape kCfg[kGemmConfigs] = {
     {128, 128}, {128, 128}, {128, 64}, {64, 64},
     {64, 64}, {128, 64}, {128, 128},
     {64, 64}, {128, 64}, {128, 128}, {64, 128},
+    {32, 32},
 };
 
 } // namespace
@@ -784,6 +1016,9 @@ hipError_t launch_gemm(int cfg, const GemmArgs &args, int grid, hipStream_t stre
     case 15: return launch_lds<128, 64, 2, 2, 16>(args, grid, stream);
     case 16: return launch_lds<128, 128, 2, 2, 16>(args, grid, stream);
     case 17: return launch_lds<64, 128, 2, 2, 16>(args, grid, stream);
+    case kGemmSplitK:
+        gemm_f64_ksplit_kernel<<<grid, kSplitWaves * 64, 0, stream>>>(args);
+        return hipGetLastError();
     default: return hipErrorInvalidValue;
     }
 }

@@ -48,6 +48,13 @@ struct BatchImage {
     std::vector<unsigned char> host;
     size_t o_tiles = 0, o_tasks = 0, o_pairs = 0, o_tab = 0, o_parts = 0;
     int cfg = 0, ntiles = 0, ntasks = 0, npairs = 0, real_tiles = 0;
+    // One GEMM launch per tile configuration: tiles [first, first + count).
+    struct Launch {
+        int cfg, first, count;
+    };
+    static constexpr int kMaxLaunches = 2;
+    Launch launch[kMaxLaunches] = {};
+    int nlaunches = 0;
     // Result blocks cut into pair groups (a small batch): the GEMM tasks of
     // groups after the first write workspace copies of their block, at
     // ws_off[i] doubles for task ws_task[i]; nparts entries at o_parts add
@@ -75,6 +82,18 @@ struct BatchImage {
         return a;
     }
 };
+
+// The GEMM launches of a batch image whose tiles stand at args.tiles.
+inline hipError_t launch_batch_gemm(GemmArgs args, const BatchImage::Launch *l, int n,
+                                    hipStream_t s) {
+    const GemmTile *tiles = args.tiles;
+    for (int i = 0; i < n; ++i) {
+        args.tiles = tiles + l[i].first;
+        args.ntiles = l[i].count;
+        if (hipError_t e = launch_gemm(l[i].cfg, args, l[i].count, s)) return e;
+    }
+    return hipSuccess;
+}
 
 // Plans a list of block contractions (same rules as sipgpu_batch_plan) for
 // the table kernel; cfg >= 0 pins its tile configuration.  split_cus > 0:

@@ -52,6 +52,7 @@ struct GemmPair {
     int K;
     int kL, mL, kR, nR;           // offsets of koffL, moffL, koffR, noffR
     int flags;                    // bit0: L k-fast, bit1: R k-fast
+    int s0;                       // k-steps (of 4 k) of the task's earlier pairs
 };
 
 // One destination block: D(m, n) at D[moffD[m] + noffD[n]].
@@ -80,7 +81,7 @@ struct GemmArgs {
     int tilesM;
     GemmTask task0;
     GemmPair pair0;
-    // single contraction split along K (ksplit > 1, 64 x 64 kernel only):
+    // single contraction in K segments (ksplit > 1, split-K tiles only):
     // tile t computes segment s = t / (ntiles / ksplit) of kseg k values;
     // segment 0 goes to task0.D, segment s > 0 is assigned to ws + (s - 1) *
     // ws_stride with task0's destination tables
@@ -98,7 +99,9 @@ struct GemmArgs {
 //   11: 64x64 (4)     12: 128x64 (2)      13: 128x128 (2)
 // direct-to-LDS kernel (2x2 waves, BK 16):
 //   14: 64x64  15: 128x64  16: 128x128  17: 64x128
-enum GemmConfig { kGemm64x64 = 0, kGemm128x128 = 1, kGemm64x128 = 2, kGemmConfigs = 18 };
+// K split over the waves of a workgroup (eight waves):
+//   18: 32x32
+enum GemmConfig { kGemm64x64 = 0, kGemm128x128 = 1, kGemm64x128 = 2, kGemmSplitK = 18, kGemmConfigs = 19 };
 int gemm_tile_m(int cfg);
 int gemm_tile_n(int cfg);
 hipError_t launch_gemm(int cfg, const GemmArgs &args, int grid, hipStream_t stream);

@@ -223,26 +223,36 @@ void make_task_pair(const ContractionShape &s, int kL, int mL, int kR, int nR, i
     const int fl = (s.l_kfast ? 1 : 0) | (s.r_kfast ? 2 : 0);
     if (!s.swap) {
         task = GemmTask{d, (int)s.M, (int)s.N, mD, nD, 0, 0, beta, 0};
-        pair = GemmPair{l, r, (int)s.K, kL, mL, kR, nR, fl};
+        pair = GemmPair{l, r, (int)s.K, kL, mL, kR, nR, fl, 0};
     } else {
         task = GemmTask{d, (int)s.N, (int)s.M, nD, mD, 0, 0, beta, 0};
-        pair = GemmPair{r, l, (int)s.K, kR, nR, kL, mL, ((fl & 1) << 1) | ((fl & 2) >> 1)};
+        pair = GemmPair{r, l, (int)s.K, kR, nR, kL, mL, ((fl & 1) << 1) | ((fl & 2) >> 1), 0};
     }
 }
 
-int pick_config(int64_t M, int64_t N) {
+// A single contraction of at most so many 32 x 32 tiles and at least so long
+// a K runs in K segments.
+constexpr int64_t kSegmentTiles = 128, kSegmentK = 768;
+
+// Tile configuration for an M x N block; `kfast`: GemmPair::flags of its
+// first pair.
+int pick_config(int64_t M, int64_t N, int kfast) {
     // SIPGPU_GEMM_CONFIG=<n> pins the tile configuration (tuning runs).
     static const int forced = [] {
         const char *e = std::getenv("SIPGPU_GEMM_CONFIG");
         return e ? std::atoi(e) : -1;
     }();
     if (forced >= 0 && forced < kGemmConfigs) return forced;
-    // Config 0 (64x64 tile, four waves of 32x32, no occupancy hint) measured
-    // fastest on every block shape of the benchmark terms; the larger tiles
-    // fit fewer workgroups per CU.
-    (void)M;
-    (void)N;
-    return kGemm64x64;
+    // By the block alone, so that its bits do not depend on its batch.  The
+    // 32 x 32 tiles with K split over the waves win until the 64 x 64 tiles
+    // fill the chip about twice over, or earlier where both operands are read
+    // along k (a wave's load then touches 16 cache lines instead of 4).
+    // Single contractions, 64 x 64 against split K: 375 tiles (1600 x 900 x
+    // 1600) 205 against 182 us, 361 (1200^3) 153 against 115, 1000 (2304 x
+    // 1600 x 2304) 430 against 618; both along k, 105 tiles (900 x 441 x 1089)
+    // 101 against 52, 361 140 against 211.
+    const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64);
+    return tiles <= ((kfast & 3) == 3 ? 160 : 512) ? kGemmSplitK : kGemm64x64;
 }
 
 // One contraction on device pointers (no locking; caller holds the lock).
@@ -262,7 +272,7 @@ int contract_device(Context &c, sipgpu_stream_s &st, const int *ptrn, const doub
         GemmPair pair;
         make_task_pair(s, ds->kL, ds->mL, ds->kR, ds->nR, ds->mD, ds->nD, l, r, d,
                        accumulate ? 1 : 0, task, pair);
-        const int cfg = pick_config(task.M, task.N);
+        const int cfg = pick_config(task.M, task.N, pair.flags);
         const int bm = gemm_tile_m(cfg), bn = gemm_tile_n(cfg);
         GemmArgs a{};
         a.tab = tab;
@@ -274,19 +284,21 @@ int contract_device(Context &c, sipgpu_stream_s &st, const int *ptrn, const doub
         task.npairs = 1;
         a.task0 = task;
         a.pair0 = pair;
-        // Too few tiles to fill the CUs and a long K: split K into segments
-        // that run side by side, segment s > 0 into the stream's workspace,
-        // then add the segments to D in order (a fixed summation order).
-        // Up to 8 segments of at least 64 k, two workgroups per CU (a ring
-        // block pair: p50 47.6 -> 44.5 us against 4 segments of 128, one per
-        // CU), and no more than the 16 MiB of the no-allocation workspace
-        // holds, so both entry points split every shape the same way.
+        // Few tiles and a long K: split K into segments that run side by
+        // side, segment s > 0 into the stream's workspace, then add the
+        // segments to D in order (a fixed summation order).  Up to 8 segments
+        // of at least 256 k, a workgroup per CU, and no more than the 16 MiB
+        // of the no-allocation workspace holds, so both entry points split
+        // every shape the same way.  The summing pass and its launch cost
+        // about 6 us, a workgroup about 27 ns per k: 225 x 225 x 2000 (64
+        // tiles) 58 us in one segment, 20 + 4 in four; 200 x 200 x 4000 112
+        // and 28 + 4.
         const int64_t K = pair.K;
         int nseg = 1, kseg = (int)K;
-        if (cfg == kGemm64x64 && ntiles * 2 <= g_device_cus && K >= 256) {
+        if (cfg == kGemmSplitK && ntiles <= kSegmentTiles && K >= kSegmentK) {
             const int64_t fit = 1 + (int64_t)(kNoAllocWsDoubles / std::max<int64_t>(s.dsize, 1));
             const int want = (int)std::max<int64_t>(
-                1, std::min<int64_t>({8, 2 * g_device_cus / ntiles, K / 64, fit}));
+                1, std::min<int64_t>({8, g_device_cus / ntiles, K / 256, fit}));
             kseg = (int)(((K + want - 1) / want + 15) / 16 * 16);
             nseg = (int)((K + kseg - 1) / kseg);
         }
@@ -377,8 +389,10 @@ using sipgpu::rt::SplitData;
 using sipgpu::rt::PanelPlan;
 
 struct sipgpu_batch_s {
-    int cfg = kGemm64x64;
+    int cfg = kGemm64x64; // of all blocks (-1: by block)
     int ntiles = 0;     // including XCD padding slots
+    sipgpu::rt::BatchImage::Launch launch[sipgpu::rt::BatchImage::kMaxLaunches] = {};
+    int nlaunches = 0;
     int ntasks = 0, npairs = 0, real_tiles = 0;
     int ngroups = 0;    // panel paths: GEMM tasks after merging result blocks
     double flops = 0.0;
@@ -742,7 +756,6 @@ int sipgpu::rt::build_batch_image(const sipgpu_contraction *list, int n, BatchIm
     std::vector<GemmTask> tasks;
     std::vector<GemmPair> pairs;
     std::vector<double> task_cost;
-    int64_t maxM = 0, maxN = 0, sumM = 0, sumN = 0;
     b.flops = 0.0;
     for (const double *dp : dest_order) {
         const auto &idx = by_dest[dp];
@@ -758,6 +771,7 @@ int sipgpu::rt::build_batch_image(const sipgpu_contraction *list, int n, BatchIm
                        const_cast<double *>(dp), beta, task, unused);
         task.first = (int)pairs.size();
         double cost = 0.0;
+        int steps = 0;
         for (size_t j = start; j < idx.size(); ++j) {
             const int i = idx[j];
             const ContractionShape &s = *shapes[shape_of[i]];
@@ -769,22 +783,25 @@ int sipgpu::rt::build_batch_image(const sipgpu_contraction *list, int n, BatchIm
             GemmPair pr;
             make_task_pair(s, t[0], t[1], t[2], t[3], t[4], t[5], list[i].l, list[i].r,
                            const_cast<double *>(dp), beta, tk, pr);
-            pairs.push_back(pr);
+            pr.s0 = steps;
+            steps += (pr.K + 3) / 4;
+            if (pr.K > 0) pairs.push_back(pr); // an empty product adds nothing
             cost += 2.0 * (double)s.M * (double)s.N * (double)s.K;
         }
         task.npairs = (int)pairs.size() - task.first;
         b.flops += cost;
         tasks.push_back(task);
         task_cost.push_back(cost);
-        maxM = std::max<int64_t>(maxM, task.M);
-        maxN = std::max<int64_t>(maxN, task.N);
-        sumM += task.M;
-        sumN += task.N;
     }
     const int nblocks = (int)tasks.size();
-    b.cfg = cfg >= 0 && cfg < kGemmConfigs
-                ? cfg
-                : pick_config(nblocks ? sumM / nblocks : 0, nblocks ? sumN / nblocks : 0);
+    // one configuration for all blocks where it is given (or pair groups are
+    // asked for), else each block's own: the split-K tiles and, launched
+    // beside them, 64 x 64 tiles for large blocks
+    const bool own = !(cfg >= 0 && cfg < kGemmConfigs) && split_cus <= 0;
+    b.cfg = cfg >= 0 && cfg < kGemmConfigs ? cfg : own ? kGemmSplitK : kGemm64x64;
+    auto cfg_of = [&](const GemmTask &t) {
+        return own ? pick_config(t.M, t.N, t.npairs ? pairs[t.first].flags : 0) : b.cfg;
+    };
     const int bm = gemm_tile_m(b.cfg), bn = gemm_tile_n(b.cfg);
 
     // Too few tiles to fill the CUs: each result block's pairs are cut into
@@ -834,14 +851,32 @@ int sipgpu::rt::build_batch_image(const sipgpu_contraction *list, int n, BatchIm
     }
     const int ntasks = (int)tasks.size();
 
-    std::vector<int> tms(ntasks), tns(ntasks);
-    for (int t = 0; t < ntasks; ++t) {
-        tms[t] = (tasks[t].M + bm - 1) / bm;
-        tns[t] = (tasks[t].N + bn - 1) / bn;
+    // launch `l`: the tiles of the blocks with configuration cfgs[l]
+    std::vector<int> cfgs;
+    for (int t = 0; t < ntasks; ++t)
+        if (std::find(cfgs.begin(), cfgs.end(), cfg_of(tasks[t])) == cfgs.end())
+            cfgs.push_back(cfg_of(tasks[t]));
+    if (cfgs.empty()) cfgs.push_back(b.cfg);
+    std::sort(cfgs.rbegin(), cfgs.rend());
+    std::vector<GemmTile> tiles;
+    b.nlaunches = 0;
+    b.real_tiles = 0;
+    for (int c : cfgs) {
+        std::vector<int> tms(ntasks, 0), tns(ntasks, 0);
+        for (int t = 0; t < ntasks; ++t) {
+            if (cfg_of(tasks[t]) != c) continue;
+            tms[t] = (tasks[t].M + gemm_tile_m(c) - 1) / gemm_tile_m(c);
+            tns[t] = (tasks[t].N + gemm_tile_n(c) - 1) / gemm_tile_n(c);
+        }
+        int real = 0;
+        const auto part = xcd_schedule<GemmTile>(tms, tns, task_cost, real);
+        if (b.nlaunches >= BatchImage::kMaxLaunches)
+            return fail(SIPGPU_EARG, "batch: too many tile configurations");
+        b.launch[b.nlaunches++] = {c, (int)tiles.size(), (int)part.size()};
+        b.real_tiles += real;
+        tiles.insert(tiles.end(), part.begin(), part.end());
     }
-    int real_tiles = 0;
-    const std::vector<GemmTile> tiles = xcd_schedule<GemmTile>(tms, tns, task_cost, real_tiles);
-    b.real_tiles = real_tiles;
+    b.cfg = cfgs.size() == 1 ? cfgs[0] : -1;
 
     // Upload: tiles | tasks | pairs | tables | parts, each 256-byte aligned.
     auto align = [](size_t v) { return (v + 255) & ~(size_t)255; };
@@ -868,8 +903,6 @@ int sipgpu::rt::build_batch_image(const sipgpu_contraction *list, int n, BatchIm
     b.ntiles = (int)tiles.size();
     b.ntasks = nblocks;
     b.npairs = (int)pairs.size();
-    (void)maxM;
-    (void)maxN;
     return 0;
 }
 
@@ -887,6 +920,8 @@ int plan_batch_locked(Context &, const sipgpu_contraction *list, int n, sipgpu_b
     HIP_TRY(hipMalloc(&b.dev, img.host.size()));
     HIP_TRY(hipMemcpy(b.dev, img.host.data(), img.host.size(), hipMemcpyHostToDevice));
     b.args = img.args_at(b.dev);
+    std::copy(img.launch, img.launch + img.nlaunches, b.launch);
+    b.nlaunches = img.nlaunches;
     b.parts = img.nparts ? reinterpret_cast<const AddPartsEntry *>(
                                static_cast<unsigned char *>(b.dev) + img.o_parts)
                          : nullptr;
@@ -1570,7 +1605,7 @@ int execute_batch(Context &c, sipgpu_batch_s &b, int stages, sipgpu_stream_t s) 
     const hipStream_t hs = resolve(c, s).s;
     if (b.split || b.packed) return sipgpu::rt::execute_panels(b.sd, b.split, stages, hs);
     if (stages & SIPGPU_STAGE_PRODUCT) {
-        HIP_TRY(launch_gemm(b.cfg, b.args, b.ntiles, hs));
+        HIP_TRY(sipgpu::rt::launch_batch_gemm(b.args, b.launch, b.nlaunches, hs));
         if (b.nparts) HIP_TRY(launch_add_parts(b.parts, b.nparts, b.parts_max_n, hs));
     }
     return 0;
@@ -1687,7 +1722,7 @@ int plan_default_locked(Context &c, const sipgpu_contraction *list, int n,
         if (!std::strcmp(e, "packed")) packed = b->ntasks > 0;
     }
     PlanChoice used = tab;
-    used.cfg = b->cfg;
+    used.cfg = b->cfg; // -1: by block
     if (packed) {
         PlanChoice pk;
         pk.path = 1;
@@ -2399,7 +2434,7 @@ int sipgpu_batch_tune(const sipgpu_contraction *list, int n, int nmoduli, sipgpu
     hipError_t he = hipMemset(scratch, 0, total * sizeof(double));
     std::vector<PlanChoice> cands;
     if (nmoduli == 0) {
-        for (int cfg : {0, 1, 2, 3, 5, 6, 11, 12, 14}) {
+        for (int cfg : {0, 1, 2, 3, 5, 6, 11, 12, 14, 18}) {
             PlanChoice ch;
             ch.path = 0;
             ch.cfg = cfg;

@@ -990,8 +990,8 @@ int server_batch(sipgpu_server_s &S, int lane, std::vector<Pending> &batch) {
             hipError_t e = hipMemcpyAsync(S.slot_dev[slot], S.slot_host[slot], img.host.size(),
                                           hipMemcpyHostToDevice, stream);
             if (e == hipSuccess)
-                e = sipgpu::launch_gemm(img.cfg, img.args_at(S.slot_dev[slot]), img.ntiles,
-                                        stream);
+                e = sipgpu::rt::launch_batch_gemm(img.args_at(S.slot_dev[slot]), img.launch,
+                                                  img.nlaunches, stream);
             if (e == hipSuccess) e = hipEventRecord(S.slot_free[slot], stream);
             if (e != hipSuccess) rc = hip_fail(e, "server: launch");
             S.slot_used[slot] = true;
