@@ -16,33 +16,38 @@ struct PermArgs {
     const double *in;
     double *out;
     int nU, nV;                   // tile-row dims (leading input dims), other dims
-    int extU[kPermMaxDims];       // extents of U dims (input order)
+    FastDiv extU[kPermMaxDims];   // extents of U dims (input order)
     int soutU[kPermMaxDims];      // their output strides
-    int extV[kPermMaxDims];       // extents of V dims (output order)
+    FastDiv extV[kPermMaxDims];   // extents of V dims (output order)
     int sinV[kPermMaxDims];       // their input strides
     int soutV[kPermMaxDims];      // their output strides
     int sizeU, sizeV;
     int TU, TV, pitch;            // tile extents and LDS row pitch
-    int tilesU;                   // tiles along U
+    int tilesU, tilesV;           // tiles along U and V
+    // Tile order: patches of patchU x (patch / patchU) tiles (U fastest inside),
+    // patchesU of them along U, dealt to the XCDs in turn from XCD `turn` on.
+    FastDiv patch, patchU, patchesU;
+    FastDiv round;                // 8 patches
+    int turn;
     int row_mode;                 // U is contiguous in the output as well
+    int stream;                   // store past the caches
 };
 
 struct PermutePlan;
 hipError_t launch_permute(const PermutePlan &plan, const double *in, double *out,
                           hipStream_t stream);
 // Batched permutes: fills args[0..n), the workgroup offsets first[0..n]
-// (first[n] the grid), the launch's LDS needs (largest staged tile in
-// doubles, largest tile v extent) and its elements per thread (8 or 16)
-// from the plans; returns the total workgroup count.
+// (first[n] the grid) and the launch's LDS needs (largest staged tile in
+// doubles, largest tile v extent) from the plans; returns the total workgroup
+// count.
 int64_t permute_batch_args(const PermutePlan *plans, const double *const *in,
                            double *const *out, int n, PermArgs *args, int *first,
-                           int *tile_cap, int *tv_cap, int *items);
+                           int *tile_cap, int *tv_cap);
 // One launch of `grid` workgroups over the device copies of args, first and
 // the per-workgroup entry table entry[0..grid) (entry[b] = the e with
 // first[e] <= b < first[e + 1]).
 hipError_t launch_permute_batch(const PermArgs *args, const int *first, const int *entry,
-                                int grid, int tile_cap, int tv_cap, int items,
-                                hipStream_t stream);
+                                int grid, int tile_cap, int tv_cap, hipStream_t stream);
 
 // ------------------------------------------------------------- contraction --
 // One operand pair of a task.  Table offsets index the plan's int32 pool.

@@ -28,9 +28,15 @@ namespace sipgpu {
 namespace {
 
 constexpr int kPermThreads = 256;
-constexpr int kPermMaxItems = 16;          // elements per thread (at most)
+// Tiles of at most 2048 elements, u at most 32 wide: on 2-D to 6-D transposes
+// (64^4 reversal, 40^4, 20^6, 120^3, 30^5) they beat 4096-element tiles on
+// every shape, since more workgroups per CU keep more loads in flight (64^4 6.3
+// against 4.7 TB/s).
+constexpr int kPermItems = 8;              // elements per thread (at most)
 constexpr int kPermMaxTV = 1024;
-constexpr int kPermMaxTU = 64;             // transpose mode only
+constexpr int kPermMaxTU = 32;             // transpose mode only
+constexpr int64_t kLargeElems = 1 << 25;   // input and output fill the 256 MB cache twice
+constexpr int kXcds = 8;                   // workgroup b runs on XCD b % 8
 
 // Dynamic LDS of a launch: the staged tile (tile_cap doubles; none in row
 // mode), then the tile's v input and output offsets (tv_cap ints each) and
@@ -40,16 +46,30 @@ __host__ __device__ constexpr size_t perm_lds_bytes(int tile_cap, int tv_cap) {
     return (size_t)tile_cap * sizeof(double) + (size_t)(2 * tv_cap + kPermMaxTU) * sizeof(int);
 }
 
-// Tile `blk` of the permute `a` (at most ITEMS * kPermThreads elements),
-// staged through the workgroup's LDS.
-template <int ITEMS>
+template <bool STREAM>
+__device__ __forceinline__ void put(double v, double *p) {
+    if (STREAM)
+        __builtin_nontemporal_store(v, p);
+    else
+        *p = v;
+}
+
+// Tile of workgroup `blk` of the permute `a` (at most kPermItems * kPermThreads
+// elements), staged through the workgroup's LDS.
+template <bool STREAM>
 __device__ __forceinline__ void permute_tile(const PermArgs &a, int blk, double *lds,
                                              int tile_cap, int tv_cap) {
     double *tile = lds;
     int *sh_inV = reinterpret_cast<int *>(lds + tile_cap);
     int *sh_outV = sh_inV + tv_cap, *sh_outU = sh_outV + tv_cap;
-    const int bu = blk % a.tilesU;
-    const int bv = blk / a.tilesU;
+    // the patch (workgroups of one XCD) and the tile in it
+    const int r = (int)fastdiv(blk, a.round), q = blk - r * (int)a.round.d;
+    const int at = r * kXcds + ((q - a.turn) & (kXcds - 1)), in_patch = q >> 3;
+    const int pv = (int)fastdiv(at, a.patchesU), pu = at - pv * (int)a.patchesU.d;
+    const int iv = (int)fastdiv(in_patch, a.patchU), iu = in_patch - iv * (int)a.patchU.d;
+    const int bu = pu * (int)a.patchU.d + iu;
+    const int bv = pv * (int)fastdiv(a.patch.d, a.patchU) + iv;
+    if (bu >= a.tilesU || bv >= a.tilesV) return;
     const int u0 = bu * a.TU, v0 = bv * a.TV;
     const int tu = min(a.TU, a.sizeU - u0);
     const int tv = min(a.TV, a.sizeV - v0);
@@ -59,9 +79,8 @@ __device__ __forceinline__ void permute_tile(const PermArgs &a, int blk, double 
     for (int i = tid; i < tv; i += kPermThreads) {
         int v = v0 + i, oin = 0, oout = 0;
         for (int d = 0; d < a.nV; ++d) {
-            const int e = a.extV[d];
-            const int q = v / e;
-            const int r = v - q * e;
+            const int q = (int)fastdiv(v, a.extV[d]);
+            const int r = v - q * (int)a.extV[d].d;
             oin += r * a.sinV[d];
             oout += r * a.soutV[d];
             v = q;
@@ -73,9 +92,8 @@ __device__ __forceinline__ void permute_tile(const PermArgs &a, int blk, double 
         for (int i = tid; i < tu; i += kPermThreads) {
             int u = u0 + i, oout = 0;
             for (int d = 0; d < a.nU; ++d) {
-                const int e = a.extU[d];
-                const int q = u / e;
-                oout += (u - q * e) * a.soutU[d];
+                const int q = (int)fastdiv(u, a.extU[d]);
+                oout += (u - q * (int)a.extU[d].d) * a.soutU[d];
                 u = q;
             }
             sh_outU[i] = oout;
@@ -86,7 +104,7 @@ __device__ __forceinline__ void permute_tile(const PermArgs &a, int blk, double 
     const int n = tu * tv;
     const double *__restrict__ in = a.in;
     double *__restrict__ out = a.out;
-    double val[ITEMS];
+    double val[kPermItems];
     // Element e = tid + i * kPermThreads of the tile, as (v, u) = (e / tu,
     // e % tu) or (u, v) = (e / tv, e % tv): one division per thread, then
     // the stride kPermThreads is added in mixed radix (no division per item).
@@ -96,7 +114,7 @@ __device__ __forceinline__ void permute_tile(const PermArgs &a, int blk, double 
         // u is contiguous in both the input and the output.
         int vv = vu0, uu = uu0;
 #pragma unroll
-        for (int i = 0; i < ITEMS; ++i) {
+        for (int i = 0; i < kPermItems; ++i) {
             if (tid + i * kPermThreads < n) val[i] = in[u0 + uu + sh_inV[vv]];
             uu += ru;
             vv += qu;
@@ -105,9 +123,9 @@ __device__ __forceinline__ void permute_tile(const PermArgs &a, int blk, double 
         vv = vu0;
         uu = uu0;
 #pragma unroll
-        for (int i = 0; i < ITEMS; ++i) {
+        for (int i = 0; i < kPermItems; ++i) {
             if (tid + i * kPermThreads < n)
-                __builtin_nontemporal_store(val[i], &out[u0 + uu + sh_outV[vv]]);
+                put<STREAM>(val[i], &out[u0 + uu + sh_outV[vv]]);
             uu += ru;
             vv += qu;
             if (uu >= tu) { uu -= tu; ++vv; }
@@ -118,7 +136,7 @@ __device__ __forceinline__ void permute_tile(const PermArgs &a, int blk, double 
     {
         int vv = vu0, uu = uu0;
 #pragma unroll
-        for (int i = 0; i < ITEMS; ++i) {
+        for (int i = 0; i < kPermItems; ++i) {
             if (tid + i * kPermThreads < n) val[i] = in[u0 + uu + sh_inV[vv]];
             uu += ru;
             vv += qu;
@@ -127,7 +145,7 @@ __device__ __forceinline__ void permute_tile(const PermArgs &a, int blk, double 
         vv = vu0;
         uu = uu0;
 #pragma unroll
-        for (int i = 0; i < ITEMS; ++i) {
+        for (int i = 0; i < kPermItems; ++i) {
             if (tid + i * kPermThreads < n) tile[vv * pitch + uu] = val[i];
             uu += ru;
             vv += qu;
@@ -139,7 +157,7 @@ __device__ __forceinline__ void permute_tile(const PermArgs &a, int blk, double 
     const int uv0 = tid / tv, vv0 = tid - uv0 * tv;
     int uu = uv0, vv = vv0;
 #pragma unroll
-    for (int i = 0; i < ITEMS; ++i) {
+    for (int i = 0; i < kPermItems; ++i) {
         if (tid + i * kPermThreads < n) val[i] = tile[vv * pitch + uu];
         vv += rv;
         uu += qv;
@@ -148,35 +166,39 @@ __device__ __forceinline__ void permute_tile(const PermArgs &a, int blk, double 
     uu = uv0;
     vv = vv0;
 #pragma unroll
-    for (int i = 0; i < ITEMS; ++i) {
+    for (int i = 0; i < kPermItems; ++i) {
         if (tid + i * kPermThreads < n)
-            __builtin_nontemporal_store(val[i], &out[sh_outU[uu] + sh_outV[vv]]);
+            put<STREAM>(val[i], &out[sh_outU[uu] + sh_outV[vv]]);
         vv += rv;
         uu += qv;
         if (vv >= tv) { vv -= tv; ++uu; }
     }
 }
 
-template <int ITEMS>
+template <bool STREAM>
 __global__ __launch_bounds__(kPermThreads) void permute_kernel(PermArgs a, int tile_cap,
                                                                int tv_cap) {
     extern __shared__ double perm_lds[];
-    permute_tile<ITEMS>(a, blockIdx.x, perm_lds, tile_cap, tv_cap);
+    permute_tile<STREAM>(a, blockIdx.x, perm_lds, tile_cap, tv_cap);
 }
 
 // Many permutes in one launch: workgroup b runs tile b - first[e] of entry
 // e = entry[b] (a table of one int per workgroup, so a workgroup's set-up is
-// two dependent loads, not a search).
-template <int ITEMS>
-__global__ __launch_bounds__(kPermThreads) void permute_batch_kernel(const PermArgs *args,
-                                                                     const int *first,
-                                                                     const int *entry,
-                                                                     int tile_cap, int tv_cap) {
+// two dependent loads, not a search).  The entry's arguments are read where
+// they are: a local copy, indexed at run time, would be kept in private
+// memory, 224 bytes a lane written and read per tile (144 blocks of 30 and 15,
+// (3,4,1,2), 20.25 M elements: 127 us so, 84 now, 76 in patches).
+__global__ __launch_bounds__(kPermThreads) void permute_batch_kernel(
+    const PermArgs *__restrict__ args, const int *__restrict__ first,
+    const int *__restrict__ entry, int tile_cap, int tv_cap) {
     extern __shared__ double perm_lds[];
     const int b = blockIdx.x;
     const int e = entry[b];
-    const PermArgs a = args[e];
-    permute_tile<ITEMS>(a, b - first[e], perm_lds, tile_cap, tv_cap);
+    const PermArgs &a = args[e];
+    if (a.stream)
+        permute_tile<true>(a, b - first[e], perm_lds, tile_cap, tv_cap);
+    else
+        permute_tile<false>(a, b - first[e], perm_lds, tile_cap, tv_cap);
 }
 
 // Tile extent for `size` elements with at most `cap` per tile: the count of
@@ -187,41 +209,74 @@ int even_tile(int64_t size, int64_t cap) {
     return (int)((size + n - 1) / n);
 }
 
-// Tile shape of one permute: elements per thread (8 or 16, so a tile holds
-// at most 2048 or 4096 elements) and the cap on the tile's u extent in
-// transpose mode.
-struct TileShape {
-    int items = kPermMaxItems;
-    int tu_cap = kPermMaxTU;
-};
+// Sets the tile order to patches of su x sv tiles; the workgroups of one
+// permute then number whole rounds of 8 patches.
+void patches(PermArgs &a, int su, int sv, int turn, int64_t &grid) {
+    const int64_t nu = (a.tilesU + su - 1) / su, nv = (a.tilesV + sv - 1) / sv;
+    a.patch = make_fastdiv((uint32_t)(su * sv));
+    a.patchU = make_fastdiv((uint32_t)su);
+    a.patchesU = make_fastdiv((uint32_t)nu);
+    a.round = make_fastdiv((uint32_t)(kXcds * su * sv));
+    a.turn = turn;
+    grid = (nu * nv + kXcds - 1) / kXcds * kXcds * su * sv;
+}
 
-// Measured on MI355X over 2-D to 6-D transposes (64^4 reversal, 40^4,
-// 20^6, 120^3, 30^5): for a single launch, tiles of 2048 elements with u at
-// most 32 wide beat 4096-element tiles on every shape (more workgroups per
-// CU keep more loads in flight: 64^4 6.3 against 4.7 TB/s).  In a batched
-// launch a workgroup first loads its entry and the entry's arguments from
-// memory (two dependent loads that a single launch has in its kernel
-// arguments), and the larger tiles amortise that: 144 ring blocks of up to
-// 450 x 450 run at 3.0 TB/s with 4096-element tiles, 1.9 with 2048.
-TileShape tile_shape(const PermutePlan &p, bool batched) {
-    (void)p;
-    TileShape t;
-    t.items = batched ? 16 : 8;
-    t.tu_cap = batched ? 64 : 32;
-    return t;
+// True if every row of every tile, read and written, is whole cache lines.
+bool whole_lines(const PermArgs &a) {
+    constexpr int kLine = 16; // doubles
+    bool ok = !a.row_mode && a.TU % kLine == 0 && a.TV % kLine == 0 && a.sizeU % kLine == 0 &&
+              a.sizeV % kLine == 0 &&
+              ((reinterpret_cast<uintptr_t>(a.in) | reinterpret_cast<uintptr_t>(a.out)) &
+               (kLine * sizeof(double) - 1)) == 0;
+    // the V dims' runs start at sums of the input strides, the U dims' at
+    // sums of the output strides; a tile of V stays in its first dim
+    for (int i = 0; i < a.nV; ++i) ok = ok && a.sinV[i] % kLine == 0;
+    for (int i = 0; i < a.nU; ++i) ok = ok && a.soutU[i] % kLine == 0;
+    ok = ok && a.nV > 0 && a.extV[0].d % kLine == 0;
+    return ok;
+}
+
+// The order of a permute's tiles over the XCDs and how it stores.
+//
+// Rows of a tile that begin or end inside a cache line share it with the
+// tile's neighbours, along U for the reads and along V for the writes.  In
+// launch order the neighbours run on other XCDs, each with an L2 of its own,
+// and the line is fetched (written) twice; patches of 8 x 8 tiles keep both
+// neighbours on one XCD at about the same time.  Stores past the caches then
+// only fit blocks that the 256 MB cache holds (30^5, 389 MB in all: 86 us
+// against 94 stored through it); larger ones store through it, so that the
+// halves of a line meet (113 x 97 x 109 x 101 reversed, 1.9 GB: launch order
+// 543 us, patches 494, stored through the cache 425; 7001 x 5003 transposed
+// 154 -> 142).  Rows of whole lines have nothing to share and run in launch
+// order with streaming stores (64^4 reversed 56 us, in patches 57).  A batch
+// takes smaller patches, since its blocks have few tiles (144 blocks of 30,
+// 15: 81 us with 8 x 8, 76 with 4 x 8).
+void tile_order(bool large, bool batched, int turn, PermArgs &a, int64_t &grid) {
+    const bool lines = whole_lines(a);
+    a.stream = lines || !large;
+    // at least 64 patches of a single block (8 an XCD), and none in a batch's
+    // smallest blocks, whose patches would not fill a round of the XCDs
+    const int64_t tiles = (int64_t)a.tilesU * a.tilesV;
+    const int64_t in_all = batched ? (tiles < 64 ? 1 : 32)
+                                   : std::min<int64_t>(large ? 256 : 64, tiles / 64);
+    if (lines || in_all <= 1) return patches(a, 1, 1, turn, grid);
+    const int64_t along_u = std::min<int64_t>(batched ? 4 : large ? 16 : 8, in_all);
+    const int su = even_tile(a.tilesU, along_u);
+    const int sv = even_tile(a.tilesV, std::max<int64_t>(1, in_all / su));
+    patches(a, su, sv, turn, grid);
 }
 
 // Kernel arguments and workgroup count of one permute (an identity as a
 // single contiguous run in row mode).
 void fill_args(const PermutePlan &p, const double *in, double *out, PermArgs &a,
-               int64_t &grid, const TileShape &ts) {
-    const int tile_elems = ts.items * kPermThreads;
+               int64_t &grid, bool large, bool batched, int turn) {
+    const int tile_elems = kPermItems * kPermThreads;
     a = PermArgs{};
     a.in = in;
     a.out = out;
     if (p.identity) {
         a.nU = 1;
-        a.extU[0] = (int)p.size;
+        a.extU[0] = make_fastdiv((uint32_t)p.size);
         a.soutU[0] = 1;
         a.nV = 0;
         a.sizeU = (int)p.size;
@@ -231,13 +286,15 @@ void fill_args(const PermutePlan &p, const double *in, double *out, PermArgs &a,
         a.TV = 1;
         a.pitch = a.TU;
         a.tilesU = (a.sizeU + a.TU - 1) / a.TU;
-        grid = a.tilesU;
+        a.tilesV = 1;
+        a.stream = 1;
+        patches(a, 1, 1, turn, grid);
         return;
     }
     a.nU = p.nU;
     a.nV = p.nV;
     for (int i = 0; i < p.nU; ++i) {
-        a.extU[i] = p.ext[i];
+        a.extU[i] = make_fastdiv((uint32_t)p.ext[i]);
         a.soutU[i] = (int)p.sout[i];
     }
     // Input strides of the canonical dims are their column-major products.
@@ -246,20 +303,24 @@ void fill_args(const PermutePlan &p, const double *in, double *out, PermArgs &a,
     for (int i = 0; i < p.rank; ++i) { sin[i] = acc; acc *= p.ext[i]; }
     for (int i = 0; i < p.nV; ++i) {
         const int d = p.vdim[i];
-        a.extV[i] = p.ext[d];
+        a.extV[i] = make_fastdiv((uint32_t)p.ext[d]);
         a.sinV[i] = (int)sin[d];
         a.soutV[i] = (int)p.sout[d];
     }
     a.sizeU = (int)p.sizeU;
     a.sizeV = (int)p.sizeV;
     a.row_mode = p.row_mode ? 1 : 0;
-    a.TU = even_tile(p.sizeU, p.row_mode ? tile_elems : ts.tu_cap);
+    a.TU = even_tile(p.sizeU, p.row_mode ? tile_elems : kPermMaxTU);
     a.TV = even_tile(p.sizeV, std::max<int64_t>(1, std::min<int64_t>(tile_elems / a.TU,
                                                                       kPermMaxTV)));
     a.pitch = p.row_mode ? a.TU : (a.TU | 1);
-    a.tilesU = (a.sizeU + a.TU - 1) / a.TU;
+    const int64_t tilesU = (a.sizeU + a.TU - 1) / a.TU;
     const int64_t tilesV = (a.sizeV + a.TV - 1) / a.TV;
-    grid = (int64_t)a.tilesU * tilesV;
+    grid = tilesU * tilesV;
+    if (grid >= ((int64_t)1 << 31)) return; // refused by the callers
+    a.tilesU = (int)tilesU;
+    a.tilesV = (int)tilesV;
+    tile_order(large, batched, turn, a, grid);
 }
 
 } // namespace
@@ -272,35 +333,34 @@ hipError_t launch_permute(const PermutePlan &p, const double *in, double *out,
                               hipMemcpyDeviceToDevice, stream);
     PermArgs a;
     int64_t grid = 0;
-    const TileShape ts = tile_shape(p, false);
-    fill_args(p, in, out, a, grid, ts);
+    fill_args(p, in, out, a, grid, p.size >= kLargeElems, false, 0);
     if (grid <= 0 || grid >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
     const int tile_cap = a.row_mode ? 0 : a.TV * a.pitch;
     const size_t lds = perm_lds_bytes(tile_cap, a.TV);
-    if (ts.items <= 8)
-        hipLaunchKernelGGL(permute_kernel<8>, dim3((unsigned)grid), dim3(kPermThreads), lds,
-                           stream, a, tile_cap, a.TV);
+    if (a.stream)
+        permute_kernel<true><<<(unsigned)grid, kPermThreads, lds, stream>>>(a, tile_cap, a.TV);
     else
-        hipLaunchKernelGGL(permute_kernel<16>, dim3((unsigned)grid), dim3(kPermThreads), lds,
-                           stream, a, tile_cap, a.TV);
+        permute_kernel<false><<<(unsigned)grid, kPermThreads, lds, stream>>>(a, tile_cap, a.TV);
     return hipGetLastError();
 }
 
 int64_t permute_batch_args(const PermutePlan *plans, const double *const *in,
                            double *const *out, int n, PermArgs *args, int *first,
-                           int *tile_cap, int *tv_cap, int *items) {
-    int64_t total = 0;
+                           int *tile_cap, int *tv_cap) {
+    int64_t total = 0, all = 0;
+    int turn = 0;
+    for (int e = 0; e < n; ++e) all += plans[e].size;
     *tile_cap = 0;
     *tv_cap = 1;
-    *items = 8;
     for (int e = 0; e < n; ++e) {
         int64_t g = 0;
         if (plans[e].size > 0) {
-            const TileShape ts = tile_shape(plans[e], true);
-            *items = std::max(*items, ts.items);
-            fill_args(plans[e], in[e], out[e], args[e], g, ts);
+            fill_args(plans[e], in[e], out[e], args[e], g, all >= kLargeElems, true, turn);
             if (!args[e].row_mode) *tile_cap = std::max(*tile_cap, args[e].TV * args[e].pitch);
             *tv_cap = std::max(*tv_cap, args[e].TV);
+            // the next entry's patches go on with the next XCD
+            const int64_t row = args[e].patchesU.d, sv = args[e].patch.d / args[e].patchU.d;
+            turn = (int)((turn + row * ((args[e].tilesV + sv - 1) / sv)) % kXcds);
         } else {
             args[e] = PermArgs{};
         }
@@ -312,16 +372,10 @@ int64_t permute_batch_args(const PermutePlan *plans, const double *const *in,
 }
 
 hipError_t launch_permute_batch(const PermArgs *args, const int *first, const int *entry,
-                                int grid, int tile_cap, int tv_cap, int items,
-                                hipStream_t stream) {
+                                int grid, int tile_cap, int tv_cap, hipStream_t stream) {
     if (grid <= 0) return hipSuccess;
-    const size_t lds = perm_lds_bytes(tile_cap, tv_cap);
-    if (items <= 8)
-        hipLaunchKernelGGL(permute_batch_kernel<8>, dim3((unsigned)grid), dim3(kPermThreads), lds,
-                           stream, args, first, entry, tile_cap, tv_cap);
-    else
-        hipLaunchKernelGGL(permute_batch_kernel<16>, dim3((unsigned)grid), dim3(kPermThreads),
-                           lds, stream, args, first, entry, tile_cap, tv_cap);
+    permute_batch_kernel<<<(unsigned)grid, kPermThreads, perm_lds_bytes(tile_cap, tv_cap),
+                           stream>>>(args, first, entry, tile_cap, tv_cap);
     return hipGetLastError();
 }
 

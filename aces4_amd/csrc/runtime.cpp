@@ -2204,7 +2204,6 @@ struct sipgpu_permute_batch_s {
     size_t first_off = 0, entry_off = 0;
     int n = 0, grid = 0;
     int tile_cap = 0, tv_cap = 1; // LDS of the launch
-    int items = 16;               // elements per thread
     long long elements = 0;
 };
 
@@ -2239,10 +2238,10 @@ int sipgpu_permute_batch_plan(const sipgpu_permutation *list, int n,
     const size_t first_off = round256((size_t)n * sizeof(PermArgs));
     const size_t entry_off = first_off + round256((size_t)(n + 1) * sizeof(int));
     std::vector<unsigned char> host(entry_off);
-    int tile_cap = 0, tv_cap = 1, items = 16;
+    int tile_cap = 0, tv_cap = 1;
     const int64_t grid = permute_batch_args(
         plans.data(), in.data(), out.data(), n, reinterpret_cast<PermArgs *>(host.data()),
-        reinterpret_cast<int *>(host.data() + first_off), &tile_cap, &tv_cap, &items);
+        reinterpret_cast<int *>(host.data() + first_off), &tile_cap, &tv_cap);
     if (grid >= ((int64_t)1 << 31)) return fail(SIPGPU_ESIZE, "permute batch: too many tiles");
     // the entry of every workgroup
     host.resize(entry_off + (size_t)grid * sizeof(int));
@@ -2258,7 +2257,6 @@ int sipgpu_permute_batch_plan(const sipgpu_permutation *list, int n,
     b->n = n;
     b->tile_cap = tile_cap;
     b->tv_cap = tv_cap;
-    b->items = items;
     b->grid = (int)grid;
     b->elements = elements;
     if (grid > 0) {
@@ -2281,7 +2279,7 @@ int sipgpu_permute_batch_execute(sipgpu_permute_batch_t b, sipgpu_stream_t s) {
     HIP_TRY(launch_permute_batch(reinterpret_cast<const PermArgs *>(base),
                                  reinterpret_cast<const int *>(base + b->first_off),
                                  reinterpret_cast<const int *>(base + b->entry_off), b->grid,
-                                 b->tile_cap, b->tv_cap, b->items, resolve(c, s).s));
+                                 b->tile_cap, b->tv_cap, resolve(c, s).s));
     return 0;
 }
 

@@ -867,11 +867,11 @@ int server_permutes(sipgpu_server_s &S, int lane, const std::vector<Pending> &ba
         const size_t first_off = round256((size_t)n * sizeof(sipgpu::PermArgs));
         const size_t entry_off = first_off + round256((size_t)(n + 1) * sizeof(int));
         std::vector<unsigned char> host(entry_off);
-        int tile_cap = 0, tv_cap = 1, items = 16;
+        int tile_cap = 0, tv_cap = 1;
         const int64_t grid = sipgpu::permute_batch_args(
             plans.data(), in.data(), out.data(), n,
             reinterpret_cast<sipgpu::PermArgs *>(host.data()),
-            reinterpret_cast<int *>(host.data() + first_off), &tile_cap, &tv_cap, &items);
+            reinterpret_cast<int *>(host.data() + first_off), &tile_cap, &tv_cap);
         const size_t bytes = entry_off + (size_t)std::max<int64_t>(grid, 0) * sizeof(int);
         if (grid >= ((int64_t)1 << 31) || bytes > kSlotBytes) {
             // tables beyond a descriptor slot: one launch per permute
@@ -897,7 +897,7 @@ int server_permutes(sipgpu_server_s &S, int lane, const std::vector<Pending> &ba
                         reinterpret_cast<const sipgpu::PermArgs *>(dev),
                         reinterpret_cast<const int *>(dev + first_off),
                         reinterpret_cast<const int *>(dev + entry_off), (int)grid, tile_cap,
-                        tv_cap, items, stream);
+                        tv_cap, stream);
                 if (e == hipSuccess) e = hipEventRecord(S.slot_free[slot], stream);
                 if (e != hipSuccess) rc = hip_fail(e, "server: permute launch");
                 S.slot_used[slot] = true;
