@@ -21,7 +21,9 @@ constexpr int oz_tile_size(int code) { return code == kOzWideTile ? kOzBigTile :
 constexpr int kOzChunk = 16;            // bytes of k per panel chunk
 constexpr int kOzStage = 128;           // bytes of k per GEMM pipeline stage
 constexpr int kOzStageChunks = kOzStage / kOzChunk;
-constexpr int kOzZero = 256;            // zero bytes at the start of every plane
+constexpr int kOzZero = 256;            // zero bytes at the start of every residue plane
+// FP64 panels: units of 16 rows x 8 k, 1 KiB in MFMA operand order (packed.hip)
+constexpr int kPanelRows = 16, kPanelK = 8, kPanelUnit = 1024;
 constexpr int kOzTileX = 32, kOzTileK = 128; // conversion tile (rows x k)
 constexpr int kOzRecChunk = 2048;       // result elements per reconstruction workgroup
 
@@ -49,13 +51,14 @@ struct OzBlock {
     int ktab, xtab;        // offsets of its k / x tables in the pool
     int exp_off;           // first exponent of its row component
     int xfast;             // 1: consecutive rows are adjacent in memory
-    int pad;
-    long long panel_off;   // byte offset inside each modulus plane
+    int row0;              // FP64: its first row in the panel (stacked operands)
+    long long panel_off;   // byte offset of the panel inside each plane
 };
 
-// 16 bytes of a task's virtual K: where the left and right operand rows
-// hold them (plane offsets of row 0 -- bytes in a residue plane, 16-byte
-// units in a plane of doubles; row r adds r * stride bytes).
+// A piece of a task's virtual K.  Residue planes: 16 bytes of k, the left and
+// right operands' row 0 at bytes a and b, row r at r * stride bytes more.
+// Planes of doubles: 8 k, the operands' first 16 rows in the 1 KiB units a and
+// b, the next 16 rows `stride` units on.
 struct OzChunkRef {
     uint32_t a, b;
     int32_t stride;
@@ -79,6 +82,7 @@ struct OzTask {
     int M, N;
     int mD, nD;
     int chunk0, nchunks;  // virtual K: chunks [chunk0, chunk0 + nchunks), whole stages
+                          // (an FP64 stage is one chunk)
     int beta;
     int expA, expB;       // first row / column exponent
     int nfast;            // 1: result elements ordered with n fastest

@@ -2,19 +2,19 @@
 //
 // For large batches the operand permutations are applied once per block
 // instead of once per tile: every operand instance (block + its k / x
-// tables) is packed into X row-major rows of Kp doubles (K rounded up to
-// an even count, zero filled), and the grouped GEMM runs over each task's
-// virtual K -- its pairs' panels concatenated in 16-byte chunks through the
-// same chunk map as the split-precision path -- with no table lookups in
-// the K loop.  The product is scattered into the destination block through
-// its tables, accumulating when the task does.
+// tables) is packed into a panel of X rows (a merged task's instances one
+// after another in one panel) by K rounded up to 8, zero filled, and the
+// grouped GEMM runs over each task's virtual K -- its pairs' panels one after
+// another, 8 k a stage -- with no table lookups in the K loop.  The product is
+// scattered into the destination block through its tables, accumulating when
+// the task does.
 //
-// MFMA v_mfma_f64_16x16x4_f64: lane l holds A(i = l%16, k = l/16); register
-// r of lane l holds C(4r + l/16, l%16).  A 16-byte LDS read gives a lane two
-// consecutive k of its row; the pair feeds two MFMAs (the first double to the
-// first, the second to the second), so MFMA t of a 64-byte step sums
-// k = 2 (4 s + l/16) + t over l/16 = 0..3: the same permutation of k for both
-// operands, so the sum over all MFMAs is the full dot product.
+// A panel is made of 1 KiB units of 16 rows x 8 k in the operand order of
+// v_mfma_f64_16x16x4_f64 (lane l holds A(i = l%16, k = l/16); register r of
+// lane l holds C(4r + l/16, l%16)): element (row i, k) sits at 2 (i + 16 (k %
+// 4)) + k / 4, so one 16-byte load per lane, 1 KiB contiguous per wave, gives
+// a wave its operand for two MFMAs.  Unit (row block, k block) of a panel is
+// number row block * (Kp / 8) + k block.
 #include "kernels.h"
 #include "ozaki.h"
 
@@ -22,10 +22,10 @@ namespace sipgpu {
 
 namespace {
 
-typedef int int32x4 __attribute__((ext_vector_type(4)));
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 typedef double f64x2 __attribute__((ext_vector_type(2)));
 typedef const __attribute__((address_space(1))) int8_t gi8_t;
+typedef const __attribute__((address_space(4))) OzChunkRef cref_t;
 
 // Workgroups over 32 x 128 tiles of operand blocks, each done as two halves
 // of 64 k (half the LDS of a whole tile, so twice the workgroups per CU keep
@@ -70,18 +70,20 @@ __global__ __launch_bounds__(256) void pack_kernel(OzConvArgs a) {
                 for (int j = 0; j < 8; ++j) S[(tid >> 6) + 4 * j][tid & 63] = v[j];
             }
             __syncthreads();
-            // 8 lanes per row, 4 pairs each: a row's 8 lanes cover 128 bytes
-            const int xx = tid >> 3, l = tid & 7;
-            const int x = w.x0 + xx;
-            if (x < b.X) {
-                double *dst = reinterpret_cast<double *>(a.planes + b.panel_off) +
-                              (long long)x * b.Kp + kb;
+            // 16 bytes (k, k + 4) per thread, rows fastest: 16 rows x 4 k are
+            // the 1 KiB of a unit, in address order
+            const int nk = b.Kp / kPanelK;
+            double *dst = reinterpret_cast<double *>(a.planes + b.panel_off);
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int k = 2 * (8 * j + l);
-                    if (kb + k < b.Kp) // Kp is even: whole 16-byte pairs
-                        *reinterpret_cast<f64x2 *>(dst + k) =
-                            *reinterpret_cast<const f64x2 *>(&S[xx][k]);
+            for (int j = 0; j < 4; ++j) {
+                const int e = j * 256 + tid;
+                const int xx = (e & 15) + 16 * ((e >> 9) & 1), kl = (e >> 4) & 3, ku = (e >> 6) & 7;
+                const int x = w.x0 + xx, kk = 8 * ku + kl;
+                if (x < b.X && kb + kk < b.Kp) {
+                    const int row = b.row0 + x;
+                    const long long unit = (long long)(row >> 4) * nk + (kb >> 3) + ku;
+                    *reinterpret_cast<f64x2 *>(dst + unit * 128 + 2 * ((row & 15) + 16 * kl)) =
+                        f64x2{S[xx][kk], S[xx][kk + 4]};
                 }
             }
         }
@@ -91,29 +93,24 @@ __global__ __launch_bounds__(256) void pack_kernel(OzConvArgs a) {
 // Grouped FP64 GEMM over packed panels.  Workgroup tile BM x BN = 128 x 128
 // (4 waves, 2 x 2, each 64 x 64: 16 accumulator fragments) or 64 x 64 (each
 // wave 32 x 32: for small batches, whose tiles are cut into K segments:
-// a segment's partial sums are a quarter of the bytes); stages of
-// 128 bytes (16 k) double-buffered in LDS with rows XOR-swizzled by 16-byte
-// chunk; loads run one stage ahead through registers; chunk entries come
-// from an LDS window (their plane offsets count 16-byte units, so panels may
-// reach 64 GiB).  Rows past the task's M / N read row M-1 / N-1 and are
-// never stored; chunks past the pairs' K read the plane's zero bytes.
+// a segment's partial sums are a quarter of the bytes).  Operands go from the
+// panels straight into registers: no LDS, no barrier, so a wave waits for its
+// own loads alone, which run one stage (32 MFMAs of 64 cycles) ahead in a
+// second register set.  Chunk entries are wave-uniform and come through the
+// scalar cache.  What bounds it is the FP64 matrix rate at the clock that the
+// card's power leaves: 4500^3 in 450 x 450 blocks 3.03 ms with the operands
+// staged through LDS (matrix units busy 82%), 2.82 so (91%; 93% and 2.06 GHz on
+// the block-sparse ladder, 7.31 -> 7.04 ms).  Rows past the task's M / N lie in its last row block or
+// repeat it and are never stored.
 template <int BM, int BN>
 __global__ __launch_bounds__(256, 2) void gemm_f64_packed_kernel(OzGemmArgs a) {
     constexpr int WM = 2, WN = 2;
     constexpr int TM = BM / WM, TN = BN / WN, FM = TM / 16, FN = TN / 16;
-    constexpr int KS = kOzStage, CH = kOzStageChunks;
-    constexpr int IA = BM / 32, IB = BN / 32;
-    constexpr int kWin = 512;
-    static_assert(CH == 8 && KS == 128, "a stage is 8 chunks of 16 bytes");
-    __shared__ __attribute__((aligned(1024))) int8_t As[2][BM * KS];
-    __shared__ __attribute__((aligned(1024))) int8_t Bs[2][BN * KS];
-    __shared__ __attribute__((aligned(16))) OzChunkRef Es[kWin];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave % WM, wn = wave / WM;
     const int li = lane & 15, lk = lane >> 4;
-    const int g = (lane & 7) ^ (lane >> 3);
     gi8_t *plane = (gi8_t *)a.planes;
 
     const int u0 = a.wg_first ? a.wg_first[blockIdx.x] : (int)blockIdx.x;
@@ -123,11 +120,12 @@ __global__ __launch_bounds__(256, 2) void gemm_f64_packed_kernel(OzGemmArgs a) {
         if (tile.task < 0) continue;
         const OzTask task = a.tasks[tile.task];
         const int m0 = tile.mt * BM, n0 = tile.nt * BN;
-        int ra[IA], rb[IB];
+        // this wave's row blocks of the operands, clamped into the panels
+        int ra[FM], rb[FN];
 #pragma unroll
-        for (int i = 0; i < IA; ++i) ra[i] = min(m0 + 8 * (wave * IA + i) + (lane >> 3), task.M - 1);
+        for (int i = 0; i < FM; ++i) ra[i] = (min(m0 + wm * TM + i * 16, task.M - 1)) >> 4;
 #pragma unroll
-        for (int i = 0; i < IB; ++i) rb[i] = min(n0 + 8 * (wave * IB + i) + (lane >> 3), task.N - 1);
+        for (int j = 0; j < FN; ++j) rb[j] = (min(n0 + wn * TN + j * 16, task.N - 1)) >> 4;
 
         f64x4 acc[FM][FN];
 #pragma unroll
@@ -135,82 +133,44 @@ __global__ __launch_bounds__(256, 2) void gemm_f64_packed_kernel(OzGemmArgs a) {
 #pragma unroll
             for (int j = 0; j < FN; ++j) acc[i][j] = f64x4{0.0, 0.0, 0.0, 0.0};
 
-        const OzChunkRef *ch = a.chunks + task.chunk0;
-        const int sb = tile.s0, se = tile.s1; // stages of this unit, se > sb
-        // windows of kWin chunk entries start at stage sb + 64 j
-        auto load_window = [&](int st0) {
-            __syncthreads();
-            const int c0 = st0 * CH, n = min(kWin, se * CH - c0);
-            for (int i = tid; i < n; i += 256)
-                *reinterpret_cast<int32x4 *>(&Es[i]) = *reinterpret_cast<const int32x4 *>(&ch[c0 + i]);
-            __syncthreads();
-        };
-        struct Sel {
-            uint32_t a, b;
-            int stride;
-        };
-        auto entry = [&](int st) {
-            const OzChunkRef e = Es[((min(st, se - 1) - sb) * CH + g) % kWin];
-            return Sel{e.a, e.b, e.stride};
-        };
-        int32x4 xa[IA], xb[IB];
-        auto fetch = [&](const Sel &e) {
+        cref_t *ch = (cref_t *)(a.chunks + task.chunk0);
+        const int sb = tile.s0, se = tile.s1; // stages of this unit
+        f64x2 fa[2][FM], fb[2][FN];
+        // stage s into register set `set` (past the unit's last stage that
+        // one again: the loads stay unconditional, nothing reads them)
+        auto fetch = [&](int set, int s) {
+            const int at = min(s, se - 1);
+            const uint32_t ea = ch[at].a, eb = ch[at].b;
+            const int stride = ch[at].stride;
 #pragma unroll
-            for (int i = 0; i < IA; ++i)
-                xa[i] = *reinterpret_cast<const __attribute__((address_space(1))) int32x4 *>(
-                    plane + (long long)e.a * kOzChunk + (long long)ra[i] * e.stride);
+            for (int i = 0; i < FM; ++i)
+                fa[set][i] = *reinterpret_cast<const __attribute__((address_space(1))) f64x2 *>(
+                    plane + ((long long)ea + (long long)ra[i] * stride) * kPanelUnit + lane * 16);
 #pragma unroll
-            for (int i = 0; i < IB; ++i)
-                xb[i] = *reinterpret_cast<const __attribute__((address_space(1))) int32x4 *>(
-                    plane + (long long)e.b * kOzChunk + (long long)rb[i] * e.stride);
+            for (int j = 0; j < FN; ++j)
+                fb[set][j] = *reinterpret_cast<const __attribute__((address_space(1))) f64x2 *>(
+                    plane + ((long long)eb + (long long)rb[j] * stride) * kPanelUnit + lane * 16);
         };
-        auto put = [&](int buf) {
+        auto mma = [&](int set) {
 #pragma unroll
-            for (int i = 0; i < IA; ++i)
-                *reinterpret_cast<int32x4 *>(&As[buf][(wave * IA + i) * 1024 + lane * 16]) = xa[i];
-#pragma unroll
-            for (int i = 0; i < IB; ++i)
-                *reinterpret_cast<int32x4 *>(&Bs[buf][(wave * IB + i) * 1024 + lane * 16]) = xb[i];
-        };
-        auto compute = [&](int buf) {
-            const int8_t *sa = As[buf], *sb = Bs[buf];
-#pragma unroll
-            for (int ks = 0; ks < KS / 64; ++ks) {
-                const int slot = ((ks * 4 + lk) ^ (li & 7)) * 16;
-                f64x2 fa[FM], fb[FN];
+            for (int h = 0; h < 2; ++h)
 #pragma unroll
                 for (int i = 0; i < FM; ++i)
-                    fa[i] = *reinterpret_cast<const f64x2 *>(sa + (wm * TM + i * 16 + li) * KS + slot);
 #pragma unroll
-                for (int j = 0; j < FN; ++j)
-                    fb[j] = *reinterpret_cast<const f64x2 *>(sb + (wn * TN + j * 16 + li) * KS + slot);
-#pragma unroll
-                for (int h = 0; h < 2; ++h)
-#pragma unroll
-                    for (int i = 0; i < FM; ++i)
-#pragma unroll
-                        for (int j = 0; j < FN; ++j)
-                            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[i][h], fb[j][h],
-                                                                             acc[i][j], 0, 0, 0);
-            }
+                    for (int j = 0; j < FN; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[set][i][h], fb[set][j][h],
+                                                                         acc[i][j], 0, 0, 0);
         };
-
-        // One stage of loads ahead is enough here: a stage is 64 MFMAs of
-        // 64 cycles per wave.  Loads are unconditional (the last stage is
-        // fetched twice) so the staged registers need no merge copies.
-        load_window(sb);
-        fetch(entry(sb));
-        put(0);
-        __syncthreads();
-        int buf = 0;
-        for (int s = sb; s < se; ++s) {
-            if (s + 1 < se && ((s + 1 - sb) * CH) % kWin == 0) load_window(s + 1);
-            fetch(entry(s + 1));
-            __builtin_amdgcn_sched_barrier(0);
-            compute(buf);
-            put(buf ^ 1); // after the last stage this writes a copy nothing reads
-            __syncthreads();
-            buf ^= 1;
+        if (sb < se) {
+            fetch(0, sb);
+            int s = sb;
+            for (; s + 1 < se; s += 2) {
+                fetch(1, s + 1);
+                mma(0);
+                fetch(0, s + 2);
+                mma(1);
+            }
+            if (s < se) mma(0);
         }
 
         if (tile.part >= 0) {

@@ -558,7 +558,7 @@ void persistent_schedule(const std::vector<std::vector<OzTile>> &lists,
                          std::vector<OzTile> &units, std::vector<int> &first,
                          std::vector<OzTile> &fix, int &nslots) {
     std::vector<std::vector<OzTile>> wg((size_t)slots * kXcds);
-    constexpr int kMinSeg = 4; // stages
+    constexpr int kMinSeg = 8; // stages (of 8 k)
     for (int x = 0; x < kXcds; ++x) {
         const auto &L = lists[x];
         const auto &c = costs[x];
@@ -1000,7 +1000,6 @@ int sipgpu::rt::build_panel_plan(const sipgpu_contraction *list, int n, int nmod
                                  const PanelOptions &opt) {
     if (nmod != 0 && (nmod < kOzMinModuli || nmod > kOzMaxUsable))
         return fail(SIPGPU_EARG, "split path: nmoduli must be in 6..14");
-    const int eb = nmod ? 1 : 8; // bytes per panel element
     // shapes
     std::unordered_map<std::string, int> shape_index;
     std::vector<std::unique_ptr<ContractionShape>> shapes;
@@ -1038,7 +1037,7 @@ int sipgpu::rt::build_panel_plan(const sipgpu_contraction *list, int n, int nmod
     struct Inst { const double *ptr; int K, X, Kp, ktab, xtab, xfast; };
     std::map<std::tuple<const double *, int, int, int, int>, int> inst_index;
     std::vector<Inst> insts;
-    const int kq = kOzChunk / eb; // panel elements per 16-byte chunk
+    const int kq = nmod ? kOzChunk : kPanelK; // k per chunk
     auto instance = [&](const double *ptr, int si, int side) {
         const ContractionShape &sh = *shapes[si];
         const int ktab = tabs[si][side == 0 ? 0 : 2], xtab = tabs[si][side == 0 ? 1 : 3];
@@ -1252,7 +1251,7 @@ int sipgpu::rt::build_panel_plan(const sipgpu_contraction *list, int n, int nmod
     // pairs) are united into components with one exponent slot each.
     std::vector<OzBlock> blocks;
     std::map<std::pair<int, int>, int> shared_copy; // (instance, side) -> block
-    long long panel = kOzZero;
+    long long panel = nmod ? kOzZero : 0;
     int nexpo = 0;
     std::vector<int> uf(2 * insts.size());
     std::iota(uf.begin(), uf.end(), 0);
@@ -1273,7 +1272,9 @@ int sipgpu::rt::build_panel_plan(const sipgpu_contraction *list, int n, int nmod
         if (it.second) nexpo += insts[ii].X;
         return it.first->second;
     };
-    auto place = [&](int ii, int exp_off) {
+    // places instance ii at `panel` (split path), or as rows row0, row0 + 1, ..
+    // of the FP64 panel there
+    auto place = [&](int ii, int exp_off, int row0) {
         const Inst &in = insts[ii];
         OzBlock ob{};
         ob.data = in.ptr;
@@ -1284,14 +1285,19 @@ int sipgpu::rt::build_panel_plan(const sipgpu_contraction *list, int n, int nmod
         ob.xtab = in.xtab;
         ob.xfast = in.xfast;
         ob.exp_off = exp_off;
+        ob.row0 = row0;
         ob.panel_off = panel;
-        panel += (long long)in.X * in.Kp * eb;
+        if (nmod) panel += (long long)in.X * in.Kp;
         blocks.push_back(ob);
         return (int)blocks.size() - 1;
     };
-    auto align_panel = [&]() { panel = (panel + 255) / 256 * 256; };
-    // chunk offsets: bytes in a residue plane, 16-byte units in an FP64 one
-    const long long unit = nmod ? 1 : kOzChunk;
+    // the end of a panel of `rows` rows of Kp k
+    auto close_panel = [&](int rows, int Kp) {
+        if (nmod)
+            panel = (panel + 255) / 256 * 256;
+        else
+            panel += (long long)((rows + kPanelRows - 1) / kPanelRows) * (Kp / kPanelK) * kPanelUnit;
+    };
     std::vector<OzChunkRef> chunks;
     for (int t = 0; t < ntasks; ++t) {
         const auto &rs = task_rows[t], &cs = task_cols[t];
@@ -1317,8 +1323,8 @@ int sipgpu::rt::build_panel_plan(const sipgpu_contraction *list, int n, int nmod
                 const auto key = std::make_pair(ii, nmod ? side : 0);
                 auto it = shared_copy.find(key);
                 if (it == shared_copy.end()) {
-                    it = shared_copy.emplace(key, place(ii, exp0)).first;
-                    align_panel();
+                    it = shared_copy.emplace(key, place(ii, exp0, 0)).first;
+                    close_panel(insts[ii].X, insts[ii].Kp);
                 }
                 return blocks[it->second].panel_off;
             }
@@ -1326,29 +1332,30 @@ int sipgpu::rt::build_panel_plan(const sipgpu_contraction *list, int n, int nmod
             int off = 0;
             for (int key : keys) {
                 const int ii = vec[key][p];
-                place(ii, exp0 + off);
+                place(ii, exp0 + off, nmod ? 0 : off);
                 off += insts[ii].X;
             }
-            align_panel();
+            close_panel(off, insts[vec[keys[0]][p]].Kp);
             return base;
         };
-        // virtual K: the pairs' panel chunks, padded with chunks of the zero
-        // bytes to whole stages (FP64) or whole pairs of stages (the INT8
-        // GEMM runs two stages per loop trip)
+        // virtual K: the pairs' panel chunks; the INT8 GEMM runs two stages of
+        // kOzStageChunks per loop trip and is padded to that with chunks of
+        // the zero bytes
         tasks[t].chunk0 = (int)chunks.size();
         const int np = (int)rvec[rs[0]].size();
         for (int p = 0; p < np; ++p) {
             const long long la = stack(0, p), lb = stack(1, p);
             const int Kp = insts[rvec[rs[0]][p]].Kp;
             for (int k = 0; k < Kp; k += kq)
-                chunks.push_back(OzChunkRef{(uint32_t)((la + (long long)k * eb) / unit),
-                                            (uint32_t)((lb + (long long)k * eb) / unit), Kp * eb,
-                                            0});
-            if (panel >= (1LL << 32) * unit - 65536)
+                chunks.push_back(nmod ? OzChunkRef{(uint32_t)(la + k), (uint32_t)(lb + k), Kp, 0}
+                                      : OzChunkRef{(uint32_t)(la / kPanelUnit + k / kPanelK),
+                                                   (uint32_t)(lb / kPanelUnit + k / kPanelK),
+                                                   Kp / kPanelK, 0});
+            if (panel >= (nmod ? 1LL << 32 : 1LL << 36) - (nmod ? 65536 : 16 * 65536))
                 return fail(SIPGPU_ESIZE, nmod ? "split path: operand panels exceed 4 GiB per modulus"
                                                : "packed path: operand panels exceed 64 GiB");
         }
-        while ((chunks.size() - tasks[t].chunk0) % ((nmod ? 2 : 1) * kOzStageChunks))
+        while (nmod && (chunks.size() - tasks[t].chunk0) % (2 * kOzStageChunks))
             chunks.push_back(OzChunkRef{0u, 0u, 0, 0});
         tasks[t].nchunks = (int)chunks.size() - tasks[t].chunk0;
     }
@@ -1404,7 +1411,7 @@ int sipgpu::rt::build_panel_plan(const sipgpu_contraction *list, int n, int nmod
         for (OzTile &u : lists[x]) {
             u.part = -1;
             u.s0 = 0;
-            u.s1 = tasks[u.task].nchunks / kOzStageChunks;
+            u.s1 = nmod ? tasks[u.task].nchunks / kOzStageChunks : tasks[u.task].nchunks;
             costs[x].push_back(task_cost[u.task] / ((double)tms[u.task] * tns[u.task]));
         }
     std::vector<OzTile> tiles, fix;
@@ -1695,6 +1702,13 @@ int plan_choice_locked(Context &c, const sipgpu_contraction *list, int n, int nm
     return 0;
 }
 
+// Untuned FP64 batches of this many flop (and 5e7 per result block) run on packed
+// panels.  Below, packing and the merged tiles' K segments cost more than the
+// table kernel's gathers: 1.5e9 flop into 16 blocks 98 us packed, 75 in
+// tables; 3.9e9 into 64 141 and 135; above, 7.3e9 into 144 181 and 237, 3.3e10
+// into 64 944 and 1440.
+constexpr double kPackedFlops = 5e9;
+
 // The plan sipgpu_batch_plan makes without a tuned choice.  Large batches
 // run on packed operand panels: the permutations are applied once per
 // block (one streaming pass) instead of per tile, and the GEMM runs over
@@ -1716,7 +1730,7 @@ int plan_default_locked(Context &c, const sipgpu_contraction *list, int n,
         out = std::move(b);
         return 0;
     }
-    bool packed = b->ntasks > 0 && b->flops >= 1e9 && b->flops / b->ntasks >= 5e7;
+    bool packed = b->ntasks > 0 && b->flops >= kPackedFlops && b->flops / b->ntasks >= 5e7;
     if (const char *e = std::getenv("SIPGPU_FP64_PATH")) {
         if (!std::strcmp(e, "tables")) packed = false;
         if (!std::strcmp(e, "packed")) packed = b->ntasks > 0;

@@ -773,8 +773,8 @@ int server_panels(sipgpu_server_s &S, int lane, const sipgpu::rt::PanelPlan &pla
     hipError_t e = hipMemcpyAsync(S.slot_dev[slot], S.slot_host[slot], desc.size(),
                                   hipMemcpyHostToDevice, st);
     S.slot_used[slot] = true;
-    if (e == hipSuccess)
-        e = sipgpu::oz_zero_heads(planes, plan.plane_bytes, plan.nmod ? plan.nmod : 1, st);
+    if (e == hipSuccess && plan.nmod)
+        e = sipgpu::oz_zero_heads(planes, plan.plane_bytes, plan.nmod, st);
     if (e != hipSuccess) return hip_fail(e, "server: split batch");
     sipgpu::rt::SplitData sd;
     sipgpu::rt::bind_panel_plan(plan, S.slot_dev[slot], planes, res, work, sd);
@@ -971,8 +971,8 @@ int server_batch(sipgpu_server_s &S, int lane, std::vector<Pending> &batch) {
             rc = sipgpu::rt::build_panel_plan(list.data(), (int)list.size(), nmod, plan);
         } else {
             rc = sipgpu::rt::build_batch_image(list.data(), (int)list.size(), img);
-            // large FP64 batches run on packed panels, as sipgpu_batch_plan
-            // plans them (the table kernel gathers per tile)
+            // large FP64 batches run on packed panels (the table kernel
+            // gathers per tile)
             if (!rc && img.ntasks > 0 && img.flops >= 1e9 && img.flops / img.ntasks >= 5e7 &&
                 sipgpu::rt::build_panel_plan(list.data(), (int)list.size(), 0, plan) == 0)
                 panels = true;
