@@ -25,7 +25,7 @@ constexpr int kOzZero = 256;            // zero bytes at the start of every resi
 // FP64 panels: units of 16 rows x 8 k, 1 KiB in MFMA operand order (packed.hip)
 constexpr int kPanelRows = 16, kPanelK = 8, kPanelUnit = 1024;
 constexpr int kOzTileX = 32, kOzTileK = 128; // conversion tile (rows x k)
-constexpr int kOzRecChunk = 2048;       // result elements per reconstruction workgroup
+constexpr int kOzRecChunk = 1024;       // result elements per reconstruction workgroup
 
 // Moduli and reconstruction constants (host-computed).
 struct OzConst {
@@ -34,12 +34,15 @@ struct OzConst {
     int p[kOzMaxModuli];          // pairwise coprime, <= 255
     int u[kOzMaxModuli];          // (M / p_i)^-1 mod p_i
     int c17[kOzMaxModuli];        // 2^17 mod p_i
-    int c34[kOzMaxModuli];        // 2^34 mod p_i
-    int off[kOzMaxModuli];        // p_i * 2^19: makes the limb sum positive
     uint32_t bar[kOzMaxModuli];   // floor(2^32 / p_i) (Barrett reciprocal)
-    double rp[kOzMaxModuli];      // 1 / p_i (rounded)
-    uint64_t mi[kOzMaxModuli][2]; // M / p_i exactly, {low, high} 64-bit halves
-    uint64_t m[2];                // M = prod p_i exactly (< 2^112)
+    // residues: 256^0 .. 256^3 and 256^4 .. 256^6 mod p_i, balanced (|.| <= 127),
+    // a byte each; 1 / p_i (rounded)
+    int32_t d0[kOzMaxModuli], d1[kOzMaxModuli];
+    float rpf[kOzMaxModuli];
+    // reconstruction, byte k of word g for modulus i = 4 g + k, and after the last
+    // modulus for -M: byte b of M / p_i and of 2^128 - M (M = prod p_i < 2^112);
+    // the two bytes of round(2^16 / p_i)
+    uint32_t crt[16][kOzMaxModuli / 4], inv[2][kOzMaxModuli / 4];
 };
 
 // One operand block as the split path sees it: K x X through its tables,

@@ -50,32 +50,32 @@ __global__ void zero_heads_kernel(int8_t *planes, long long plane_bytes, int npl
 // values along the index that is adjacent in memory (32 lanes on 32
 // consecutive rows, or 128 on consecutive k); entries outside the block read
 // as 0.  Thread t holds (row, k) = (t % 32, t / 32 + 8 j) when rows are
-// adjacent, else (t / 128 + 2 j, t % 128).
+// adjacent, else (t / 128 + 2 j, t % 128).  Places outside the block load its
+// last element's instead, so that nothing branches and all table entries,
+// then all values, are in flight together.
 struct SubTile {
     double v[16];
 };
 
 __device__ __forceinline__ void fetch_subtile(const OzBlock &b, const int32_t *tab, int x0, int k0,
                                               int tid, SubTile &t) {
-    if (b.xfast) {
-        const int x = x0 + (tid & 31);
-        const bool xin = x < b.X;
-        const int xo = xin ? tab[b.xtab + x] : 0;
+    typedef const __attribute__((address_space(1))) double gdouble_t;
+    gdouble_t *data = (gdouble_t *)b.data;
+    const bool xf = b.xfast;
+    // this thread's index along the adjacent side, and its 16 along the other
+    const int fast = xf ? x0 + (tid & 31) : k0 + (tid & 127);
+    const int slow = xf ? k0 + (tid >> 5) : x0 + (tid >> 7), step = xf ? 8 : 2;
+    const int nfast = xf ? b.X : b.K, nslow = xf ? b.K : b.X;
+    const int32_t *ftab = tab + (xf ? b.xtab : b.ktab), *stab = tab + (xf ? b.ktab : b.xtab);
+    const int off = ftab[min(fast, nfast - 1)];
+    int at[16];
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const int k = k0 + (tid >> 5) + 8 * j;
-            t.v[j] = (xin && k < b.K) ? b.data[tab[b.ktab + k] + xo] : 0.0;
-        }
-    } else {
-        const int k = k0 + (tid & 127);
-        const bool kin = k < b.K;
-        const int ko = kin ? tab[b.ktab + k] : 0;
+    for (int j = 0; j < 16; ++j) at[j] = stab[min(slow + step * j, nslow - 1)] + off;
+    double v[16];
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const int x = x0 + (tid >> 7) + 2 * j;
-            t.v[j] = (kin && x < b.X) ? b.data[ko + tab[b.xtab + x]] : 0.0;
-        }
-    }
+    for (int j = 0; j < 16; ++j) v[j] = data[at[j]];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) t.v[j] = fast < nfast && slow + step * j < nslow ? v[j] : 0.0;
 }
 
 __device__ __forceinline__ void store_subtile(const OzBlock &b, int tid, const SubTile &t,
@@ -92,9 +92,11 @@ __device__ __forceinline__ void store_subtile(const OzBlock &b, int tid, const S
 // One workgroup per 32-row tile of a block: max |value| of each row over
 // the block's K, as a binary exponent folded into the row's component with
 // atomicMax (order-independent, so the result is deterministic).  Maxima
-// stay in registers across the K sweep (two sub-tiles in flight per step);
-// one LDS reduction per tile folds them per row.
-__global__ __launch_bounds__(256) void row_exponent_kernel(OzConvArgs a, const OzConvTile *items,
+// stay in registers across the K sweep; one LDS reduction per tile folds them
+// per row.  Bound by the reads: the full ring batch (0.32 GB) in 80 us, four
+// workgroups per CU with 16 loads a thread in flight; 128 us with a branch at
+// every load.
+__global__ __launch_bounds__(256, 4) void row_exponent_kernel(OzConvArgs a, const OzConvTile *items,
                                                            int nitems) {
     __shared__ double part[kOzTileX][129];
     const int tid = threadIdx.x;
@@ -104,12 +106,12 @@ __global__ __launch_bounds__(256) void row_exponent_kernel(OzConvArgs a, const O
         double mx[16];
 #pragma unroll
         for (int j = 0; j < 16; ++j) mx[j] = 0.0;
-        for (int k0 = 0; k0 < b.K; k0 += 2 * kOzTileK) {
-            SubTile t0, t1;
-            fetch_subtile(b, a.tab, w.x0, k0, tid, t0);
-            fetch_subtile(b, a.tab, w.x0, k0 + kOzTileK, tid, t1);
+#pragma unroll 1
+        for (int k0 = 0; k0 < b.K; k0 += kOzTileK) {
+            SubTile t;
+            fetch_subtile(b, a.tab, w.x0, k0, tid, t);
 #pragma unroll
-            for (int j = 0; j < 16; ++j) mx[j] = fmax(mx[j], fmax(fabs(t0.v[j]), fabs(t1.v[j])));
+            for (int j = 0; j < 16; ++j) mx[j] = fmax(mx[j], fabs(t.v[j]));
         }
         // rows adjacent: thread holds row tid%32 for 16 k; else 16 rows
         __syncthreads();
@@ -152,24 +154,18 @@ __device__ __forceinline__ uint32_t crt_digit(int v, int p, int c17, int u, uint
     return tt;
 }
 
-// Residue of an exact integer |v| < 2^52 held in a double, in [0, p):
-// q = floor(v / p) from the rounded reciprocal is off by at most one, and
-// v - p q is exact (fma of integers below 2^53).  (The residue panels use
-// the cheaper limb / Barrett form below; this serves the GEMM epilogue.)
-__device__ __forceinline__ int mod_exact(double v, double p, double rp) {
-    const double q = floor(v * rp);
-    double r = fma(-p, q, v);
-    if (r < 0.0) r += p;
-    if (r >= p) r -= p;
-    return (int)r;
-}
-
 // Persistent workgroups over 32 x 128 conversion tiles: the next tile's
 // values are loaded into registers while the current one (transposed
 // through LDS) is converted to balanced residues (|r| <= 127) for every
 // modulus and written as 16-byte row pieces of the block's panel in each
 // modulus plane.  Panel bytes for k in [K, Kp) are written as zeros.
-__global__ __launch_bounds__(256) void to_residues_kernel(OzConvArgs a) {
+//
+// A residue costs two four-byte dot products, an FP32 quotient and one 24-bit
+// multiply-add (FP32 and 24-bit products run at full rate, the high half of a
+// 32-bit product at a quarter of it): the full ring batch (40 million operand
+// elements, 14 moduli, 0.9 GB) takes 297 us, and took 406 with Barrett
+// reduction of three limbs and a branch at every load.
+__global__ __launch_bounds__(256, 4) void to_residues_kernel(OzConvArgs a) {
     __shared__ double S[kOzTileX][kOzTileK + 1];
     const int tid = threadIdx.x;
     int it = blockIdx.x;
@@ -195,33 +191,44 @@ __global__ __launch_bounds__(256) void to_residues_kernel(OzConvArgs a) {
         if (x >= cb.X || k >= cb.Kp) continue;
         const int e = a.expo[cb.exp_off + x];
         const int shift = e == INT_MIN ? 0 : (a.c.P - 1) - e;
-        // each scaled integer v (|v| <= 2^51, exact in FP64) split once into
-        // v = h2 2^34 + h1 2^17 + h0 with h0, h1 in [0, 2^17), |h2| <= 2^17
-        int h0[16], h1[16], h2[16];
+        // each scaled value, rounded to an integer V (|V| <= 2^51; the sum with
+        // 1.5 2^52 rounds to nearest even and leaves V in the low bits), as seven
+        // digits base 256 in [-128, 127]: the bytes of V + 128 (1 + 256 + ..
+        // + 256^5), the six low ones less 128
+        int lo[16], hi[16];
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
-            const double v = e == INT_MIN ? 0.0 : rint(ldexp(S[xx][kc + j], shift));
-            const double d2 = floor(v * 0x1p-34);
-            const double r1 = fma(-d2, 0x1p34, v); // exact, in [0, 2^34)
-            const double d1 = floor(r1 * 0x1p-17);
-            h2[j] = (int)d2;
-            h1[j] = (int)d1;
-            h0[j] = (int)fma(-d1, 0x1p17, r1);
+            const double v = e == INT_MIN ? 0.0 : ldexp(S[xx][kc + j], shift);
+            const unsigned long long digits =
+                (unsigned long long)__double_as_longlong(v + 0x1.8p52) +
+                (0x0000808080808080ull - 0x4338000000000000ull);
+            lo[j] = (int)((uint32_t)digits ^ 0x80808080u);
+            hi[j] = (int)((uint32_t)(digits >> 32) ^ 0x00008080u);
         }
         int8_t *dst = a.planes + cb.panel_off + (long long)x * cb.Kp + k;
         for (int i = 0; i < a.c.n; ++i) {
-            const int p = a.c.p[i], c17 = a.c.c17[i], c34 = a.c.c34[i], off = a.c.off[i];
-            const uint32_t bar = a.c.bar[i];
-            uint32_t word[4] = {0u, 0u, 0u, 0u};
+            const int c0 = a.c.d0[i], c1 = a.c.d1[i], np = -a.c.p[i];
+            const float rp = a.c.rpf[i];
+            uint32_t word[4];
 #pragma unroll
-            for (int j = 0; j < 16; ++j) {
-                // t = v mod p up to a multiple of p, in (0, 2^28): 24-bit products
-                const int t = __mul24(h2[j], c34) + __mul24(h1[j], c17) + h0[j] + off;
-                const uint32_t q = __umulhi((uint32_t)t, bar); // floor(t/p) or one less
-                int r = t - __mul24((int)q, p);                  // in [0, 2p)
-                if (r >= p) r -= p;
-                if (r > p / 2) r -= p; // balanced, |r| <= 127
-                word[j >> 2] |= (uint32_t)(uint8_t)(int8_t)r << (8 * (j & 3));
+            for (int j = 0; j < 16; j += 4) {
+                uint32_t res[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    // t = digits . (256^j mod p), |t| < 2^17, congruent to V; as the
+                    // low bits of the float 1.5 2^23 + t, since 0x4b400000 is 1.5 2^23
+                    const int t = __builtin_amdgcn_sdot4(
+                        hi[j + q], c1,
+                        __builtin_amdgcn_sdot4(lo[j + q], c0, 0x4b400000, false), false);
+                    // round(t / p) in the low bits: the quotient is at least 1/510 from
+                    // a half (p = 254: or on it, and either neighbour will do), its
+                    // error below 2^-13, so |t - p round(t / p)| <= 127
+                    const float f = __fmaf_rn(__int_as_float(t) - 0x1.8p23f, rp, 0x1.8p23f);
+                    // the two 0x4b400000 leave the low byte as it is
+                    res[q] = (uint32_t)(t + __mul24(__float_as_int(f), np));
+                }
+                word[j >> 2] = __builtin_amdgcn_perm(res[1], res[0], 0x0c0c0400u) |
+                               __builtin_amdgcn_perm(res[3], res[2], 0x04000c0cu);
             }
             *reinterpret_cast<int32x4 *>(dst + (long long)i * a.plane_bytes) =
                 int32x4{(int)word[0], (int)word[1], (int)word[2], (int)word[3]};
@@ -427,14 +434,6 @@ struct U128 {
     unsigned long long lo, hi;
 };
 
-__device__ __forceinline__ void mad_small(U128 &acc, unsigned long long t, const uint64_t m[2]) {
-    const unsigned long long plo = t * m[0];
-    const unsigned long long phi = __umul64hi(t, m[0]) + t * m[1];
-    const unsigned long long lo = acc.lo + plo;
-    acc.hi += phi + (lo < plo ? 1ull : 0ull);
-    acc.lo = lo;
-}
-
 // A signed 128-bit value correctly rounded to FP64.
 __device__ __forceinline__ double to_double(U128 v) {
     const bool neg = (long long)v.hi < 0;
@@ -457,77 +456,117 @@ __device__ __forceinline__ double to_double(U128 v) {
     return neg ? -d : d;
 }
 
-// One workgroup per kOzRecChunk result elements of a task, walked in the
-// task's element order (the destination's memory order where it has a
-// unit-stride index).  Explicit CRT: with t_i = r_i u_i mod p_i,
-// C = sum_i t_i (M/p_i) - q M for q = round(sum_i t_i / p_i), exact in FP64
-// because |C| <= M/4 keeps that sum a quarter away from the rounding
-// boundary.  C is formed exactly modulo 2^128 (|C| < 2^111), rounded once
-// to FP64 and scaled by the operands' powers of two.
+// One workgroup per kOzRecChunk result elements of a task, four to a thread,
+// walked in the task's element order (the destination's memory order where it
+// has a unit-stride index).  Explicit CRT: with t_i = r_i u_i mod p_i,
+// C = sum_i t_i (M/p_i) - q M for q = round(sum_i t_i / p_i); |C| <= M/4 keeps
+// that sum a quarter away from the rounding boundary, so 1/p_i in 16 bits
+// (0.03 off over 14 moduli) gives q.  C is formed exactly modulo 2^128
+// (|C| < 2^111), rounded once to FP64 and scaled by the operands' powers of
+// two.
+//
+// Both sums are byte dot products: the planes' words of four elements are
+// transposed into words of four moduli's t_i each, q takes the place after
+// the last modulus, and byte b of every M/p_i and of -M gives the sum S_b
+// (< 2^20) of weight 256^b.
+// Bound by instruction issue: 64 dot products an element, about as many more
+// to put the sums together and to find the destination.  A full ring batch
+// (15 blocks of up to 450 x 900, 20 million elements, 14 moduli, 0.6 GB): 189
+// us; with 128-bit products per modulus (64-bit integer and FP64 units) 282.
+// One round of 1024 elements a workgroup, all planes loaded at once: a batch
+// of 4800 elements takes 7 us instead of 20, which were load latencies.
+template <int NW>
 __global__ __launch_bounds__(256) void reconstruct_kernel(OzRecArgs a) {
-    for (int it = blockIdx.x; it < a.nitems; it += gridDim.x) {
-        const OzRecItem w = a.items[it];
-        const OzTask task = a.tasks[w.task];
-        const int total = task.M * task.N;
-        const int e1 = min(w.e0 + kOzRecChunk, total);
-        const uint8_t *res = a.res_planes + task.res_off;
-        // four consecutive elements per thread: one 32-bit load per plane
-        // (task regions start 16-byte aligned and planes end 16 bytes past
-        // the last region, so the word never leaves the plane)
-        for (int e0 = w.e0 + 4 * (int)threadIdx.x; e0 < e1; e0 += 4 * (int)blockDim.x) {
-            U128 acc[4] = {{0ull, 0ull}, {0ull, 0ull}, {0ull, 0ull}, {0ull, 0ull}};
-            double s[4] = {0.0, 0.0, 0.0, 0.0};
-            // moduli four at a time: the four planes' words are loaded
-            // before any is used, so their latencies overlap
-            for (int i0 = 0; i0 < a.c.n; i0 += 4) {
-                uint32_t w4[4];
+    typedef double f64x2 __attribute__((ext_vector_type(2), aligned(8)));
+    typedef __attribute__((address_space(1))) double gdouble_t;
+    typedef __attribute__((address_space(1))) f64x2 gf64x2_t;
+    const OzRecItem w = a.items[blockIdx.x];
+    const OzTask task = a.tasks[w.task];
+    const int e1 = min(w.e0 + kOzRecChunk, task.M * task.N);
+    const int e0 = w.e0 + 4 * (int)threadIdx.x;
+    if (e0 >= e1) return;
+    // one 32-bit load per plane for the thread's four elements, all before any
+    // is used (task regions start 16-byte aligned and planes end 16 bytes past
+    // the last region, so the word never leaves the plane)
+    const uint8_t *res = a.res_planes + task.res_off + e0;
+    uint32_t w4[4 * NW];
 #pragma unroll
-                for (int d = 0; d < 4; ++d)
-                    w4[d] = i0 + d < a.c.n
-                                ? *reinterpret_cast<const uint32_t *>(
-                                      res + (long long)(i0 + d) * a.res_plane_bytes + e0)
-                                : 0u;
+    for (int i = 0; i < 4 * NW; ++i)
+        w4[i] = i < 4 * (NW - 1) || i < a.c.n
+                    ? *reinterpret_cast<const uint32_t *>(res + (long long)i * a.res_plane_bytes)
+                    : 0u;
+    // destinations and exponents (past the end the last element's again, which
+    // is not stored)
+    gdouble_t *dst[4];
+    int beta[4], ea[4], eb[4];
+    {
+        const int fast = task.nfast ? task.N : task.M;
+        int slow = e0 / fast, quick = e0 - slow * fast;
 #pragma unroll
-                for (int d = 0; d < 4; ++d) {
-                    if (i0 + d >= a.c.n) break;
-                    const int i = i0 + d;
-                    const double rp = a.c.rp[i];
-                    const uint64_t mi[2] = {a.c.mi[i][0], a.c.mi[i][1]};
+        for (int q = 0; q < 4; ++q) {
+            const int m = task.nfast ? slow : quick, n = task.nfast ? quick : slow;
+            ea[q] = a.expo[task.expA + m];
+            eb[q] = a.expo[task.expB + n];
+            dst[q] = (gdouble_t *)oz_dest(task, a.subs, a.tab, m, n, beta[q]);
+            if (e0 + q + 1 < e1 && ++quick == fast) quick = 0, ++slow;
+        }
+    }
+    // byte k of t[q][g]: t_i of element q, modulus i = 4 g + k
+    uint32_t t[4][NW];
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const unsigned t = (w4[d] >> (8 * q)) & 0xffu;
-                        s[q] += (double)t * rp;
-                        mad_small(acc[q], (unsigned long long)t, mi);
-                    }
-                }
+    for (int q = 0; q < 4; ++q) {
+        uint32_t s0 = 1u << 15, s1 = 0u;
+#pragma unroll
+        for (int g = 0; g < NW; ++g) {
+            const uint32_t sel = 0x0c0c0400u + 0x0101u * q;
+            t[q][g] = __builtin_amdgcn_perm(w4[4 * g + 1], w4[4 * g], sel) |
+                      __builtin_amdgcn_perm(w4[4 * g + 3], w4[4 * g + 2], sel) << 16;
+            s0 = __builtin_amdgcn_udot4(t[q][g], a.c.inv[0][g], s0, false);
+            s1 = __builtin_amdgcn_udot4(t[q][g], a.c.inv[1][g], s1, false);
+        }
+        t[q][NW - 1] |= ((s0 + (s1 << 8)) >> 16) << (8 * (a.c.n & 3));
+    }
+    uint32_t pr[4][8]; // S_2k + 256 S_2k+1, weight 2^16k
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            uint32_t even = 0u, odd = 0u;
+            // M < 2^112: bytes 14 and 15 are those of -M alone
+#pragma unroll
+            for (int g = k < 7 ? 0 : NW - 1; g < NW; ++g) {
+                even = __builtin_amdgcn_udot4(t[q][g], a.c.crt[2 * k][g], even, false);
+                odd = __builtin_amdgcn_udot4(t[q][g], a.c.crt[2 * k + 1][g], odd, false);
             }
+            pr[q][k] = even + (odd << 8);
+        }
+        __builtin_amdgcn_sched_barrier(0); // the constants in turn: all at once spill
+    }
+    double v[4];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int e = e0 + q;
-                if (e >= e1) break;
-                int m, n;
-                if (task.nfast) {
-                    m = e / task.N;
-                    n = e - m * task.N;
-                } else {
-                    n = e / task.M;
-                    m = e - n * task.M;
-                }
-                U128 qm{0ull, 0ull};
-                mad_small(qm, (unsigned long long)rint(s[q]), a.c.m);
-                const U128 C{acc[q].lo - qm.lo,
-                             acc[q].hi - qm.hi - (acc[q].lo < qm.lo ? 1ull : 0ull)};
-                const int ea = a.expo[task.expA + m], eb = a.expo[task.expB + n];
-                double v = 0.0;
-                if (ea != INT_MIN && eb != INT_MIN) {
-                    const int sa = (a.c.P - 1) - ea, sb = (a.c.P - 1) - eb;
-                    v = ldexp(to_double(C), -(sa + sb));
-                }
-                int beta;
-                double *p = oz_dest(task, a.subs, a.tab, m, n, beta);
-                if (beta) v += *p;
-                *p = v;
-            }
+    for (int q = 0; q < 4; ++q) {
+        auto two = [](uint32_t x, uint32_t y) {
+            return (unsigned long long)x + ((unsigned long long)y << 16);
+        };
+        const unsigned long long low = two(pr[q][0], pr[q][1]), mid = two(pr[q][2], pr[q][3]);
+        U128 C{low + (mid << 32),
+               two(pr[q][4], pr[q][5]) + (two(pr[q][6], pr[q][7]) << 32) + (mid >> 32)};
+        C.hi += C.lo < low ? 1ull : 0ull;
+        v[q] = 0.0;
+        if (ea[q] != INT_MIN && eb[q] != INT_MIN)
+            v[q] = ldexp(to_double(C), -((a.c.P - 1) - ea[q] + ((a.c.P - 1) - eb[q])));
+    }
+    if (e0 + 4 <= e1 && dst[1] == dst[0] + 1 && dst[2] == dst[0] + 2 && dst[3] == dst[0] + 3 &&
+        beta[0] == beta[1] && beta[0] == beta[2] && beta[0] == beta[3]) {
+        gf64x2_t *p = (gf64x2_t *)dst[0];
+        f64x2 x = {v[0], v[1]}, y = {v[2], v[3]};
+        if (beta[0]) x += p[0], y += p[1];
+        p[0] = x, p[1] = y;
+    } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            if (e0 + q >= e1) break;
+            *dst[q] = beta[q] ? v[q] + *dst[q] : v[q];
         }
     }
 }
@@ -581,7 +620,15 @@ hipError_t oz_gemm(const OzGemmArgs &a, hipStream_t s) {
 
 hipError_t oz_reconstruct(const OzRecArgs &a, hipStream_t s) {
     if (a.nitems <= 0) return hipSuccess;
-    hipLaunchKernelGGL(reconstruct_kernel, dim3(grid_for(a.nitems, 65535)), dim3(256), 0, s, a);
+    const dim3 grid(a.nitems);
+    const int words = a.c.n / 4 + 1; // of four: the moduli and q
+    if (words > 4) return hipErrorInvalidValue;
+    if (words == 4)
+        hipLaunchKernelGGL(reconstruct_kernel<4>, grid, dim3(256), 0, s, a);
+    else if (words == 3)
+        hipLaunchKernelGGL(reconstruct_kernel<3>, grid, dim3(256), 0, s, a);
+    else
+        hipLaunchKernelGGL(reconstruct_kernel<2>, grid, dim3(256), 0, s, a);
     return hipGetLastError();
 }
 

@@ -966,6 +966,11 @@ int oz_constants(int n, long long kmax, OzConst &c) {
         M *= (unsigned __int128)kModuli[i];
         log2M += std::log2((double)kModuli[i]);
     }
+    // the bytes of x, lowest first, in place i of each row's words
+    auto put = [](uint32_t (*rows)[kOzMaxModuli / 4], int bytes, int i, unsigned __int128 x) {
+        for (int b = 0; b < bytes; ++b)
+            rows[b][i / 4] |= (uint32_t)(uint8_t)(x >> (8 * b)) << (8 * (i % 4));
+    };
     for (int i = 0; i < n; ++i) {
         const int p = c.p[i];
         long long mi = 1; // (M / p_i) mod p_i
@@ -973,16 +978,17 @@ int oz_constants(int n, long long kmax, OzConst &c) {
             if (j != i) mi = (mi * (c.p[j] % p)) % p;
         c.u[i] = inv_mod((int)mi, p);
         c.c17[i] = (int)((1LL << 17) % p);
-        c.c34[i] = (int)((1LL << 34) % p);
-        c.off[i] = p << 19;
         c.bar[i] = (uint32_t)((1ULL << 32) / (unsigned long long)p);
-        c.rp[i] = 1.0 / p;
-        const unsigned __int128 Mi = M / (unsigned __int128)p;
-        c.mi[i][0] = (uint64_t)Mi;
-        c.mi[i][1] = (uint64_t)(Mi >> 64);
+        for (int j = 0; j < 7; ++j) {
+            int d = (int)((1LL << (8 * j)) % p);
+            if (2 * d > p) d -= p;
+            (j < 4 ? c.d0 : c.d1)[i] |= (int32_t)((uint32_t)(uint8_t)d << (8 * (j & 3)));
+        }
+        c.rpf[i] = 1.0f / (float)p;
+        put(c.inv, 2, i, (unsigned __int128)((65536 + p / 2) / p));
+        put(c.crt, 16, i, M / (unsigned __int128)p);
     }
-    c.m[0] = (uint64_t)M;
-    c.m[1] = (uint64_t)(M >> 64);
+    put(c.crt, 16, n, -M);
     // |C| <= K 2^(2P-2) <= M / 4
     const double lk = std::log2((double)std::max<long long>(kmax, 1));
     int P = (int)std::floor((log2M - 2.0 - lk) / 2.0) + 1;
