@@ -18,11 +18,14 @@ constexpr int kOzSmallTile = 64;
 constexpr int kOzWorkSlot = kOzBM * kOzBN;
 // edge of the output tile a GEMM tile code stands for
 constexpr int oz_tile_size(int code) { return code == kOzWideTile ? kOzBigTile : code; }
+// most workgroups of one launch over a tile list (a multiple of the XCDs)
+constexpr int kOzMaxGrid = 1 << 22;
 constexpr int kOzChunk = 16;            // bytes of k per panel chunk
 constexpr int kOzStage = 128;           // bytes of k per GEMM pipeline stage
 constexpr int kOzStageChunks = kOzStage / kOzChunk;
 constexpr int kOzZero = 256;            // zero bytes at the start of every residue plane
-// FP64 panels: units of 16 rows x 8 k, 1 KiB in MFMA operand order (packed.hip)
+// Panels hold 16 rows together: residue panels 16 bytes of k of each (256-byte
+// units), FP64 panels 8 k of each, 1 KiB in MFMA operand order (packed.hip)
 constexpr int kPanelRows = 16, kPanelK = 8, kPanelUnit = 1024;
 constexpr int kOzTileX = 32, kOzTileK = 128; // conversion tile (rows x k)
 constexpr int kOzRecChunk = 1024;       // result elements per reconstruction workgroup
@@ -46,27 +49,35 @@ struct OzConst {
 };
 
 // One operand block as the split path sees it: K x X through its tables,
-// converted once per execution into X row-major residue rows of Kp bytes
-// (K rounded up to a whole chunk, zero filled).
+// converted once per execution into X residue rows of Kp bytes (K rounded up
+// to a whole chunk, zero filled).
 struct OzBlock {
     const double *data;
     int K, X, Kp;
     int ktab, xtab;        // offsets of its k / x tables in the pool
     int exp_off;           // first exponent of its row component
     int xfast;             // 1: consecutive rows are adjacent in memory
-    int row0;              // FP64: its first row in the panel (stacked operands)
+    int row0;              // its first row in the panel (stacked operands)
     long long panel_off;   // byte offset of the panel inside each plane
 };
 
 // A piece of a task's virtual K.  Residue planes: 16 bytes of k, the left and
-// right operands' row 0 at bytes a and b, row r at r * stride bytes more.
+// right operands' first 16 rows in the 256-byte units a and b (16 bytes a row).
 // Planes of doubles: 8 k, the operands' first 16 rows in the 1 KiB units a and
-// b, the next 16 rows `stride` units on.
+// b.  The next 16 rows are `stride` units on; it stands beside either, so that
+// a lane that reads one operand takes what it needs with one 8-byte load.
 struct OzChunkRef {
-    uint32_t a, b;
+    uint32_t a;
     int32_t stride;
-    int32_t pad;
+    uint32_t b;
+    int32_t stride_b; // = stride
 };
+
+// Byte of a residue plane where row r of the chunk at unit `at` lies.
+__device__ __forceinline__ long long oz_row(uint32_t at, int r, int32_t stride) {
+    return (long long)(at + (uint32_t)(r >> 4) * (uint32_t)stride) * (kPanelRows * kOzChunk) +
+           (r & 15) * kOzChunk;
+}
 
 // One result block of a merged task: where its elements go.
 struct OzSub {
@@ -115,7 +126,8 @@ __device__ __forceinline__ double *oz_dest(const OzTask &t, const OzSub *subs, c
 // fixup list, part is the tile's first slot and s0 its number of segments.
 struct OzTile {
     int task, mt, nt, part;
-    int s0, s1, pad0, pad1;
+    int s0, s1;
+    int mod, pad; // split path: the tile's modulus
 };
 
 // Conversion work item: rows [x0, x0 + kOzTileX) and k [k0, k0 + kOzTileK) of a block.

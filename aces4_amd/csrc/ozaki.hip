@@ -157,14 +157,15 @@ __device__ __forceinline__ uint32_t crt_digit(int v, int p, int c17, int u, uint
 // Persistent workgroups over 32 x 128 conversion tiles: the next tile's
 // values are loaded into registers while the current one (transposed
 // through LDS) is converted to balanced residues (|r| <= 127) for every
-// modulus and written as 16-byte row pieces of the block's panel in each
-// modulus plane.  Panel bytes for k in [K, Kp) are written as zeros.
+// modulus and written to the block's panel in each modulus plane, the 16-byte
+// pieces of 16 rows next to each other (a unit, 256 bytes).  Panel bytes for k
+// in [K, Kp) are written as zeros.
 //
 // A residue costs two four-byte dot products, an FP32 quotient and one 24-bit
 // multiply-add (FP32 and 24-bit products run at full rate, the high half of a
 // 32-bit product at a quarter of it): the full ring batch (40 million operand
-// elements, 14 moduli, 0.9 GB) takes 297 us, and took 406 with Barrett
-// reduction of three limbs and a branch at every load.
+// elements, 14 moduli, 0.9 GB) takes 225 us; panels of rows instead of units
+// 297, and with Barrett reduction of three limbs and a branch at every load 406.
 __global__ __launch_bounds__(256, 4) void to_residues_kernel(OzConvArgs a) {
     __shared__ double S[kOzTileX][kOzTileK + 1];
     const int tid = threadIdx.x;
@@ -186,7 +187,7 @@ __global__ __launch_bounds__(256, 4) void to_residues_kernel(OzConvArgs a) {
             b = a.blocks[w.block];
             fetch_subtile(b, a.tab, w.x0, w.k0, tid, next);
         }
-        const int xx = tid >> 3, kc = (tid & 7) * 16; // 8 lanes: one 128-byte row piece
+        const int xx = tid & 31, kc = (tid >> 5) * 16; // 16 lanes: the 256 bytes of a unit
         const int x = cw.x0 + xx, k = cw.k0 + kc;
         if (x >= cb.X || k >= cb.Kp) continue;
         const int e = a.expo[cb.exp_off + x];
@@ -205,7 +206,9 @@ __global__ __launch_bounds__(256, 4) void to_residues_kernel(OzConvArgs a) {
             lo[j] = (int)((uint32_t)digits ^ 0x80808080u);
             hi[j] = (int)((uint32_t)(digits >> 32) ^ 0x00008080u);
         }
-        int8_t *dst = a.planes + cb.panel_off + (long long)x * cb.Kp + k;
+        const int row = cb.row0 + x;
+        int8_t *dst = a.planes + cb.panel_off + (long long)(row >> 4) * cb.Kp * kPanelRows +
+                      (k / kOzChunk) * (kPanelRows * kOzChunk) + (row & 15) * kOzChunk;
         for (int i = 0; i < a.c.n; ++i) {
             const int c0 = a.c.d0[i], c1 = a.c.d1[i], np = -a.c.p[i];
             const float rp = a.c.rpf[i];
@@ -236,7 +239,7 @@ __global__ __launch_bounds__(256, 4) void to_residues_kernel(OzConvArgs a) {
     }
 }
 
-// INT8 GEMM over residue panels, one modulus per blockIdx.y.  Workgroup tile
+// INT8 GEMM over residue panels, a tile of one modulus per entry of the list.  Workgroup tile
 // BM x BN (4 waves, 2 x 2, each (BM/2) x (BN/2)); the task's virtual K runs
 // in stages of 128 bytes = 8 chunks, double-buffered in LDS; loads run two
 // stages ahead through two register sets (16 bytes per lane each): the
@@ -249,7 +252,7 @@ __global__ __launch_bounds__(256, 4) void to_residues_kernel(OzConvArgs a) {
 // bytes.  MFMA v_mfma_i32_16x16x64_i8: lane l holds row l%16, bytes
 // 16*(l/16) .. +15 of a 64-byte k step; accumulator register r of lane l is
 // C(4*(l/16) + r, l%16).
-template <int BM, int BN, int WM, int WN, int MINB, int SETS>
+template <int BM, int BN, int WM, int WN, int MINB>
 __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_i8_kernel(OzGemmArgs a) {
     constexpr int NT = 64 * WM * WN; // threads
     constexpr int TM = BM / WM, TN = BN / WN, FM = TM / 16, FN = TN / 16;
@@ -270,14 +273,13 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_i8_kernel(OzGemmArgs 
     const int wm = wave % WM, wn = wave / WM;
     const int li = lane & 15, lk = lane >> 4;
     const int g = (lane & 7) ^ (lane >> 3); // chunk of the stage this lane loads
-    const int mod = blockIdx.y;
-    const int p = a.c.p[mod], u = a.c.u[mod], c17 = a.c.c17[mod];
-    const uint32_t bar = a.c.bar[mod];
-    gi8_t *plane = (gi8_t *)(a.planes + (long long)mod * a.plane_bytes);
-
     for (int t = blockIdx.x; t < a.ntiles; t += gridDim.x) {
         const OzTile tile = a.tiles[t];
         if (tile.task < 0) continue;
+        const int mod = tile.mod;
+        const int p = a.c.p[mod], u = a.c.u[mod], c17 = a.c.c17[mod];
+        const uint32_t bar = a.c.bar[mod];
+        gi8_t *plane = (gi8_t *)(a.planes + (long long)mod * a.plane_bytes);
         const OzTask task = a.tasks[tile.task];
         const int m0 = tile.mt * BM, n0 = tile.nt * BN;
         int ra[IA], rb[IB];
@@ -294,10 +296,9 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_i8_kernel(OzGemmArgs 
 
         const OzChunkRef *ch = a.chunks + task.chunk0;
         const int nst = task.nchunks / CH; // even: the planner pads to pairs of stages
-        // SETS == 2: two register sets, the loads of stage s + 2 are issued
-        // while stage s is multiplied and land in LDS after stage s + 1;
-        // SETS == 1 (the 64 x 128 wave tiles): one set, one stage ahead
-        int32x4 xa[IA], xb[IB], ya[SETS == 2 ? IA : 1], yb[SETS == 2 ? IB : 1];
+        // two register sets: the loads of stage s + 2 are issued while stage s
+        // is multiplied and land in LDS after stage s + 1
+        int32x4 xa[IA], xb[IB], ya[IA], yb[IB];
         auto put = [&](int buf, const int32x4 *va, const int32x4 *vb) {
 #pragma unroll
             for (int i = 0; i < IA; ++i)
@@ -362,28 +363,13 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_i8_kernel(OzGemmArgs 
 #pragma unroll
             for (int i = 0; i < IA; ++i)
                 va[i] = *reinterpret_cast<const __attribute__((address_space(1))) int32x4 *>(
-                    plane + e.a + ra[i] * e.stride);
+                    plane + oz_row(e.a, ra[i], e.stride));
 #pragma unroll
             for (int i = 0; i < IB; ++i)
                 vb[i] = *reinterpret_cast<const __attribute__((address_space(1))) int32x4 *>(
-                    plane + e.b + rb[i] * e.stride);
+                    plane + oz_row(e.b, rb[i], e.stride));
         };
         load_window(0);
-        if constexpr (SETS == 1) {
-            fetch2(entry(0), xa, xb);
-            put(0, xa, xb);
-            __syncthreads();
-            int buf = 0;
-            for (int s = 0; s < nst; ++s) {
-                if (s + 1 < nst && ((s + 1) * CH) % kWin == 0) load_window(s + 1);
-                fetch2(entry(s + 1), xa, xb);
-                __builtin_amdgcn_sched_barrier(0); // keep the loads ahead of the MFMAs
-                compute(buf);
-                put(buf ^ 1, xa, xb); // after the last stage this writes a copy nothing reads
-                __syncthreads();
-                buf ^= 1;
-            }
-        } else {
         fetch2(entry(0), xa, xb);
         fetch2(entry(1), ya, yb);
         put(0, xa, xb);
@@ -404,7 +390,6 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_i8_kernel(OzGemmArgs 
             compute(1);
             put(0, xa, xb); // after the last pair of stages this writes a copy nothing reads
             __syncthreads();
-        }
         }
 
         // t = (C mod p) u mod p of the tile into this modulus' result plane,
@@ -427,6 +412,163 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_i8_kernel(OzGemmArgs 
                 }
             }
     }
+}
+
+// The INT8 GEMM with a 256 x 256 workgroup tile, eight waves of 64 x 128.
+//
+// Operands go from memory into LDS directly (buffer_load_dwordx4 .. lds: no
+// registers, no LDS store instructions), 64 bytes of virtual K a stage, through
+// four stage buffers of 32 KiB: the loads of stage s + 3 are issued while
+// stage s is multiplied.  A wave waits for its own loads of stage s (those of
+// the two stages behind it stay in flight), then one barrier says that
+// everybody's have landed and that nobody still reads stage s - 1, whose
+// buffer the new loads fill.  A unit of a buffer is 16 rows x 64 bytes in MFMA
+// operand order (lane l: row l % 16, bytes 16 (l / 16) ..), so both the loads
+// and the fragment reads are linear in the lane.  The buffers are separate
+// variables: the compiler then knows that a read of one does not depend on the
+// loads into the others.  A lane holds the chunk entries of the next four
+// stages.
+//
+// The product is formed transposed (B as the MFMA's row operand), so a lane's
+// four accumulators are four consecutive columns of one row and leave as one
+// 4-byte store.
+//
+// Bound by the card's power: the full ring batch (2.55e12 INT8 operations in
+// 14 moduli) takes 1.27 ms, 2.0e15 operations a second, what a library's large
+// INT8 product reaches here.  Operands staged through registers, with one LDS
+// latency every eight MFMAs, took 0.32 ms longer.
+__global__ __launch_bounds__(512, 1) void gemm_i8_wide_kernel(OzGemmArgs a) {
+    constexpr int BT = kOzBigTile, FM = 4, FN = 8; // wave grid 4 x 2
+    constexpr int KS = 64, CH = KS / kOzChunk, kUnit = 16 * KS;
+    __shared__ __attribute__((aligned(1024))) int8_t S0[2 * BT * KS], S1[2 * BT * KS],
+        S2[2 * BT * KS], S3[2 * BT * KS];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave & 3, wn = wave >> 2;
+    const int li = lane & 15, lk = lane >> 4;
+    const OzTile tile = a.tiles[blockIdx.x];
+    if (tile.task < 0) return;
+    const int mod = tile.mod;
+    const int p = a.c.p[mod], u = a.c.u[mod], c17 = a.c.c17[mod];
+    const uint32_t bar = a.c.bar[mod];
+    // (buffer loads: the compiler takes a global load into LDS for a flat access
+    // and then waits for all loads at once)
+    const __amdgpu_buffer_rsrc_t plane = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<int8_t *>(a.planes) + (long long)mod * a.plane_bytes, 0,
+        (int)(uint32_t)a.plane_bytes, 0x00020000);
+
+    const OzTask task = a.tasks[tile.task];
+    const int m0 = tile.mt * BT, n0 = tile.nt * BT;
+    // this wave loads four of the stage's 32 units: waves 0-3 those of A,
+    // waves 4-7 those of B; a lane's rows, clamped into the panel
+    const bool side_b = wave >= 4;
+    int row[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int r = ((wave & 3) * 4 + i) * 16 + li;
+        row[i] = side_b ? min(n0 + r, task.N - 1) : min(m0 + r, task.M - 1);
+    }
+    const int nst = task.nchunks / CH; // a multiple of four (the planner pads)
+    // this lane's chunk entry (unit, stride) of stage st on its wave's side (past
+    // the last one: that one's again, whose loads nothing reads)
+    typedef int32_t int32x2 __attribute__((ext_vector_type(2)));
+    typedef const __attribute__((address_space(1))) int32x2 gentry_t;
+    gentry_t *ch = (gentry_t *)(a.chunks + task.chunk0 + lk) + (side_b ? 1 : 0);
+    auto entry = [&](int st) { return ch[min(st, nst - 1) * CH * 2]; };
+    auto fill = [&](int8_t *S, const int32x2 &e) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                plane, (__attribute__((address_space(3))) void *)(S + (wave * 4 + i) * kUnit), 16,
+                (int)oz_row(e[0], row[i], e[1]), 0, 0, 0);
+    };
+    int32x4 acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[i][j] = int32x4{0, 0, 0, 0};
+    // stage st from `cur`; the loads of stage st + 3, whose entry is in `e`, go
+    // to `next`, then e becomes the entry of stage st + 7
+    auto stage = [&](const int8_t *cur, int8_t *next, int32x2 &e, int st) {
+        // vmcnt <= 10, lgkmcnt 0: this wave's loads of stage st have landed (each
+        // stage issues four and an entry; those of two stages are behind them)
+        // and its reads of stage st - 1 are done.  (A fence would wait for all
+        // loads; the empty statements keep the compiler from moving any.)
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0x007a);
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        fill(next, e);
+        asm volatile("" ::: "memory");
+        e = entry(st + 7);
+        __builtin_amdgcn_sched_barrier(0);
+        const int8_t *sa = cur + wm * FM * kUnit + lane * 16;
+        const int8_t *sb = cur + BT * KS + wn * FN * kUnit + lane * 16;
+        // all fragments of the stage at once, the first MFMAs' first: one LDS
+        // latency a stage instead of one every eight MFMAs
+        int32x4 fa[FM], fb[FN];
+        fb[0] = *reinterpret_cast<const int32x4 *>(sb);
+#pragma unroll
+        for (int i = 0; i < FM; ++i) fa[i] = *reinterpret_cast<const int32x4 *>(sa + i * kUnit);
+#pragma unroll
+        for (int j = 1; j < FN; ++j) fb[j] = *reinterpret_cast<const int32x4 *>(sb + j * kUnit);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+                acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fb[j], fa[i], acc[i][j], 0, 0, 0);
+    };
+    if (nst > 0) {
+        // issued in the order of the loop's stages: its waits count loads
+        const int32x2 e0 = entry(0), e1 = entry(1), e2 = entry(2);
+        int32x2 e6 = entry(6), e3, e4, e5;
+        asm volatile("" ::: "memory");
+        fill(S0, e0);
+        asm volatile("" ::: "memory");
+        e3 = entry(3);
+        asm volatile("" ::: "memory");
+        fill(S1, e1);
+        asm volatile("" ::: "memory");
+        e4 = entry(4);
+        asm volatile("" ::: "memory");
+        fill(S2, e2);
+        asm volatile("" ::: "memory");
+        e5 = entry(5);
+        asm volatile("" ::: "memory");
+        for (int st = 0; st < nst; st += 4) {
+            stage(S0, S3, e3, st);
+            stage(S1, S0, e4, st + 1);
+            stage(S2, S1, e5, st + 2);
+            stage(S3, S2, e6, st + 3);
+        }
+    }
+    // t = (C mod p) u mod p of the tile into this modulus' result plane, in
+    // the task's element order
+    uint8_t *res = a.res_planes + (long long)mod * a.res_plane_bytes + task.res_off;
+#pragma unroll
+    for (int i = 0; i < FM; ++i) {
+        const int m = m0 + (wm * FM + i) * 16 + li;
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+            const int n = n0 + (wn * FN + j) * 16 + 4 * lk;
+            uint32_t word = 0;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) word |= crt_digit(acc[i][j][r], p, c17, u, bar) << (8 * r);
+            if (m >= task.M || n >= task.N) continue;
+            if (task.nfast && n + 4 <= task.N) {
+                __builtin_memcpy(res + (long long)m * task.N + n, &word, 4);
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (n + r < task.N)
+                        res[task.nfast ? (long long)m * task.N + n + r
+                                       : (long long)(n + r) * task.M + m] = (uint8_t)(word >> (8 * r));
+            }
+        }
+    }
+    __builtin_amdgcn_s_waitcnt(0); // no load into LDS outlives the workgroup
 }
 
 // 128-bit helpers on {low, high} 64-bit halves (two's complement, mod 2^128).
@@ -609,12 +751,11 @@ hipError_t oz_gemm(const OzGemmArgs &a, hipStream_t s) {
     if (a.ntiles <= 0) return hipSuccess;
     if (a.tile == kOzBigTile) return oz_gemm_big(a, s);
     if (a.tile == kOzWideTile) {
-        hipLaunchKernelGGL((gemm_i8_kernel<kOzBigTile, kOzBigTile, 4, 2, 1, 1>),
-                           dim3(a.ntiles, a.c.n), dim3(512), 0, s, a);
+        gemm_i8_wide_kernel<<<dim3(a.ntiles), 512, 0, s>>>(a);
         return hipGetLastError();
     }
-    hipLaunchKernelGGL((gemm_i8_kernel<kOzBM, kOzBN, 2, 2, 2, 2>), dim3(a.ntiles, a.c.n), dim3(256),
-                       0, s, a);
+    hipLaunchKernelGGL((gemm_i8_kernel<kOzBM, kOzBN, 2, 2, 2>), dim3(grid_for(a.ntiles, kOzMaxGrid)),
+                       dim3(256), 0, s, a);
     return hipGetLastError();
 }
 

@@ -41,14 +41,14 @@ __global__ __launch_bounds__(256, 1) void gemm_i8_big_kernel(OzGemmArgs a) {
     const int wm = wave % WM, wn = wave / WM;
     const int li = lane & 15, lk = lane >> 4;
     const int g = (lane & 3) ^ ((lane >> 3) & 3); // chunk of the stage this lane loads
-    const int mod = blockIdx.y;
-    const int p = a.c.p[mod], u = a.c.u[mod];
-    const uint32_t bar = a.c.bar[mod];
-    gi8_t *plane = (gi8_t *)(a.planes + (long long)mod * a.plane_bytes);
 
     for (int t = blockIdx.x; t < a.ntiles; t += gridDim.x) {
         const OzTile tile = a.tiles[t];
         if (tile.task < 0) continue;
+        const int mod = tile.mod;
+        const int p = a.c.p[mod], u = a.c.u[mod];
+        const uint32_t bar = a.c.bar[mod];
+        gi8_t *plane = (gi8_t *)(a.planes + (long long)mod * a.plane_bytes);
         const OzTask task = a.tasks[tile.task];
         const int m0 = tile.mt * BM, n0 = tile.nt * BN;
         const OzChunkRef *ch = a.chunks + task.chunk0;
@@ -86,11 +86,11 @@ __global__ __launch_bounds__(256, 1) void gemm_i8_big_kernel(OzGemmArgs a) {
 #pragma unroll
             for (int i = 0; i < IA; ++i)
                 va[i] = *reinterpret_cast<const __attribute__((address_space(1))) int32x4 *>(
-                    plane + e.a + ra[i] * e.stride);
+                    plane + oz_row(e.a, ra[i], e.stride));
 #pragma unroll
             for (int i = 0; i < IB; ++i)
                 vb[i] = *reinterpret_cast<const __attribute__((address_space(1))) int32x4 *>(
-                    plane + e.b + rb[i] * e.stride);
+                    plane + oz_row(e.b, rb[i], e.stride));
         };
         auto put = [&](int buf, const int32x4 (&va)[IA], const int32x4 (&vb)[IB]) {
 #pragma unroll
@@ -190,7 +190,8 @@ __global__ __launch_bounds__(256, 1) void gemm_i8_big_kernel(OzGemmArgs a) {
 
 hipError_t oz_gemm_big(const OzGemmArgs &a, hipStream_t s) {
     if (a.ntiles <= 0) return hipSuccess;
-    hipLaunchKernelGGL(gemm_i8_big_kernel, dim3(a.ntiles, a.c.n), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(gemm_i8_big_kernel, dim3(a.ntiles < kOzMaxGrid ? a.ntiles : kOzMaxGrid), dim3(256),
+                       0, s, a);
     return hipGetLastError();
 }
 

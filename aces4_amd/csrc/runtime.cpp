@@ -522,6 +522,36 @@ std::vector<Tile> interleave(const std::vector<std::vector<Tile>> &per_xcd) {
     return tiles;
 }
 
+// The split path's work lists: every tile of `lists` once per modulus.  The
+// pairs, tile after tile in list order, are cut into one piece per XCD of equal
+// stages (a list may end on some of a tile's moduli), and each piece runs
+// modulus by modulus, so that the tiles an XCD runs together share panels.
+// With the lists of xcd_lists for every modulus an XCD got up to a fifth more
+// than its share or a round too many: the 324 tiles of a full ring batch (lists
+// of up to 50) 1.46 ms against 1.27, 20 tiles with 12 moduli 86 us against 52.
+std::vector<std::vector<OzTile>> deal_moduli(const std::vector<std::vector<OzTile>> &lists,
+                                             const OzTask *tasks, int nmod) {
+    // (about 16 chunks' time to start and store a tile)
+    auto cost = [&](const OzTile &u) { return (double)tasks[u.task].nchunks + 16.0; };
+    double total = 0.0, done = 0.0;
+    for (const auto &list : lists)
+        for (const OzTile &u : list) total += cost(u) * nmod;
+    std::vector<std::vector<OzTile>> per(kXcds);
+    for (const auto &list : lists)
+        for (const OzTile &u : list)
+            for (int mod = 0; mod < nmod; ++mod) {
+                const double c = cost(u);
+                const int x = std::min(kXcds - 1, (int)((done + c / 2) / total * kXcds));
+                per[x].push_back(u);
+                per[x].back().mod = mod;
+                done += c;
+            }
+    for (auto &list : per)
+        std::stable_sort(list.begin(), list.end(),
+                         [](const OzTile &a, const OzTile &b) { return a.mod < b.mod; });
+    return per;
+}
+
 template <class Tile>
 std::vector<Tile> xcd_schedule(const std::vector<int> &tm, const std::vector<int> &tn,
                                const std::vector<double> &cost, int &real_tiles) {
@@ -1278,8 +1308,7 @@ int sipgpu::rt::build_panel_plan(const sipgpu_contraction *list, int n, int nmod
         if (it.second) nexpo += insts[ii].X;
         return it.first->second;
     };
-    // places instance ii at `panel` (split path), or as rows row0, row0 + 1, ..
-    // of the FP64 panel there
+    // instance ii as rows row0, row0 + 1, .. of the panel at `panel`
     auto place = [&](int ii, int exp_off, int row0) {
         const Inst &in = insts[ii];
         OzBlock ob{};
@@ -1293,16 +1322,14 @@ int sipgpu::rt::build_panel_plan(const sipgpu_contraction *list, int n, int nmod
         ob.exp_off = exp_off;
         ob.row0 = row0;
         ob.panel_off = panel;
-        if (nmod) panel += (long long)in.X * in.Kp;
         blocks.push_back(ob);
         return (int)blocks.size() - 1;
     };
-    // the end of a panel of `rows` rows of Kp k
+    // the end of a panel of `rows` rows of Kp k; `unit` bytes of panel per 16
+    // rows x kq k
+    const long long unit = nmod ? kPanelRows * kOzChunk : kPanelUnit;
     auto close_panel = [&](int rows, int Kp) {
-        if (nmod)
-            panel = (panel + 255) / 256 * 256;
-        else
-            panel += (long long)((rows + kPanelRows - 1) / kPanelRows) * (Kp / kPanelK) * kPanelUnit;
+        panel += (long long)((rows + kPanelRows - 1) / kPanelRows) * (Kp / kq) * unit;
     };
     std::vector<OzChunkRef> chunks;
     for (int t = 0; t < ntasks; ++t) {
@@ -1338,7 +1365,7 @@ int sipgpu::rt::build_panel_plan(const sipgpu_contraction *list, int n, int nmod
             int off = 0;
             for (int key : keys) {
                 const int ii = vec[key][p];
-                place(ii, exp0 + off, nmod ? 0 : off);
+                place(ii, exp0 + off, off);
                 off += insts[ii].X;
             }
             close_panel(off, insts[vec[keys[0]][p]].Kp);
@@ -1353,16 +1380,13 @@ int sipgpu::rt::build_panel_plan(const sipgpu_contraction *list, int n, int nmod
             const long long la = stack(0, p), lb = stack(1, p);
             const int Kp = insts[rvec[rs[0]][p]].Kp;
             for (int k = 0; k < Kp; k += kq)
-                chunks.push_back(nmod ? OzChunkRef{(uint32_t)(la + k), (uint32_t)(lb + k), Kp, 0}
-                                      : OzChunkRef{(uint32_t)(la / kPanelUnit + k / kPanelK),
-                                                   (uint32_t)(lb / kPanelUnit + k / kPanelK),
-                                                   Kp / kPanelK, 0});
-            if (panel >= (nmod ? 1LL << 32 : 1LL << 36) - (nmod ? 65536 : 16 * 65536))
-                return fail(SIPGPU_ESIZE, nmod ? "split path: operand panels exceed 4 GiB per modulus"
-                                               : "packed path: operand panels exceed 64 GiB");
+                chunks.push_back(OzChunkRef{(uint32_t)(la / unit + k / kq), Kp / kq,
+                                            (uint32_t)(lb / unit + k / kq), Kp / kq});
+            if (panel >= (1LL << 36))
+                return fail(SIPGPU_ESIZE, "operand panels exceed 64 GiB");
         }
         while (nmod && (chunks.size() - tasks[t].chunk0) % (2 * kOzStageChunks))
-            chunks.push_back(OzChunkRef{0u, 0u, 0, 0});
+            chunks.push_back(OzChunkRef{0u, 0, 0u, 0});
         tasks[t].nchunks = (int)chunks.size() - tasks[t].chunk0;
     }
     // conversion work
@@ -1382,23 +1406,31 @@ int sipgpu::rt::build_panel_plan(const sipgpu_contraction *list, int n, int nmod
         for (long long e0 = 0; e0 < mn; e0 += kOzRecChunk) rec.push_back(OzRecItem{t, (int)e0});
         res_elems += (mn + 15) / 16 * 16;
     }
-    // GEMM tile: 256 x 256 with eight waves of 64 x 128 (two per SIMD, two
-    // thirds of the LDS traffic per MFMA of the 128 x 128 tile) when the batch has at
-    // least one such tile per CU over all moduli, else 128 x 128.  Measured
-    // with 14 moduli: ring 1.98 ms against 2.24 (128) and 2.97 (256, four
-    // waves of 128 x 128, one per SIMD); the block-sparse ladder likewise.
-    // SIPGPU_OZ_TILE=128|256|257 or the tuner pins it.
-    long long big_tiles = 0;
-    for (const OzTask &t : tasks)
+    // GEMM tile: 256 x 256 with eight waves of 64 x 128, or 128 x 128 with four,
+    // by the rounds of workgroups over the CUs that each takes: a round of the
+    // large tile costs 1.4 of one round of the small (34 against 24 us at K =
+    // 2048, 15.5 against 11.5 at K = 256), or 0.84 of two (two of its workgroups
+    // share a CU: 35 against 42, 16.4 against 17.1), so 1.7 against 1 each.
+    // Measured with 14 moduli at K = 2048: 512 x 512 34 us against 26 (one round
+    // of each), 512 x 768 34 against 42, 1024 x 1024 43 against 75, 2048 x 2048
+    // 145 against 239.  SIPGPU_OZ_TILE=128|256|257 or the tuner pins it.
+    long long big_tiles = 0, small_tiles = 0;
+    for (const OzTask &t : tasks) {
         big_tiles += (long long)((t.M + kOzBigTile - 1) / kOzBigTile) *
                      ((t.N + kOzBigTile - 1) / kOzBigTile);
-    int tile = (nmod && big_tiles * nmod >= 256) ? kOzWideTile : kOzBM;
+        small_tiles += (long long)((t.M + kOzBM - 1) / kOzBM) * ((t.N + kOzBN - 1) / kOzBN);
+    }
+    auto rounds = [&](long long tiles) { return (tiles * nmod + 255) / 256; };
+    int tile = nmod && 17 * rounds(big_tiles) < 10 * rounds(small_tiles) ? kOzWideTile : kOzBM;
     if (const char *e = std::getenv("SIPGPU_OZ_TILE")) {
         const int v = std::atoi(e);
         if (nmod && (v == kOzBM || v == kOzBigTile || v == kOzWideTile)) tile = v;
     }
     if (nmod && (opt.tile == kOzBM || opt.tile == kOzBigTile || opt.tile == kOzWideTile))
         tile = opt.tile;
+    // (the wide kernel's buffer loads reach 4 GiB)
+    if (tile == kOzWideTile && panel >= (1LL << 32) - 256) tile = kOzBigTile;
+    if (tile == kOzWideTile && big_tiles * nmod > kOzMaxGrid) tile = kOzBM;
     // the packed FP64 GEMM: 128 x 128 tiles, or 64 x 64 when chosen (small
     // batches cut into K segments write a quarter of the partial sums)
     if (!nmod && opt.tile == kOzSmallTile) tile = kOzSmallTile;
@@ -1432,7 +1464,7 @@ int sipgpu::rt::build_panel_plan(const sipgpu_contraction *list, int n, int nmod
         const int slots = 64 >> (std::min(std::max(opt.tail, 1), 4) - 1);
         persistent_schedule(lists, costs, slots, tiles, wg_first, fix, nslots);
     } else {
-        tiles = interleave(lists);
+        tiles = interleave(nmod ? deal_moduli(lists, tasks.data(), nmod) : lists);
     }
     if (tiles.size() >= (size_t)INT_MAX) return fail(SIPGPU_ESIZE, "split path: too many tiles");
 
