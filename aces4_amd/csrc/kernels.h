@@ -86,7 +86,7 @@ struct GemmArgs {
     int tilesM;
     GemmTask task0;
     GemmPair pair0;
-    // single contraction in K segments (ksplit > 1, split-K tiles only):
+    // single contraction in K segments (ksplit > 1; 64 x 64 and split-K tiles):
     // tile t computes segment s = t / (ntiles / ksplit) of kseg k values;
     // segment 0 goes to task0.D, segment s > 0 is assigned to ws + (s - 1) *
     // ws_stride with task0's destination tables

@@ -118,9 +118,8 @@ Context &ctx() {
 // per device, held until the process ends.  On the host `scratch` names a
 // stand-in, not device memory: init resolves each device's address with
 // hipGetSymbolAddress, and host code only ever passes that address on.
-// A split contraction has at most g_device_cus / 2 tiles of 64 x 64 and
-// four K segments, so its three workspace segments hold at most
-// 3 * 128 * 4096 doubles (12 MiB) on 256 CUs.
+// A split contraction takes at most as many K segments as fit here (all but
+// the first), so both entry points split it the same way.
 constexpr size_t kNoAllocWsDoubles = (size_t)2 << 20; // 16 MiB
 constexpr size_t kNoAllocPartDoubles = (size_t)std::max(kDotBlocks, kEnergyBlocks);
 static __device__ __align__(256) double scratch[kNoAllocWsDoubles + kNoAllocPartDoubles];
@@ -230,10 +229,6 @@ void make_task_pair(const ContractionShape &s, int kL, int mL, int kR, int nR, i
     }
 }
 
-// A single contraction of at most so many 32 x 32 tiles and at least so long
-// a K runs in K segments.
-constexpr int64_t kSegmentTiles = 128, kSegmentK = 768;
-
 // Tile configuration for an M x N block; `kfast`: GemmPair::flags of its
 // first pair.
 int pick_config(int64_t M, int64_t N, int kfast) {
@@ -255,6 +250,54 @@ int pick_config(int64_t M, int64_t N, int kfast) {
     return tiles <= ((kfast & 3) == 3 ? 160 : 512) ? kGemmSplitK : kGemm64x64;
 }
 
+// Tiles and K segments of a single contraction whose block pick_config gave
+// `cfg`.  Where the 64 x 64 tiles fill less than half the chip and K is long,
+// K runs in segments side by side: segment s > 0 into the stream's workspace,
+// then the segments are added to D in order (a fixed summation order).  Either
+// the 32 x 32 tiles (split K) in segments of at least 256 k, which occupy a CU
+// for 18 ns a k (27 where both operands are read along k) whether one or two
+// run there, plus 4 us and the segments' traffic at 5 TB/s for the sums; or
+// the 64 x 64 tiles in up to 8 segments of at least 64 k and two workgroups per
+// CU, 128 ns a k each (100 along k; a fifth less with a CU of their own) plus
+// 13 us of launches, ramp and sums.  The faster by these estimates was within
+// 8% of the faster measured over 100 to 361 small tiles and K of 512 to 4096;
+// in us, 32 x 32 and 64 x 64: 100 tiles, K = 4096 45 and 65; 270 tiles 98 and
+// 92; along k 100 tiles, K = 1024 23 and 24, K = 4096 63 and 55; 270 tiles, K =
+// 2048 79 and 47, and 115 in one segment of 32 x 32 tiles.
+struct SegmentPlan {
+    int cfg, nseg;
+    int64_t kseg;
+};
+SegmentPlan plan_segments(int cfg, int64_t M, int64_t N, int64_t K, int kfast, int64_t dsize,
+                          int64_t cus) {
+    const int64_t big = ((M + 63) / 64) * ((N + 63) / 64);
+    if ((cfg != kGemmSplitK && cfg != kGemm64x64) || big * 2 > cus || K < 256)
+        return {cfg, 1, K};
+    // no more than the 16 MiB of the no-allocation workspace holds, so both
+    // entry points split every shape the same way
+    const int64_t fit = 1 + (int64_t)(kNoAllocWsDoubles / std::max<int64_t>(dsize, 1));
+    const int64_t most = std::max<int64_t>(1, std::min<int64_t>({8, 2 * cus / big, K / 64, fit}));
+    const bool both = (kfast & 3) == 3;
+    int64_t want = most;
+    if (cfg == kGemmSplitK) {
+        const int64_t small = ((M + 31) / 32) * ((N + 31) / 32);
+        double best = 0.0;
+        for (int64_t w = 1; w <= std::min(most, std::max<int64_t>(1, K / 256)); ++w) {
+            const double sums = w > 1 ? 4.0 + 16e-6 / 5.0 * (double)(dsize * w) : 0.0;
+            const double t = 4.0 + sums + (double)((small * w + cus - 1) / cus) * (double)K / w *
+                                              (both ? 0.027 : 0.018);
+            if (w == 1 || t < best) best = t, want = w;
+        }
+        const double each = (both ? 0.1 : 0.128) * (big * most <= cus ? 0.82 : 1.0);
+        if (13.0 + (double)K / most * each < 0.97 * best) {
+            cfg = kGemm64x64;
+            want = most;
+        }
+    }
+    const int64_t kseg = ((K + want - 1) / want + 15) / 16 * 16;
+    return {cfg, (int)((K + kseg - 1) / kseg), kseg};
+}
+
 // One contraction on device pointers (no locking; caller holds the lock).
 // `fx` (may be null) replaces the stream's workspace and partials; with it
 // the call allocates nothing and refuses shapes it would have to plan.
@@ -272,7 +315,11 @@ int contract_device(Context &c, sipgpu_stream_s &st, const int *ptrn, const doub
         GemmPair pair;
         make_task_pair(s, ds->kL, ds->mL, ds->kR, ds->nR, ds->mD, ds->nD, l, r, d,
                        accumulate ? 1 : 0, task, pair);
-        const int cfg = pick_config(task.M, task.N, pair.flags);
+        const SegmentPlan sp =
+            plan_segments(pick_config(task.M, task.N, pair.flags), task.M, task.N, pair.K,
+                          pair.flags, s.dsize, g_device_cus);
+        const int cfg = sp.cfg;
+        int nseg = sp.nseg;
         const int bm = gemm_tile_m(cfg), bn = gemm_tile_n(cfg);
         GemmArgs a{};
         a.tab = tab;
@@ -284,24 +331,6 @@ int contract_device(Context &c, sipgpu_stream_s &st, const int *ptrn, const doub
         task.npairs = 1;
         a.task0 = task;
         a.pair0 = pair;
-        // Few tiles and a long K: split K into segments that run side by
-        // side, segment s > 0 into the stream's workspace, then add the
-        // segments to D in order (a fixed summation order).  Up to 8 segments
-        // of at least 256 k, a workgroup per CU, and no more than the 16 MiB
-        // of the no-allocation workspace holds, so both entry points split
-        // every shape the same way.  The summing pass and its launch cost
-        // about 6 us, a workgroup about 27 ns per k: 225 x 225 x 2000 (64
-        // tiles) 58 us in one segment, 20 + 4 in four; 200 x 200 x 4000 112
-        // and 28 + 4.
-        const int64_t K = pair.K;
-        int nseg = 1, kseg = (int)K;
-        if (cfg == kGemmSplitK && ntiles <= kSegmentTiles && K >= kSegmentK) {
-            const int64_t fit = 1 + (int64_t)(kNoAllocWsDoubles / std::max<int64_t>(s.dsize, 1));
-            const int want = (int)std::max<int64_t>(
-                1, std::min<int64_t>({8, g_device_cus / ntiles, K / 256, fit}));
-            kseg = (int)(((K + want - 1) / want + 15) / 16 * 16);
-            nseg = (int)((K + kseg - 1) / kseg);
-        }
         if (nseg > 1) {
             const size_t need = (size_t)(nseg - 1) * (size_t)s.dsize * sizeof(double);
             if (fx) {
@@ -341,7 +370,7 @@ int contract_device(Context &c, sipgpu_stream_s &st, const int *ptrn, const doub
         if (nseg > 1) {
             double *ws = fx ? fx->ws : st.ws;
             a.ksplit = nseg;
-            a.kseg = kseg;
+            a.kseg = (int)sp.kseg;
             a.ws = ws;
             a.ws_stride = s.dsize;
             a.ntiles = (int)ntiles * nseg;

@@ -104,3 +104,29 @@ def test_blocks_of_both_configurations_in_one_batch():
         sg.synchronize()
         assert np.array_equal(d.download().view(np.uint64), g.view(np.uint64))
         alone.destroy()
+
+
+# single contractions in K segments: of 32 x 32 tiles (fewer and more tiles
+# than CUs), of 64 x 64 tiles, and of neither (K one below the shortest)
+SINGLES = [(320, 320, 1025), (600, 600, 770), (450, 320, 1030), (850, 296, 515), (500, 500, 255),
+           (33, 31, 2500), (1, 1, 5000)]
+
+
+@pytest.mark.parametrize("form", range(3))
+@pytest.mark.parametrize("M, N, K", SINGLES)
+def test_single_contraction_segments(M, N, K, form):
+    sg.init(0)
+    rng = np.random.default_rng([M, N, K, form])
+    print("segments", M, N, K, form, flush=True)
+    ptrn, pairs = pairs_of(rng, FORMS[form], M, N, [K])
+    ld, rd, l, r = pairs[0]
+    D0 = rng.standard_normal(M * N)
+    dl, dr = sg.DeviceArray.from_host(l), sg.DeviceArray.from_host(r)
+    for accumulate in (False, True):
+        d = sg.DeviceArray.from_host(D0)
+        sg.contract(ptrn, dl.ptr, ld, dr.ptr, rd, d.ptr, [M, N], accumulate=accumulate)
+        sg.synchronize()
+        assert rel_fro(d.download(), expected(ptrn, pairs, M, N, D0, accumulate)) <= 1e-13
+        d.free()
+    dl.free()
+    dr.free()
