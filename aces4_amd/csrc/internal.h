@@ -139,6 +139,7 @@ struct PanelPlan {
     long long plane_bytes = 0, res_plane_bytes = 0;
     int nslots = 0; // workspace slots of kOzBM * kOzBN doubles
     OzConst c{};
+    bool skip_halves = false; // OzGemmArgs::skip_halves
     int tile = 0, ntiles = 0, nconv = 0, nrows = 0, nrec = 0, nfix = 0, nwg = 0, nexpo = 0;
     int ndest = 0, ngroups = 0, npairs = 0, real_tiles = 0;
     double flops = 0.0;

@@ -64,13 +64,14 @@ struct OzBlock {
 // A piece of a task's virtual K.  Residue planes: 16 bytes of k, the left and
 // right operands' first 16 rows in the 256-byte units a and b (16 bytes a row).
 // Planes of doubles: 8 k, the operands' first 16 rows in the 1 KiB units a and
-// b.  The next 16 rows are `stride` units on; it stands beside either, so that
-// a lane that reads one operand takes what it needs with one 8-byte load.
+// b.  The next 16 rows are `stride` units on; in a residue panel it stands
+// beside either, so that a lane that reads one operand takes what it needs
+// with one 8-byte load.
 struct OzChunkRef {
     uint32_t a;
     int32_t stride;
     uint32_t b;
-    int32_t stride_b; // = stride
+    int32_t aux; // residues: = stride; doubles: k-steps of four that hold k (1 or 2)
 };
 
 // Byte of a residue plane where row r of the chunk at unit `at` lies.
@@ -150,6 +151,7 @@ struct OzGemmArgs {
     long long res_plane_bytes;
     int ntiles;
     int tile; // tile code: kOzBM (= kOzBN), kOzBigTile, kOzWideTile, kOzSmallTile (FP64)
+    bool skip_halves;   // packed FP64 path: heed OzChunkRef::aux
     const int32_t *tab; // destination tables (packed FP64 path)
     const OzSub *subs;  // result blocks of merged tasks (packed FP64 path)
     double *work;       // split-tile partial products, kOzWorkSlot per slot

@@ -30,7 +30,7 @@ typedef const __attribute__((address_space(4))) OzChunkRef cref_t;
 // Workgroups over 32 x 128 tiles of operand blocks, each done as two halves
 // of 64 k (half the LDS of a whole tile, so twice the workgroups per CU keep
 // their loads in flight): read along the index adjacent in memory,
-// transposed through LDS, written as 128-byte row pieces of the panel.
+// transposed through LDS, written unit by unit.
 __global__ __launch_bounds__(256) void pack_kernel(OzConvArgs a) {
     constexpr int HK = kOzTileK / 2;
     __shared__ __attribute__((aligned(16))) double S[kOzTileX][HK + 2];
@@ -102,7 +102,9 @@ __global__ __launch_bounds__(256) void pack_kernel(OzConvArgs a) {
 // staged through LDS (matrix units busy 82%), 2.82 so (91%; 93% and 2.06 GHz on
 // the block-sparse ladder, 7.31 -> 7.04 ms).  Rows past the task's M / N lie in its last row block or
 // repeat it and are never stored.
-template <int BM, int BN>
+// SKIP: heed the chunks' k-step counts (a pair's last 8 k may hold four or
+// fewer: their second MFMAs would multiply zeros).
+template <int BM, int BN, bool SKIP>
 __global__ __launch_bounds__(256, 2) void gemm_f64_packed_kernel(OzGemmArgs a) {
     constexpr int WM = 2, WN = 2;
     constexpr int TM = BM / WM, TN = BN / WN, FM = TM / 16, FN = TN / 16;
@@ -136,12 +138,14 @@ __global__ __launch_bounds__(256, 2) void gemm_f64_packed_kernel(OzGemmArgs a) {
         cref_t *ch = (cref_t *)(a.chunks + task.chunk0);
         const int sb = tile.s0, se = tile.s1; // stages of this unit
         f64x2 fa[2][FM], fb[2][FN];
+        int steps[2]; // MFMA k-steps of the stage
         // stage s into register set `set` (past the unit's last stage that
         // one again: the loads stay unconditional, nothing reads them)
         auto fetch = [&](int set, int s) {
             const int at = min(s, se - 1);
             const uint32_t ea = ch[at].a, eb = ch[at].b;
             const int stride = ch[at].stride;
+            steps[set] = SKIP ? ch[at].aux : 2;
 #pragma unroll
             for (int i = 0; i < FM; ++i)
                 fa[set][i] = *reinterpret_cast<const __attribute__((address_space(1))) f64x2 *>(
@@ -153,13 +157,15 @@ __global__ __launch_bounds__(256, 2) void gemm_f64_packed_kernel(OzGemmArgs a) {
         };
         auto mma = [&](int set) {
 #pragma unroll
-            for (int h = 0; h < 2; ++h)
+            for (int h = 0; h < 2; ++h) {
+                if (SKIP && h >= steps[set]) break;
 #pragma unroll
                 for (int i = 0; i < FM; ++i)
 #pragma unroll
                     for (int j = 0; j < FN; ++j)
                         acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[set][i][h], fb[set][j][h],
                                                                          acc[i][j], 0, 0, 0);
+            }
         };
         if (sb < se) {
             fetch(0, sb);
@@ -297,11 +303,12 @@ hipError_t oz_pack(const OzConvArgs &a, hipStream_t s) {
 hipError_t oz_gemm_f64(const OzGemmArgs &a, hipStream_t s) {
     if (a.ntiles <= 0) return hipSuccess;
     const dim3 grid(a.wg_first ? a.nwg : a.ntiles);
-    if (a.tile == kOzSmallTile)
-        hipLaunchKernelGGL((gemm_f64_packed_kernel<kOzSmallTile, kOzSmallTile>), grid, dim3(256), 0,
-                           s, a);
-    else
-        hipLaunchKernelGGL((gemm_f64_packed_kernel<kOzBM, kOzBN>), grid, dim3(256), 0, s, a);
+    const bool small = a.tile == kOzSmallTile;
+    auto kernel = small ? (a.skip_halves ? gemm_f64_packed_kernel<kOzSmallTile, kOzSmallTile, true>
+                                         : gemm_f64_packed_kernel<kOzSmallTile, kOzSmallTile, false>)
+                        : (a.skip_halves ? gemm_f64_packed_kernel<kOzBM, kOzBN, true>
+                                         : gemm_f64_packed_kernel<kOzBM, kOzBN, false>);
+    kernel<<<grid, 256, 0, s>>>(a);
     return hipGetLastError();
 }
 

@@ -1408,9 +1408,11 @@ int sipgpu::rt::build_panel_plan(const sipgpu_contraction *list, int n, int nmod
         for (int p = 0; p < np; ++p) {
             const long long la = stack(0, p), lb = stack(1, p);
             const int Kp = insts[rvec[rs[0]][p]].Kp;
+            const int K = insts[rvec[rs[0]][p]].K;
             for (int k = 0; k < Kp; k += kq)
                 chunks.push_back(OzChunkRef{(uint32_t)(la / unit + k / kq), Kp / kq,
-                                            (uint32_t)(lb / unit + k / kq), Kp / kq});
+                                            (uint32_t)(lb / unit + k / kq),
+                                            nmod ? Kp / kq : K - k > 4 ? 2 : 1});
             if (panel >= (1LL << 36))
                 return fail(SIPGPU_ESIZE, "operand panels exceed 64 GiB");
         }
@@ -1539,6 +1541,13 @@ int sipgpu::rt::build_panel_plan(const sipgpu_contraction *list, int n, int nmod
     P.res_plane_bytes = nmod ? (res_elems + 16 + 255) / 256 * 256 : 0; // a word past the last region
     P.nslots = nslots;
     P.tile = tile;
+    // Skipping the empty MFMAs of a pair's last 8 k costs the other stages 3% (a
+    // branch each: the ring term, pairs of 450 k, 3032 us without and 3128 with
+    // it); a (T) tuple's pairs of 20 k (a sixth of the MFMAs empty) take 764 us
+    // without and 696 with it.  The line lies at 5% of the MFMAs.
+    long long halves = 0;
+    for (const OzChunkRef &c : chunks) halves += !nmod && c.aux == 1;
+    P.skip_halves = halves * 10 > (long long)chunks.size();
     P.ntiles = (int)tiles.size();
     P.nconv = (int)conv.size();
     P.nrows = (int)rows.size();
@@ -1590,6 +1599,7 @@ void sipgpu::rt::bind_panel_plan(const PanelPlan &P, void *desc, int8_t *planes,
     g.res_plane_bytes = P.res_plane_bytes;
     g.ntiles = P.ntiles;
     g.tile = P.tile;
+    g.skip_halves = P.skip_halves;
     g.tab = dtab;
     g.subs = dsubs;
     g.work = work;
