@@ -808,7 +808,7 @@ def tune_report(w):
 
 GEMM_KERNEL = {"tables": "gemm_f64_kernel", "packed": "gemm_f64_packed_kernel"}
 PATH_NAME = {"tables": "plain FP64 MFMA, grouped batch, permutations fused into the GEMM loads",
-             "packed": "plain FP64 MFMA, operands packed into K-contiguous panels once per "
+             "packed": "plain FP64 MFMA, operands packed into panels in MFMA operand order once per "
                        "step (pack_kernel), then one grouped GEMM over the panels"}
 
 

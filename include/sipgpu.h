@@ -281,8 +281,8 @@ int sipgpu_batch_plan_split_tol(const sipgpu_contraction *list, int n, double re
 int sipgpu_batch_split_info(sipgpu_batch_t batch, int *nmoduli, int *bits);
 /* How a planned batch runs.  sipgpu_batch_plan picks the packed path for
  * batches of at least 5e9 flop averaging 5e7 flop per result block: each
- * operand block is first packed once into K-contiguous panels, then one
- * grouped GEMM runs over whole 16-k stages of every task's concatenated K
+ * operand block is first packed once into panels in MFMA operand order, then
+ * one grouped GEMM runs over the 8-k stages of every task's concatenated K
  * (SIPGPU_FP64_PATH=tables|packed in the environment pins the choice). */
 enum { SIPGPU_BATCH_TABLES = 0, SIPGPU_BATCH_PACKED = 1, SIPGPU_BATCH_SPLIT = 2 };
 int sipgpu_batch_kind(sipgpu_batch_t batch, int *kind);
