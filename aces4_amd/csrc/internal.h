@@ -156,6 +156,12 @@ void bind_panel_plan(const PanelPlan &p, void *desc, int8_t *planes, uint8_t *re
 // Enqueues the stages (SIPGPU_STAGE_* bits) of a bound panel batch.
 int execute_panels(SplitData &sd, bool split, int stages, hipStream_t s);
 
+// The boxes of a tuple of segments (of the virtual, then the occupied index
+// range): their count, and the tuple fields of the box kernel's arguments.
+// SIPGPU_ESIZE where the kernel's work items could not number them.
+int triples_tuple_boxes(const std::vector<int> &vseg, const std::vector<int> &oseg,
+                        const int *tuple, TriplesArgs &a, long long &boxes);
+
 } // namespace rt
 } // namespace sipgpu
 

@@ -117,6 +117,26 @@ int max_seg_blocks(const std::vector<int> &seg) {
 
 } // namespace
 
+int sipgpu::rt::triples_tuple_boxes(const std::vector<int> &vseg, const std::vector<int> &oseg,
+                                    const int *tuple, TriplesArgs &a, long long &boxes) {
+    // (the kernel counts work items in 32 bits and adds a stride to them)
+    constexpr long long kMost = 1LL << 31;
+    boxes = 1;
+    for (int d = 0; d < 6; ++d) {
+        const std::vector<int> &seg = d < 3 ? vseg : oseg;
+        if (tuple[d] < 0 || tuple[d] >= (int)seg.size())
+            return fail(SIPGPU_EARG, "triples: tuple outside the segments");
+        a.lo[d] = std::accumulate(seg.begin(), seg.begin() + tuple[d], 0);
+        a.wdims[d] = seg[tuple[d]];
+        seg_blocks(a.lo[d], a.wdims[d], a.first[d], a.count[d]);
+        boxes *= a.count[d];
+        if (boxes >= kMost)
+            return fail(SIPGPU_ESIZE, "triples: the tuple has 2^31 boxes or more");
+    }
+    a.end[0] = (unsigned)boxes;
+    return 0;
+}
+
 extern "C" {
 
 int sipgpu_triples_create(int nv, const int *v_seg, int no, const int *o_seg,
@@ -178,6 +198,10 @@ int sipgpu_triples_create(int nv, const int *v_seg, int no, const int *o_seg,
     if (e != hipSuccess) return no_memory();
     // built once the device holds a partial per slot: the host's classes are
     // then at most a hundredth of that
+    if (pairs * (pairs + 1) * (pairs + 2) / 6 >= 1LL << 26) { // items hold class * 64
+        (void)no_memory();
+        return fail(SIPGPU_ESIZE, "triples: too many super-box classes");
+    }
     try {
         P->orbits = super_box_classes((int)pairs);
         list_boxes(*P);
@@ -359,20 +383,11 @@ int sipgpu_triples_tuple(sipgpu_triples_t P, const int *tuple, double factor, do
     a.tuple_mode = 1;
     a.partial = P->tuple_partial;
     a.wout = w_out;
-    long long grid = 1;
-    for (int d = 0; d < 6; ++d) {
-        const std::vector<int> &seg = d < 3 ? P->vseg : P->oseg;
-        if (tuple[d] < 0 || tuple[d] >= (int)seg.size())
-            return fail(SIPGPU_EARG, "triples: tuple outside the segments");
-        a.lo[d] = std::accumulate(seg.begin(), seg.begin() + tuple[d], 0);
-        a.wdims[d] = seg[tuple[d]];
-        seg_blocks(a.lo[d], a.wdims[d], a.first[d], a.count[d]);
-        grid *= a.count[d];
-    }
+    long long boxes = 0;
+    if (int rc = sipgpu::rt::triples_tuple_boxes(P->vseg, P->oseg, tuple, a, boxes)) return rc;
     const hipStream_t hs = sipgpu::rt::stream_of(s);
-    a.end[0] = (unsigned)grid;
     SIPGPU_HIP_TRY(sipgpu::launch_triples_boxes(a, hs));
-    SIPGPU_HIP_TRY(sipgpu::launch_triples_reduce(P->tuple_partial, grid, P->sums, factor, out, hs));
+    SIPGPU_HIP_TRY(sipgpu::launch_triples_reduce(P->tuple_partial, boxes, P->sums, factor, out, hs));
     return 0;
 }
 
