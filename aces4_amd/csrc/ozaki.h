@@ -29,6 +29,7 @@ constexpr int kOzZero = 256;            // zero bytes at the start of every resi
 constexpr int kPanelRows = 16, kPanelK = 8, kPanelUnit = 1024;
 constexpr int kOzTileX = 32, kOzTileK = 128; // conversion tile (rows x k)
 constexpr int kOzRecChunk = 1024;       // result elements per reconstruction workgroup
+constexpr int kOzRecPer = 2;            // workgroups per work item
 
 // Moduli and reconstruction constants (host-computed).
 struct OzConst {
@@ -128,21 +129,39 @@ __device__ __forceinline__ double *oz_dest(const OzTask &t, const OzSub *subs, c
 struct OzTile {
     int task, mt, nt, part;
     int s0, s1;
-    int mod, pad; // split path: the tile's modulus
 };
+
+// A GEMM work unit of the split path: one tile of a task in one modulus.  Eight
+// bytes: every tile is listed once per modulus, and a list that has outgrown a
+// descriptor slot costs its upload too.
+struct OzUnit {
+    int task;      // < 0: none (padding of the XCD schedule)
+    uint32_t tile; // 16 (mt + nt * tiles along M) + modulus
+};
+
+// Tile (mt, nt) and modulus of a unit of a task with M rows, in tiles of `edge`.
+__device__ __forceinline__ void oz_unit(const OzUnit &u, int M, int edge, int &mt, int &nt,
+                                        int &mod) {
+    const uint32_t along = (uint32_t)(M + edge - 1) / (uint32_t)edge, q = u.tile >> 4;
+    mod = (int)(u.tile & 15u);
+    nt = (int)(q / along);
+    mt = (int)(q - (uint32_t)nt * along);
+}
 
 // Conversion work item: rows [x0, x0 + kOzTileX) and k [k0, k0 + kOzTileK) of a block.
 struct OzConvTile {
     int block, x0, k0, pad;
 };
 
-// Reconstruction work item: elements [e0, e0 + kOzRecChunk) of a task.
+// Reconstruction work item: elements [e0, e0 + kOzRecPer * kOzRecChunk) of a
+// task, one workgroup per kOzRecChunk of them.
 struct OzRecItem {
     int task, e0;
 };
 
 struct OzGemmArgs {
-    const OzTile *tiles;
+    const OzTile *tiles; // packed FP64 path
+    const OzUnit *units; // split path
     const OzTask *tasks;
     const OzChunkRef *chunks;
     const int8_t *planes;

@@ -274,14 +274,15 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_i8_kernel(OzGemmArgs 
     const int li = lane & 15, lk = lane >> 4;
     const int g = (lane & 7) ^ (lane >> 3); // chunk of the stage this lane loads
     for (int t = blockIdx.x; t < a.ntiles; t += gridDim.x) {
-        const OzTile tile = a.tiles[t];
-        if (tile.task < 0) continue;
-        const int mod = tile.mod;
+        const OzUnit unit = a.units[t];
+        if (unit.task < 0) continue;
+        const OzTask task = a.tasks[unit.task];
+        int mt, nt, mod;
+        oz_unit(unit, task.M, BM, mt, nt, mod);
         const int p = a.c.p[mod], u = a.c.u[mod], c17 = a.c.c17[mod];
         const uint32_t bar = a.c.bar[mod];
         gi8_t *plane = (gi8_t *)(a.planes + (long long)mod * a.plane_bytes);
-        const OzTask task = a.tasks[tile.task];
-        const int m0 = tile.mt * BM, n0 = tile.nt * BN;
+        const int m0 = mt * BM, n0 = nt * BN;
         int ra[IA], rb[IB];
 #pragma unroll
         for (int i = 0; i < IA; ++i) ra[i] = min(m0 + 8 * (wave * IA + i) + (lane >> 3), task.M - 1);
@@ -447,9 +448,11 @@ __global__ __launch_bounds__(512, 1) void gemm_i8_wide_kernel(OzGemmArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave & 3, wn = wave >> 2;
     const int li = lane & 15, lk = lane >> 4;
-    const OzTile tile = a.tiles[blockIdx.x];
-    if (tile.task < 0) return;
-    const int mod = tile.mod;
+    const OzUnit unit = a.units[blockIdx.x];
+    if (unit.task < 0) return;
+    const OzTask task = a.tasks[unit.task];
+    int mt, nt, mod;
+    oz_unit(unit, task.M, BT, mt, nt, mod);
     const int p = a.c.p[mod], u = a.c.u[mod], c17 = a.c.c17[mod];
     const uint32_t bar = a.c.bar[mod];
     // (buffer loads: the compiler takes a global load into LDS for a flat access
@@ -458,8 +461,7 @@ __global__ __launch_bounds__(512, 1) void gemm_i8_wide_kernel(OzGemmArgs a) {
         const_cast<int8_t *>(a.planes) + (long long)mod * a.plane_bytes, 0,
         (int)(uint32_t)a.plane_bytes, 0x00020000);
 
-    const OzTask task = a.tasks[tile.task];
-    const int m0 = tile.mt * BT, n0 = tile.nt * BT;
+    const int m0 = mt * BT, n0 = nt * BT;
     // this wave loads four of the stage's 32 units: waves 0-3 those of A,
     // waves 4-7 those of B; a lane's rows, clamped into the panel
     const bool side_b = wave >= 4;
@@ -622,10 +624,11 @@ __global__ __launch_bounds__(256) void reconstruct_kernel(OzRecArgs a) {
     typedef double f64x2 __attribute__((ext_vector_type(2), aligned(8)));
     typedef __attribute__((address_space(1))) double gdouble_t;
     typedef __attribute__((address_space(1))) f64x2 gf64x2_t;
-    const OzRecItem w = a.items[blockIdx.x];
+    const OzRecItem w = a.items[blockIdx.x / kOzRecPer];
     const OzTask task = a.tasks[w.task];
-    const int e1 = min(w.e0 + kOzRecChunk, task.M * task.N);
-    const int e0 = w.e0 + 4 * (int)threadIdx.x;
+    const int first = w.e0 + (int)(blockIdx.x % kOzRecPer) * kOzRecChunk;
+    const int e1 = min(first + kOzRecChunk, task.M * task.N);
+    const int e0 = first + 4 * (int)threadIdx.x;
     if (e0 >= e1) return;
     // one 32-bit load per plane for the thread's four elements, all before any
     // is used (task regions start 16-byte aligned and planes end 16 bytes past
@@ -761,7 +764,7 @@ hipError_t oz_gemm(const OzGemmArgs &a, hipStream_t s) {
 
 hipError_t oz_reconstruct(const OzRecArgs &a, hipStream_t s) {
     if (a.nitems <= 0) return hipSuccess;
-    const dim3 grid(a.nitems);
+    const dim3 grid(a.nitems * kOzRecPer);
     const int words = a.c.n / 4 + 1; // of four: the moduli and q
     if (words > 4) return hipErrorInvalidValue;
     if (words == 4)

@@ -43,14 +43,15 @@ __global__ __launch_bounds__(256, 1) void gemm_i8_big_kernel(OzGemmArgs a) {
     const int g = (lane & 3) ^ ((lane >> 3) & 3); // chunk of the stage this lane loads
 
     for (int t = blockIdx.x; t < a.ntiles; t += gridDim.x) {
-        const OzTile tile = a.tiles[t];
-        if (tile.task < 0) continue;
-        const int mod = tile.mod;
+        const OzUnit unit = a.units[t];
+        if (unit.task < 0) continue;
+        const OzTask task = a.tasks[unit.task];
+        int mt, nt, mod;
+        oz_unit(unit, task.M, BM, mt, nt, mod);
         const int p = a.c.p[mod], u = a.c.u[mod];
         const uint32_t bar = a.c.bar[mod];
         gi8_t *plane = (gi8_t *)(a.planes + (long long)mod * a.plane_bytes);
-        const OzTask task = a.tasks[tile.task];
-        const int m0 = tile.mt * BM, n0 = tile.nt * BN;
+        const int m0 = mt * BM, n0 = nt * BN;
         const OzChunkRef *ch = a.chunks + task.chunk0;
         const int nst = task.nchunks / CH; // even
         // rows this lane loads: group i of the wave covers 16 rows

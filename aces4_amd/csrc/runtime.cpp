@@ -558,26 +558,28 @@ std::vector<Tile> interleave(const std::vector<std::vector<Tile>> &per_xcd) {
 // With the lists of xcd_lists for every modulus an XCD got up to a fifth more
 // than its share or a round too many: the 324 tiles of a full ring batch (lists
 // of up to 50) 1.46 ms against 1.27, 20 tiles with 12 moduli 86 us against 52.
-std::vector<std::vector<OzTile>> deal_moduli(const std::vector<std::vector<OzTile>> &lists,
-                                             const OzTask *tasks, int nmod) {
+std::vector<std::vector<OzUnit>> deal_moduli(const std::vector<std::vector<OzTile>> &lists,
+                                             const OzTask *tasks, const std::vector<int> &tms,
+                                             int nmod) {
     // (about 16 chunks' time to start and store a tile)
     auto cost = [&](const OzTile &u) { return (double)tasks[u.task].nchunks + 16.0; };
     double total = 0.0, done = 0.0;
     for (const auto &list : lists)
         for (const OzTile &u : list) total += cost(u) * nmod;
-    std::vector<std::vector<OzTile>> per(kXcds);
+    std::vector<std::vector<OzUnit>> per(kXcds);
     for (const auto &list : lists)
         for (const OzTile &u : list)
             for (int mod = 0; mod < nmod; ++mod) {
                 const double c = cost(u);
                 const int x = std::min(kXcds - 1, (int)((done + c / 2) / total * kXcds));
-                per[x].push_back(u);
-                per[x].back().mod = mod;
+                per[x].push_back(OzUnit{
+                    u.task, (uint32_t)(u.mt + u.nt * tms[u.task]) * 16u + (uint32_t)mod});
                 done += c;
             }
     for (auto &list : per)
-        std::stable_sort(list.begin(), list.end(),
-                         [](const OzTile &a, const OzTile &b) { return a.mod < b.mod; });
+        std::stable_sort(list.begin(), list.end(), [](const OzUnit &a, const OzUnit &b) {
+            return (a.tile & 15u) < (b.tile & 15u);
+        });
     return per;
 }
 
@@ -1434,7 +1436,8 @@ int sipgpu::rt::build_panel_plan(const sipgpu_contraction *list, int n, int nmod
     for (int t = 0; t < ntasks && nmod; ++t) {
         tasks[t].res_off = res_elems; // 16-byte aligned: the reconstruction reads words
         const long long mn = (long long)tasks[t].M * tasks[t].N;
-        for (long long e0 = 0; e0 < mn; e0 += kOzRecChunk) rec.push_back(OzRecItem{t, (int)e0});
+        for (long long e0 = 0; e0 < mn; e0 += kOzRecPer * kOzRecChunk)
+            rec.push_back(OzRecItem{t, (int)e0});
         res_elems += (mn + 15) / 16 * 16;
     }
     // GEMM tile: 256 x 256 with eight waves of 64 x 128, or 128 x 128 with four,
@@ -1484,6 +1487,7 @@ int sipgpu::rt::build_panel_plan(const sipgpu_contraction *list, int n, int nmod
             costs[x].push_back(task_cost[u.task] / ((double)tms[u.task] * tns[u.task]));
         }
     std::vector<OzTile> tiles, fix;
+    std::vector<OzUnit> split_units;
     std::vector<int> wg_first;
     int nslots = 0;
     const bool tail = opt.tail >= 0 ? opt.tail != 0 : !(tail_env && !std::strcmp(tail_env, "0"));
@@ -1494,10 +1498,16 @@ int sipgpu::rt::build_panel_plan(const sipgpu_contraction *list, int n, int nmod
         // through the fixup pass where the segments are short
         const int slots = 64 >> (std::min(std::max(opt.tail, 1), 4) - 1);
         persistent_schedule(lists, costs, slots, tiles, wg_first, fix, nslots);
+    } else if (nmod) {
+        for (int t = 0; t < ntasks; ++t)
+            if ((long long)tms[t] * tns[t] >= 1 << 28)
+                return fail(SIPGPU_ESIZE, "split path: too many tiles");
+        split_units = interleave(deal_moduli(lists, tasks.data(), tms, nmod));
     } else {
-        tiles = interleave(nmod ? deal_moduli(lists, tasks.data(), nmod) : lists);
+        tiles = interleave(lists);
     }
-    if (tiles.size() >= (size_t)INT_MAX) return fail(SIPGPU_ESIZE, "split path: too many tiles");
+    const size_t ntiles = nmod ? split_units.size() : tiles.size();
+    if (ntiles >= (size_t)INT_MAX) return fail(SIPGPU_ESIZE, "split path: too many tiles");
 
     OzConst oc{};
     if (nmod) {
@@ -1510,7 +1520,8 @@ int sipgpu::rt::build_panel_plan(const sipgpu_contraction *list, int n, int nmod
     size_t off = 0;
     P.o_blocks = off; off = align(off + blocks.size() * sizeof(OzBlock));
     P.o_tasks = off; off = align(off + tasks.size() * sizeof(OzTask));
-    P.o_tiles = off; off = align(off + tiles.size() * sizeof(OzTile));
+    P.o_tiles = off;
+    off = align(off + (nmod ? ntiles * sizeof(OzUnit) : ntiles * sizeof(OzTile)));
     P.o_chunks = off; off = align(off + chunks.size() * sizeof(OzChunkRef));
     P.o_tab = off; off = align(off + pool.size() * sizeof(int32_t));
     P.o_conv = off; off = align(off + conv.size() * sizeof(OzConvTile));
@@ -1526,7 +1537,10 @@ int sipgpu::rt::build_panel_plan(const sipgpu_contraction *list, int n, int nmod
     };
     put(P.o_blocks, blocks.data(), blocks.size() * sizeof(OzBlock));
     put(P.o_tasks, tasks.data(), tasks.size() * sizeof(OzTask));
-    put(P.o_tiles, tiles.data(), tiles.size() * sizeof(OzTile));
+    if (nmod)
+        put(P.o_tiles, split_units.data(), ntiles * sizeof(OzUnit));
+    else
+        put(P.o_tiles, tiles.data(), ntiles * sizeof(OzTile));
     put(P.o_chunks, chunks.data(), chunks.size() * sizeof(OzChunkRef));
     put(P.o_tab, pool.data(), pool.size() * sizeof(int32_t));
     put(P.o_conv, conv.data(), conv.size() * sizeof(OzConvTile));
@@ -1548,7 +1562,7 @@ int sipgpu::rt::build_panel_plan(const sipgpu_contraction *list, int n, int nmod
     long long halves = 0;
     for (const OzChunkRef &c : chunks) halves += !nmod && c.aux == 1;
     P.skip_halves = halves * 10 > (long long)chunks.size();
-    P.ntiles = (int)tiles.size();
+    P.ntiles = (int)ntiles;
     P.nconv = (int)conv.size();
     P.nrows = (int)rows.size();
     P.nrec = (int)rec.size();
@@ -1590,7 +1604,10 @@ void sipgpu::rt::bind_panel_plan(const PanelPlan &P, void *desc, int8_t *planes,
     ca.c = P.c;
     OzGemmArgs &g = sd.gargs;
     g = OzGemmArgs{};
-    g.tiles = reinterpret_cast<const OzTile *>(base + P.o_tiles);
+    if (P.nmod)
+        g.units = reinterpret_cast<const OzUnit *>(base + P.o_tiles);
+    else
+        g.tiles = reinterpret_cast<const OzTile *>(base + P.o_tiles);
     g.tasks = dtasks;
     g.chunks = reinterpret_cast<const OzChunkRef *>(base + P.o_chunks);
     g.planes = planes;

@@ -656,7 +656,10 @@ int sipgpu_cache_get_stats(sipgpu_cache_t c, sipgpu_cache_stats *out) {
 namespace {
 
 constexpr int kSlots = 4;
-constexpr size_t kSlotBytes = 32u << 20;
+// A descriptor slot begins with the size that most batches stay below; one
+// that needs more makes its slot grow, up to the size beyond which a batch is
+// refused (256 split contractions of 50^4, 60^4 or 64^4 blocks take 24 to 31 MiB).
+constexpr size_t kSlotBytes = 32u << 20, kSlotMaxBytes = 256u << 20;
 constexpr int kLanes = 2; // device streams the batches run on
 
 enum { kKindContract = 0, kKindPermute = 1 };
@@ -701,6 +704,7 @@ struct sipgpu_server_s {
     void *slot_host[kSlots] = {};
     hipEvent_t slot_free[kSlots] = {};
     bool slot_used[kSlots] = {};
+    size_t slot_bytes[kSlots] = {};
     int next_slot = 0;
 
     std::mutex mu;
@@ -734,15 +738,31 @@ struct sipgpu_server_s {
 
 namespace {
 
-// A descriptor slot whose previous batch has finished reading it.
-int take_slot(sipgpu_server_s &S, int &slot) {
+// Device and host memory of a slot, at least `bytes`.  On failure the slot is
+// empty and the next batch that takes it tries again.
+int size_slot(sipgpu_server_s &S, int slot, size_t bytes) {
+    if (bytes <= S.slot_bytes[slot]) return 0;
+    if (S.slot_dev[slot]) (void)hipFree(S.slot_dev[slot]);
+    if (S.slot_host[slot]) (void)hipHostFree(S.slot_host[slot]);
+    S.slot_dev[slot] = S.slot_host[slot] = nullptr;
+    S.slot_bytes[slot] = 0;
+    SIPGPU_HIP_TRY(hipMalloc(&S.slot_dev[slot], bytes));
+    SIPGPU_HIP_TRY(hipHostMalloc(&S.slot_host[slot], bytes, hipHostMallocDefault));
+    S.slot_bytes[slot] = bytes;
+    return 0;
+}
+
+// A descriptor slot for `bytes` whose previous batch has finished reading it.
+int take_slot(sipgpu_server_s &S, size_t bytes, int &slot) {
     slot = S.next_slot;
     S.next_slot = (S.next_slot + 1) % kSlots;
     if (S.slot_used[slot]) {
         hipError_t e = hipEventSynchronize(S.slot_free[slot]);
         if (e != hipSuccess) return hip_fail(e, "server: slot");
     }
-    return 0;
+    size_t room = kSlotBytes;
+    while (room < bytes) room *= 2;
+    return size_slot(S, slot, room);
 }
 
 // A panel batch (split precision, or packed FP64): its descriptors through a
@@ -765,7 +785,7 @@ int server_panels(sipgpu_server_s &S, int lane, const sipgpu::rt::PanelPlan &pla
         S.scratch_bytes[lane] = bytes;
     }
     int slot = 0;
-    if (int rc = take_slot(S, slot)) return rc;
+    if (int rc = take_slot(S, desc.size(), slot)) return rc;
     int8_t *planes = static_cast<int8_t *>(S.scratch[lane]);
     uint8_t *res = reinterpret_cast<uint8_t *>(planes + up(plan.plane_total()));
     double *work = plan.nslots ? reinterpret_cast<double *>(res + up(plan.res_total())) : nullptr;
@@ -873,7 +893,7 @@ int server_permutes(sipgpu_server_s &S, int lane, const std::vector<Pending> &ba
             reinterpret_cast<sipgpu::PermArgs *>(host.data()),
             reinterpret_cast<int *>(host.data() + first_off), &tile_cap, &tv_cap);
         const size_t bytes = entry_off + (size_t)std::max<int64_t>(grid, 0) * sizeof(int);
-        if (grid >= ((int64_t)1 << 31) || bytes > kSlotBytes) {
+        if (grid >= ((int64_t)1 << 31) || bytes > kSlotMaxBytes) {
             // tables beyond a descriptor slot: one launch per permute
             for (int e = 0; e < n && !rc; ++e) {
                 const hipError_t he = sipgpu::launch_permute(plans[e], in[e], out[e], stream);
@@ -886,7 +906,7 @@ int server_permutes(sipgpu_server_s &S, int lane, const std::vector<Pending> &ba
             for (int e = 0; e < n; ++e)
                 for (int w = first[e]; w < first[e + 1]; ++w) entry[w] = e;
             int slot = 0;
-            rc = take_slot(S, slot);
+            rc = take_slot(S, bytes, slot);
             if (!rc) {
                 std::memcpy(S.slot_host[slot], host.data(), bytes);
                 const unsigned char *dev = static_cast<const unsigned char *>(S.slot_dev[slot]);
@@ -979,12 +999,12 @@ int server_batch(sipgpu_server_s &S, int lane, std::vector<Pending> &batch) {
         }
     }
     const std::vector<unsigned char> &desc = panels ? plan.host : img.host;
-    if (!rc && desc.size() > kSlotBytes)
+    if (!rc && desc.size() > kSlotMaxBytes)
         rc = fail(SIPGPU_ESIZE, "server: batch work list exceeds its descriptor slot");
     if (!rc && panels) rc = server_panels(S, lane, plan, desc);
     if (!rc && !panels && img.ntiles > 0) {
         int slot = 0;
-        rc = take_slot(S, slot);
+        rc = take_slot(S, desc.size(), slot);
         if (!rc) {
             std::memcpy(S.slot_host[slot], img.host.data(), img.host.size());
             hipError_t e = hipMemcpyAsync(S.slot_dev[slot], S.slot_host[slot], img.host.size(),
@@ -1272,8 +1292,7 @@ int sipgpu_server_create(sipgpu_cache_t cache, int max_batch, sipgpu_server_t *s
     for (int l = 0; l < S->lanes; ++l)
         SIPGPU_HIP_TRY(hipStreamCreateWithFlags(&S->stream[l], hipStreamNonBlocking));
     for (int i = 0; i < kSlots; ++i) {
-        SIPGPU_HIP_TRY(hipMalloc(&S->slot_dev[i], kSlotBytes));
-        SIPGPU_HIP_TRY(hipHostMalloc(&S->slot_host[i], kSlotBytes, hipHostMallocDefault));
+        if (int rc = size_slot(*S, i, kSlotBytes)) return rc;
         SIPGPU_HIP_TRY(hipEventCreateWithFlags(&S->slot_free[i], hipEventDisableTiming));
     }
     S->sched = std::thread(scheduler_loop, S.get());

@@ -1,0 +1,78 @@
+// Host-only check of the split path's plans (no device calls): the descriptors
+// of large batches fit the server's first slot size, every tile stands in the
+// work list once per modulus, and the reconstruction items cover every result.
+// Block addresses are stand-in integers (the planner only compares them).
+#include <cstdio>
+#include <map>
+#include <tuple>
+#include <vector>
+#include "internal.h"
+using namespace sipgpu;
+
+static int fails = 0;
+#define CHECK(c) do { if (!(c)) { std::printf("FAIL %s:%d %s\n", __FILE__, __LINE__, #c); ++fails; } } while (0)
+
+// n contractions D(a,b,i,j) = V(a,b,c,d) T(c,d,i,j) of seg^4 blocks over
+// `shared` left and right blocks (0: each its own)
+static rt::PanelPlan plan_of(int n, int seg, int shared, int nmod) {
+    int dr = 4, lr = 4, rr = 4, ptrn[8], ierr = 0;
+    int aces[12] = {1, 2, 3, 4, 1, 2, 5, 6, 5, 6, 3, 4};
+    get_contraction_ptrn_(&dr, &lr, &rr, aces, ptrn, &ierr);
+    CHECK(ierr == 0);
+    auto ptr = [&](int id) { return (double *)(((uintptr_t)id + 1) << 32); };
+    std::vector<sipgpu_contraction> list;
+    for (int i = 0; i < n; ++i) {
+        sipgpu_contraction e{};
+        e.l = ptr(shared ? i % shared : i);
+        e.r = ptr(10000 + (shared ? i / shared : i));
+        e.d = ptr(20000 + i);
+        e.lrank = e.rrank = e.drank = 4;
+        for (int k = 0; k < 4; ++k) e.ldims[k] = e.rdims[k] = e.ddims[k] = seg;
+        for (int k = 0; k < 8; ++k) e.ptrn[k] = ptrn[k];
+        e.accumulate = 1;
+        list.push_back(e);
+    }
+    rt::PanelPlan p;
+    CHECK(rt::build_panel_plan(list.data(), n, nmod, p) == 0);
+    return p;
+}
+
+static void check_lists(const rt::PanelPlan &p) {
+    const OzTask *tasks = (const OzTask *)(p.host.data() + p.o_tasks);
+    const OzUnit *units = (const OzUnit *)(p.host.data() + p.o_tiles);
+    const int edge = oz_tile_size(p.tile);
+    std::map<std::tuple<int, int, int>, int> seen; // (task, tile, modulus)
+    for (int i = 0; i < p.ntiles; ++i)
+        if (units[i].task >= 0)
+            seen[{units[i].task, (int)(units[i].tile >> 4), (int)(units[i].tile & 15)}]++;
+    size_t want = 0;
+    for (int t = 0; t < p.ngroups; ++t) {
+        const int tiles = ((tasks[t].M + edge - 1) / edge) * ((tasks[t].N + edge - 1) / edge);
+        want += (size_t)tiles * p.nmod;
+        for (int q = 0; q < tiles; ++q)
+            for (int m = 0; m < p.nmod; ++m) CHECK((seen[{t, q, m}]) == 1);
+    }
+    CHECK(seen.size() == want);
+    const OzRecItem *rec = (const OzRecItem *)(p.host.data() + p.o_rec);
+    std::vector<long long> next(p.ngroups, 0);
+    for (int i = 0; i < p.nrec; ++i) {
+        CHECK(rec[i].e0 == next[rec[i].task]);
+        next[rec[i].task] += kOzRecPer * kOzRecChunk;
+    }
+    for (int t = 0; t < p.ngroups; ++t) CHECK(next[t] >= (long long)tasks[t].M * tasks[t].N);
+}
+
+int main() {
+    const size_t slot = 32u << 20;
+    const int batches[3][3] = {{256, 50, 0}, {256, 60, 16}, {120, 64, 0}};
+    for (const auto &b : batches) {
+        const rt::PanelPlan p = plan_of(b[0], b[1], b[2], 14);
+        std::printf("%d of %d^4: %.1f MiB\n", b[0], b[1], p.host.size() / 1048576.0);
+        CHECK(p.host.size() <= slot);
+    }
+    check_lists(plan_of(3, 7, 0, 6));
+    check_lists(plan_of(5, 17, 2, 14));
+    check_lists(plan_of(40, 23, 0, 13));
+    std::printf(fails ? "FAILED %d\n" : "all ok\n", fails);
+    return fails != 0;
+}
