@@ -1004,6 +1004,19 @@ constexpr CfgShape kCfg[kGemmConfigs] = {
     {32, 32},
 };
 
+// One workgroup of 512 per tile, 2^22 tiles a launch (a launch holds fewer than
+// 2^32 work-items).
+hipError_t launch_ksplit(GemmArgs args, int grid, hipStream_t stream) {
+    constexpr int kMost = 1 << 22;
+    if (grid > kMost && !args.tiles) return hipErrorInvalidConfiguration;
+    for (; grid > 0; grid -= kMost) {
+        gemm_f64_ksplit_kernel<<<std::min(grid, kMost), kSplitWaves * 64, 0, stream>>>(args);
+        if (hipError_t e = hipGetLastError()) return e;
+        if (args.tiles) args.tiles += kMost;
+    }
+    return hipSuccess;
+}
+
 } // namespace
 
 int gemm_tile_m(int cfg) { return cfg >= 0 && cfg < kGemmConfigs ? kCfg[cfg].bm : 0; }
@@ -1031,8 +1044,7 @@ hipError_t launch_gemm(int cfg, const GemmArgs &args, int grid, hipStream_t stre
     case 16: return launch_lds<128, 128, 2, 2, 16>(args, grid, stream);
     case 17: return launch_lds<64, 128, 2, 2, 16>(args, grid, stream);
     case kGemmSplitK:
-        gemm_f64_ksplit_kernel<<<grid, kSplitWaves * 64, 0, stream>>>(args);
-        return hipGetLastError();
+        return launch_ksplit(args, grid, stream);
     default: return hipErrorInvalidValue;
     }
 }

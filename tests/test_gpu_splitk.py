@@ -130,3 +130,26 @@ def test_single_contraction_segments(M, N, K, form):
         d.free()
     dl.free()
     dr.free()
+
+
+def test_more_tiles_than_one_launch_holds():
+    """8193 rows of 32768 as 32 x 32 tiles: over 2^23 workgroups of 512."""
+    sg.init(0)
+    print("split K, two launches", flush=True)
+    n, N = 8193, 32768
+    rng = np.random.default_rng(8)
+    l, r = rng.standard_normal(n), rng.standard_normal(N)
+    dl, dr, d = sg.DeviceArray.from_host(l), sg.DeviceArray.from_host(r), sg.DeviceArray(n * N)
+    ptrn, _ = FORMS[0]
+    cs = [sg.make_contraction(ptrn, dl.at(i), [1, 1], dr.ptr, [1, N], d.at(i * N), [1, N])
+          for i in range(n)]
+    b = sg.plan_choice(cs, "tables", config=SPLIT_K)
+    b.execute()
+    sg.synchronize()
+    b.destroy()
+    for i in range(0, n, 64):
+        m = min(64, n - i)
+        got = d.download_range(i * N, m * N).reshape(m, N)
+        assert np.array_equal(got, l[i:i + m, None] * r)  # one product, rounded once
+    for a in (dl, dr, d):
+        a.free()
