@@ -474,11 +474,14 @@ __global__ __launch_bounds__(WM *WN * 64) void gemm_f64_db_kernel(GemmArgs args)
         __syncthreads();
 
         // prologue: stage 0 to LDS, stage 1 loads and stage 2 lookups in flight
+        // (a task without pairs, its K empty: nothing to load)
         Cursor C = at_pair(task.first);
-        lookup(C);
-        issue(C);
-        store(C, 0);
-        Cursor L = advance(C);
+        if (C.p < pend) {
+            lookup(C);
+            issue(C);
+            store(C, 0);
+        }
+        Cursor L = C.p < pend ? advance(C) : C;
         if (L.p < pend) { lookup(L); issue(L); }
         Cursor Kn = L.p < pend ? advance(L) : L;
         if (Kn.p < pend) lookup(Kn);

@@ -328,7 +328,7 @@ int contract_device(Context &c, sipgpu_stream_s &st, const int *ptrn, const doub
         if (ntiles >= ((int64_t)1 << 31)) return fail(SIPGPU_ESIZE, "too many tiles");
         a.ntiles = (int)ntiles;
         task.first = 0;
-        task.npairs = 1;
+        task.npairs = pair.K > 0 ? 1 : 0; // an empty sum has nothing to load
         a.task0 = task;
         a.pair0 = pair;
         if (nseg > 1) {
@@ -664,7 +664,7 @@ void persistent_schedule(const std::vector<std::vector<OzTile>> &lists,
             if (j == slots - 1) target = 1e300; // the last takes the rest
             while (i < n) {
                 const int nst = L[i].s1 - L[i].s0;
-                const double cs = c[i] / nst; // cost per stage
+                const double cs = nst ? c[i] / nst : 0.0; // cost per stage
                 const int rem = L[i].s1 - st;
                 if (pos + rem * cs <= target + 0.5 * kMinSeg * cs) {
                     segs[i - full].push_back({j, st, L[i].s1});
@@ -672,7 +672,7 @@ void persistent_schedule(const std::vector<std::vector<OzTile>> &lists,
                     if (++i < n) st = L[i].s0;
                     continue;
                 }
-                int k = (int)std::lround((target - pos) / cs / kMinSeg) * kMinSeg;
+                int k = cs > 0.0 ? (int)std::lround((target - pos) / cs / kMinSeg) * kMinSeg : 0;
                 if (k > 0 && L[i].s1 - (st + k) < kMinSeg) k = rem;
                 if (k > 0) {
                     segs[i - full].push_back({j, st, st + k});
@@ -1403,8 +1403,8 @@ int sipgpu::rt::build_panel_plan(const sipgpu_contraction *list, int n, int nmod
             return base;
         };
         // virtual K: the pairs' panel chunks; the INT8 GEMM runs two stages of
-        // kOzStageChunks per loop trip and is padded to that with chunks of
-        // the zero bytes
+        // kOzStageChunks per loop trip, at least once, and is padded to that
+        // with chunks of the zero bytes (all of them where K is empty)
         tasks[t].chunk0 = (int)chunks.size();
         const int np = (int)rvec[rs[0]].size();
         for (int p = 0; p < np; ++p) {
@@ -1418,7 +1418,8 @@ int sipgpu::rt::build_panel_plan(const sipgpu_contraction *list, int n, int nmod
             if (panel >= (1LL << 36))
                 return fail(SIPGPU_ESIZE, "operand panels exceed 64 GiB");
         }
-        while (nmod && (chunks.size() - tasks[t].chunk0) % (2 * kOzStageChunks))
+        auto listed = [&]() { return (int)chunks.size() - tasks[t].chunk0; };
+        while (nmod && (listed() == 0 || listed() % (2 * kOzStageChunks)))
             chunks.push_back(OzChunkRef{0u, 0, 0u, 0});
         tasks[t].nchunks = (int)chunks.size() - tasks[t].chunk0;
     }

@@ -1,6 +1,7 @@
-// Host-only check of the split path's plans (no device calls): the descriptors
-// of large batches fit the server's first slot size, every tile stands in the
-// work list once per modulus, and the reconstruction items cover every result.
+// Host-only check of the panel planner (no device calls): the descriptors of
+// large split batches fit the server's first slot size, every tile stands in the
+// work list once per modulus, the reconstruction items cover every result, and
+// products with an empty K keep their tiles.
 // Block addresses are stand-in integers (the planner only compares them).
 #include <cstdio>
 #include <map>
@@ -62,6 +63,44 @@ static void check_lists(const rt::PanelPlan &p) {
     for (int t = 0; t < p.ngroups; ++t) CHECK(next[t] >= (long long)tasks[t].M * tasks[t].N);
 }
 
+// Batches of n products D(m,n) = L(k,m) R(k,n), every third with an empty K.
+static void check_empty(int n, int nmod) {
+    auto ptr = [&](int id) { return (double *)(((uintptr_t)id + 1) << 24); };
+    std::vector<sipgpu_contraction> list;
+    for (int i = 0; i < n; ++i) {
+        sipgpu_contraction e{};
+        const int K = i % 3 == 2 ? 0 : 40, ptrn[4] = {-1, 1, -1, 2};
+        e.l = ptr(3 * i), e.r = ptr(3 * i + 1), e.d = ptr(3 * i + 2);
+        e.lrank = e.rrank = e.drank = 2;
+        e.ldims[0] = e.rdims[0] = K;
+        e.ldims[1] = e.ddims[0] = 150, e.rdims[1] = e.ddims[1] = 130;
+        for (int k = 0; k < 4; ++k) e.ptrn[k] = ptrn[k];
+        list.push_back(e);
+    }
+    rt::PanelPlan p;
+    CHECK(rt::build_panel_plan(list.data(), n, nmod, p) == 0);
+    const OzTask *tasks = (const OzTask *)(p.host.data() + p.o_tasks);
+    if (nmod) {
+        check_lists(p);
+        for (int t = 0; t < p.ngroups; ++t) CHECK(tasks[t].nchunks > 0 && tasks[t].nchunks % 16 == 0);
+        return;
+    }
+    // packed: every tile once in the units or, in one or more parts, in the fixups
+    const OzTile *units = (const OzTile *)(p.host.data() + p.o_tiles);
+    std::map<std::tuple<int, int, int>, int> stages;
+    for (int i = 0; i < p.ntiles; ++i)
+        if (units[i].task >= 0)
+            stages[{units[i].task, units[i].mt, units[i].nt}] += units[i].s1 - units[i].s0;
+    size_t want = 0;
+    for (int t = 0; t < p.ngroups; ++t)
+        for (int m = 0; m < (tasks[t].M + p.tile - 1) / p.tile; ++m)
+            for (int q = 0; q < (tasks[t].N + p.tile - 1) / p.tile; ++q, ++want) {
+                CHECK(stages.count({t, m, q}) == 1);
+                CHECK((stages[{t, m, q}]) == tasks[t].nchunks);
+            }
+    CHECK(stages.size() == want);
+}
+
 int main() {
     const size_t slot = 32u << 20;
     const int batches[3][3] = {{256, 50, 0}, {256, 60, 16}, {120, 64, 0}};
@@ -73,6 +112,8 @@ int main() {
     check_lists(plan_of(3, 7, 0, 6));
     check_lists(plan_of(5, 17, 2, 14));
     check_lists(plan_of(40, 23, 0, 13));
+    for (int n : {1, 3, 20, 900})
+        for (int nmod : {0, 6, 14}) check_empty(n, nmod);
     std::printf(fails ? "FAILED %d\n" : "all ok\n", fails);
     return fails != 0;
 }
