@@ -695,7 +695,7 @@ __global__ __launch_bounds__(WM *WN * 64) void gemm_f64_lds_kernel(GemmArgs args
 // k-steps (all its pairs, four k a step) straight from global memory into
 // registers: no LDS staging, no barrier in the loop.  The eight partial tiles
 // are added through LDS in wave order at the end.  The split depends on the
-// task alone, so a block's bits do not depend on its batch.
+// task alone.
 //
 // What bounds it: for few tiles the latency of a wave's chain (tables, loads,
 // MFMAs of its eighth), for many the cache lines its gathers touch.  107

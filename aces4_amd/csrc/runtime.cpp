@@ -229,17 +229,21 @@ void make_task_pair(const ContractionShape &s, int kL, int mL, int kR, int nR, i
     }
 }
 
-// Tile configuration for an M x N block; `kfast`: GemmPair::flags of its
-// first pair.
-int pick_config(int64_t M, int64_t N, int kfast) {
-    // SIPGPU_GEMM_CONFIG=<n> pins the tile configuration (tuning runs).
+// The tile configuration that SIPGPU_GEMM_CONFIG=<n> pins (tuning runs), else -1.
+int pinned_config() {
     static const int forced = [] {
         const char *e = std::getenv("SIPGPU_GEMM_CONFIG");
-        return e ? std::atoi(e) : -1;
+        const int n = e ? std::atoi(e) : -1;
+        return n < kGemmConfigs ? n : -1;
     }();
-    if (forced >= 0 && forced < kGemmConfigs) return forced;
-    // By the block alone, so that its bits do not depend on its batch.  The
-    // 32 x 32 tiles with K split over the waves win until the 64 x 64 tiles
+    return forced;
+}
+
+// Tile configuration for an M x N block on its own; `kfast`: GemmPair::flags of
+// its first pair.
+int pick_config(int64_t M, int64_t N, int kfast) {
+    if (pinned_config() >= 0) return pinned_config();
+    // The 32 x 32 tiles with K split over the waves win until the 64 x 64 tiles
     // fill the chip about twice over, or earlier where both operands are read
     // along k (a wave's load then touches 16 cache lines instead of 4).
     // Single contractions, 64 x 64 against split K: 375 tiles (1600 x 900 x
@@ -249,6 +253,51 @@ int pick_config(int64_t M, int64_t N, int kfast) {
     const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64);
     return tiles <= ((kfast & 3) == 3 ? 160 : 512) ? kGemmSplitK : kGemm64x64;
 }
+
+// Estimated time (us) of a batch's blocks in split-K tiles and in 64 x 64 tiles.
+// A tile is a chain of k-steps, which bounds few tiles, and occupies its CU,
+// which bounds many: a batch takes about the root of the two squares' sum.  The
+// 64 x 64 tiles' chain is eight times as long, and they pay for whole stages of
+// 16 k and for every pair; but once they fill the chip, one of them costs less
+// than the four split-K tiles of its area, which gather every operand element
+// twice as often.  In us for 64 x 64 and split-K tiles:
+// 1000 blocks of 320 x 320, K = 200, 1165 and 2084 (both along k), 1337 and 1899
+// (one), 1465 and 1789 (neither); 30 of them 53 and 66, 54 and 62, 57 and 58;
+// 1000 of 100^3 117 and 197; 16 of 100 x 100, K = 1600, 187 and 27; 285 of 31 x
+// 37, K = 2574, 383 and 172.  Over 806 batches of 32 to 16384 tiles of 64 x 64
+// the choice by these estimates took 0.7% longer than the faster of the two on
+// average, 1.45 times as long at worst (13 x 191, K = 6672 along k); 64 x 64 tiles
+// throughout 68% longer, split-K tiles throughout 10%.
+struct TileTimes {
+    double chain[2] = {}, work[2] = {}; // split-K, 64 x 64
+    bool beta = false;
+    // a block of M x N, the k of its pairs (also rounded up to 8 and 16 per pair)
+    void add(const GemmTask &t, const GemmPair *list) {
+        double k = 0.0, k8 = 0.0, k16 = 0.0;
+        for (int p = 0; p < t.npairs; ++p) {
+            const int K = list[p].K;
+            k += K, k8 += (K + 7) / 8 * 8, k16 += (K + 15) / 16 * 16;
+        }
+        const int pairs = t.npairs, kfast = pairs ? list[0].flags : 0;
+        const int along = (kfast & 1) + (kfast >> 1 & 1); // operands read along k
+        static constexpr double kSmall[3] = {0.0055, 0.0075, 0.009};
+        static constexpr double kChain[3] = {0.091, 0.084, 0.067}, kBig[3] = {0.03, 0.0256, 0.019};
+        auto tiles = [&](int e) {
+            return (double)((t.M + e - 1) / e) * (double)((t.N + e - 1) / e);
+        };
+        const double mfma = tiles(16) * 0.003 * k;
+        chain[0] = std::max(chain[0], 0.009 * k8 + 0.1 * pairs);
+        work[0] += tiles(32) * (1.3 + kSmall[along] * k8 + 0.02 * pairs) + mfma;
+        chain[1] = std::max(chain[1], kChain[along] * k16 + 0.3 * pairs);
+        work[1] += tiles(64) * (0.75 + kBig[along] * k16 + 0.12 * pairs) + mfma;
+        beta = beta || t.beta;
+    }
+    // (a 64 x 64 tile adds to its block one load after another)
+    double us(bool big) const {
+        const double c = (double)std::max<int64_t>(g_device_cus, 1);
+        return (big ? beta ? 5.9 : 3.9 : 2.6) + std::hypot(chain[big], work[big] / c);
+    }
+};
 
 // Tiles and K segments of a single contraction whose block pick_config gave
 // `cfg`.  Where the 64 x 64 tiles fill less than half the chip and K is long,
@@ -860,8 +909,18 @@ int sipgpu::rt::build_batch_image(const sipgpu_contraction *list, int n, BatchIm
     // beside them, 64 x 64 tiles for large blocks
     const bool own = !(cfg >= 0 && cfg < kGemmConfigs) && split_cus <= 0;
     b.cfg = cfg >= 0 && cfg < kGemmConfigs ? cfg : own ? kGemmSplitK : kGemm64x64;
+    // ... unless the batch has so many small blocks that 64 x 64 tiles of them
+    // fill the chip (a pinned configuration stays)
+    auto kfast = [&](const GemmTask &t) { return t.npairs ? pairs[t.first].flags : 0; };
+    TileTimes times;
+    if (own && pinned_config() < 0)
+        for (const GemmTask &t : tasks)
+            if (pick_config(t.M, t.N, kfast(t)) == kGemmSplitK)
+                times.add(t, pairs.data() + t.first);
+    const bool full = times.work[0] > 0.0 && times.us(true) < times.us(false);
     auto cfg_of = [&](const GemmTask &t) {
-        return own ? pick_config(t.M, t.N, t.npairs ? pairs[t.first].flags : 0) : b.cfg;
+        const int c = own ? pick_config(t.M, t.N, kfast(t)) : b.cfg;
+        return full && c == kGemmSplitK ? (int)kGemm64x64 : c;
     };
     const int bm = gemm_tile_m(b.cfg), bn = gemm_tile_n(b.cfg);
 
