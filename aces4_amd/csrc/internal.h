@@ -65,6 +65,8 @@ struct BatchImage {
     int nparts = 0;
     long long parts_max_n = 0, ws_doubles = 0;
     double flops = 0.0;
+    // A batch without a choice of its own runs on packed panels instead.
+    bool prefer_packed = false;
     void bind_workspace(double *ws) {
         GemmTask *t = reinterpret_cast<GemmTask *>(host.data() + o_tasks);
         for (size_t i = 0; i < ws_task.size(); ++i) t[ws_task[i]].D = ws + ws_off[i];

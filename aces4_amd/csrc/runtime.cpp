@@ -24,6 +24,7 @@
 #include <set>
 #include <string>
 #include <unordered_map>
+#include <unordered_set>
 #include <vector>
 
 #include "../../include/sipgpu.h"
@@ -299,6 +300,43 @@ struct TileTimes {
     }
 };
 
+// Untuned FP64 batches of kPackedFlops and more (and 5e7 per result block) run on
+// packed panels, those of kPackedLeast and more where the estimates say that
+// panels are faster: 1.5e9 flop into 16 blocks 98 us packed, 75 in tables, 3.9e9
+// into 64 141 and 135; but 2.6e9 into 5 of 45 x 84, K = 36 pairs of 1949, 450 and
+// 1540, 1.0e9 into one of 68 x 118, K = 36 of 1760, 290 and 990 (long chains, which
+// the packed path cuts into K segments).  From 5e9 on 7.3e9 into 144 181 and 237,
+// 3.3e10 into 64 944 and 1440.
+constexpr double kPackedFlops = 5e9, kPackedLeast = 1e9;
+
+// Estimated time (us) of a batch on packed panels: launches, the operands' bytes
+// read and written, the 128 x 128 tiles' k over 512 workgroups (blocks that share
+// operands are merged and leave no ragged tiles), the results.  Over 73 batches
+// of 1e9 to 5e9 flop the faster of this and the tables' estimate took 1.7% longer
+// than the faster of the two, 1.28 times as long at worst; tables throughout 21%
+// and 3.5 times.
+double packed_us(const std::vector<GemmTask> &tasks, const std::vector<GemmPair> &pairs) {
+    std::unordered_set<const double *> seen;
+    double operands = 0.0, whole = 0.0, ragged = 0.0, results = 0.0;
+    auto use = [&](const double *p, double elems) {
+        if (seen.insert(p).second) operands += elems;
+    };
+    for (const GemmTask &t : tasks) {
+        double k8 = 0.0;
+        for (int p = t.first; p < t.first + t.npairs; ++p) {
+            use(pairs[p].L, (double)t.M * pairs[p].K);
+            use(pairs[p].R, (double)t.N * pairs[p].K);
+            k8 += (pairs[p].K + 7) / 8 * 8;
+        }
+        whole += 1.1 * t.M * (double)t.N / (128.0 * 128.0) * k8;
+        ragged += (double)((t.M + 127) / 128) * (double)((t.N + 127) / 128) * k8;
+        results += (double)t.M * (double)t.N;
+    }
+    const bool merged = 2.0 * pairs.size() > 1.3 * seen.size();
+    return 27.0 + 16e-6 * 0.24 * operands + 0.21 / 512.0 * (merged ? whole : ragged) +
+           8e-6 * 2.0 * results;
+}
+
 // Tiles and K segments of a single contraction whose block pick_config gave
 // `cfg`.  Where the 64 x 64 tiles fill less than half the chip and K is long,
 // K runs in segments side by side: segment s > 0 into the stream's workspace,
@@ -472,6 +510,7 @@ struct sipgpu_batch_s {
     sipgpu::rt::BatchImage::Launch launch[sipgpu::rt::BatchImage::kMaxLaunches] = {};
     int nlaunches = 0;
     int ntasks = 0, npairs = 0, real_tiles = 0;
+    bool prefer_packed = false; // BatchImage::prefer_packed
     int ngroups = 0;    // panel paths: GEMM tasks after merging result blocks
     double flops = 0.0;
     void *dev = nullptr; // tiles | tasks | pairs | tab | parts
@@ -912,12 +951,16 @@ int sipgpu::rt::build_batch_image(const sipgpu_contraction *list, int n, BatchIm
     // ... unless the batch has so many small blocks that 64 x 64 tiles of them
     // fill the chip (a pinned configuration stays)
     auto kfast = [&](const GemmTask &t) { return t.npairs ? pairs[t.first].flags : 0; };
-    TileTimes times;
+    TileTimes times, large;
     if (own && pinned_config() < 0)
         for (const GemmTask &t : tasks)
-            if (pick_config(t.M, t.N, kfast(t)) == kGemmSplitK)
-                times.add(t, pairs.data() + t.first);
+            (pick_config(t.M, t.N, kfast(t)) == kGemmSplitK ? times : large)
+                .add(t, pairs.data() + t.first);
     const bool full = times.work[0] > 0.0 && times.us(true) < times.us(false);
+    if (nblocks > 0 && b.flops >= kPackedLeast && b.flops / nblocks >= 5e7)
+        b.prefer_packed = b.flops >= kPackedFlops ||
+                          packed_us(tasks, pairs) < (times.work[0] > 0.0 ? times.us(full) : 0.0) +
+                                                        (large.work[0] > 0.0 ? large.us(true) : 0.0);
     auto cfg_of = [&](const GemmTask &t) {
         const int c = own ? pick_config(t.M, t.N, kfast(t)) : b.cfg;
         return full && c == kGemmSplitK ? (int)kGemm64x64 : c;
@@ -1048,6 +1091,7 @@ int plan_batch_locked(Context &, const sipgpu_contraction *list, int n, sipgpu_b
     b.nparts = img.nparts;
     b.parts_max_n = img.parts_max_n;
     b.cfg = img.cfg;
+    b.prefer_packed = img.prefer_packed;
     b.flops = img.flops;
     b.ntiles = img.ntiles;
     b.ntasks = img.ntasks;
@@ -1856,17 +1900,10 @@ int plan_choice_locked(Context &c, const sipgpu_contraction *list, int n, int nm
     return 0;
 }
 
-// Untuned FP64 batches of this many flop (and 5e7 per result block) run on packed
-// panels.  Below, packing and the merged tiles' K segments cost more than the
-// table kernel's gathers: 1.5e9 flop into 16 blocks 98 us packed, 75 in
-// tables; 3.9e9 into 64 141 and 135; above, 7.3e9 into 144 181 and 237, 3.3e10
-// into 64 944 and 1440.
-constexpr double kPackedFlops = 5e9;
-
 // The plan sipgpu_batch_plan makes without a tuned choice.  Large batches
 // run on packed operand panels: the permutations are applied once per
 // block (one streaming pass) instead of per tile, and the GEMM runs over
-// whole 16-k stages of each task's virtual K.  Small batches (and single
+// whole 8-k stages of each task's virtual K.  Small batches (and single
 // contractions) keep the table-driven kernel: no extra pass, no panel
 // memory.  SIPGPU_FP64_PATH=tables|packed pins it.
 int plan_default_locked(Context &c, const sipgpu_contraction *list, int n,
@@ -1884,7 +1921,7 @@ int plan_default_locked(Context &c, const sipgpu_contraction *list, int n,
         out = std::move(b);
         return 0;
     }
-    bool packed = b->ntasks > 0 && b->flops >= kPackedFlops && b->flops / b->ntasks >= 5e7;
+    bool packed = b->prefer_packed;
     if (const char *e = std::getenv("SIPGPU_FP64_PATH")) {
         if (!std::strcmp(e, "tables")) packed = false;
         if (!std::strcmp(e, "packed")) packed = b->ntasks > 0;

@@ -991,9 +991,8 @@ int server_batch(sipgpu_server_s &S, int lane, std::vector<Pending> &batch) {
             rc = sipgpu::rt::build_panel_plan(list.data(), (int)list.size(), nmod, plan);
         } else {
             rc = sipgpu::rt::build_batch_image(list.data(), (int)list.size(), img);
-            // large FP64 batches run on packed panels (the table kernel
-            // gathers per tile)
-            if (!rc && img.ntasks > 0 && img.flops >= 1e9 && img.flops / img.ntasks >= 5e7 &&
+            // on packed panels where sipgpu_batch_plan would plan them
+            if (!rc && img.prefer_packed &&
                 sipgpu::rt::build_panel_plan(list.data(), (int)list.size(), 0, plan) == 0)
                 panels = true;
         }

@@ -280,7 +280,8 @@ int sipgpu_batch_plan_split_tol(const sipgpu_contraction *list, int n, double re
 /* Moduli count and operand bits P of a split batch (0 and 53 for FP64 batches). */
 int sipgpu_batch_split_info(sipgpu_batch_t batch, int *nmoduli, int *bits);
 /* How a planned batch runs.  sipgpu_batch_plan picks the packed path for
- * batches of at least 5e9 flop averaging 5e7 flop per result block: each
+ * batches of at least 5e9 flop averaging 5e7 flop per result block, and from
+ * 1e9 flop on for those with few tiles and a long K: each
  * operand block is first packed once into panels in MFMA operand order, then
  * one grouped GEMM runs over the 8-k stages of every task's concatenated K
  * (SIPGPU_FP64_PATH=tables|packed in the environment pins the choice). */

@@ -1,6 +1,7 @@
-// Host-only check of the table planner's choice of tiles (no device calls): few
+// Host-only check of the planner's choice of tiles and path (no device calls): few
 // small blocks run in 32 x 32 tiles with K split, batches whose 64 x 64 tiles
-// fill the chip in those, large blocks in 64 x 64 tiles beside few small ones.
+// fill the chip in those, large blocks in 64 x 64 tiles beside few small ones;
+// batches of 1e9 to 5e9 flop on packed panels where their tables' chains are long.
 #include <cstdio>
 #include <vector>
 #include "internal.h"
@@ -43,6 +44,14 @@ static std::vector<int> batch(int n, int M, int N, int K, int pairs, int form) {
     return configs(list);
 }
 
+static bool packed(int n, int M, int N, int K, int pairs, int form) {
+    std::vector<sipgpu_contraction> list;
+    add(list, n, M, N, K, pairs, form);
+    rt::BatchImage img;
+    CHECK(rt::build_batch_image(list.data(), (int)list.size(), img) == 0);
+    return img.prefer_packed;
+}
+
 int main() {
     const std::vector<int> split{kGemmSplitK}, big{kGemm64x64};
     for (int form = 0; form < 3; ++form) {
@@ -57,6 +66,18 @@ int main() {
         add(mixed, 3, 40, 50, 70, 1, form);
         CHECK((configs(mixed) == std::vector<int>{kGemmSplitK, kGemm64x64}));
     }
+    // measured, us in tables and packed: 1540 and 450, 990 and 290, 320 and 131
+    CHECK(packed(5, 45, 84, 1949, 36, 0));
+    CHECK(packed(1, 68, 118, 1760, 36, 1));
+    CHECK(packed(8, 80, 78, 1326, 16, 1));
+    // 39 and 72, 71 and 151, 191 and 499
+    CHECK(!packed(4, 224, 268, 249, 9, 1));
+    CHECK(!packed(4, 83, 1164, 320, 9, 2));
+    CHECK(!packed(61, 31, 1095, 57, 16, 1));
+    // below 1e9 flop, below 5e7 a block; from 5e9 on
+    CHECK(!packed(1, 68, 118, 1600, 36, 1));
+    CHECK(!packed(200, 100, 100, 100, 10, 0));
+    CHECK(packed(64, 450, 450, 450, 1, 2));
     std::printf(fails ? "FAILED %d\n" : "all ok\n", fails);
     return fails != 0;
 }
