@@ -31,8 +31,8 @@ struct FastDiv {
 };
 
 inline FastDiv make_fastdiv(uint32_t d) {
-    uint32_t s = 0;
-    while ((uint64_t(1) << s) < d) ++s;
+    const uint32_t s = d > 1 ? 32 - uint32_t(__builtin_clz(d - 1)) : 0;
+    if ((d & (d - 1)) == 0) return FastDiv{d, 1, s};
     const uint64_t m = ((uint64_t(1) << 32) * ((uint64_t(1) << s) - d)) / d + 1;
     return FastDiv{d, uint32_t(m), s};
 }
