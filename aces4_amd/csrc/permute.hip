@@ -227,18 +227,26 @@ void patches(PermArgs &a, int su, int sv, int turn, int64_t &grid) {
     grid = rounds ? (nu * nv + kXcds - 1) / kXcds * kXcds * su * sv : nu * nv;
 }
 
-// True if every row of every tile, read and written, is whole cache lines.
-bool whole_lines(const PermArgs &a) {
-    constexpr int kLine = 16; // doubles
-    bool ok = !a.row_mode && a.TU % kLine == 0 && a.TV % kLine == 0 && a.sizeU % kLine == 0 &&
-              a.sizeV % kLine == 0 &&
-              ((reinterpret_cast<uintptr_t>(a.in) | reinterpret_cast<uintptr_t>(a.out)) &
-               (kLine * sizeof(double) - 1)) == 0;
-    // the V dims' runs start at sums of the input strides, the U dims' at
-    // sums of the output strides; a tile of V stays in its first dim
+constexpr int kLine = 16; // doubles
+
+bool on_line(const void *p) {
+    return (reinterpret_cast<uintptr_t>(p) & (kLine * sizeof(double) - 1)) == 0;
+}
+
+// True if every row that a tile reads is whole cache lines: runs of U, which
+// start at sums of the input strides of V.
+bool whole_lines_in(const PermArgs &a) {
+    bool ok = !a.row_mode && a.TU % kLine == 0 && a.sizeU % kLine == 0 && on_line(a.in);
     for (int i = 0; i < a.nV; ++i) ok = ok && a.sinV[i] % kLine == 0;
+    return ok;
+}
+
+// True if every row that a tile writes is: runs of V inside its first dim, which
+// start at sums of the output strides of U.
+bool whole_lines_out(const PermArgs &a) {
+    bool ok = !a.row_mode && a.TV % kLine == 0 && a.sizeV % kLine == 0 && on_line(a.out) &&
+              a.nV > 0 && a.extV[0].d % kLine == 0;
     for (int i = 0; i < a.nU; ++i) ok = ok && a.soutU[i] % kLine == 0;
-    ok = ok && a.nV > 0 && a.extV[0].d % kLine == 0;
     return ok;
 }
 
@@ -253,13 +261,17 @@ bool whole_lines(const PermArgs &a) {
 // against 94 stored through it); larger ones store through it, so that the
 // halves of a line meet (113 x 97 x 109 x 101 reversed, 1.9 GB: launch order
 // 543 us, patches 494, stored through the cache 425; 7001 x 5003 transposed
-// 154 -> 142).  Rows of whole lines have nothing to share and run in launch
+// 154 -> 142), unless a tile writes whole lines (36 x 14 x 18 x 18 x 20 x 16
+// reversed in part, runs of 16 doubles: 163 us past the cache, 172 through it) or
+// whole rows (row mode: 63 x 82 x 81 x 94 as (1,3,4,2) 110 and 128; over 27 such
+// shapes 0.97 of launch order, 1.09 through the cache).  Rows of whole lines on
+// both sides have nothing to share and run in launch
 // order with streaming stores (64^4 reversed 56 us, in patches 57).  A batch
 // takes smaller patches, since its blocks have few tiles (144 blocks of 30,
 // 15: 81 us with 8 x 8, 76 with 4 x 8).
 void tile_order(bool large, bool batched, int turn, PermArgs &a, int64_t &grid) {
-    const bool lines = whole_lines(a);
-    a.stream = lines || !large;
+    const bool out = whole_lines_out(a), lines = out && whole_lines_in(a);
+    a.stream = out || a.row_mode || !large;
     // at least 64 patches of a single block (8 an XCD), and none in a batch's
     // smallest blocks, whose patches would not fill a round of the XCDs
     const int64_t tiles = (int64_t)a.tilesU * a.tilesV;

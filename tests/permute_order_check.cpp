@@ -1,7 +1,7 @@
 // Host-only check of the permutes' tile order (no device calls): over a batch's
 // workgroups every tile of every entry is visited once, workgroup numbers decoded
 // as the kernel decodes them; entries of fewer than 8 tiles have no empty
-// workgroup.
+// workgroup; blocks beyond the cache stream whole lines and whole rows only.
 #include <cstdio>
 #include <vector>
 #include "kernels.h"
@@ -75,6 +75,20 @@ int main() {
             all.push_back(mid[(i * 5 + c) % mid.size()]);
         }
     check(all);
+    // stores of a batch beyond the cache: whole lines written (reads ragged or
+    // not), whole rows, identity; ragged runs, and a block off its line
+    std::vector<int> first;
+    auto streams = [&](const Shape &s, uintptr_t base) {
+        return args_of({s, {{7001, 5003}, {2, 1}}}, first, base)[0].stream;
+    };
+    CHECK(streams({{512, 1024}, {2, 1}}, 1 << 20) == 1);
+    CHECK(streams({{511, 1024}, {2, 1}}, 1 << 20) == 1);
+    CHECK(streams({{512, 1041}, {2, 1}}, 1 << 20) == 0);
+    CHECK(streams({{36, 14, 18, 18, 20, 15}, {6, 2, 4, 3, 5, 1}}, 1 << 20) == 0);
+    CHECK(streams({{36, 14, 18, 18, 20, 16}, {6, 2, 4, 3, 5, 1}}, 1 << 20) == 1);
+    CHECK(streams({{512, 1024}, {2, 1}}, (1 << 20) + 8) == 0);
+    CHECK(streams({{41, 30, 29, 7}, {1, 3, 2, 4}}, 1 << 20) == 1);
+    CHECK(streams({{13, 11, 17}, {1, 2, 3}}, 1 << 20) == 1);
     std::printf(fails ? "FAILED %d\n" : "all ok\n", fails);
     return fails != 0;
 }

@@ -68,3 +68,27 @@ def test_permute_batch_tile_orders(copies):
     b.destroy()
     src.free()
     dst.free()
+
+
+def test_permute_batch_beyond_the_cache():
+    """2^25 elements and more: entries that store through the cache (ragged runs)
+    beside those that stream (whole lines, whole rows, identity, one tile) in one
+    launch."""
+    sg.init(0)
+    shapes = SHAPES + [([36, 14, 18, 18, 20, 16], [6, 2, 4, 3, 5, 1])] + SHAPES[:4]
+    sizes = [int(np.prod(d)) for d, _ in shapes]
+    at = np.concatenate([[0], np.cumsum([(s + 15) // 16 * 16 for s in sizes])])
+    assert sum(sizes) >= 1 << 25
+    x = uniform(10, int(at[-1]))
+    src, dst = sg.DeviceArray.from_host(x), sg.DeviceArray(x.size)
+    print("permute batch beyond the cache", len(shapes), flush=True)
+    b = sg.PermuteBatch([sg.permutation(d, [1] + p, src.at(int(o)), dst.at(int(o)))
+                         for (d, p), o in zip(shapes, at)])
+    b.execute()
+    sg.synchronize()
+    got = dst.download()
+    for (d, p), o, n in zip(shapes, at, sizes):
+        assert np.array_equal(got[o:o + n], transposed(x[o:o + n], d, p)), (d, p)
+    b.destroy()
+    src.free()
+    dst.free()
