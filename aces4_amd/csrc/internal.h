@@ -105,6 +105,14 @@ inline hipError_t launch_batch_gemm(GemmArgs args, const BatchImage::Launch *l, 
 int build_batch_image(const sipgpu_contraction *list, int n, BatchImage &img, int cfg = -1,
                       int split_cus = 0);
 
+// Tile configuration and K segments (kseg k each) of a single contraction whose
+// block holds dsize elements.
+struct SegmentPlan {
+    int cfg, nseg;
+    int64_t kseg;
+};
+SegmentPlan plan_single(const GemmTask &task, const GemmPair &pair, int64_t dsize);
+
 // Choices of the panel planner; -1 takes the default (environment, then the
 // built-in rule).
 struct PanelOptions {

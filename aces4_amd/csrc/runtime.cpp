@@ -61,6 +61,7 @@ int hip_fail(hipError_t e, const char *what) {
 namespace {
 
 using sipgpu::rt::BatchImage;
+using sipgpu::rt::SegmentPlan;
 using sipgpu::rt::fail;
 using sipgpu::rt::hip_fail;
 double g_last_clock_mhz = 0.0; // shader clock seen by the last MFMA calibration
@@ -351,10 +352,7 @@ double packed_us(const std::vector<GemmTask> &tasks, const std::vector<GemmPair>
 // in us, 32 x 32 and 64 x 64: 100 tiles, K = 4096 45 and 65; 270 tiles 98 and
 // 92; along k 100 tiles, K = 1024 23 and 24, K = 4096 63 and 55; 270 tiles, K =
 // 2048 79 and 47, and 115 in one segment of 32 x 32 tiles.
-struct SegmentPlan {
-    int cfg, nseg;
-    int64_t kseg;
-};
+// A pinned configuration keeps its tiles.
 SegmentPlan plan_segments(int cfg, int64_t M, int64_t N, int64_t K, int kfast, int64_t dsize,
                           int64_t cus) {
     const int64_t big = ((M + 63) / 64) * ((N + 63) / 64);
@@ -376,7 +374,7 @@ SegmentPlan plan_segments(int cfg, int64_t M, int64_t N, int64_t K, int kfast, i
             if (w == 1 || t < best) best = t, want = w;
         }
         const double each = (both ? 0.1 : 0.128) * (big * most <= cus ? 0.82 : 1.0);
-        if (13.0 + (double)K / most * each < 0.97 * best) {
+        if (pinned_config() < 0 && 13.0 + (double)K / most * each < 0.97 * best) {
             cfg = kGemm64x64;
             want = most;
         }
@@ -384,6 +382,16 @@ SegmentPlan plan_segments(int cfg, int64_t M, int64_t N, int64_t K, int kfast, i
     const int64_t kseg = ((K + want - 1) / want + 15) / 16 * 16;
     return {cfg, (int)((K + kseg - 1) / kseg), kseg};
 }
+
+} // namespace
+
+sipgpu::rt::SegmentPlan sipgpu::rt::plan_single(const GemmTask &task, const GemmPair &pair,
+                                                int64_t dsize) {
+    return plan_segments(pick_config(task.M, task.N, pair.flags), task.M, task.N, pair.K,
+                         pair.flags, dsize, g_device_cus);
+}
+
+namespace {
 
 // One contraction on device pointers (no locking; caller holds the lock).
 // `fx` (may be null) replaces the stream's workspace and partials; with it
@@ -402,9 +410,7 @@ int contract_device(Context &c, sipgpu_stream_s &st, const int *ptrn, const doub
         GemmPair pair;
         make_task_pair(s, ds->kL, ds->mL, ds->kR, ds->nR, ds->mD, ds->nD, l, r, d,
                        accumulate ? 1 : 0, task, pair);
-        const SegmentPlan sp =
-            plan_segments(pick_config(task.M, task.N, pair.flags), task.M, task.N, pair.K,
-                          pair.flags, s.dsize, g_device_cus);
+        const SegmentPlan sp = sipgpu::rt::plan_single(task, pair, s.dsize);
         const int cfg = sp.cfg;
         int nseg = sp.nseg;
         const int bm = gemm_tile_m(cfg), bn = gemm_tile_n(cfg);
