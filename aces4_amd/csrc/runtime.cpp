@@ -387,8 +387,21 @@ SegmentPlan plan_segments(int cfg, int64_t M, int64_t N, int64_t K, int kfast, i
 
 sipgpu::rt::SegmentPlan sipgpu::rt::plan_single(const GemmTask &task, const GemmPair &pair,
                                                 int64_t dsize) {
-    return plan_segments(pick_config(task.M, task.N, pair.flags), task.M, task.N, pair.K,
-                         pair.flags, dsize, g_device_cus);
+    int cfg = pick_config(task.M, task.N, pair.flags);
+    // With more 64 x 64 tiles than CUs the shorter chains of the split-K tiles
+    // gain little where K is short: 945 x 2065, K = 9, 10.7 us in 64 x 64 tiles,
+    // 12.6 in split-K tiles; 1453 x 1358, K = 51, 15.3 and 16.8.  The estimates
+    // (made for batches) are 25% low for 64 x 64 tiles here: with that the choice
+    // was within 3% of the faster in 30 products of 264 to 510 tiles.
+    if (cfg == kGemmSplitK && pinned_config() < 0 &&
+        (int64_t)((task.M + 63) / 64) * ((task.N + 63) / 64) > g_device_cus) {
+        GemmTask one = task;
+        one.npairs = 1;
+        TileTimes times;
+        times.add(one, &pair);
+        if (times.us(true) < 0.75 * times.us(false)) cfg = kGemm64x64;
+    }
+    return plan_segments(cfg, task.M, task.N, pair.K, pair.flags, dsize, g_device_cus);
 }
 
 namespace {

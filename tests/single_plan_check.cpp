@@ -31,6 +31,11 @@ int main(int argc, char **argv) {
         CHECK(plan(850, 296, 2048, 3).cfg == kGemm64x64 && plan(850, 296, 2048, 3).nseg > 1);
         CHECK(plan(1200, 1200, 1200, 0).cfg == kGemmSplitK);
         CHECK(plan(2304, 2304, 1600, 0).cfg == kGemm64x64);
+        // more 64 x 64 tiles than CUs: by K
+        CHECK(plan(945, 2065, 9, 1).cfg == kGemm64x64);
+        CHECK(plan(1453, 1358, 51, 1).cfg == kGemm64x64);
+        CHECK(plan(675, 2184, 54, 1, 1).cfg == kGemmSplitK);
+        CHECK(plan(1600, 900, 1600, 1).cfg == kGemmSplitK);
     }
     std::printf(fails ? "FAILED %d\n" : "all ok\n", fails);
     return fails != 0;
