@@ -5,14 +5,13 @@
 // row sets (x, y1, y2), PB over column sets (x2, x3, y3)), and one energy
 // partial per box slot.  sipgpu_triples_pack fills the panels from the T, V1 and V2
 // blocks; sipgpu_triples_run computes the partials of a range of box
-// slots (one workgroup per box); sipgpu_triples_energy sums all partials in
-// slot order into the energy (deterministic).
+// slots (one workgroup per CU, each over many boxes); sipgpu_triples_energy sums
+// all partials in slot order into the energy (deterministic).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <cstring>
+#include <exception>
 #include <memory>
-#include <new>
 #include <numeric>
 #include <vector>
 
@@ -47,6 +46,12 @@ struct sipgpu_triples_s {
     long long slots = 0;   // box slots of the super-box order
     int super_v = 0;       // super-boxes along a virtual index
     bool packed = false;
+
+    ~sipgpu_triples_s() {
+        for (void *p : {tables, (void *)PA, (void *)PB, (void *)partial, (void *)sums,
+                        (void *)tuple_partial})
+            if (p) (void)hipFree(p);
+    }
 };
 
 namespace {
@@ -137,16 +142,12 @@ int sipgpu::rt::triples_tuple_boxes(const std::vector<int> &vseg, const std::vec
     return 0;
 }
 
-extern "C" {
+namespace {
 
-int sipgpu_triples_create(int nv, const int *v_seg, int no, const int *o_seg,
-                          const double *const *T, const double *const *V1,
-                          const double *const *V2, const double *e_occ, const double *e_vir,
-                          sipgpu_triples_t *plan) {
-    if (int rc = sipgpu::rt::refuse_in_capture("planning the triples")) return rc;
-    if (nv < 1 || no < 1 || !v_seg || !o_seg || !T || !V1 || !V2 || !e_occ || !e_vir || !plan)
-        return fail(SIPGPU_EARG, "triples: bad arguments");
-    if (int rc = sipgpu::rt::ensure_ready()) return rc;
+// sipgpu_triples_create after its checks.  Host memory that runs out throws.
+int create(int nv, const int *v_seg, int no, const int *o_seg, const double *const *T,
+           const double *const *V1, const double *const *V2, const double *e_occ,
+           const double *e_vir, sipgpu_triples_t *plan) {
     auto P = std::make_unique<sipgpu_triples_s>();
     P->nv = nv;
     P->no = no;
@@ -183,9 +184,6 @@ int sipgpu_triples_create(int nv, const int *v_seg, int no, const int *o_seg,
         if (!V2[i]) return fail(SIPGPU_EARG, "triples: null V2 block");
 
     auto no_memory = [&]() {
-        for (void *p : {(void *)P->tables, (void *)P->PA, (void *)P->PB, (void *)P->partial,
-                        (void *)P->sums, (void *)P->tuple_partial})
-            if (p) (void)hipFree(p);
         (void)hipGetLastError();
         return fail(SIPGPU_ENOMEM, "triples: device memory for the packed operands");
     };
@@ -196,18 +194,13 @@ int sipgpu_triples_create(int nv, const int *v_seg, int no, const int *o_seg,
     if (e == hipSuccess)
         e = hipMalloc(&P->tuple_partial, (size_t)max_tuple_boxes * sizeof(double));
     if (e != hipSuccess) return no_memory();
-    // built once the device holds a partial per slot: the host's classes are
-    // then at most a hundredth of that
-    if (pairs * (pairs + 1) * (pairs + 2) / 6 >= 1LL << 26) { // items hold class * 64
-        (void)no_memory();
+    // built once the device holds a partial per slot: a class (24 bytes) and its
+    // items (4 bytes a box, 64 at most) take up to an eleventh of its slots'
+    // partials (6 arrangements of 64)
+    if (pairs * (pairs + 1) * (pairs + 2) / 6 >= 1LL << 26) // items hold class * 64
         return fail(SIPGPU_ESIZE, "triples: too many super-box classes");
-    }
-    try {
-        P->orbits = super_box_classes((int)pairs);
-        list_boxes(*P);
-    } catch (const std::bad_alloc &) {
-        return no_memory();
-    }
+    P->orbits = super_box_classes((int)pairs);
+    list_boxes(*P);
 
     // tables: super-box classes, then int arrays, then pointer tables (16-byte aligned)
     std::vector<int> vseg_of(P->kd), oseg_of(P->kl), vstart(nv), ostart(no);
@@ -219,11 +212,16 @@ int sipgpu_triples_create(int nv, const int *v_seg, int no, const int *o_seg,
         ostart[s] = g;
         for (int q = 0; q < P->oseg[s]; ++q) oseg_of[g + q] = s;
     }
-    std::vector<unsigned char> img;
+    struct Piece {
+        const void *p;
+        size_t at, bytes;
+    };
+    std::vector<Piece> pieces;
+    size_t size = 0;
     auto put = [&](const void *p, size_t bytes) {
-        const size_t at = (img.size() + 15) & ~(size_t)15;
-        img.resize(at + bytes);
-        std::memcpy(img.data() + at, p, bytes);
+        const size_t at = (size + 15) & ~(size_t)15;
+        pieces.push_back(Piece{p, at, bytes});
+        size = at + bytes;
         return at;
     };
     const size_t o_orbits = put(P->orbits.data(), P->orbits.size() * sizeof(TriplesOrbit));
@@ -237,9 +235,11 @@ int sipgpu_triples_create(int nv, const int *v_seg, int no, const int *o_seg,
     const size_t o_T = put(T, nT * sizeof(double *));
     const size_t o_V1 = put(V1, nV1 * sizeof(double *));
     const size_t o_V2 = put(V2, nV2 * sizeof(double *));
-    e = hipMalloc(&P->tables, img.size());
-    if (e == hipSuccess)
-        e = hipMemcpy(P->tables, img.data(), img.size(), hipMemcpyHostToDevice);
+    e = hipMalloc(&P->tables, size);
+    for (const Piece &x : pieces)
+        if (e == hipSuccess && x.bytes)
+            e = hipMemcpy(static_cast<unsigned char *>(P->tables) + x.at, x.p, x.bytes,
+                          hipMemcpyHostToDevice);
     if (e != hipSuccess) return no_memory();
     const unsigned char *base = static_cast<const unsigned char *>(P->tables);
     P->d_orbits = reinterpret_cast<const TriplesOrbit *>(base + o_orbits);
@@ -259,13 +259,29 @@ int sipgpu_triples_create(int nv, const int *v_seg, int no, const int *o_seg,
     return 0;
 }
 
+} // namespace
+
+extern "C" {
+
+int sipgpu_triples_create(int nv, const int *v_seg, int no, const int *o_seg,
+                          const double *const *T, const double *const *V1,
+                          const double *const *V2, const double *e_occ, const double *e_vir,
+                          sipgpu_triples_t *plan) {
+    if (int rc = sipgpu::rt::refuse_in_capture("planning the triples")) return rc;
+    if (nv < 1 || no < 1 || !v_seg || !o_seg || !T || !V1 || !V2 || !e_occ || !e_vir || !plan)
+        return fail(SIPGPU_EARG, "triples: bad arguments");
+    if (int rc = sipgpu::rt::ensure_ready()) return rc;
+    try {
+        return create(nv, v_seg, no, o_seg, T, V1, V2, e_occ, e_vir, plan);
+    } catch (const std::exception &) { // std::bad_alloc, std::length_error
+        return fail(SIPGPU_ENOMEM, "triples: host memory for the plan");
+    }
+}
+
 int sipgpu_triples_destroy(sipgpu_triples_t P) {
     if (int rc = sipgpu::rt::refuse_in_capture("freeing the triples")) return rc;
     if (!P) return fail(SIPGPU_EARG, "null triples plan");
     SIPGPU_HIP_TRY(hipDeviceSynchronize());
-    for (void *p : {(void *)P->tables, (void *)P->PA, (void *)P->PB, (void *)P->partial,
-                    (void *)P->sums, (void *)P->tuple_partial})
-        if (p) (void)hipFree(p);
     delete P;
     return 0;
 }
