@@ -388,7 +388,8 @@ __global__ __launch_bounds__(kThreads) void triples_box_kernel(TriplesArgs a) {
     // apart: 20.9).  Each passes one
     // barrier a product, the first four waves at its end, the others at its
     // middle: behind it every wave has added the product before.
-    const bool late = wave >= 4;
+    // (a scalar: the barriers stand under scalar branches)
+    const bool late = __builtin_amdgcn_readfirstlane(wave) >= 4;
     const int middle = nkp / 2 / 3 * 3;
     // Permutation g, its first k-pair in register set S: nkp = 3 n + REST
     // k-pairs, so that the sets of three permutations are known here.
