@@ -166,6 +166,20 @@ void bind_panel_plan(const PanelPlan &p, void *desc, int8_t *planes, uint8_t *re
 // Enqueues the stages (SIPGPU_STAGE_* bits) of a bound panel batch.
 int execute_panels(SplitData &sd, bool split, int stages, hipStream_t s);
 
+// Boxes of the whole (T) sum over nvb virtual and nob occupied 5-blocks: the
+// classes of super-boxes, ascending in `first`, and the boxes to compute (class *
+// 64 + position), XCD by XCD (xcd_first[0 .. 8]), ascending in each.
+struct TriplesBoxes {
+    int super_v = 0;
+    std::vector<TriplesOrbit> orbits;
+    std::vector<unsigned> items;
+    size_t xcd_first[9] = {};
+};
+void triples_boxes(int nvb, int nob, TriplesBoxes &b);
+// The boxes that have an image among slots [box0, box0 + nbox), if they are at
+// most kTriplesGroups; else 0.
+int triples_short_range(const TriplesBoxes &b, long long box0, long long nbox,
+                        unsigned (&list)[kTriplesGroups]);
 // The boxes of a tuple of segments (of the virtual, then the occupied index
 // range): their count, and the tuple fields of the box kernel's arguments.
 // SIPGPU_ESIZE where the kernel's work items could not number them.

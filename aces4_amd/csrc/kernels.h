@@ -231,6 +231,8 @@ struct TriplesPackArgs {
     const int *vseg_start, *oseg_start; // global index of each segment's start
     const double *const *T, *const *V1, *const *V2;
 };
+// One workgroup of 512 per CU (fewer for fewer boxes).
+constexpr unsigned kTriplesGroups = 256;
 struct TriplesArgs {
     const double *PA, *PB;
     int nkp, nvb, nob;
@@ -245,6 +247,9 @@ struct TriplesArgs {
     unsigned begin[8], end[8];
     long long box0, nbox;
     int super_v;
+    // ... or, for a short range of slots (nlist > 0), the boxes list[0 .. nlist)
+    int nlist;
+    unsigned list[kTriplesGroups];
     // tuple mode: boxes 0 .. end[0] - 1 of first[d] .. first[d] + count[d] - 1
     // (first index fastest).  Elements count that lie in the global index
     // ranges [lo[d], lo[d] + wdims[d]) (both modes)
@@ -254,8 +259,6 @@ struct TriplesArgs {
     int lo[6], wdims[6];
 };
 hipError_t launch_triples_pack(const TriplesPackArgs &a, hipStream_t s);
-// One workgroup of 512 per CU (fewer for fewer boxes).
-constexpr unsigned kTriplesGroups = 256;
 hipError_t launch_triples_boxes(const TriplesArgs &a, hipStream_t s);
 // out[0] += factor * sum of partial[0 .. n) in a fixed order (sums: kTriplesSums doubles)
 hipError_t launch_triples_reduce(const double *partial, long long n, double *sums, double factor,

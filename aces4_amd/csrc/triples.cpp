@@ -26,10 +26,7 @@ using sipgpu::rt::hip_fail;
 struct sipgpu_triples_s {
     int nv = 0, no = 0;
     std::vector<int> vseg, oseg;
-    std::vector<TriplesOrbit> orbits; // ascending in `first`
-    // boxes to compute (class * 64 + position), XCD by XCD, ascending in each
-    std::vector<unsigned> items;
-    size_t xcd_first[9] = {};
+    sipgpu::rt::TriplesBoxes boxes;
     int nvb = 0, nob = 0;             // 5-blocks of the virtual / occupied range
     int kd = 0, kl = 0, nkp = 0;
     // device memory
@@ -44,7 +41,6 @@ struct sipgpu_triples_s {
     long long pa_doubles = 0, pb_doubles = 0;
     double *partial = nullptr, *sums = nullptr, *tuple_partial = nullptr;
     long long slots = 0;   // box slots of the super-box order
-    int super_v = 0;       // super-boxes along a virtual index
     bool packed = false;
 
     ~sipgpu_triples_s() {
@@ -56,50 +52,39 @@ struct sipgpu_triples_s {
 
 namespace {
 
-// Classes of super-boxes over n super pairs and, per class, its first
-// super-box: the 6, 3 or 1 distinct arrangements of a class are consecutive.
-std::vector<TriplesOrbit> super_box_classes(int n) {
-    std::vector<TriplesOrbit> out;
-    long long first = 0;
-    for (int p = 0; p < n; ++p)
-        for (int q = p; q < n; ++q)
-            for (int r = q; r < n; ++r) {
-                out.push_back(TriplesOrbit{{p, q, r}, 0, first});
-                first += p == q && q == r ? 1 : p == q || q == r ? 3 : 6;
-            }
-    return out;
+// The 5-blocks of pair m at position q of a super-box (bit 0 virtual, bit 1 occupied).
+int sub_of(unsigned q, int m) { return (int)((q >> m) & 1) | (int)((q >> (3 + m)) & 1) << 1; }
+
+// Class that holds a slot's super-box.
+long long class_of(const sipgpu::rt::TriplesBoxes &b, long long slot) {
+    return std::upper_bound(b.orbits.begin(), b.orbits.end(), slot / 64,
+                            [](long long s, const TriplesOrbit &o) { return s < o.first; }) -
+           b.orbits.begin() - 1;
 }
 
-// The boxes to compute: positions whose 5-blocks exist and whose pairs are
-// ascending (another order of equal super pairs is an image), the classes
-// dealt to the XCDs in turn.  Bit q of a mask stands for position q.
-void list_boxes(sipgpu_triples_s &P) {
-    uint64_t zero[6] = {}, asc01 = 0, asc12 = 0; // zero[d]: positions with bit d clear
-    for (unsigned q = 0; q < 64; ++q) {
-        const uint64_t bit = 1ull << q;
-        int sub[3];
-        for (int m = 0; m < 3; ++m) sub[m] = ((q >> m) & 1) | ((q >> (3 + m)) & 1) << 1;
-        for (int d = 0; d < 6; ++d)
-            if (!((q >> d) & 1)) zero[d] |= bit;
-        if (sub[0] <= sub[1]) asc01 |= bit;
-        if (sub[1] <= sub[2]) asc12 |= bit;
-    }
-    for (int x = 0; x < 8; ++x) {
-        P.xcd_first[x] = P.items.size();
-        for (size_t c = x; c < P.orbits.size(); c += 8) {
-            const int *p = P.orbits[c].p;
-            uint64_t boxes = ~0ull;
-            for (int m = 0; m < 3; ++m) {
-                if (2 * (p[m] % P.super_v) + 1 >= P.nvb) boxes &= zero[m];
-                if (2 * (p[m] / P.super_v) + 1 >= P.nob) boxes &= zero[3 + m];
-            }
-            if (p[0] == p[1]) boxes &= asc01;
-            if (p[1] == p[2]) boxes &= asc12;
-            for (; boxes; boxes &= boxes - 1)
-                P.items.push_back((unsigned)(c * 64) | (unsigned)__builtin_ctzll(boxes));
+// True if an arrangement of the pairs of the box at position q of class o lies
+// among slots [box0, box0 + nbox) (the kernel's image_slot).
+bool has_image(const TriplesOrbit &o, unsigned q, long long box0, long long nbox) {
+    static constexpr int kPerm[6][3] = {{0, 1, 2}, {0, 2, 1}, {1, 0, 2}, {1, 2, 0}, {2, 0, 1}, {2, 1, 0}};
+    const bool eq01 = o.p[0] == o.p[1], eq12 = o.p[1] == o.p[2];
+    for (int g = 0; g < 6; ++g) {
+        const int *t = kPerm[g];
+        int rank = g;
+        if (eq01 && eq12)
+            rank = 0;
+        else if (eq01)
+            rank = t[0] == 2 ? 0 : t[1] == 2 ? 1 : 2;
+        else if (eq12)
+            rank = t[0] == 0 ? 0 : t[1] == 0 ? 1 : 2;
+        unsigned at = 0;
+        for (int m = 0; m < 3; ++m) {
+            const int s = sub_of(q, t[m]);
+            at |= (unsigned)(s & 1) << m | (unsigned)(s >> 1) << (3 + m);
         }
+        const long long slot = (o.first + rank) * 64 + at;
+        if (slot >= box0 && slot < box0 + nbox) return true;
     }
-    P.xcd_first[8] = P.items.size();
+    return false;
 }
 
 // the 5-blocks that a segment at global index g touches
@@ -121,6 +106,68 @@ int max_seg_blocks(const std::vector<int> &seg) {
 }
 
 } // namespace
+
+void sipgpu::rt::triples_boxes(int nvb, int nob, TriplesBoxes &b) {
+    b = TriplesBoxes{};
+    b.super_v = (nvb + 1) / 2;
+    // the classes and, per class, its first super-box: the 6, 3 or 1 distinct
+    // arrangements of a class are consecutive
+    const int n = b.super_v * ((nob + 1) / 2);
+    long long first = 0;
+    for (int p = 0; p < n; ++p)
+        for (int q = p; q < n; ++q)
+            for (int r = q; r < n; ++r) {
+                b.orbits.push_back(TriplesOrbit{{p, q, r}, 0, first});
+                first += p == q && q == r ? 1 : p == q || q == r ? 3 : 6;
+            }
+    // The boxes to compute: positions whose 5-blocks exist and whose pairs are
+    // ascending (another order of equal super pairs is an image), the classes
+    // dealt to the XCDs in turn.  Bit q of a mask stands for position q.
+    uint64_t zero[6] = {}, asc01 = 0, asc12 = 0; // zero[d]: positions with bit d clear
+    for (unsigned q = 0; q < 64; ++q) {
+        const uint64_t bit = 1ull << q;
+        int sub[3];
+        for (int m = 0; m < 3; ++m) sub[m] = sub_of(q, m);
+        for (int d = 0; d < 6; ++d)
+            if (!((q >> d) & 1)) zero[d] |= bit;
+        if (sub[0] <= sub[1]) asc01 |= bit;
+        if (sub[1] <= sub[2]) asc12 |= bit;
+    }
+    for (int x = 0; x < 8; ++x) {
+        b.xcd_first[x] = b.items.size();
+        for (size_t c = x; c < b.orbits.size(); c += 8) {
+            const int *p = b.orbits[c].p;
+            uint64_t boxes = ~0ull;
+            for (int m = 0; m < 3; ++m) {
+                if (2 * (p[m] % b.super_v) + 1 >= nvb) boxes &= zero[m];
+                if (2 * (p[m] / b.super_v) + 1 >= nob) boxes &= zero[3 + m];
+            }
+            if (p[0] == p[1]) boxes &= asc01;
+            if (p[1] == p[2]) boxes &= asc12;
+            for (; boxes; boxes &= boxes - 1)
+                b.items.push_back((unsigned)(c * 64) | (unsigned)__builtin_ctzll(boxes));
+        }
+    }
+    b.xcd_first[8] = b.items.size();
+}
+
+int sipgpu::rt::triples_short_range(const TriplesBoxes &b, long long box0, long long nbox,
+                                    unsigned (&list)[kTriplesGroups]) {
+    if (nbox <= 0) return 0;
+    const long long c0 = class_of(b, box0), c1 = class_of(b, box0 + nbox - 1);
+    if (c1 - c0 >= kTriplesGroups) return 0;
+    unsigned n = 0;
+    for (long long c = c0; c <= c1; ++c) {
+        const auto f = b.items.begin() + b.xcd_first[c % 8],
+                   l = b.items.begin() + b.xcd_first[c % 8 + 1];
+        for (auto i = std::lower_bound(f, l, (unsigned)c * 64); i != l && *i / 64 == c; ++i) {
+            if (!has_image(b.orbits[c], *i % 64, box0, nbox)) continue;
+            if (n == kTriplesGroups) return 0;
+            list[n++] = *i;
+        }
+    }
+    return (int)n;
+}
 
 int sipgpu::rt::triples_tuple_boxes(const std::vector<int> &vseg, const std::vector<int> &oseg,
                                     const int *tuple, TriplesArgs &a, long long &boxes) {
@@ -168,8 +215,7 @@ int create(int nv, const int *v_seg, int no, const int *o_seg, const double *con
     const long long per_set = 8LL * P->nkp * 128;
     P->pa_doubles = nvb * nob * nob * per_set;
     P->pb_doubles = nvb * nvb * nob * per_set;
-    P->super_v = (P->nvb + 1) / 2;
-    const long long pairs = (long long)P->super_v * ((P->nob + 1) / 2);
+    const long long pairs = ((nvb + 1) / 2) * ((nob + 1) / 2);
     P->slots = 64 * pairs * pairs * pairs;
     const long long vmax = max_seg_blocks(P->vseg), omax = max_seg_blocks(P->oseg);
     const long long max_tuple_boxes = vmax * vmax * vmax * omax * omax * omax;
@@ -199,8 +245,7 @@ int create(int nv, const int *v_seg, int no, const int *o_seg, const double *con
     // partials (6 arrangements of 64)
     if (pairs * (pairs + 1) * (pairs + 2) / 6 >= 1LL << 26) // items hold class * 64
         return fail(SIPGPU_ESIZE, "triples: too many super-box classes");
-    P->orbits = super_box_classes((int)pairs);
-    list_boxes(*P);
+    sipgpu::rt::triples_boxes(P->nvb, P->nob, P->boxes);
 
     // tables: super-box classes, then int arrays, then pointer tables (16-byte aligned)
     std::vector<int> vseg_of(P->kd), oseg_of(P->kl), vstart(nv), ostart(no);
@@ -224,8 +269,8 @@ int create(int nv, const int *v_seg, int no, const int *o_seg, const double *con
         size = at + bytes;
         return at;
     };
-    const size_t o_orbits = put(P->orbits.data(), P->orbits.size() * sizeof(TriplesOrbit));
-    const size_t o_items = put(P->items.data(), P->items.size() * sizeof(unsigned));
+    const size_t o_orbits = put(P->boxes.orbits.data(), P->boxes.orbits.size() * sizeof(TriplesOrbit));
+    const size_t o_items = put(P->boxes.items.data(), P->boxes.items.size() * sizeof(unsigned));
     const size_t o_vext = put(P->vseg.data(), nv * sizeof(int));
     const size_t o_oext = put(P->oseg.data(), no * sizeof(int));
     const size_t o_vso = put(vseg_of.data(), vseg_of.size() * sizeof(int));
@@ -339,7 +384,7 @@ sipgpu::TriplesArgs box_args(const sipgpu_triples_s &P) {
     a.nob = P.nob;
     a.kd = P.kd;
     a.kl = P.kl;
-    a.super_v = P.super_v;
+    a.super_v = P.boxes.super_v;
     a.orbits = P.d_orbits;
     a.items = P.d_items;
     for (int d = 0; d < 6; ++d) a.wdims[d] = d < 3 ? P.kd : P.kl;
@@ -359,25 +404,21 @@ int sipgpu_triples_run(sipgpu_triples_t P, long long box0, long long nbox, sipgp
     sipgpu::TriplesArgs a = box_args(*P);
     a.partial = P->partial;
     const hipStream_t hs = sipgpu::rt::stream_of(s);
-    // class that holds a slot's super-box
-    auto class_of = [&](long long slot) {
-        return std::upper_bound(P->orbits.begin(), P->orbits.end(), slot / 64,
-                                [](long long s, const TriplesOrbit &o) { return s < o.first; }) -
-               P->orbits.begin() - 1;
-    };
     // one launch per SIPGPU_TRIPLES_LAUNCH_BOXES slots (about 0.3 s of the
     // whole sum at o = 30, v = 240).  A class that a cut divides is computed
     // by both launches.
     for (long long b = box0; b < box0 + nbox; b += SIPGPU_TRIPLES_LAUNCH_BOXES) {
         a.box0 = b;
         a.nbox = std::min<long long>(SIPGPU_TRIPLES_LAUNCH_BOXES, box0 + nbox - b);
-        const unsigned i0 = (unsigned)class_of(b) * 64,
-                       i1 = ((unsigned)class_of(b + a.nbox - 1) + 1) * 64;
+        const sipgpu::rt::TriplesBoxes &B = P->boxes;
+        a.nlist = sipgpu::rt::triples_short_range(B, b, a.nbox, a.list);
+        const unsigned i0 = (unsigned)class_of(B, b) * 64,
+                       i1 = ((unsigned)class_of(B, b + a.nbox - 1) + 1) * 64;
         for (int x = 0; x < 8; ++x) {
-            const auto f = P->items.begin() + P->xcd_first[x],
-                       l = P->items.begin() + P->xcd_first[x + 1];
-            a.begin[x] = (unsigned)(std::lower_bound(f, l, i0) - P->items.begin());
-            a.end[x] = (unsigned)(std::lower_bound(f, l, i1) - P->items.begin());
+            const auto f = B.items.begin() + B.xcd_first[x],
+                       l = B.items.begin() + B.xcd_first[x + 1];
+            a.begin[x] = (unsigned)(std::lower_bound(f, l, i0) - B.items.begin());
+            a.end[x] = (unsigned)(std::lower_bound(f, l, i1) - B.items.begin());
         }
         SIPGPU_HIP_TRY(sipgpu::launch_triples_boxes(a, hs));
     }

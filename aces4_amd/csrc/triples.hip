@@ -135,7 +135,9 @@ __global__ __launch_bounds__(256) void triples_pack_kernel(TriplesPackArgs a) {
 // index ranges, their pairs ascending) XCD by XCD, the classes dealt to the
 // XCDs in turn.  Slots number the 64 boxes of every super-box, the
 // arrangements of a class next to each other, so that any range of slots
-// holds most images of the boxes it computes.
+// holds most images of the boxes it computes.  A range of few boxes comes as a
+// list instead, only boxes with an image in it, one to a workgroup over all
+// XCDs (one slot 93 us; 177 with its whole class on one XCD).
 struct BoxId {
     int p[3];        // the class's super pairs
     long long first; // its first super-box
@@ -179,7 +181,7 @@ __device__ __forceinline__ void box_of(const TriplesArgs &a, unsigned t, int (&b
         }
         return;
     }
-    const unsigned item = a.items[t];
+    const unsigned item = a.nlist ? a.list[t] : a.items[t];
     const TriplesOrbit o = a.orbits[item >> 6];
     id.first = o.first;
 #pragma unroll
@@ -233,9 +235,9 @@ __global__ __launch_bounds__(kThreads) void triples_box_kernel(TriplesArgs a) {
     const int wm = wave & 1, wn = wave >> 1;
     // this workgroup's work items: item, item + stride, ... < end
     unsigned item, end, stride;
-    if (a.tuple_mode) {
+    if (a.tuple_mode || a.nlist) {
         item = blockIdx.x;
-        end = a.end[0];
+        end = a.tuple_mode ? a.end[0] : (unsigned)a.nlist;
         stride = gridDim.x;
     } else {
         const int x = blockIdx.x & 7;
@@ -549,11 +551,12 @@ hipError_t launch_triples_pack(const TriplesPackArgs &a, hipStream_t s) {
 }
 
 hipError_t launch_triples_boxes(const TriplesArgs &a, hipStream_t s) {
-    unsigned most = 0; // work items of the longest list
-    for (int x = 0; x < (a.tuple_mode ? 1 : 8); ++x) most = std::max(most, a.end[x] - a.begin[x]);
+    const bool one_list = a.tuple_mode || a.nlist;
+    unsigned most = a.nlist; // work items of the longest list
+    for (int x = 0; x < (one_list ? 1 : 8); ++x) most = std::max(most, a.end[x] - a.begin[x]);
     if (most == 0) return hipSuccess;
-    const unsigned grid = a.tuple_mode ? std::min(most, kTriplesGroups)
-                                       : 8 * std::min(most, kTriplesGroups / 8);
+    const unsigned grid = one_list ? std::min(most, kTriplesGroups)
+                                   : 8 * std::min(most, kTriplesGroups / 8);
     if (a.nkp < 4) return hipErrorInvalidValue;
     if (a.nkp % 3 == 0)
         triples_box_kernel<0><<<grid, kThreads, 0, s>>>(a);

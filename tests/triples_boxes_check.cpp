@@ -1,14 +1,57 @@
-// Host-only check of a tuple's boxes (sipgpu::rt::triples_tuple_boxes): their
+// Host-only check of the boxes of (T) sums: of a tuple (triples_tuple_boxes: their
 // count and ranges, and the refusal of tuples whose boxes 32-bit work items
-// cannot number.
+// cannot number) and of short ranges of slots (triples_short_range: a slot has at
+// most one box, a range the boxes of its slots, all slots all boxes).
+#include <algorithm>
 #include <cstdio>
+#include <set>
 #include <vector>
 #include "internal.h"
 
 static int fails = 0;
 #define CHECK(c) do { if (!(c)) { std::printf("FAIL %s:%d %s\n", __FILE__, __LINE__, #c); ++fails; } } while (0)
 
+static void check_ranges(int nvb, int nob) {
+    using namespace sipgpu;
+    rt::TriplesBoxes b;
+    rt::triples_boxes(nvb, nob, b);
+    const long long n = ((nvb + 1) / 2) * ((nob + 1) / 2), slots = 64 * n * n * n;
+    std::set<unsigned> items(b.items.begin(), b.items.end()), seen;
+    CHECK(items.size() == b.items.size());
+    // boxes that differ by a permutation of their (virtual, occupied) pairs
+    const long long pairs = (long long)nvb * nob;
+    CHECK((long long)items.size() == pairs * (pairs + 1) * (pairs + 2) / 6);
+    std::vector<std::vector<unsigned>> of(slots);
+    unsigned list[kTriplesGroups];
+    long long boxes = 0;
+    for (long long s = 0; s < slots; ++s) {
+        const int k = rt::triples_short_range(b, s, 1, list);
+        CHECK(k <= 1);
+        boxes += k;
+        of[s].assign(list, list + k);
+        seen.insert(list, list + k);
+        for (int i = 0; i < k; ++i) CHECK(items.count(list[i]));
+    }
+    CHECK(boxes == pairs * pairs * pairs);
+    CHECK(seen == items);
+    for (long long s = 0; s < slots; s += 29)
+        for (long long m : {2LL, 37LL, 64LL, 300LL, 1000LL}) {
+            if (s + m > slots) continue;
+            std::set<unsigned> want;
+            for (long long t = s; t < s + m; ++t) want.insert(of[t].begin(), of[t].end());
+            const int k = rt::triples_short_range(b, s, m, list);
+            if (want.size() > kTriplesGroups)
+                CHECK(k == 0);
+            else
+                CHECK(k == (int)want.size() && std::set<unsigned>(list, list + k) == want);
+        }
+}
+
 int main() {
+    check_ranges(1, 1);
+    check_ranges(3, 2);
+    check_ranges(4, 3);
+    check_ranges(5, 4);
     auto boxes = [](const std::vector<int> &v, const std::vector<int> &o, std::vector<int> tuple,
                     sipgpu::TriplesArgs &a, long long &n) {
         n = 0;
