@@ -181,10 +181,11 @@ void triples_boxes(int nvb, int nob, TriplesBoxes &b);
 int triples_short_range(const TriplesBoxes &b, long long box0, long long nbox,
                         unsigned (&list)[kTriplesGroups]);
 // The boxes of a tuple of segments (of the virtual, then the occupied index
-// range): their count, and the tuple fields of the box kernel's arguments.
-// SIPGPU_ESIZE where the kernel's work items could not number them.
+// range), in the 5-blocks of the whole ranges or cut from the tuple's own start:
+// their count, and the tuple fields of the box kernel's arguments.  SIPGPU_ESIZE
+// where the kernel's work items could not number them.
 int triples_tuple_boxes(const std::vector<int> &vseg, const std::vector<int> &oseg,
-                        const int *tuple, TriplesArgs &a, long long &boxes);
+                        const int *tuple, bool cut, TriplesArgs &a, long long &boxes);
 
 } // namespace rt
 } // namespace sipgpu

@@ -203,8 +203,9 @@ hipError_t launch_slice(const SliceArgs &a, bool insert, double *tens, double *s
 // occupied index range are each cut into 5-blocks (block s starts at global
 // index 5 s, across segment boundaries, so only the last is shorter: cut
 // inside each segment instead, segments of 17, 18, 17, 14 | 13, 14 had
-// 729,000 partly empty boxes, not 592,704, 296 ms a sum against 40 with the
-// images of a box shared); a box is one 5-block per W index.
+// 729,000 partly empty boxes, not 592,704); a box is one 5-block per W index.
+// A tuple whose segments begin inside 5-blocks has more boxes than its own
+// extents need, so its panels are cut again from the tuple's own start.
 constexpr int kTriplesBox = 5;
 constexpr int kTriplesSums = 4096; // partial sums of the final reduction
 // A class of super-boxes (two 5-blocks per index) that differ by a
@@ -257,7 +258,15 @@ struct TriplesArgs {
     int first[6], count[6];
     double *wout;   // tuple mode, optional: W of the tuple (column-major)
     int lo[6], wdims[6];
+    // tuple mode: block 0 of index d starts at org[d] (0, or lo[d] with panels
+    // cut for the tuple); permutation g's set (x1, y1, y2) in PA is number
+    // base_a[g] + (x1 na1[g] + y1) na2[g] + y2, its set (x2, x3, y3) in PB likewise
+    int org[6], base_a[6], na1[6], na2[6], base_b[6], nb1[6], nb2[6];
 };
+// Cuts the panels of one tuple (the tuple fields of `t`) out of PA and PB of the
+// whole ranges, into `out`.
+hipError_t launch_triples_cut(const TriplesArgs &t, const double *PA, const double *PB, double *out,
+                              hipStream_t s);
 hipError_t launch_triples_pack(const TriplesPackArgs &a, hipStream_t s);
 hipError_t launch_triples_boxes(const TriplesArgs &a, hipStream_t s);
 // out[0] += factor * sum of partial[0 .. n) in a fixed order (sums: kTriplesSums doubles)

@@ -40,17 +40,23 @@ struct sipgpu_triples_s {
     double *PA = nullptr, *PB = nullptr;
     long long pa_doubles = 0, pb_doubles = 0;
     double *partial = nullptr, *sums = nullptr, *tuple_partial = nullptr;
+    // panels cut for one tuple at a time (sipgpu_triples_tuple), allocated by the
+    // first tuple that needs them, for the largest
+    double *cut = nullptr;
+    bool no_cut = false; // there is no room for them
     long long slots = 0;   // box slots of the super-box order
     bool packed = false;
 
     ~sipgpu_triples_s() {
         for (void *p : {tables, (void *)PA, (void *)PB, (void *)partial, (void *)sums,
-                        (void *)tuple_partial})
+                        (void *)tuple_partial, (void *)cut})
             if (p) (void)hipFree(p);
     }
 };
 
 namespace {
+
+constexpr int kPerm[6][3] = {{0, 1, 2}, {0, 2, 1}, {1, 0, 2}, {1, 2, 0}, {2, 0, 1}, {2, 1, 0}};
 
 // The 5-blocks of pair m at position q of a super-box (bit 0 virtual, bit 1 occupied).
 int sub_of(unsigned q, int m) { return (int)((q >> m) & 1) | (int)((q >> (3 + m)) & 1) << 1; }
@@ -65,7 +71,6 @@ long long class_of(const sipgpu::rt::TriplesBoxes &b, long long slot) {
 // True if an arrangement of the pairs of the box at position q of class o lies
 // among slots [box0, box0 + nbox) (the kernel's image_slot).
 bool has_image(const TriplesOrbit &o, unsigned q, long long box0, long long nbox) {
-    static constexpr int kPerm[6][3] = {{0, 1, 2}, {0, 2, 1}, {1, 0, 2}, {1, 2, 0}, {2, 0, 1}, {2, 1, 0}};
     const bool eq01 = o.p[0] == o.p[1], eq12 = o.p[1] == o.p[2];
     for (int g = 0; g < 6; ++g) {
         const int *t = kPerm[g];
@@ -170,7 +175,7 @@ int sipgpu::rt::triples_short_range(const TriplesBoxes &b, long long box0, long 
 }
 
 int sipgpu::rt::triples_tuple_boxes(const std::vector<int> &vseg, const std::vector<int> &oseg,
-                                    const int *tuple, TriplesArgs &a, long long &boxes) {
+                                    const int *tuple, bool cut, TriplesArgs &a, long long &boxes) {
     // (the kernel counts work items in 32 bits and adds a stride to them)
     constexpr long long kMost = 1LL << 31;
     boxes = 1;
@@ -180,16 +185,53 @@ int sipgpu::rt::triples_tuple_boxes(const std::vector<int> &vseg, const std::vec
             return fail(SIPGPU_EARG, "triples: tuple outside the segments");
         a.lo[d] = std::accumulate(seg.begin(), seg.begin() + tuple[d], 0);
         a.wdims[d] = seg[tuple[d]];
-        seg_blocks(a.lo[d], a.wdims[d], a.first[d], a.count[d]);
+        a.org[d] = cut ? a.lo[d] : 0;
+        seg_blocks(a.lo[d] - a.org[d], a.wdims[d], a.first[d], a.count[d]);
         boxes *= a.count[d];
         if (boxes >= kMost)
             return fail(SIPGPU_ESIZE, "triples: the tuple has 2^31 boxes or more");
     }
     a.end[0] = (unsigned)boxes;
+    // where the sets of the permutations are: in the whole ranges' panels, or
+    // one array of sets after the other
+    long long sets = 0;
+    for (int g = 0; g < 6; ++g) {
+        const int *p = kPerm[g];
+        a.na1[g] = cut ? a.count[3 + p[0]] : a.nob;
+        a.na2[g] = cut ? a.count[3 + p[1]] : a.nob;
+        a.nb1[g] = cut ? a.count[p[2]] : a.nvb;
+        a.nb2[g] = cut ? a.count[3 + p[2]] : a.nob;
+        a.base_a[g] = (int)sets;
+        if (cut) sets += (long long)a.count[p[0]] * a.na1[g] * a.na2[g];
+        a.base_b[g] = (int)sets;
+        if (cut) sets += (long long)a.count[p[1]] * a.nb1[g] * a.nb2[g];
+        if (sets >= kMost) return fail(SIPGPU_ESIZE, "triples: too many sets in a tuple");
+    }
     return 0;
 }
 
 namespace {
+
+// Room for the panels of any tuple cut from its own start: true if there is (not
+// where it would take more than the whole ranges' panels, and a capture does not
+// allocate).
+bool cut_room(sipgpu_triples_s &P, hipStream_t s) {
+    if (P.cut) return true;
+    if (P.no_cut || sipgpu::rt::thread_captures() || sipgpu::rt::capturing(s)) return false;
+    auto blocks = [](const std::vector<int> &seg) {
+        return (long long)(*std::max_element(seg.begin(), seg.end()) + sipgpu::kTriplesBox - 1) /
+               sipgpu::kTriplesBox;
+    };
+    const long long v = blocks(P.vseg), o = blocks(P.oseg);
+    const long long doubles = 6 * (v * o * o + v * v * o) * 8LL * P.nkp * 128;
+    P.no_cut = doubles > P.pa_doubles + P.pb_doubles ||
+               hipMalloc(&P.cut, (size_t)doubles * sizeof(double)) != hipSuccess;
+    if (P.no_cut) {
+        P.cut = nullptr;
+        (void)hipGetLastError();
+    }
+    return !P.no_cut;
+}
 
 // sipgpu_triples_create after its checks.  Host memory that runs out throws.
 int create(int nv, const int *v_seg, int no, const int *o_seg, const double *const *T,
@@ -441,8 +483,20 @@ int sipgpu_triples_tuple(sipgpu_triples_t P, const int *tuple, double factor, do
     a.partial = P->tuple_partial;
     a.wout = w_out;
     long long boxes = 0;
-    if (int rc = sipgpu::rt::triples_tuple_boxes(P->vseg, P->oseg, tuple, a, boxes)) return rc;
+    if (int rc = sipgpu::rt::triples_tuple_boxes(P->vseg, P->oseg, tuple, false, a, boxes)) return rc;
     const hipStream_t hs = sipgpu::rt::stream_of(s);
+    // Segments that begin inside 5-blocks touch one more each: panels cut from the
+    // tuple's own start save those boxes for a pass over its sets (segments of 17,
+    // 18, 17, 14 | 13, 14, tuple (1,1,1,1,1,1): 4096 boxes, or 1728).
+    sipgpu::TriplesArgs own = a;
+    long long own_boxes = 0;
+    if (sipgpu::rt::triples_tuple_boxes(P->vseg, P->oseg, tuple, true, own, own_boxes) == 0 &&
+        own_boxes < boxes && cut_room(*P, hs)) {
+        a = own;
+        boxes = own_boxes;
+        a.PA = a.PB = P->cut;
+        SIPGPU_HIP_TRY(sipgpu::launch_triples_cut(a, P->PA, P->PB, P->cut, hs));
+    }
     SIPGPU_HIP_TRY(sipgpu::launch_triples_boxes(a, hs));
     SIPGPU_HIP_TRY(sipgpu::launch_triples_reduce(P->tuple_partial, boxes, P->sums, factor, out, hs));
     return 0;

@@ -45,6 +45,7 @@ static_assert(kTriplesSums % kFinalThreads == 0, "the final sum's split");
 
 // the permutations P of (0, 1, 2), in the order W sums them
 __constant__ int kPerm[6][3] = {{0, 1, 2}, {0, 2, 1}, {1, 0, 2}, {1, 2, 0}, {2, 0, 1}, {2, 1, 0}};
+constexpr int kPermHost[6][3] = {{0, 1, 2}, {0, 2, 1}, {1, 0, 2}, {1, 2, 0}, {2, 0, 1}, {2, 1, 0}};
 
 // box digit strides in LDS: a fastest, then b, c, i, j, k
 __device__ __forceinline__ int box_stride(int d) {
@@ -120,6 +121,42 @@ __global__ __launch_bounds__(256) void triples_pack_kernel(TriplesPackArgs a) {
     }
 }
 
+// The sets of a tuple cut from its own start (TriplesArgs::org = lo): blockIdx.y
+// = 2 g + side.  One thread per 16 bytes, a row's elements k and k + 4, which
+// stand together in the whole ranges' panels as well.
+__global__ __launch_bounds__(256) void triples_cut_kernel(TriplesArgs t, const double *PA,
+                                                          const double *PB, double *out) {
+    const int g = blockIdx.y >> 1, side = blockIdx.y & 1;
+    const int p0 = kPerm[g][0], p1 = kPerm[g][1], p2 = kPerm[g][2];
+    // the set's three indices: (x1, y1, y2) or (x2, x3, y3)
+    const int d0 = side ? p1 : p0, d1 = side ? p2 : 3 + p0, d2 = 3 + (side ? p2 : p1);
+    const int n1 = side ? t.nb1[g] : t.na1[g], n2 = side ? t.nb2[g] : t.na2[g];
+    const long long total = (long long)t.count[d0] * n1 * n2 * 8 * t.nkp * 64;
+    const f64x2 *from = reinterpret_cast<const f64x2 *>(side ? PB : PA);
+    f64x2 *to = reinterpret_cast<f64x2 *>(out) +
+                (long long)(side ? t.base_b[g] : t.base_a[g]) * 8 * t.nkp * 64;
+    for (long long e = (long long)blockIdx.x * 256 + threadIdx.x; e < total;
+         e += (long long)gridDim.x * 256) {
+        const int lane = (int)(e & 63);
+        const long long u = e >> 6; // (set, row block, k-pair)
+        const int kp = (int)(u % t.nkp);
+        const long long sr = u / t.nkp;
+        const int row = (int)(sr & 7) * 16 + (lane & 15), set = (int)(sr >> 3);
+        const int l0 = set / (n1 * n2) * kBoxE + row % kBoxE,
+                  l1 = set / n2 % n1 * kBoxE + row / kBoxE % kBoxE,
+                  l2 = set % n2 * kBoxE + row / (kBoxE * kBoxE);
+        f64x2 v = {0.0, 0.0};
+        if (row < kBoxRows && l0 < t.wdims[d0] && l1 < t.wdims[d1] && l2 < t.wdims[d2]) {
+            const int g0 = t.lo[d0] + l0, g1 = t.lo[d1] + l1, g2 = t.lo[d2] + l2;
+            const long long s = ((long long)(g0 / kBoxE) * (side ? t.nvb : t.nob) + g1 / kBoxE) * t.nob +
+                                g2 / kBoxE;
+            const int r = g0 % kBoxE + kBoxE * (g1 % kBoxE + kBoxE * (g2 % kBoxE));
+            v = from[((s * 8 + (r >> 4)) * t.nkp + kp) * 64 + (r & 15) + (lane & 48)];
+        }
+        to[e] = v;
+    }
+}
+
 // ---------------------------------------------------------------- boxes --
 
 // W is unchanged when the pairs (a,i), (b,j), (c,k) are permuted together
@@ -171,8 +208,9 @@ __device__ __forceinline__ long long image_slot(const BoxId &b, int g) {
 
 // Box coordinates (5-block indices of a, b, c, i, j, k) of work item t.
 // Tuple mode: the boxes of one tuple, first index fastest.
+template <bool TUPLE>
 __device__ __forceinline__ void box_of(const TriplesArgs &a, unsigned t, int (&bc)[6], BoxId &id) {
-    if (a.tuple_mode) {
+    if (TUPLE) {
         unsigned q = t;
 #pragma unroll
         for (int d = 0; d < 6; ++d) {
@@ -219,7 +257,7 @@ __device__ __forceinline__ void group_barrier() {
 // the bounds tested per element, the waits between them and both waves of a
 // SIMD adding at once, the sum of o = 30, v = 60 took 24.9 ms; 20.9 now, of
 // which the MFMAs alone take 15.8 (76% busy; was 65%).
-template <int REST>
+template <int REST, bool TUPLE>
 __global__ __launch_bounds__(kThreads) void triples_box_kernel(TriplesArgs a) {
     __shared__ double W[kBoxElems + 64]; // 64: where the padded rows and columns go
     __shared__ double eps[6][kBoxE];
@@ -235,9 +273,9 @@ __global__ __launch_bounds__(kThreads) void triples_box_kernel(TriplesArgs a) {
     const int wm = wave & 1, wn = wave >> 1;
     // this workgroup's work items: item, item + stride, ... < end
     unsigned item, end, stride;
-    if (a.tuple_mode || a.nlist) {
+    if (TUPLE || a.nlist) {
         item = blockIdx.x;
-        end = a.tuple_mode ? a.end[0] : (unsigned)a.nlist;
+        end = TUPLE ? a.end[0] : (unsigned)a.nlist;
         stride = gridDim.x;
     } else {
         const int x = blockIdx.x & 7;
@@ -248,7 +286,7 @@ __global__ __launch_bounds__(kThreads) void triples_box_kernel(TriplesArgs a) {
     if (item >= end) return;
     int bc[6]; // the box being loaded
     BoxId id;
-    box_of(a, item, bc, id);
+    box_of<TUPLE>(a, item, bc, id);
 
     for (int t = tid; t < 6 * 128; t += kThreads) {
         const int g = t >> 7, x = t & 127;
@@ -271,8 +309,10 @@ __global__ __launch_bounds__(kThreads) void triples_box_kernel(TriplesArgs a) {
         const int x1 = pick(bc[0], bc[1], bc[2], p0), y1 = pick(bc[3], bc[4], bc[5], p0);
         const int x2 = pick(bc[0], bc[1], bc[2], p1), y2 = pick(bc[3], bc[4], bc[5], p1);
         const int x3 = pick(bc[0], bc[1], bc[2], p2), y3 = pick(bc[3], bc[4], bc[5], p2);
-        const long long rowset = ((long long)x1 * a.nob + y1) * a.nob + y2;
-        const long long colset = ((long long)x2 * a.nvb + x3) * a.nob + y3;
+        const long long rowset = TUPLE ? a.base_a[g] + ((long long)x1 * a.na1[g] + y1) * a.na2[g] + y2
+                                       : ((long long)x1 * a.nob + y1) * a.nob + y2;
+        const long long colset = TUPLE ? a.base_b[g] + ((long long)x2 * a.nb1[g] + x3) * a.nb2[g] + y3
+                                       : ((long long)x2 * a.nvb + x3) * a.nob + y3;
         pa = reinterpret_cast<const f64x2 *>(a.PA) + ((rowset * 8 + wm * 4) * nkp) * 64 + lane;
         pb = reinterpret_cast<const f64x2 *>(a.PB) + ((colset * 8 + wn * 2) * nkp) * 64 + lane;
     };
@@ -319,22 +359,24 @@ __global__ __launch_bounds__(kThreads) void triples_box_kernel(TriplesArgs a) {
     auto fetch_tables = [&]() {
         if (tid < 30) {
             const int d = tid / kBoxE;
-            int blk = bc[0];
+            int at = bc[0] * kBoxE + (TUPLE ? a.org[0] : 0);
 #pragma unroll
-            for (int e = 1; e < 6; ++e) blk = d == e ? bc[e] : blk;
-            const int g = blk * kBoxE + tid % kBoxE, total = d < 3 ? a.kd : a.kl;
+            for (int e = 1; e < 6; ++e)
+                at = d == e ? bc[e] * kBoxE + (TUPLE ? a.org[e] : 0) : at;
+            const int g = at + tid % kBoxE, total = d < 3 ? a.kd : a.kl;
             my_eps = g < total ? (d < 3 ? a.e_vir : a.e_occ)[g] : 0.0;
         }
         if (tid < 6) {
-            int g0 = bc[0], first = a.lo[0], ext = a.wdims[0];
+            // the first element that counts, from the box's own first
+            auto from = [&](int e) { return a.lo[e] - (TUPLE ? a.org[e] : 0) - bc[e] * kBoxE; };
+            int first = from(0), ext = a.wdims[0];
 #pragma unroll
             for (int e = 1; e < 6; ++e) {
-                g0 = tid == e ? bc[e] : g0;
-                first = tid == e ? a.lo[e] : first;
+                first = tid == e ? from(e) : first;
                 ext = tid == e ? a.wdims[e] : ext;
             }
-            my_lo = max(0, first - g0 * kBoxE);
-            my_hi = min(kBoxE, first + ext - g0 * kBoxE);
+            my_lo = max(0, first);
+            my_hi = min(kBoxE, first + ext);
         }
     };
     // add permutation g's product into the box: row (x1, y1, y2), column
@@ -399,7 +441,7 @@ __global__ __launch_bounds__(kThreads) void triples_box_kernel(TriplesArgs a) {
         constexpr int S = decltype(first_set)::value;
         // what is loaded after this permutation: the next one, then the next
         // box (after the last box its own operands, which nothing reads)
-        if (g == 5 && item + stride < end) box_of(a, item + stride, bc, id);
+        if (g == 5 && item + stride < end) box_of<TUPLE>(a, item + stride, bc, id);
         panels(g == 5 ? 0 : g + 1, npa, npb);
         for (int kp = 0; kp + 3 <= nkp; kp += 3) {
             if (late && kp == middle) group_barrier();
@@ -438,7 +480,7 @@ __global__ __launch_bounds__(kThreads) void triples_box_kernel(TriplesArgs a) {
         // and runs over ijk.
         double sum = 0.0;
         __syncthreads(); // the box is complete
-        if (!a.wout) {
+        if (!TUPLE || !a.wout) {
             const int abc = tid & 127;
             const int ea_i = abc % kBoxE, eb_i = (abc / kBoxE) % kBoxE, ec_i = abc / (kBoxE * kBoxE);
             if (abc < kBoxRows && ea_i >= lo[0] && ea_i < hi[0] && eb_i >= lo[1] && eb_i < hi[1] &&
@@ -454,8 +496,8 @@ __global__ __launch_bounds__(kThreads) void triples_box_kernel(TriplesArgs a) {
             }
         }
         // tuple mode with W written out: every element's global position
-        if (a.wout) box_of(a, item, bc, id);
-        for (int e = a.wout ? tid : kBoxElems; e < kBoxElems; e += kThreads) {
+        if (TUPLE && a.wout) box_of<TUPLE>(a, item, bc, id);
+        for (int e = TUPLE && a.wout ? tid : kBoxElems; e < kBoxElems; e += kThreads) {
             int q = e, dg[6];
             bool in = true;
 #pragma unroll
@@ -470,13 +512,11 @@ __global__ __launch_bounds__(kThreads) void triples_box_kernel(TriplesArgs a) {
             const double D = eps[3][dg[3]] + eps[4][dg[4]] + eps[5][dg[5]] - eps[0][dg[0]] -
                              eps[1][dg[1]] - eps[2][dg[2]];
             sum += (w / D) * w;
-            if (a.wout) {
-                long long o = 0;
+            long long o = 0;
 #pragma unroll
-                for (int d = 5; d >= 0; --d)
-                    o = o * a.wdims[d] + (bc[d] * kBoxE + dg[d] - a.lo[d]);
-                a.wout[o] = w;
-            }
+            for (int d = 5; d >= 0; --d)
+                o = o * a.wdims[d] + (a.org[d] + bc[d] * kBoxE + dg[d] - a.lo[d]);
+            a.wout[o] = w;
         }
         // fixed-order reduction: lanes by xor butterfly, then waves in order
 #pragma unroll
@@ -486,12 +526,12 @@ __global__ __launch_bounds__(kThreads) void triples_box_kernel(TriplesArgs a) {
         if (tid == 0) {
             double t = red[0];
             for (int w = 1; w < kThreads / 64; ++w) t += red[w];
-            if (a.tuple_mode) {
+            if (TUPLE) {
                 a.partial[item] = t;
             } else {
                 int unused[6];
                 BoxId id;
-                box_of(a, item, unused, id);
+                box_of<TUPLE>(a, item, unused, id);
                 // images that coincide store the same value twice
                 for (int g = 0; g < 6; ++g) {
                     const long long slot = image_slot(id, g);
@@ -501,7 +541,7 @@ __global__ __launch_bounds__(kThreads) void triples_box_kernel(TriplesArgs a) {
         }
         item += stride;
         if (item >= end) break;
-        if (a.wout) box_of(a, item, bc, id);
+        if (TUPLE && a.wout) box_of<TUPLE>(a, item, bc, id);
     }
 }
 
@@ -558,12 +598,26 @@ hipError_t launch_triples_boxes(const TriplesArgs &a, hipStream_t s) {
     const unsigned grid = one_list ? std::min(most, kTriplesGroups)
                                    : 8 * std::min(most, kTriplesGroups / 8);
     if (a.nkp < 4) return hipErrorInvalidValue;
-    if (a.nkp % 3 == 0)
-        triples_box_kernel<0><<<grid, kThreads, 0, s>>>(a);
-    else if (a.nkp % 3 == 1)
-        triples_box_kernel<1><<<grid, kThreads, 0, s>>>(a);
-    else
-        triples_box_kernel<2><<<grid, kThreads, 0, s>>>(a);
+    auto kernel = a.nkp % 3 == 0   ? a.tuple_mode ? triples_box_kernel<0, true> : triples_box_kernel<0, false>
+                  : a.nkp % 3 == 1 ? a.tuple_mode ? triples_box_kernel<1, true> : triples_box_kernel<1, false>
+                  : a.tuple_mode   ? triples_box_kernel<2, true>
+                                   : triples_box_kernel<2, false>;
+    kernel<<<grid, kThreads, 0, s>>>(a);
+    return hipGetLastError();
+}
+
+hipError_t launch_triples_cut(const TriplesArgs &t, const double *PA, const double *PB, double *out,
+                              hipStream_t s) {
+    // enough workgroups for the largest of the twelve set arrays
+    long long most = 0;
+    for (int g = 0; g < 6; ++g) {
+        const long long a = (long long)t.count[kPermHost[g][0]] * t.na1[g] * t.na2[g];
+        const long long b = (long long)t.count[kPermHost[g][1]] * t.nb1[g] * t.nb2[g];
+        most = std::max(most, std::max(a, b));
+    }
+    const long long blocks = (most * 8 * t.nkp * 64 + 255) / 256;
+    triples_cut_kernel<<<dim3((unsigned)std::min<long long>(blocks, 4096), 12), 256, 0, s>>>(t, PA, PB,
+                                                                                            out);
     return hipGetLastError();
 }
 

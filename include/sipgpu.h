@@ -640,8 +640,10 @@ int sipgpu_permute_rhs_to_lhs(int lrank, const int *lhs_ids, const int *rhs_ids,
  * sipgpu_triples_energy adds factor * (sum of all partials, in slot order)
  * to *out (a device double).  sipgpu_triples_tuple computes one tuple's
  * energy into *out (+=) and, if w_out is not null, writes its W block
- * (column-major a, b, c, i, j, k).  All calls on one plan must be ordered
- * (one stream). */
+ * (column-major a, b, c, i, j, k); the first tuple whose segments begin inside
+ * 5-blocks allocates panels for one tuple (not within a capture; without room
+ * for them the tuple runs on the whole ranges' panels, in more boxes).  All
+ * calls on one plan must be ordered (one stream). */
 #define SIPGPU_TRIPLES_LAUNCH_BOXES (1LL << 21)
 typedef struct sipgpu_triples_s *sipgpu_triples_t;
 int sipgpu_triples_create(int nv, const int *v_seg, int no, const int *o_seg,

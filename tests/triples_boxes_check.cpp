@@ -53,10 +53,10 @@ int main() {
     check_ranges(4, 3);
     check_ranges(5, 4);
     auto boxes = [](const std::vector<int> &v, const std::vector<int> &o, std::vector<int> tuple,
-                    sipgpu::TriplesArgs &a, long long &n) {
+                    sipgpu::TriplesArgs &a, long long &n, bool cut = false) {
         n = 0;
         a = sipgpu::TriplesArgs{};
-        return sipgpu::rt::triples_tuple_boxes(v, o, tuple.data(), a, n);
+        return sipgpu::rt::triples_tuple_boxes(v, o, tuple.data(), cut, a, n);
     };
     sipgpu::TriplesArgs a{};
     long long n = 0;
@@ -65,6 +65,16 @@ int main() {
     CHECK(n == 4LL * 4 * 4 * 4 * 3 * 3 && a.end[0] == (unsigned)n);
     CHECK(a.lo[1] == 17 && a.first[1] == 3 && a.count[1] == 4 && a.wdims[1] == 18);
     CHECK(a.lo[3] == 13 && a.first[3] == 2 && a.count[3] == 4 && a.wdims[3] == 14);
+    // cut from the tuple's own start: the boxes its extents need, its sets one
+    // array after the other
+    CHECK(boxes({17, 18}, {13, 14}, {0, 1, 0, 1, 0, 0}, a, n, true) == 0);
+    CHECK(n == 4LL * 4 * 4 * 3 * 3 * 3 && a.end[0] == (unsigned)n);
+    CHECK(a.lo[1] == 17 && a.org[1] == 17 && a.first[1] == 0 && a.count[1] == 4);
+    CHECK(a.lo[3] == 13 && a.org[3] == 13 && a.first[3] == 0 && a.count[3] == 3);
+    for (int g = 0; g < 6; ++g) {
+        CHECK(a.base_b[g] == a.base_a[g] + 4 * 3 * 3 && a.na1[g] == 3 && a.na2[g] == 3);
+        CHECK(a.nb1[g] == 4 && a.nb2[g] == 3 && (g == 0 || a.base_a[g] == a.base_b[g - 1] + 4 * 4 * 3));
+    }
     CHECK(boxes({17, 18}, {13, 14}, {0, 2, 0, 1, 0, 0}, a, n) == SIPGPU_EARG);
     CHECK(boxes({17, 18}, {13, 14}, {0, 1, 0, -1, 0, 0}, a, n) == SIPGPU_EARG);
     // one segment each: 35, 36 and 41 5-blocks in every index
