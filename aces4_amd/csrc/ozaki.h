@@ -76,7 +76,7 @@ struct OzChunkRef {
 };
 
 // Byte of a residue plane where row r of the chunk at unit `at` lies.
-__device__ __forceinline__ long long oz_row(uint32_t at, int r, int32_t stride) {
+__host__ __device__ __forceinline__ long long oz_row(uint32_t at, int r, int32_t stride) {
     return (long long)(at + (uint32_t)(r >> 4) * (uint32_t)stride) * (kPanelRows * kOzChunk) +
            (r & 15) * kOzChunk;
 }

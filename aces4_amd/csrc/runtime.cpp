@@ -1585,9 +1585,12 @@ int sipgpu::rt::build_panel_plan(const sipgpu_contraction *list, int n, int nmod
     }
     if (nmod && (opt.tile == kOzBM || opt.tile == kOzBigTile || opt.tile == kOzWideTile))
         tile = opt.tile;
-    // (the wide kernel's buffer loads reach 4 GiB)
-    if (tile == kOzWideTile && panel >= (1LL << 32) - 256) tile = kOzBigTile;
-    if (tile == kOzWideTile && big_tiles * nmod > kOzMaxGrid) tile = kOzBM;
+    // The wide kernel's buffer loads reach 4 GiB of a plane, and it runs one tile
+    // a workgroup.  Beyond, the 128 x 128 tiles: a ring batch (13 moduli) 2.74 ms
+    // with them, 2.79 with 256 x 256 in four waves; a small one 54 and 100 us.
+    if (tile == kOzWideTile &&
+        (panel >= (1LL << 32) - 256 || big_tiles * nmod > kOzMaxGrid))
+        tile = kOzBM;
     // the packed FP64 GEMM: 128 x 128 tiles, or 64 x 64 when chosen (small
     // batches cut into K segments write a quarter of the partial sums)
     if (!nmod && opt.tile == kOzSmallTile) tile = kOzSmallTile;

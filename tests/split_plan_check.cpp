@@ -1,8 +1,10 @@
 // Host-only check of the panel planner (no device calls): the descriptors of
 // large split batches fit the server's first slot size, every tile stands in the
-// work list once per modulus, the reconstruction items cover every result, and
-// products with an empty K keep their tiles.
+// work list once per modulus, the reconstruction items cover every result,
+// products with an empty K keep their tiles, and planes of 4 GiB and more run in
+// tiles that reach all of them.
 // Block addresses are stand-in integers (the planner only compares them).
+#include <algorithm>
 #include <cstdio>
 #include <map>
 #include <tuple>
@@ -112,6 +114,23 @@ int main() {
     check_lists(plan_of(3, 7, 0, 6));
     check_lists(plan_of(5, 17, 2, 14));
     check_lists(plan_of(40, 23, 0, 13));
+    {
+        const rt::PanelPlan below = plan_of(100, 64, 0, 6), above = plan_of(140, 64, 0, 6);
+        CHECK(below.plane_bytes < 1LL << 32 && below.tile == kOzWideTile);
+        CHECK(above.plane_bytes > 1LL << 32 && above.tile == kOzBM);
+        check_lists(above);
+        // every chunk's rows lie inside the plane, at offsets past 32 bits too
+        const OzTask *tasks = (const OzTask *)(above.host.data() + above.o_tasks);
+        const OzChunkRef *chunks = (const OzChunkRef *)(above.host.data() + above.o_chunks);
+        long long last = 0;
+        for (int t = 0; t < above.ngroups; ++t)
+            for (int c = 0; c < tasks[t].nchunks; ++c) {
+                const OzChunkRef &r = chunks[tasks[t].chunk0 + c];
+                last = std::max({last, oz_row(r.a, tasks[t].M - 1, r.stride),
+                                 oz_row(r.b, tasks[t].N - 1, r.stride)});
+            }
+        CHECK(last > 1LL << 32 && last + kOzChunk <= above.plane_bytes);
+    }
     for (int n : {1, 3, 20, 900})
         for (int nmod : {0, 6, 14}) check_empty(n, nmod);
     std::printf(fails ? "FAILED %d\n" : "all ok\n", fails);
