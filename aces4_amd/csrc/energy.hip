@@ -8,7 +8,7 @@
 // the virtual ones in index order (the order energy_denominator_rhf.F
 // do_rhf_den2/4/6 add them in).  Kernels: x /= D in place, and the fixed-
 // order reduction E += factor * sum (x / D) * y, whose per-workgroup
-// partials are summed by one thread in workgroup order (deterministic).
+// partials one workgroup sums in a fixed order (deterministic).
 #include "kernels.h"
 
 #include <type_traits>
@@ -20,28 +20,16 @@ namespace {
 constexpr int kEnergyThreads = 256;
 
 // Mixed-radix digits (index values) of element e, first index fastest.
-__device__ __forceinline__ void decode(const EnergyArgs &a, long long e, int (&idx)[kEnergyMaxRank]) {
-    // (e is a first element or a stride, below the launch's threads; 32-bit
-    // divisions take a fifth of the instructions of 64-bit ones)
-    if (e <= 0x7fffffff) {
-        unsigned r = (unsigned)e;
-#pragma unroll
-        for (int d = 0; d < kEnergyMaxRank; ++d) {
-            idx[d] = 0;
-            if (d < a.rank) {
-                const unsigned q = r / (unsigned)a.dims[d];
-                idx[d] = (int)(r - q * (unsigned)a.dims[d]);
-                r = q;
-            }
-        }
-        return;
-    }
+// (e is a first element or the grid's stride, at most kEnergyBlocks *
+// kEnergyThreads; 32-bit divisions take a fifth of the instructions of 64-bit ones)
+__device__ __forceinline__ void decode(const EnergyArgs &a, unsigned e, int (&idx)[kEnergyMaxRank]) {
 #pragma unroll
     for (int d = 0; d < kEnergyMaxRank; ++d) {
         idx[d] = 0;
         if (d < a.rank) {
-            idx[d] = (int)(e % a.dims[d]);
-            e /= a.dims[d];
+            const unsigned q = e / (unsigned)a.dims[d];
+            idx[d] = (int)(e - q * (unsigned)a.dims[d]);
+            e = q;
         }
     }
 }
@@ -132,8 +120,8 @@ __global__ __launch_bounds__(kEnergyThreads) void denominator_divide_kernel(Ener
     const long long e0 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     const long long S = (long long)gridDim.x * blockDim.x;
     int idx[kEnergyMaxRank], step[kEnergyMaxRank];
-    decode(a, e0, idx);
-    decode(a, S, step);
+    decode(a, (unsigned)e0, idx);
+    decode(a, (unsigned)S, step);
     double q[kEnergyAhead];
 #pragma unroll
     for (int u = 0; u < kEnergyAhead; ++u) q[u] = e0 + u * S < a.n ? x[e0 + u * S] : 0.0;
@@ -162,8 +150,8 @@ __global__ __launch_bounds__(kEnergyThreads) void energy_partial_kernel(EnergyAr
     const long long S = (long long)gridDim.x * blockDim.x;
     const bool same = x == y;
     int idx[kEnergyMaxRank], step[kEnergyMaxRank];
-    decode(a, e0, idx);
-    decode(a, S, step);
+    decode(a, (unsigned)e0, idx);
+    decode(a, (unsigned)S, step);
     double qx[kEnergyAhead], qy[kEnergyAhead];
 #pragma unroll
     for (int u = 0; u < kEnergyAhead; ++u) {
@@ -206,8 +194,8 @@ __global__ __launch_bounds__(kEnergyThreads) void energy_parts_kernel(EnergyArgs
     const long long e0 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     const long long S = (long long)gridDim.x * blockDim.x;
     int idx[kEnergyMaxRank], step[kEnergyMaxRank];
-    decode(a, e0, idx);
-    decode(a, S, step);
+    decode(a, (unsigned)e0, idx);
+    decode(a, (unsigned)S, step);
     double v = 0.0;
     for (long long e = e0; e < a.n; e += S) {
         double x[kAddManyMax];

@@ -46,3 +46,14 @@ def test_denominator_and_energy(dims, signs):
     assert np.array_equal(xd.download(), x / D)
     for v in [xd, yd, out] + ed:
         v.free()
+
+
+# over 4 x 4096 x 256 elements: every thread's queue of loads is refilled, and its
+# digits advance more than four times
+LARGE = [([67, 63, 37, 29], [-1, 1, -1, 1]), ([2101, 23, 9, 11], [-1, -1, 1, 1])]
+
+
+@pytest.mark.parametrize("dims, signs", LARGE, ids=lambda v: str(v))
+def test_blocks_longer_than_the_loads_ahead(dims, signs):
+    assert np.prod(dims) > 4 * 4096 * 256
+    test_denominator_and_energy(dims, signs)
