@@ -10,6 +10,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstring>
 #include <exception>
 #include <memory>
 #include <numeric>
@@ -299,20 +300,18 @@ int create(int nv, const int *v_seg, int no, const int *o_seg, const double *con
         ostart[s] = g;
         for (int q = 0; q < P->oseg[s]; ++q) oseg_of[g + q] = s;
     }
-    struct Piece {
-        const void *p;
-        size_t at, bytes;
-    };
-    std::vector<Piece> pieces;
-    size_t size = 0;
+    // (the two long lists are uploaded from where they are)
+    auto up16 = [](size_t v) { return (v + 15) & ~(size_t)15; };
+    const size_t orbit_bytes = P->boxes.orbits.size() * sizeof(TriplesOrbit),
+                 item_bytes = P->boxes.items.size() * sizeof(unsigned);
+    const size_t o_orbits = 0, o_items = up16(orbit_bytes), o_img = up16(o_items + item_bytes);
+    std::vector<unsigned char> img;
     auto put = [&](const void *p, size_t bytes) {
-        const size_t at = (size + 15) & ~(size_t)15;
-        pieces.push_back(Piece{p, at, bytes});
-        size = at + bytes;
-        return at;
+        const size_t at = up16(img.size());
+        img.resize(at + bytes);
+        std::memcpy(img.data() + at, p, bytes);
+        return o_img + at;
     };
-    const size_t o_orbits = put(P->boxes.orbits.data(), P->boxes.orbits.size() * sizeof(TriplesOrbit));
-    const size_t o_items = put(P->boxes.items.data(), P->boxes.items.size() * sizeof(unsigned));
     const size_t o_vext = put(P->vseg.data(), nv * sizeof(int));
     const size_t o_oext = put(P->oseg.data(), no * sizeof(int));
     const size_t o_vso = put(vseg_of.data(), vseg_of.size() * sizeof(int));
@@ -322,11 +321,15 @@ int create(int nv, const int *v_seg, int no, const int *o_seg, const double *con
     const size_t o_T = put(T, nT * sizeof(double *));
     const size_t o_V1 = put(V1, nV1 * sizeof(double *));
     const size_t o_V2 = put(V2, nV2 * sizeof(double *));
-    e = hipMalloc(&P->tables, size);
-    for (const Piece &x : pieces)
-        if (e == hipSuccess && x.bytes)
-            e = hipMemcpy(static_cast<unsigned char *>(P->tables) + x.at, x.p, x.bytes,
+    e = hipMalloc(&P->tables, o_img + img.size());
+    auto upload = [&](size_t at, const void *p, size_t bytes) {
+        if (e == hipSuccess)
+            e = hipMemcpy(static_cast<unsigned char *>(P->tables) + at, p, bytes,
                           hipMemcpyHostToDevice);
+    };
+    upload(o_orbits, P->boxes.orbits.data(), orbit_bytes);
+    upload(o_items, P->boxes.items.data(), item_bytes);
+    upload(o_img, img.data(), img.size());
     if (e != hipSuccess) return no_memory();
     const unsigned char *base = static_cast<const unsigned char *>(P->tables);
     P->d_orbits = reinterpret_cast<const TriplesOrbit *>(base + o_orbits);
