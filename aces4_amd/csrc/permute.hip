@@ -241,13 +241,17 @@ bool whole_lines_in(const PermArgs &a) {
     return ok;
 }
 
-// True if every row that a tile writes is: runs of V inside its first dim, which
-// start at sums of the output strides of U.
-bool whole_lines_out(const PermArgs &a) {
-    bool ok = !a.row_mode && a.TV % kLine == 0 && a.sizeV % kLine == 0 && on_line(a.out) &&
-              a.nV > 0 && a.extV[0].d % kLine == 0;
+// True if the runs of V in the output (its leading dims as far as they follow
+// each other there) are whole lines, and so every row that a tile of a multiple
+// of 16 v writes.
+bool whole_runs_out(const PermArgs &a) {
+    bool ok = !a.row_mode && on_line(a.out) && a.nV > 0;
     for (int i = 0; i < a.nU; ++i) ok = ok && a.soutU[i] % kLine == 0;
-    return ok;
+    int64_t run = 1;
+    int d = 0;
+    while (d < a.nV && a.soutV[d] == run) run *= a.extV[d++].d;
+    for (; d < a.nV; ++d) ok = ok && a.soutV[d] % kLine == 0;
+    return ok && run % kLine == 0;
 }
 
 // The order of a permute's tiles over the XCDs and how it stores.
@@ -262,15 +266,16 @@ bool whole_lines_out(const PermArgs &a) {
 // halves of a line meet (113 x 97 x 109 x 101 reversed, 1.9 GB: launch order
 // 543 us, patches 494, stored through the cache 425; 7001 x 5003 transposed
 // 154 -> 142), unless a tile writes whole lines (36 x 14 x 18 x 18 x 20 x 16
-// reversed in part, runs of 16 doubles: 163 us past the cache, 172 through it) or
-// whole rows (row mode: 63 x 82 x 81 x 94 as (1,3,4,2) 110 and 128; over 27 such
-// shapes 0.97 of launch order, 1.09 through the cache).  Rows of whole lines on
+// reversed in part 163 us past the cache, 172 through it; 23 x 15 x 26 x 18 x 22
+// x 12 as (5,6,3,1,2,4) 129 and 142) or whole rows (row mode: 63 x 82 x 81 x 94
+// as (1,3,4,2) 110 and 128; over 27 such shapes 0.97 of launch order, 1.09
+// through the cache).  Rows of whole lines on
 // both sides have nothing to share and run in launch
 // order with streaming stores (64^4 reversed 56 us, in patches 57).  A batch
 // takes smaller patches, since its blocks have few tiles (144 blocks of 30,
 // 15: 81 us with 8 x 8, 76 with 4 x 8).
 void tile_order(bool large, bool batched, int turn, PermArgs &a, int64_t &grid) {
-    const bool out = whole_lines_out(a), lines = out && whole_lines_in(a);
+    const bool out = whole_runs_out(a) && a.TV % kLine == 0, lines = out && whole_lines_in(a);
     a.stream = out || a.row_mode || !large;
     // at least 64 patches of a single block (8 an XCD), and none in a batch's
     // smallest blocks, whose patches would not fill a round of the XCDs
@@ -331,6 +336,7 @@ void fill_args(const PermutePlan &p, const double *in, double *out, PermArgs &a,
     a.TU = even_tile(p.sizeU, p.row_mode ? tile_elems : kPermMaxTU);
     a.TV = even_tile(p.sizeV, std::max<int64_t>(1, std::min<int64_t>(tile_elems / a.TU,
                                                                       kPermMaxTV)));
+    if (a.TV > kLine && whole_runs_out(a)) a.TV -= a.TV % kLine; // tiles end where lines do
     a.pitch = p.row_mode ? a.TU : (a.TU | 1);
     const int64_t tilesU = (a.sizeU + a.TU - 1) / a.TU;
     const int64_t tilesV = (a.sizeV + a.TV - 1) / a.TV;

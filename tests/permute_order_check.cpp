@@ -87,6 +87,11 @@ int main() {
     CHECK(streams({{36, 14, 18, 18, 20, 15}, {6, 2, 4, 3, 5, 1}}, 1 << 20) == 0);
     CHECK(streams({{36, 14, 18, 18, 20, 16}, {6, 2, 4, 3, 5, 1}}, 1 << 20) == 1);
     CHECK(streams({{512, 1024}, {2, 1}}, (1 << 20) + 8) == 0);
+    // runs of several dims: 18 x 22, 26, 12 follow each other, 24.75 lines each
+    CHECK(streams({{23, 15, 26, 18, 22, 12}, {5, 6, 3, 1, 2, 4}}, 1 << 20) == 1);
+    CHECK(streams({{23, 15, 26, 18, 22, 11}, {5, 6, 3, 1, 2, 4}}, 1 << 20) == 0);
+    CHECK(args_of({{{25, 44, 50, 31, 36}, {5, 3, 1, 4, 2}}}, first)[0].TV % 16 == 0);
+    CHECK(streams({{42, 39, 28, 42, 22}, {3, 5, 1, 2, 4}}, 1 << 20) == 0);
     CHECK(streams({{41, 30, 29, 7}, {1, 3, 2, 4}}, 1 << 20) == 1);
     CHECK(streams({{13, 11, 17}, {1, 2, 3}}, 1 << 20) == 1);
     std::printf(fails ? "FAILED %d\n" : "all ok\n", fails);
