@@ -267,7 +267,7 @@ bool whole_runs_out(const PermArgs &a) {
 // 543 us, patches 494, stored through the cache 425; 7001 x 5003 transposed
 // 154 -> 142), unless a tile writes whole lines (36 x 14 x 18 x 18 x 20 x 16
 // reversed in part 163 us past the cache, 172 through it; 23 x 15 x 26 x 18 x 22
-// x 12 as (5,6,3,1,2,4) 129 and 142) or whole rows (row mode: 63 x 82 x 81 x 94
+// x 12 as (5,6,3,1,2,4) 133 and 142) or whole rows (row mode: 63 x 82 x 81 x 94
 // as (1,3,4,2) 110 and 128; over 27 such shapes 0.97 of launch order, 1.09
 // through the cache).  Rows of whole lines on
 // both sides have nothing to share and run in launch
