@@ -18,7 +18,7 @@
 // permute of its batch),
 // makes its blocks resident, and launches the batch as one grouped launch,
 // its work list uploaded through a small ring of descriptor slots (no
-// allocation per batch).  Two device streams ("lanes"): large batches run
+// allocation per batch, but where a slot grows to a batch's list).  Two device streams ("lanes"): large batches run
 // in order on lane 0, and a small batch admitted while lane 0 is busy runs on
 // lane 1 beside it; a batch that touches a block the other lane's
 // unfinished batches write (or writes one they touch) first waits for them

@@ -164,8 +164,9 @@ __global__ __launch_bounds__(256) void triples_cut_kernel(TriplesArgs t, const d
 // to six boxes that differ by such a permutation have one energy.  The kernel
 // computes it once, on the box whose pairs are in ascending order, and stores
 // it for every image: a whole sum runs a sixth of its boxes (o = 30, v = 60,
-// segments of 20 and 10: 373,248 slots, 64,824 boxes; 133 -> 25.8 ms).  A slot's
-// value does not depend on which range of slots a call covers.
+// segments of 20 and 10: 373,248 slots, 64,824 boxes; this step alone took 133
+// -> 25.8 ms).  A slot's value does not depend on which range of slots a call
+// covers.
 //
 // Global mode: item 64 c + q is position q (one bit per index) of class c's
 // ascending super-box; the plan lists the items that are boxes (inside the
@@ -233,7 +234,7 @@ __device__ __forceinline__ void box_of(const TriplesArgs &a, unsigned t, int (&b
 
 // *w += x in LDS, no value returned: the wave does not wait for the sum
 // before it goes on with the next product (read, add, write: 21.7 ms a sum of
-// o = 30, v = 60, this 20.9).  Each element is added to once between two
+// o = 30, v = 60, so 20.9 at that time).  Each element is added to once between two
 // barriers, so the order of the sums is fixed.
 __device__ __forceinline__ void lds_add(double *w, double x) {
     __builtin_amdgcn_ds_atomic_fadd_f64((__attribute__((address_space(3))) double *)w, x);
@@ -255,8 +256,8 @@ __device__ __forceinline__ void group_barrier() {
 // fetches its next box's first operands and energies during the present one.
 // Adding a product into the box is 16384 LDS operations without a branch: with
 // the bounds tested per element, the waits between them and both waves of a
-// SIMD adding at once, the sum of o = 30, v = 60 took 24.9 ms; 20.9 now, of
-// which the MFMAs alone take 15.8 (76% busy; was 65%).
+// SIMD adding at once, the sum of o = 30, v = 60 took 24.9 ms; 20.4 now, its
+// matrix cores 78% busy by the counters.
 template <int REST, bool TUPLE>
 __global__ __launch_bounds__(kThreads) void triples_box_kernel(TriplesArgs a) {
     __shared__ double W[kBoxElems + 64]; // 64: where the padded rows and columns go
@@ -429,7 +430,7 @@ __global__ __launch_bounds__(kThreads) void triples_box_kernel(TriplesArgs a) {
     };
     // The two waves of a SIMD (w and w + 4) run half a product apart: one adds
     // its product into the box while the other multiplies (together: 21.6 ms,
-    // apart: 20.9).  Each passes one
+    // apart: 20.9, before tuples were compiled apart).  Each passes one
     // barrier a product, the first four waves at its end, the others at its
     // middle: behind it every wave has added the product before.
     // (a scalar: the barriers stand under scalar branches)
