@@ -266,12 +266,19 @@ int pick_config(int64_t M, int64_t N, int kfast) {
 // 1000 blocks of 320 x 320, K = 200, 1165 and 2084 (both along k), 1337 and 1899
 // (one), 1465 and 1789 (neither); 30 of them 53 and 66, 54 and 62, 57 and 58;
 // 1000 of 100^3 117 and 197; 16 of 100 x 100, K = 1600, 187 and 27; 285 of 31 x
-// 37, K = 2574, 383 and 172.  Over 806 batches of 32 to 16384 tiles of 64 x 64
-// the choice by these estimates took 0.7% longer than the faster of the two on
-// average, 1.45 times as long at worst (13 x 191, K = 6672 along k); 64 x 64 tiles
-// throughout 68% longer, split-K tiles throughout 10%.
+// 37, K = 2574, 383 and 172.  Operands that are read along k, 32 bytes of a line at
+// a time, and together exceed the 256 MB cache twice over also cost what each tile
+// reads of them at 3.5 (split-K) and 4 TB/s: 318 blocks of 14 x 162, K = 10374 in 16
+// pairs, 4.6 GB, 1305 and 1899; 2663 of 29 x 135, K = 1565 in 4, 1879 and 2617.
+// Over 806 batches of 32 to 16384 tiles of 64 x 64 the choice by these estimates
+// took 0.35% longer than the faster of the two on average, over 4881 others, mostly
+// along k, 1.0% (1.22 times as long in the worst hundredth, 1.6 at worst); on the
+// 806, 64 x 64 tiles throughout took 68% longer, split-K tiles throughout 10%.
 struct TileTimes {
+    static constexpr double kBeyondCache = 500e6; // bytes
     double chain[2] = {}, work[2] = {}; // split-K, 64 x 64
+    double read[2] = {};                // bytes that tiles read along k
+    bool beyond = false;                // of operands beyond the cache
     bool beta = false;
     // a block of M x N, the k of its pairs (also rounded up to 8 and 16 per pair)
     void add(const GemmTask &t, const GemmPair *list) {
@@ -290,6 +297,12 @@ struct TileTimes {
         const double mfma = tiles(16) * 0.003 * k;
         chain[0] = std::max(chain[0], 0.009 * k8 + 0.1 * pairs);
         work[0] += tiles(32) * (1.3 + kSmall[along] * k8 + 0.02 * pairs) + mfma;
+        if (along == 2)
+            for (int big = 0; big < 2; ++big) {
+                const int e = big ? 64 : 32;
+                read[big] += 8.0 * k * (t.M * (double)((t.N + e - 1) / e) +
+                                        t.N * (double)((t.M + e - 1) / e));
+            }
         chain[1] = std::max(chain[1], kChain[along] * k16 + 0.3 * pairs);
         work[1] += tiles(64) * (0.75 + kBig[along] * k16 + 0.12 * pairs) + mfma;
         beta = beta || t.beta;
@@ -297,7 +310,9 @@ struct TileTimes {
     // (a 64 x 64 tile adds to its block one load after another)
     double us(bool big) const {
         const double c = (double)std::max<int64_t>(g_device_cus, 1);
-        return (big ? beta ? 5.9 : 3.9 : 2.6) + std::hypot(chain[big], work[big] / c);
+        const double mem = beyond ? read[big] / (big ? 4e6 : 3.5e6) : 0.0;
+        return (big ? beta ? 5.9 : 3.9 : 2.6) +
+               std::hypot(chain[big], std::max(work[big] / c, mem));
     }
 };
 
@@ -975,6 +990,17 @@ int sipgpu::rt::build_batch_image(const sipgpu_contraction *list, int n, BatchIm
         for (const GemmTask &t : tasks)
             (pick_config(t.M, t.N, kfast(t)) == kGemmSplitK ? times : large)
                 .add(t, pairs.data() + t.first);
+    if (times.read[1] > TileTimes::kBeyondCache) { // the operands themselves, each once
+        std::unordered_set<const double *> seen;
+        double bytes = 0.0;
+        for (const GemmTask &t : tasks)
+            if ((kfast(t) & 3) == 3 && pick_config(t.M, t.N, kfast(t)) == kGemmSplitK)
+                for (int p = t.first; p < t.first + t.npairs; ++p) {
+                    if (seen.insert(pairs[p].L).second) bytes += 8.0 * t.M * pairs[p].K;
+                    if (seen.insert(pairs[p].R).second) bytes += 8.0 * t.N * pairs[p].K;
+                }
+        times.beyond = bytes > TileTimes::kBeyondCache;
+    }
     const bool full = times.work[0] > 0.0 && times.us(true) < times.us(false);
     if (nblocks > 0 && b.flops >= kPackedLeast && b.flops / nblocks >= 5e7)
         b.prefer_packed = b.flops >= kPackedFlops ||

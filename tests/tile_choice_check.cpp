@@ -44,6 +44,14 @@ static std::vector<int> batch(int n, int M, int N, int K, int pairs, int form) {
     return configs(list);
 }
 
+// the same with one pair of operands for all
+static std::vector<int> shared(int n, int M, int N, int K, int pairs, int form) {
+    std::vector<sipgpu_contraction> list;
+    add(list, n, M, N, K, pairs, form);
+    for (auto &e : list) e.l = list[0].l, e.r = list[0].r;
+    return configs(list);
+}
+
 static bool packed(int n, int M, int N, int K, int pairs, int form) {
     std::vector<sipgpu_contraction> list;
     add(list, n, M, N, K, pairs, form);
@@ -66,6 +74,13 @@ int main() {
         add(mixed, 3, 40, 50, 70, 1, form);
         CHECK((configs(mixed) == std::vector<int>{kGemmSplitK, kGemm64x64}));
     }
+    // operands along k beyond the cache: the tiles that read them less often (split-K
+    // 2617 us, 64 x 64 1879); within it, or read across k, as above
+    CHECK(batch(2663, 29, 135, 391, 4, 0) == big);
+    CHECK(batch(318, 14, 162, 648, 16, 0) == big);
+    CHECK(shared(2663, 29, 135, 391, 4, 0) == split);
+    CHECK(batch(2663, 29, 135, 391, 4, 2) == split);
+    CHECK(batch(100, 29, 135, 391, 4, 0) == split);
     // measured, us in tables and packed: 1540 and 450, 990 and 290, 320 and 131
     CHECK(packed(5, 45, 84, 1949, 36, 0));
     CHECK(packed(1, 68, 118, 1760, 36, 1));
