@@ -34,6 +34,8 @@ struct PermArgs {
 };
 
 struct PermutePlan;
+// Arguments of a permute on its own; returns its workgroup count.
+int64_t permute_args(const PermutePlan &plan, const double *in, double *out, PermArgs &args);
 hipError_t launch_permute(const PermutePlan &plan, const double *in, double *out,
                           hipStream_t stream);
 // Batched permutes: fills args[0..n), the workgroup offsets first[0..n]

@@ -229,8 +229,8 @@ void patches(PermArgs &a, int su, int sv, int turn, int64_t &grid) {
 
 constexpr int kLine = 16; // doubles
 
-bool on_line(const void *p) {
-    return (reinterpret_cast<uintptr_t>(p) & (kLine * sizeof(double) - 1)) == 0;
+bool on_line(const void *p, int line = kLine) {
+    return (reinterpret_cast<uintptr_t>(p) & (line * sizeof(double) - 1)) == 0;
 }
 
 // True if every row that a tile reads is whole cache lines: runs of U, which
@@ -242,16 +242,16 @@ bool whole_lines_in(const PermArgs &a) {
 }
 
 // True if the runs of V in the output (its leading dims as far as they follow
-// each other there) are whole lines, and so every row that a tile of a multiple
-// of 16 v writes.
-bool whole_runs_out(const PermArgs &a) {
-    bool ok = !a.row_mode && on_line(a.out) && a.nV > 0;
-    for (int i = 0; i < a.nU; ++i) ok = ok && a.soutU[i] % kLine == 0;
+// each other there) are whole lines (or lines of another size), and so every row
+// that a tile of a multiple of them writes.
+bool whole_runs_out(const PermArgs &a, int line = kLine) {
+    bool ok = !a.row_mode && on_line(a.out, line) && a.nV > 0;
+    for (int i = 0; i < a.nU; ++i) ok = ok && a.soutU[i] % line == 0;
     int64_t run = 1;
     int d = 0;
     while (d < a.nV && a.soutV[d] == run) run *= a.extV[d++].d;
-    for (; d < a.nV; ++d) ok = ok && a.soutV[d] % kLine == 0;
-    return ok && run % kLine == 0;
+    for (; d < a.nV; ++d) ok = ok && a.soutV[d] % line == 0;
+    return ok && run % line == 0;
 }
 
 // The order of a permute's tiles over the XCDs and how it stores.
@@ -265,23 +265,27 @@ bool whole_runs_out(const PermArgs &a) {
 // against 94 stored through it); larger ones store through it, so that the
 // halves of a line meet (113 x 97 x 109 x 101 reversed, 1.9 GB: launch order
 // 543 us, patches 494, stored through the cache 425; 7001 x 5003 transposed
-// 154 -> 142), unless a tile writes whole lines (36 x 14 x 18 x 18 x 20 x 16
-// reversed in part 163 us past the cache, 172 through it; 23 x 15 x 26 x 18 x 22
-// x 12 as (5,6,3,1,2,4) 133 and 142) or whole rows (row mode: 63 x 82 x 81 x 94
-// as (1,3,4,2) 110 and 128; over 27 such shapes 0.97 of launch order, 1.09
-// through the cache).  Rows of whole lines on
-// both sides have nothing to share and run in launch
-// order with streaming stores (64^4 reversed 56 us, in patches 57).  A batch
-// takes smaller patches, since its blocks have few tiles (144 blocks of 30,
+// 154 -> 142), unless what a tile writes begins and ends at half lines, the 64
+// bytes that memory takes (36 x 14 x 18 x 18 x 20 x 16 reversed in part 163 us past
+// the cache, 172 through it; 5934 x 6104 transposed 109 and 123; over 96 shapes of
+// such halves 0.96, the worst 1.004, but over 30 batches 0.997 and 1.06: whole lines
+// there; tiles that end at quarters of a line go either way, 0.9 to 1.3, and stay)
+// or is whole rows (row mode: 63 x 82 x 81 x 94 as
+// (1,3,4,2) 110 and 128; over 27 such shapes 0.97 of launch order, 1.09 through the
+// cache).  Past the cache patches of 16 x 4 tiles are enough (over 96 such shapes
+// 0.983 of 16 x 16).  Rows of whole lines on both sides have nothing to share and
+// run in launch order with streaming stores (64^4 reversed 56 us, in patches 57).  A
+// batch takes smaller patches, since its blocks have few tiles (144 blocks of 30,
 // 15: 81 us with 8 x 8, 76 with 4 x 8).
 void tile_order(bool large, bool batched, int turn, PermArgs &a, int64_t &grid) {
     const bool out = whole_runs_out(a) && a.TV % kLine == 0, lines = out && whole_lines_in(a);
-    a.stream = out || a.row_mode || !large;
+    const bool halves = whole_runs_out(a, kLine / 2) && a.TV % (kLine / 2) == 0;
+    a.stream = (batched ? out : halves) || a.row_mode || !large;
     // at least 64 patches of a single block (8 an XCD), and none in a batch's
     // smallest blocks, whose patches would not fill a round of the XCDs
     const int64_t tiles = (int64_t)a.tilesU * a.tilesV;
     const int64_t in_all = batched ? (tiles < 64 ? 1 : 32)
-                                   : std::min<int64_t>(large ? 256 : 64, tiles / 64);
+                                   : std::min<int64_t>(a.stream ? 64 : 256, tiles / 64);
     if (lines || in_all <= 1) return patches(a, 1, 1, turn, grid);
     const int64_t along_u = std::min<int64_t>(batched ? 4 : large ? 16 : 8, in_all);
     const int su = even_tile(a.tilesU, along_u);
@@ -349,6 +353,12 @@ void fill_args(const PermutePlan &p, const double *in, double *out, PermArgs &a,
 
 } // namespace
 
+int64_t permute_args(const PermutePlan &p, const double *in, double *out, PermArgs &a) {
+    int64_t grid = 0;
+    fill_args(p, in, out, a, grid, p.size >= kLargeElems, false, 0);
+    return grid;
+}
+
 hipError_t launch_permute(const PermutePlan &p, const double *in, double *out,
                           hipStream_t stream) {
     if (p.size <= 0) return hipSuccess;
@@ -356,8 +366,7 @@ hipError_t launch_permute(const PermutePlan &p, const double *in, double *out,
         return hipMemcpyAsync(out, in, (size_t)p.size * sizeof(double),
                               hipMemcpyDeviceToDevice, stream);
     PermArgs a;
-    int64_t grid = 0;
-    fill_args(p, in, out, a, grid, p.size >= kLargeElems, false, 0);
+    const int64_t grid = permute_args(p, in, out, a);
     if (grid <= 0 || grid >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
     const int tile_cap = a.row_mode ? 0 : a.TV * a.pitch;
     const size_t lds = perm_lds_bytes(tile_cap, a.TV);

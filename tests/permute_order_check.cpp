@@ -1,7 +1,8 @@
 // Host-only check of the permutes' tile order (no device calls): over a batch's
 // workgroups every tile of every entry is visited once, workgroup numbers decoded
 // as the kernel decodes them; entries of fewer than 8 tiles have no empty
-// workgroup; blocks beyond the cache stream whole lines and whole rows only.
+// workgroup; blocks beyond the cache stream whole lines (a permute on its own: half
+// lines) and whole rows only.
 #include <cstdio>
 #include <vector>
 #include "kernels.h"
@@ -94,6 +95,23 @@ int main() {
     CHECK(streams({{42, 39, 28, 42, 22}, {3, 5, 1, 2, 4}}, 1 << 20) == 0);
     CHECK(streams({{41, 30, 29, 7}, {1, 3, 2, 4}}, 1 << 20) == 1);
     CHECK(streams({{13, 11, 17}, {1, 2, 3}}, 1 << 20) == 1);
+    // a permute on its own also streams whole halves of lines: 28 x 42 = 73.5 lines,
+    // blocks at half a line; not quarters, nor tiles of 66 v
+    auto alone = [&](const Shape &s, uintptr_t base) {
+        std::vector<int> t{1};
+        t.insert(t.end(), s.perm.begin(), s.perm.end());
+        PermutePlan plan;
+        CHECK(plan_permute((int)s.dims.size(), s.dims.data(), t.data(), plan) == 0);
+        PermArgs a;
+        CHECK(permute_args(plan, (const double *)base, (double *)(base + ((uintptr_t)1 << 35)), a) > 0);
+        return a.stream;
+    };
+    CHECK(alone({{42, 39, 28, 42, 22}, {3, 5, 1, 2, 4}}, 1 << 20) == 1);
+    CHECK(alone({{42, 39, 28, 42, 22}, {3, 5, 1, 2, 4}}, (1 << 20) + 64) == 1);
+    CHECK(alone({{42, 39, 28, 42, 22}, {3, 5, 1, 2, 4}}, (1 << 20) + 32) == 0);
+    CHECK(alone({{5934, 6104}, {2, 1}}, 1 << 20) == 1);
+    CHECK(alone({{33, 35, 30, 34, 31}, {3, 5, 1, 2, 4}}, 1 << 20) == 0);
+    CHECK(alone({{93, 72, 110, 73}, {2, 1, 3, 4}}, 1 << 20) == 0);
     std::printf(fails ? "FAILED %d\n" : "all ok\n", fails);
     return fails != 0;
 }
