@@ -284,7 +284,10 @@ int sipgpu_batch_split_info(sipgpu_batch_t batch, int *nmoduli, int *bits);
  * 1e9 flop on for those with few tiles and a long K: each
  * operand block is first packed once into panels in MFMA operand order, then
  * one grouped GEMM runs over the 8-k stages of every task's concatenated K
- * (SIPGPU_FP64_PATH=tables|packed in the environment pins the choice). */
+ * (SIPGPU_FP64_PATH=tables|packed in the environment pins the choice).  The
+ * path and, on the tables path, the tiles follow from the whole batch, and with
+ * them the order of a block's sums: its last bits are the same every time the
+ * batch runs, but may differ in another batch. */
 enum { SIPGPU_BATCH_TABLES = 0, SIPGPU_BATCH_PACKED = 1, SIPGPU_BATCH_SPLIT = 2 };
 int sipgpu_batch_kind(sipgpu_batch_t batch, int *kind);
 /* Runs only some stages of a planned batch on `s` (no reference
@@ -495,7 +498,9 @@ int sipgpu_cache_end_program(sipgpu_cache_t cache, unsigned long long *kept);
  * batched permute launch, one grouped FP64
  * launch, or the split-precision stages with their planes in a server-owned
  * scratch buffer per stream (grown, after that stream drains, to the
- * largest batch's need).  Two device streams: large batches (>= 1e9 flop)
+ * largest batch's need).  A batch's work list is uploaded through one of four
+ * slots of 32 MiB, which grow up to 256 MiB (SIPGPU_ESIZE beyond).
+ * Two device streams: large batches (>= 1e9 flop)
  * run in order on the first, and a small batch admitted while the first is
  * busy runs on the second, beside it on the device; a batch that reads a
  * block an unfinished batch of the other stream writes (or writes one it
